@@ -6,6 +6,7 @@ operator call fails loudly.  There is no PyTorch or CPU fallback.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 import threading
 
@@ -13,6 +14,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libsba_mi355x.so")
+NATIVE_PATH = os.path.join(_HERE, "csrc", "_sba_torch.so")
 
 SBA_DTYPE_F32, SBA_DTYPE_BF16, SBA_DTYPE_F16 = 0, 1, 2
 SBA_ABI_VERSION = 6
@@ -86,6 +88,29 @@ def load() -> C.CDLL:
             raise RuntimeError("libsba_mi355x.so ABI version mismatch; rebuild it")
         _lib = lib
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The native host layer (csrc/sba_torch.cpp), an extension module over the same library: loaded once, raises if it
+    has not been built."""
+    global _native
+    if _native is None:
+        with _lock:
+            if _native is None:
+                if not os.path.exists(NATIVE_PATH):
+                    raise RuntimeError(
+                        f"{NATIVE_PATH} is missing: build it with `make -C {os.path.dirname(NATIVE_PATH)}` "
+                        "(or __graft_entry__.build()). There is no fallback path.")
+                spec = importlib.util.spec_from_file_location("_sba_torch", NATIVE_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                _native = module
+                set_workspace_budget(_workspace_budget)
+                check_gave_up(_check_gave_up)
+    return _native
 
 
 EXPORTED_SYMBOLS = ("sba_abi_version", "sba_error_string", "sba_workspace_bytes", "sba_bwd_scratch_bytes",
@@ -187,6 +212,8 @@ def set_workspace_budget(nbytes) -> None:
     that is set, else 256 MiB); 0 never keeps anything; float('inf') always keeps the tables."""
     global _workspace_budget
     _workspace_budget = nbytes
+    if _native is not None:
+        _native.set_workspace_budget(-1.0 if nbytes is None else float(nbytes))
 
 
 def workspace_budget():
@@ -213,6 +240,8 @@ _check_gave_up = None
 def check_gave_up(on) -> None:
     global _check_gave_up
     _check_gave_up = on
+    if _native is not None:
+        _native.set_check_gave_up(-1 if on is None else int(bool(on)))
 
 
 def gave_up_checked() -> bool:

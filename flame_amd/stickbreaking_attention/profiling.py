@@ -60,6 +60,12 @@ def _on() -> bool:
     return _TIMER is not None and _TIMER.active
 
 
+def native() -> bool:
+    """Whether a call goes to the native host layer: not while torch.compile traces, and not in a step that is timed kernel
+    by kernel."""
+    return (_TIMER is None or not _TIMER.active) and not torch.compiler.is_compiling()
+
+
 def mark(name: str):
     if _on():
         _TIMER.mark(name)

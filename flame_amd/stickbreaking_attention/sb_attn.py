@@ -146,6 +146,8 @@ def _bwd(do, dr, q, k, v, ws, logit_scale, attend_current=False):
 
 
 class StickBreakingAttention(torch.autograd.Function):
+    """The operator as torch.compile traces it and as the per-kernel timer runs it; every other call takes the native
+    host layer (csrc/sba_torch.cpp), which does the same without the interpreter."""
 
     @staticmethod
     def forward(ctx, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, inv_temp: float,
@@ -184,12 +186,14 @@ class StickBreakingAttention(torch.autograd.Function):
 
 
 def sb_attn(q, k, v, inv_temp=None, zero_start=True, attend_current=False):
-    if inv_temp is None:
-        inv_temp = 1 / math.sqrt(q.size(-1))
     return sb_attn_(q, k, v, inv_temp, attend_current=attend_current)
 
 
 def sb_attn_(q, k, v, inv_temp, attend_current):
+    if profiling.native():
+        return _lib.native().attention(q, k, v, inv_temp, attend_current)
+    if inv_temp is None:
+        inv_temp = 1 / math.sqrt(q.size(-1))
     if q.numel() == 0:
         # nothing to launch (an empty batch or a zero-length sequence): empty results that stay in the graph
         return q * 0, q.sum(-1) * 0

@@ -196,6 +196,8 @@ def varlen_bwd(do, dr, q, k, v, cu_seqlens, max_seqlens, ws, logit_scale, attend
 
 
 class StickBreakingAttention(torch.autograd.Function):
+    """The operator as torch.compile traces it and as the per-kernel timer runs it; every other call takes the native
+    host layer (csrc/sba_torch.cpp), which keeps schedules of its own."""
 
     @staticmethod
     def forward(ctx, q, k, v, cu_seqlens, max_seqlens, inv_temp, attend_current):
@@ -260,12 +262,14 @@ def sb_attn_varlen(q, k, v, cu_seqlens, max_seqlens, inv_temp=None, zero_start=T
     without the 0 too: its zero-prefixed copy is made once per tensor): pass the same tensor to every layer."""
     if not zero_start:
         cu_seqlens = _with_leading_zero(cu_seqlens)
-    if inv_temp is None:
-        inv_temp = 1 / math.sqrt(q.size(-1))
     return _apply(q, k, v, cu_seqlens, max_seqlens, inv_temp, attend_current)
 
 
 def _apply(q, k, v, cu_seqlens, max_seqlens, inv_temp, attend_current):
+    if profiling.native():
+        return _lib.native().attention_varlen(q, k, v, cu_seqlens, int(max_seqlens), inv_temp, attend_current)
+    if inv_temp is None:
+        inv_temp = 1 / math.sqrt(q.size(-1))
     if q.numel() == 0:
         # no tokens (or no heads): nothing to launch; empty results that stay in the graph
         return q * 0, q.sum(-1) * 0
