@@ -1,0 +1,66 @@
+// Kernels around the attention operator in the language model (sba_model.hip): normalisation with the residual, SwiGLU, the
+// weights' casts, cross-entropy, clipping with AdamW.  Rows are dense; `f16` selects float16 instead of bf16 for the 16-bit
+// tensors; everything else is fp32.  Launches are asynchronous on `stream`.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace sba_model {
+
+constexpr int kMaxNormWidth = 2048;      // columns of a row that a wave keeps in registers
+constexpr int kCastTensors = 8;
+constexpr int kOptChunk = 16384;         // weights that one workgroup of the optimizer kernels takes
+
+// y = rms_norm(x + h) * w as 16-bit; h (16-bit) may be null; sum receives x + h when h is given.
+struct NormFwd {
+    const float* x; const void* h; const float* w;
+    float* sum; void* y; float* rstd;
+    int rows, cols; float eps;
+};
+int norm_fwd(const NormFwd& a, bool f16, hipStream_t stream);
+
+// dx = dres + the gradient through the norm; dx16 its 16-bit copy (may be null), dw_part [norm_bwd_parts(rows)][cols].
+struct NormBwd {
+    const void* dy; const float* x; const float* w; const float* rstd; const float* dres;
+    float* dx; void* dx16; float* dw_part;
+    int rows, cols;
+};
+int norm_bwd_parts(int rows);
+int norm_bwd(const NormBwd& a, bool f16, hipStream_t stream);
+int sum_parts(const float* part, float* out, int parts, int cols, hipStream_t stream);
+
+int add_residual(const float* x, const void* h, float* out, int64_t n, bool f16, hipStream_t stream);
+
+// y = [rows][2 * width] = gate | up;  out = silu(gate) * up
+int swiglu_fwd(const void* y, void* out, int64_t rows, int width, bool f16, hipStream_t stream);
+int swiglu_bwd(const void* y, const void* d_out, void* dy, int64_t rows, int width, bool f16, hipStream_t stream);
+
+// up to kCastTensors fp32 tensors, one after the other, as 16-bit
+struct CastList {
+    const float* src[kCastTensors];
+    int64_t end[kCastTensors];           // running total of elements; every length is a multiple of 8
+    int n;
+};
+int cast_list(const CastList& a, void* out, bool f16, hipStream_t stream);
+int cast_one(const float* src, void* out, int64_t n, bool f16, hipStream_t stream);
+
+// Next-token cross-entropy over rows of `classes` 16-bit logits: row r of a sequence of `len` is scored against
+// labels[r + 1], the last row of a sequence and rows whose label is `ignore` are not.  lse, row_loss [rows]; mean, count [1].
+int loss_fwd(const void* logits, const int64_t* labels, float* lse, float* row_loss, float* mean, float* count, int rows, int len,
+             int classes, int64_t ignore, bool f16, hipStream_t stream);
+int loss_bwd(const void* logits, const int64_t* labels, const float* lse, const float* count, const float* d_loss,
+             void* d_logits, int rows, int len, int classes, int64_t ignore, bool f16, hipStream_t stream);
+
+// One weight tensor of a clip + AdamW step.
+struct OptTensor {
+    float* p; float* g; float* m; float* v; float* step;
+    int64_t n; int64_t first_chunk;      // chunks of the tensors before this one
+    double lr, beta1, beta2;
+    float decay, one_minus_beta1, beta2_f, one_minus_beta2, eps;         // rounded once from the caller's doubles
+    float step_size, denom_scale;        // filled on the device: lr / (1 - beta1^step), 1 / sqrt(1 - beta2^step)
+};
+// norm [1], partial [chunks + 1] (the last one: the clip coefficient).  Three launches: partial sums, norms and step counts, update.
+int clip_and_adamw(OptTensor* tensors, int n_tensors, int64_t chunks, float max_norm, float* partial, float* norm,
+                   hipStream_t stream);
+
+}  // namespace sba_model

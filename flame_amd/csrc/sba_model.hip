@@ -1,0 +1,520 @@
+// Kernels around the attention operator in the language model.  All of them are bound by memory: what pays is that a tensor
+// is read and written once where a chain of framework kernels passes over it several times, and that the fp32 residual stream
+// and its 16-bit copies leave in the same pass.
+#include "sba_model.h"
+
+namespace sba_model {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <typename E> struct Vec;
+template <> struct Vec<__bf16> {
+    typedef __bf16 x8 __attribute__((ext_vector_type(8)));
+    typedef __bf16 x4 __attribute__((ext_vector_type(4)));
+};
+template <> struct Vec<_Float16> {
+    typedef _Float16 x8 __attribute__((ext_vector_type(8)));
+    typedef _Float16 x4 __attribute__((ext_vector_type(4)));
+};
+
+constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / 64;
+
+__device__ inline float wave_sum(float v) {
+#pragma unroll
+    for (int d = 32; d; d >>= 1) v += __shfl_xor(v, d, 64);
+    return v;
+}
+__device__ inline float wave_max(float v) {
+#pragma unroll
+    for (int d = 32; d; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
+    return v;
+}
+
+int launched() { return hipGetLastError() == hipSuccess ? 0 : -6; }
+
+// ------------------------------------------------------------------------------------------------- RMS norm
+// One wave per row, the row in registers (K groups of 256 columns, four columns a lane and group: 16-byte accesses, 1 KB per
+// wave and instruction).
+template <typename E, int K, bool kAdd>
+__global__ __launch_bounds__(kThreads) void norm_fwd_kernel(NormFwd a) {
+    const int lane = threadIdx.x & 63, row = blockIdx.x * kWaves + (threadIdx.x >> 6);
+    if (row >= a.rows) return;
+    typedef typename Vec<E>::x4 e4;
+    const int64_t base = (int64_t)row * a.cols;
+    f32x4 x[K];
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int c = (k * 64 + lane) * 4;
+        x[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (c < a.cols) {
+            x[k] = *(const f32x4*)(a.x + base + c);
+            if (kAdd) {
+                const e4 h = *(const e4*)((const E*)a.h + base + c);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[k][i] += (float)h[i];
+                *(f32x4*)(a.sum + base + c) = x[k];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ss += x[k][i] * x[k][i];
+    }
+    ss = wave_sum(ss);
+    const float rstd = rsqrtf(ss / (float)a.cols + a.eps);
+    if (lane == 0) a.rstd[row] = rstd;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int c = (k * 64 + lane) * 4;
+        if (c < a.cols) {
+            const f32x4 w = *(const f32x4*)(a.w + c);
+            e4 y;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = (E)(x[k][i] * rstd * w[i]);
+            *(e4*)((E*)a.y + base + c) = y;
+        }
+    }
+}
+
+// dx_i = dres_i + rstd * (dy_i w_i - x_i rstd^2 mean_j(dy_j w_j x_j)).  A wave walks rows and keeps its share of
+// dw = sum over rows of dy x rstd in registers; the four waves of a workgroup add theirs in LDS and write one partial row.
+template <typename E, int K>
+__global__ __launch_bounds__(kThreads) void norm_bwd_kernel(NormBwd a) {
+    typedef typename Vec<E>::x4 e4;
+    __shared__ float part[kWaves][K * 256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    f32x4 dw[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) dw[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int row = blockIdx.x * kWaves + wave; row < a.rows; row += gridDim.x * kWaves) {
+        const int64_t base = (int64_t)row * a.cols;
+        const float rstd = a.rstd[row];
+        f32x4 x[K], g[K], r[K];
+        float dot = 0.f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int c = (k * 64 + lane) * 4;
+            x[k] = g[k] = r[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (c < a.cols) {
+                x[k] = *(const f32x4*)(a.x + base + c);
+                const e4 dy = *(const e4*)((const E*)a.dy + base + c);
+                if (a.dres) r[k] = *(const f32x4*)(a.dres + base + c);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) g[k][i] = (float)dy[i];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int c = (k * 64 + lane) * 4;
+            const f32x4 w = c < a.cols ? *(const f32x4*)(a.w + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                dw[k][i] += g[k][i] * x[k][i] * rstd;
+                g[k][i] *= w[i];
+                dot += g[k][i] * x[k][i];
+            }
+        }
+        const float c1 = wave_sum(dot) / (float)a.cols * rstd * rstd;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int c = (k * 64 + lane) * 4;
+            if (c >= a.cols) continue;
+            e4 d16;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                r[k][i] += rstd * (g[k][i] - x[k][i] * c1);
+                d16[i] = (E)r[k][i];
+            }
+            *(f32x4*)(a.dx + base + c) = r[k];
+            if (a.dx16) *(e4*)((E*)a.dx16 + base + c) = d16;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) *(f32x4*)&part[wave][(k * 64 + lane) * 4] = dw[k];
+    __syncthreads();
+    for (int c = threadIdx.x; c < a.cols; c += kThreads)
+        a.dw_part[(int64_t)blockIdx.x * a.cols + c] = part[0][c] + part[1][c] + part[2][c] + part[3][c];
+}
+
+// out[c] = sum over the parts: a workgroup takes 16 columns, 64 threads share a column's parts, eight loads of each in flight
+__global__ __launch_bounds__(1024) void sum_parts_kernel(const float* part, float* out, int parts, int cols) {
+    __shared__ float acc[64][17];
+    const int lc = threadIdx.x & 15, c = blockIdx.x * 16 + lc, g = threadIdx.x >> 4;
+    float s = 0.f;
+    if (c < cols)
+#pragma unroll 8
+        for (int i = g; i < parts; i += 64) s += part[(int64_t)i * cols + c];
+    acc[g][lc] = s;
+    __syncthreads();
+    if (g == 0 && c < cols) {
+#pragma unroll
+        for (int i = 1; i < 64; ++i) s += acc[i][lc];
+        out[c] = s;
+    }
+}
+
+template <typename E>
+__global__ __launch_bounds__(kThreads) void add_residual_kernel(const float* x, const E* h, float* out, int64_t n4) {
+    typedef typename Vec<E>::x4 e4;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n4; i += (int64_t)gridDim.x * kThreads) {
+        f32x4 v = *(const f32x4*)(x + i * 4);
+        const e4 a = *(const e4*)(h + i * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += (float)a[j];
+        *(f32x4*)(out + i * 4) = v;
+    }
+}
+
+// ------------------------------------------------------------------------------------------------- SwiGLU
+// silu(gate) and d_out * up are rounded to 16 bits where the module path holds them as tensors: both paths give the same bits.
+template <typename E>
+__global__ __launch_bounds__(kThreads) void swiglu_fwd_kernel(const E* y, E* out, int64_t n8, int w8) {
+    typedef typename Vec<E>::x8 e8;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n8; i += (int64_t)gridDim.x * kThreads) {
+        const int64_t row = i / w8;
+        const int c = (int)(i - row * w8);
+        const E* r = y + (row * 2 * w8 + c) * 8;
+        const e8 g = *(const e8*)r, u = *(const e8*)(r + (int64_t)w8 * 8);
+        e8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float gf = (float)g[j];
+            o[j] = (E)((float)(E)(gf / (1.f + __expf(-gf))) * (float)u[j]);
+        }
+        *(e8*)(out + i * 8) = o;
+    }
+}
+
+template <typename E>
+__global__ __launch_bounds__(kThreads) void swiglu_bwd_kernel(const E* y, const E* d_out, E* dy, int64_t n8, int w8) {
+    typedef typename Vec<E>::x8 e8;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n8; i += (int64_t)gridDim.x * kThreads) {
+        const int64_t row = i / w8;
+        const int c = (int)(i - row * w8);
+        const int64_t at = (row * 2 * w8 + c) * 8, up = (int64_t)w8 * 8;
+        const e8 g = *(const e8*)(y + at), u = *(const e8*)(y + at + up), d = *(const e8*)(d_out + i * 8);
+        e8 dg, du;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float gf = (float)g[j], df = (float)d[j];
+            const float sg = 1.f / (1.f + __expf(-gf));
+            du[j] = (E)(df * (float)(E)(gf * sg));
+            dg[j] = (E)((float)(E)(df * (float)u[j]) * sg * (1.f + gf * (1.f - sg)));
+        }
+        *(e8*)(dy + at) = dg;
+        *(e8*)(dy + at + up) = du;
+    }
+}
+
+// ------------------------------------------------------------------------------------------------- casts
+template <typename E>
+__global__ __launch_bounds__(kThreads) void cast_kernel(CastList a, E* out, int64_t n8) {
+    typedef typename Vec<E>::x8 e8;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n8; i += (int64_t)gridDim.x * kThreads) {
+        const int64_t e = i * 8;
+        int t = 0;
+        while (e >= a.end[t]) ++t;
+        const float* s = a.src[t] + (t ? e - a.end[t - 1] : e);
+        const f32x4 lo = *(const f32x4*)s, hi = *(const f32x4*)(s + 4);
+        e8 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { o[j] = (E)lo[j]; o[4 + j] = (E)hi[j]; }
+        *(e8*)(out + e) = o;
+    }
+}
+
+// ------------------------------------------------------------------------------------------------- cross-entropy
+__device__ inline int64_t target_of(const int64_t* labels, int row, int len, int64_t ignore) {
+    return (row + 1) % len == 0 ? ignore : labels[row + 1];
+}
+
+// One workgroup per row, one pass with a running maximum: the logits are read once, as 16-bit.
+template <typename E>
+__global__ __launch_bounds__(kThreads) void loss_fwd_kernel(const E* logits, const int64_t* labels, float* lse, float* row_loss,
+                                                            int len, int classes, int64_t ignore) {
+    typedef typename Vec<E>::x8 e8;
+    __shared__ float sm[kWaves], ss[kWaves];
+    const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const E* r = logits + (int64_t)row * classes;
+    float m = -INFINITY, s = 0.f;
+    for (int c = threadIdx.x * 8; c < classes; c += kThreads * 8) {
+        const e8 v = *(const e8*)(r + c);
+        float f[8], big = m;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { f[j] = (float)v[j]; big = fmaxf(big, f[j]); }
+        const float base = big == -INFINITY ? 0.f : big;         // a row of -inf so far: nothing to rescale
+        s *= __expf(m - base);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += __expf(f[j] - base);
+        m = big;
+    }
+    const float wm = wave_max(m);
+    const float ws = wave_sum(s * __expf(m - (wm == -INFINITY ? 0.f : wm)));
+    if (lane == 0) { sm[wave] = wm; ss[wave] = ws; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float M = sm[0];
+        for (int i = 1; i < kWaves; ++i) M = fmaxf(M, sm[i]);
+        float S = 0.f;
+        for (int i = 0; i < kWaves; ++i) S += ss[i] * __expf(sm[i] - (M == -INFINITY ? 0.f : M));
+        const float l = M + __logf(S);
+        lse[row] = l;
+        const int64_t t = target_of(labels, row, len, ignore);
+        // (a label outside the classes: no number stands for its loss)
+        row_loss[row] = t == ignore ? 0.f : (t < 0 || t >= classes) ? NAN : l - (float)r[t];
+    }
+}
+
+__global__ __launch_bounds__(1024) void loss_mean_kernel(const float* row_loss, const int64_t* labels, float* mean, float* count,
+                                                         int rows, int len, int64_t ignore) {
+    __shared__ float ss[16], sc[16];
+    float s = 0.f, c = 0.f;
+    for (int r = threadIdx.x; r < rows; r += 1024) {
+        s += row_loss[r];
+        c += target_of(labels, r, len, ignore) == ignore ? 0.f : 1.f;
+    }
+    s = wave_sum(s);
+    c = wave_sum(c);
+    if ((threadIdx.x & 63) == 0) { ss[threadIdx.x >> 6] = s; sc[threadIdx.x >> 6] = c; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < 16; ++i) { s += ss[i]; c += sc[i]; }
+        *mean = s / c;
+        *count = c;
+    }
+}
+
+template <typename E>
+__global__ __launch_bounds__(kThreads) void loss_bwd_kernel(const E* logits, const int64_t* labels, const float* lse,
+                                                            const float* count, const float* d_loss, E* d_logits, int len,
+                                                            int classes, int64_t ignore) {
+    typedef typename Vec<E>::x8 e8;
+    const int row = blockIdx.x;
+    const int64_t t = target_of(labels, row, len, ignore);
+    const float scale = t == ignore ? 0.f : *d_loss / *count, l = lse[row];
+    const E* r = logits + (int64_t)row * classes;
+    E* d = d_logits + (int64_t)row * classes;
+    for (int c = threadIdx.x * 8; c < classes; c += kThreads * 8) {
+        e8 o;
+        if (t == ignore) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) o[j] = (E)0.f;
+        } else {
+            const e8 v = *(const e8*)(r + c);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) o[j] = (E)((__expf((float)v[j] - l) - (c + j == t ? 1.f : 0.f)) * scale);
+        }
+        *(e8*)(d + c) = o;
+    }
+}
+
+// ------------------------------------------------------------------------------------------------- clip + AdamW
+__device__ inline int tensor_of(const OptTensor* t, int n, int64_t chunk) {
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (t[mid].first_chunk <= chunk) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(kThreads) void square_sum_kernel(const OptTensor* tensors, int n_tensors, float* partial) {
+    __shared__ float ss[kWaves];
+    const OptTensor& t = tensors[tensor_of(tensors, n_tensors, blockIdx.x)];
+    const int64_t from = (blockIdx.x - t.first_chunk) * kOptChunk, to = from + kOptChunk < t.n ? from + kOptChunk : t.n;
+    float s = 0.f;
+    for (int64_t i = from + threadIdx.x * 4; i < to; i += kThreads * 4) {
+        if (i + 4 <= to) {
+            const f32x4 g = *(const f32x4*)(t.g + i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s += g[j] * g[j];
+        } else {
+            for (int64_t j = i; j < to; ++j) s += t.g[j] * t.g[j];
+        }
+    }
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) ss[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[blockIdx.x] = ss[0] + ss[1] + ss[2] + ss[3];
+}
+
+__global__ __launch_bounds__(1024) void norm_and_steps_kernel(OptTensor* tensors, int n_tensors, int64_t chunks,
+                                                              float* partial, float max_norm, float* norm_out) {
+    __shared__ double ss[16];
+    double s = 0.0;
+    for (int64_t i = threadIdx.x; i < chunks; i += 1024) s += (double)partial[i];
+    for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d, 64);
+    if ((threadIdx.x & 63) == 0) ss[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < 16; ++i) s += ss[i];
+        const float norm = (float)sqrt(s);
+        *norm_out = norm;
+        const float c = max_norm / (norm + 1e-6f);
+        partial[chunks] = c > 1.f ? 1.f : c;                  // (a norm that is NaN stays NaN)
+    }
+    for (int i = threadIdx.x; i < n_tensors; i += 1024) {
+        OptTensor& t = tensors[i];
+        const float step = *t.step + 1.f;
+        *t.step = step;
+        t.step_size = (float)(t.lr / (1.0 - pow(t.beta1, (double)step)));
+        t.denom_scale = (float)(1.0 / sqrt(1.0 - pow(t.beta2, (double)step)));
+    }
+}
+
+__device__ inline void adamw(float& p, float& g, float& m, float& v, float coef, const OptTensor& t) {
+    g *= coef;
+    m += t.one_minus_beta1 * (g - m);
+    v = t.beta2_f * v + t.one_minus_beta2 * g * g;
+    p = p * t.decay - t.step_size * m / (sqrtf(v) * t.denom_scale + t.eps);
+}
+
+// One pass over gradient, weight and both moments: 28 bytes a weight, and 4 more when the gradient is clipped, which is
+// written back so that a caller finds the clipped one, as after a clipping pass of its own.
+__global__ __launch_bounds__(kThreads) void adamw_kernel(const OptTensor* tensors, int n_tensors, const float* clip) {
+    const OptTensor t = tensors[tensor_of(tensors, n_tensors, blockIdx.x)];
+    const int64_t from = (blockIdx.x - t.first_chunk) * kOptChunk, to = from + kOptChunk < t.n ? from + kOptChunk : t.n;
+    const float coef = *clip;
+    const bool clipped = coef != 1.f;
+    for (int64_t i = from + threadIdx.x * 4; i < to; i += kThreads * 4) {
+        if (i + 4 <= to) {
+            f32x4 g = *(const f32x4*)(t.g + i), p = *(const f32x4*)(t.p + i), m = *(const f32x4*)(t.m + i),
+                  v = *(const f32x4*)(t.v + i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float gj = g[j], pj = p[j], mj = m[j], vj = v[j];
+                adamw(pj, gj, mj, vj, coef, t);
+                g[j] = gj; p[j] = pj; m[j] = mj; v[j] = vj;
+            }
+            *(f32x4*)(t.p + i) = p;
+            *(f32x4*)(t.m + i) = m;
+            *(f32x4*)(t.v + i) = v;
+            if (clipped) *(f32x4*)(t.g + i) = g;
+        } else {
+            for (int64_t j = i; j < to; ++j) {
+                float g = t.g[j], p = t.p[j], m = t.m[j], v = t.v[j];
+                adamw(p, g, m, v, coef, t);
+                t.p[j] = p; t.m[j] = m; t.v[j] = v;
+                if (clipped) t.g[j] = g;
+            }
+        }
+    }
+}
+
+unsigned grid_for(int64_t work_items) {
+    const int64_t blocks = (work_items + kThreads - 1) / kThreads;
+    return (unsigned)(blocks < 1 ? 1 : blocks > 16384 ? 16384 : blocks);
+}
+
+template <typename E>
+int norm_fwd_t(const NormFwd& a, hipStream_t s) {
+    const dim3 grid((a.rows + kWaves - 1) / kWaves), block(kThreads);
+#define SBA_NORM(K)                                                                                          \
+    if (a.cols <= K * 256) {                                                                                 \
+        if (a.h) hipLaunchKernelGGL((norm_fwd_kernel<E, K, true>), grid, block, 0, s, a);                    \
+        else hipLaunchKernelGGL((norm_fwd_kernel<E, K, false>), grid, block, 0, s, a);                       \
+        return launched();                                                                                   \
+    }
+    SBA_NORM(1) SBA_NORM(2) SBA_NORM(4) SBA_NORM(8)
+#undef SBA_NORM
+    return -2;
+}
+
+template <typename E>
+int norm_bwd_t(const NormBwd& a, hipStream_t s) {
+    const dim3 grid(norm_bwd_parts(a.rows)), block(kThreads);
+#define SBA_NORM(K)                                                                                          \
+    if (a.cols <= K * 256) {                                                                                 \
+        hipLaunchKernelGGL((norm_bwd_kernel<E, K>), grid, block, 0, s, a);                                   \
+        return launched();                                                                                   \
+    }
+    SBA_NORM(1) SBA_NORM(2) SBA_NORM(4) SBA_NORM(8)
+#undef SBA_NORM
+    return -2;
+}
+
+}  // namespace
+
+int norm_fwd(const NormFwd& a, bool f16, hipStream_t s) { return f16 ? norm_fwd_t<_Float16>(a, s) : norm_fwd_t<__bf16>(a, s); }
+int norm_bwd(const NormBwd& a, bool f16, hipStream_t s) { return f16 ? norm_bwd_t<_Float16>(a, s) : norm_bwd_t<__bf16>(a, s); }
+
+// two workgroups a CU, fewer when there are not four rows for each of their waves
+int norm_bwd_parts(int rows) {
+    const int by_rows = (rows + kWaves * 4 - 1) / (kWaves * 4);
+    return by_rows < 1 ? 1 : by_rows > 512 ? 512 : by_rows;
+}
+
+int sum_parts(const float* part, float* out, int parts, int cols, hipStream_t s) {
+    hipLaunchKernelGGL(sum_parts_kernel, dim3((cols + 15) / 16), dim3(1024), 0, s, part, out, parts, cols);
+    return launched();
+}
+
+int add_residual(const float* x, const void* h, float* out, int64_t n, bool f16, hipStream_t s) {
+    const dim3 grid(grid_for(n / 4)), block(kThreads);
+    if (f16) hipLaunchKernelGGL(add_residual_kernel<_Float16>, grid, block, 0, s, x, (const _Float16*)h, out, n / 4);
+    else hipLaunchKernelGGL(add_residual_kernel<__bf16>, grid, block, 0, s, x, (const __bf16*)h, out, n / 4);
+    return launched();
+}
+
+int swiglu_fwd(const void* y, void* out, int64_t rows, int width, bool f16, hipStream_t s) {
+    const int64_t n8 = rows * (width / 8);
+    const dim3 grid(grid_for(n8)), block(kThreads);
+    if (f16) hipLaunchKernelGGL(swiglu_fwd_kernel<_Float16>, grid, block, 0, s, (const _Float16*)y, (_Float16*)out, n8, width / 8);
+    else hipLaunchKernelGGL(swiglu_fwd_kernel<__bf16>, grid, block, 0, s, (const __bf16*)y, (__bf16*)out, n8, width / 8);
+    return launched();
+}
+
+int swiglu_bwd(const void* y, const void* d_out, void* dy, int64_t rows, int width, bool f16, hipStream_t s) {
+    const int64_t n8 = rows * (width / 8);
+    const dim3 grid(grid_for(n8)), block(kThreads);
+    if (f16)
+        hipLaunchKernelGGL(swiglu_bwd_kernel<_Float16>, grid, block, 0, s, (const _Float16*)y, (const _Float16*)d_out, (_Float16*)dy, n8, width / 8);
+    else
+        hipLaunchKernelGGL(swiglu_bwd_kernel<__bf16>, grid, block, 0, s, (const __bf16*)y, (const __bf16*)d_out, (__bf16*)dy, n8, width / 8);
+    return launched();
+}
+
+int cast_list(const CastList& a, void* out, bool f16, hipStream_t s) {
+    const int64_t n8 = a.end[a.n - 1] / 8;
+    const dim3 grid(grid_for(n8)), block(kThreads);
+    if (f16) hipLaunchKernelGGL(cast_kernel<_Float16>, grid, block, 0, s, a, (_Float16*)out, n8);
+    else hipLaunchKernelGGL(cast_kernel<__bf16>, grid, block, 0, s, a, (__bf16*)out, n8);
+    return launched();
+}
+
+int cast_one(const float* src, void* out, int64_t n, bool f16, hipStream_t s) {
+    CastList a = {};
+    a.src[0] = src;
+    a.end[0] = n;
+    a.n = 1;
+    return cast_list(a, out, f16, s);
+}
+
+int loss_fwd(const void* logits, const int64_t* labels, float* lse, float* row_loss, float* mean, float* count, int rows, int len,
+             int classes, int64_t ignore, bool f16, hipStream_t s) {
+    if (f16)
+        hipLaunchKernelGGL(loss_fwd_kernel<_Float16>, dim3(rows), dim3(kThreads), 0, s, (const _Float16*)logits, labels, lse, row_loss, len, classes, ignore);
+    else
+        hipLaunchKernelGGL(loss_fwd_kernel<__bf16>, dim3(rows), dim3(kThreads), 0, s, (const __bf16*)logits, labels, lse, row_loss, len, classes, ignore);
+    hipLaunchKernelGGL(loss_mean_kernel, dim3(1), dim3(1024), 0, s, row_loss, labels, mean, count, rows, len, ignore);
+    return launched();
+}
+
+int loss_bwd(const void* logits, const int64_t* labels, const float* lse, const float* count, const float* d_loss,
+             void* d_logits, int rows, int len, int classes, int64_t ignore, bool f16, hipStream_t s) {
+    if (f16)
+        hipLaunchKernelGGL(loss_bwd_kernel<_Float16>, dim3(rows), dim3(kThreads), 0, s, (const _Float16*)logits, labels, lse, count, d_loss, (_Float16*)d_logits, len, classes, ignore);
+    else
+        hipLaunchKernelGGL(loss_bwd_kernel<__bf16>, dim3(rows), dim3(kThreads), 0, s, (const __bf16*)logits, labels, lse, count, d_loss, (__bf16*)d_logits, len, classes, ignore);
+    return launched();
+}
+
+int clip_and_adamw(OptTensor* tensors, int n_tensors, int64_t chunks, float max_norm, float* partial, float* norm,
+                   hipStream_t s) {
+    hipLaunchKernelGGL(square_sum_kernel, dim3((unsigned)chunks), dim3(kThreads), 0, s, tensors, n_tensors, partial);
+    hipLaunchKernelGGL(norm_and_steps_kernel, dim3(1), dim3(1024), 0, s, tensors, n_tensors, chunks, partial, max_norm, norm);
+    hipLaunchKernelGGL(adamw_kernel, dim3((unsigned)chunks), dim3(kThreads), 0, s, tensors, n_tensors, partial + chunks);
+    return launched();
+}
+
+}  // namespace sba_model

@@ -352,6 +352,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                                  std::optional<double> inv_temp, bool attend_current) {
         return run(q, k, v, cu_seqlens, max_seqlens, scale_or_default(inv_temp, q), attend_current);
     });
+    bind_model(m);
     m.def("set_workspace_budget", [](double bytes) { g_budget = bytes; });
     m.def("set_check_gave_up", [](int on) { g_check_gave_up = on; });
 }

@@ -40,6 +40,8 @@ Tensor attention_forward(const Problem& pr, const Tensor& o, const Tensor& rem, 
 void attention_backward(const Problem& pr, const Tensor& tables, const Tensor& d_o, const Tensor& d_rem, const Tensor& dq,
                         const Tensor& dk, const Tensor& dv);
 
+void bind_model(py::module& m);          // sba_torch_model.cpp
+
 hipStream_t stream_of(const Tensor& t);
 void check_status(int rc, const char* what);
 

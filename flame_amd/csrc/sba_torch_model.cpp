@@ -1,0 +1,400 @@
+// The language model's blocks as autograd nodes of their own: one node per transformer block instead of about forty framework
+// operators, so that a block costs the host a dozen launches in each direction, the elementwise work around the matrix products
+// runs in fused kernels (sba_model.hip), and the weights' gradients come out of their products in fp32.
+//
+// What a block computes is flame_amd/modeling_sba.py's SBABlock under autocast: fp32 weights and residual stream, 16-bit
+// operands of every product, fp32 normalisation.
+#include "sba_model.h"
+#include "sba_torch.h"
+
+#include <ATen/ops/empty.h>
+#include <ATen/ops/empty_like.h>
+#include <ATen/ops/mm.h>
+#include <c10/util/SmallVector.h>
+#include <torch/csrc/autograd/custom_function.h>
+
+#include <cstring>
+
+namespace sba_torch {
+namespace {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+using namespace sba_model;
+
+void ok(int rc) { check_status(rc, "model kernel"); }
+bool is_f16(at::ScalarType t) { return t == at::kHalf; }
+
+Tensor empty(at::IntArrayRef sizes, const Tensor& like, at::ScalarType t) { return at::empty(sizes, like.options().dtype(t)); }
+
+// fp32 weights as 16-bit ones, stacked along their rows in one buffer each; `groups` says how many weights share a buffer
+std::vector<Tensor> cast_weights(at::ArrayRef<Tensor> w, at::IntArrayRef groups, at::ScalarType t) {
+    CastList list = {};
+    int64_t total = 0;
+    for (const auto& x : w) {
+        list.src[list.n] = x.data_ptr<float>();
+        total += x.numel();
+        list.end[list.n++] = total;
+    }
+    Tensor all = empty({total}, w[0], t);
+    ok(cast_list(list, all.data_ptr(), is_f16(t), stream_of(all)));
+    std::vector<Tensor> out;
+    int64_t at = 0;
+    int i = 0;
+    for (int64_t g : groups) {
+        int64_t rows = 0;
+        const int64_t cols = w[i].size(1);
+        for (int64_t j = 0; j < g; ++j) rows += w[i++].size(0);
+        out.push_back(all.narrow(0, at, rows * cols).view({rows, cols}));
+        at += rows * cols;
+    }
+    return out;
+}
+
+// d_weight = d_out^T . in, in fp32
+std::vector<Tensor> weight_grads(std::initializer_list<std::pair<Tensor, Tensor>> pairs) {
+    std::vector<Tensor> r;
+    for (const auto& [d_out, in] : pairs) r.push_back(at::mm(d_out.t(), in, at::kFloat));
+    return r;
+}
+
+struct Norm { Tensor y, rstd, sum; };
+Norm rms_norm(const Tensor& x, const Tensor& h, const Tensor& w, double eps, at::ScalarType t) {
+    Norm r;
+    const int64_t rows = x.size(0), cols = x.size(1);
+    r.y = empty({rows, cols}, x, t);
+    r.rstd = empty({rows}, x, at::kFloat);
+    NormFwd a = {};
+    a.x = x.data_ptr<float>();
+    if (h.defined()) {
+        r.sum = at::empty_like(x);
+        a.h = h.data_ptr();
+        a.sum = r.sum.data_ptr<float>();
+    }
+    a.w = w.data_ptr<float>();
+    a.y = r.y.data_ptr();
+    a.rstd = r.rstd.data_ptr<float>();
+    a.rows = (int)rows;
+    a.cols = (int)cols;
+    a.eps = (float)eps;
+    ok(norm_fwd(a, is_f16(t), stream_of(x)));
+    return r;
+}
+
+struct NormGrad { Tensor dx, dx16, dw; };
+NormGrad rms_norm_grad(const Tensor& dy, const Tensor& x, const Tensor& w, const Tensor& rstd, const Tensor& dres, bool want16) {
+    NormGrad r;
+    const int64_t rows = x.size(0), cols = x.size(1);
+    const int parts = norm_bwd_parts((int)rows);
+    Tensor part = empty({parts, cols}, x, at::kFloat);
+    r.dx = at::empty_like(x);
+    r.dw = at::empty_like(w);
+    NormBwd a = {};
+    a.dy = dy.data_ptr();
+    a.x = x.data_ptr<float>();
+    a.w = w.data_ptr<float>();
+    a.rstd = rstd.data_ptr<float>();
+    a.dres = dres.defined() ? dres.data_ptr<float>() : nullptr;
+    a.dx = r.dx.data_ptr<float>();
+    if (want16) {
+        r.dx16 = empty({rows, cols}, x, dy.scalar_type());
+        a.dx16 = r.dx16.data_ptr();
+    }
+    a.dw_part = part.data_ptr<float>();
+    a.rows = (int)rows;
+    a.cols = (int)cols;
+    const auto s = stream_of(x);
+    ok(norm_bwd(a, is_f16(dy.scalar_type()), s));
+    ok(sum_parts(part.data_ptr<float>(), r.dw.data_ptr<float>(), parts, (int)cols, s));
+    return r;
+}
+
+Tensor cast_to(const Tensor& x, at::ScalarType t) {
+    Tensor out = empty(x.sizes(), x, t);
+    ok(cast_one(x.data_ptr<float>(), out.data_ptr(), x.numel(), is_f16(t), stream_of(x)));
+    return out;
+}
+
+// -------------------------------------------------------------------------------------------------------- one block
+
+struct BlockShape {
+    int64_t B, T, hidden, heads, width;
+    double eps1, eps2, scale;
+    at::ScalarType t;
+    c10::intrusive_ptr<Plan> plan;
+};
+
+// the three column slices of a [B*T, 3*hidden] product as the operator's q, k, v
+Problem problem_of(const BlockShape& s, const Tensor& qkv) {
+    const int64_t D = s.hidden / s.heads, row = 3 * s.hidden;
+    auto view = [&](int64_t i) {
+        return s.plan ? qkv.as_strided({s.heads, s.T, D}, {D, row, 1}, qkv.storage_offset() + i * s.hidden)
+                      : qkv.as_strided({s.B, s.heads, s.T, D}, {s.T * row, D, row, 1}, qkv.storage_offset() + i * s.hidden);
+    };
+    return Problem{view(0), view(1), view(2), s.plan, s.scale, false};
+}
+// a dense [B*T, hidden] tensor as the operator's o
+Tensor heads_of(const BlockShape& s, const Tensor& o) {
+    const int64_t D = s.hidden / s.heads;
+    return s.plan ? o.as_strided({s.heads, s.T, D}, {D, s.hidden, 1})
+                  : o.as_strided({s.B, s.heads, s.T, D}, {s.T * s.hidden, D, s.hidden, 1});
+}
+
+// the operands have their types already: nothing for autocast to look at
+struct NoAutocast {
+    c10::impl::ExcludeDispatchKeyGuard guard{c10::DispatchKey::AutocastCUDA};
+};
+
+struct BlockState {
+    Tensor x1, y1, rstd1, qkv, o, tables, y2, rstd2, gu, a;
+    std::vector<Tensor> w;              // 16-bit: q|k|v stacked, o, gate|up stacked, down
+};
+
+// weights: norm1, q, k, v, o, norm2, gate, up, down
+Tensor block_forward(const BlockShape& s, const Tensor& x, at::ArrayRef<Tensor> weights, bool train, BlockState& st) {
+    const Tensor cast[] = {weights[1], weights[2], weights[3], weights[4], weights[6], weights[7], weights[8]};
+    st.w = cast_weights(cast, {3, 1, 2, 1}, s.t);
+    const int64_t N = s.B * s.T;
+    auto n1 = rms_norm(x, Tensor(), weights[0], s.eps1, s.t);
+    st.y1 = n1.y;
+    st.rstd1 = n1.rstd;
+    st.qkv = at::mm(st.y1, st.w[0].t());
+    Problem pr = problem_of(s, st.qkv);
+    st.o = empty({N, s.hidden}, x, s.t);
+    Tensor rem = s.plan ? empty({s.heads, s.T}, x, s.t) : empty({s.B, s.heads, s.T}, x, s.t);
+    st.tables = attention_forward(pr, heads_of(s, st.o), rem, train);
+    Tensor h = at::mm(st.o, st.w[1].t());
+    auto n2 = rms_norm(x, h, weights[5], s.eps2, s.t);
+    st.x1 = n2.sum;
+    st.y2 = n2.y;
+    st.rstd2 = n2.rstd;
+    st.gu = at::mm(st.y2, st.w[2].t());
+    st.a = empty({N, s.width}, x, s.t);
+    ok(swiglu_fwd(st.gu.data_ptr(), st.a.data_ptr(), N, (int)s.width, is_f16(s.t), stream_of(x)));
+    Tensor m = at::mm(st.a, st.w[3].t());
+    Tensor out = at::empty_like(x);
+    ok(add_residual(st.x1.data_ptr<float>(), m.data_ptr(), out.data_ptr<float>(), x.numel(), is_f16(s.t), stream_of(x)));
+    return out;
+}
+
+struct Block : torch::autograd::Function<Block> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& n1, const Tensor& wq, const Tensor& wk,
+                          const Tensor& wv, const Tensor& wo, const Tensor& n2, const Tensor& wg, const Tensor& wu,
+                          const Tensor& wd, const std::optional<Tensor>& cu_seqlens, const BlockShape& s) {
+        const Tensor x = x_in.contiguous().view({s.B * s.T, s.hidden});
+        BlockState st;
+        const Tensor weights[] = {n1, wq, wk, wv, wo, n2, wg, wu, wd};
+        Tensor out = block_forward(s, x, weights, true, st);
+        ctx->save_for_backward({x, n1, n2, st.x1, st.y1, st.rstd1, st.qkv, st.o, st.tables, st.y2, st.rstd2, st.gu, st.a, st.w[0],
+                                st.w[1], st.w[2], st.w[3], cu_seqlens ? *cu_seqlens : Tensor()});
+        ctx->saved_data["scale"] = s.scale;
+        ctx->saved_data["sizes"] = std::vector<int64_t>{s.B, s.T, s.hidden, s.heads, s.width};
+        if (s.plan) ctx->saved_data["plan"] = c10::IValue::make_capsule(s.plan);
+        return out.view(x_in.sizes());
+    }
+
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &x = sv[0], &n1 = sv[1], &n2 = sv[2], &x1 = sv[3], &y1 = sv[4], &rstd1 = sv[5], &qkv = sv[6], &o = sv[7],
+                     &tables = sv[8], &y2 = sv[9], &rstd2 = sv[10], &gu = sv[11], &a = sv[12], &w_qkv = sv[13], &w_o = sv[14],
+                     &w_gu = sv[15], &w_d = sv[16];
+        const auto z = ctx->saved_data["sizes"].toIntVector();
+        BlockShape s{z[0], z[1], z[2], z[3], z[4], 0, 0, ctx->saved_data["scale"].toDouble(), qkv.scalar_type(), {}};
+        const auto plan = ctx->saved_data.find("plan");
+        if (plan != ctx->saved_data.end()) s.plan = c10::static_intrusive_pointer_cast<Plan>(plan->second.toCapsule());
+        c10::DeviceGuard guard(x.device());
+        const int64_t N = s.B * s.T;
+        const Tensor dx2 = grads[0].contiguous().view({N, s.hidden});
+
+        const Tensor dm = cast_to(dx2, s.t);
+        const Tensor da = at::mm(dm, w_d);
+        const Tensor dgu = at::empty_like(gu);
+        ok(swiglu_bwd(gu.data_ptr(), da.data_ptr(), dgu.data_ptr(), N, (int)s.width, is_f16(s.t), stream_of(x)));
+        const Tensor dy2 = at::mm(dgu, w_gu);
+        auto g2 = rms_norm_grad(dy2, x1, n2, rstd2, dx2, true);
+        const Tensor d_o = at::mm(g2.dx16, w_o);
+        const Tensor dqkv = at::empty_like(qkv);
+        {
+            Problem pr = problem_of(s, qkv);
+            const Problem g = problem_of(s, dqkv);
+            attention_backward(pr, tables, heads_of(s, d_o), Tensor(), g.q, g.k, g.v);
+        }
+        const Tensor dy1 = at::mm(dqkv, w_qkv);
+        const auto dw = weight_grads({{dqkv, y1}, {g2.dx16, o}, {dgu, y2}, {dm, a}});
+        const Tensor &dwqkv = dw[0], &dwo = dw[1], &dwgu = dw[2], &dwd = dw[3];
+        auto g1 = rms_norm_grad(dy1, x, n1, rstd1, g2.dx, false);
+
+        const int64_t C = s.hidden, F = s.width;
+        return {g1.dx.view(grads[0].sizes()), g1.dw, dwqkv.narrow(0, 0, C), dwqkv.narrow(0, C, C), dwqkv.narrow(0, 2 * C, C), dwo,
+                g2.dw, dwgu.narrow(0, 0, F), dwgu.narrow(0, F, F), dwd, Tensor(), Tensor()};
+    }
+};
+
+Tensor block(const Tensor& x, const std::vector<Tensor>& w, int64_t heads, double eps1, double eps2, py::object dtype,
+             const std::optional<Tensor>& cu_seqlens, int64_t max_seqlens) {
+    BlockShape s;
+    s.B = x.size(0);
+    s.T = x.size(1);
+    s.hidden = x.size(2);
+    s.heads = heads;
+    s.width = w[6].size(0);
+    s.eps1 = eps1;
+    s.eps2 = eps2;
+    s.scale = 1.0 / std::sqrt((double)(s.hidden / heads));
+    s.t = torch::python::detail::py_object_to_dtype(dtype);
+    c10::DeviceGuard guard(x.device());
+    NoAutocast no_autocast;
+    if (cu_seqlens) {
+        s.plan = plan_for(*cu_seqlens, heads, x.device());
+        check_plan(*s.plan, s.T, max_seqlens);
+    }
+    bool train = x.requires_grad();
+    for (const auto& t : w) train = train || t.requires_grad();
+    if (at::GradMode::is_enabled() && train)
+        return Block::apply(x, w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], cu_seqlens, s);
+    at::AutoDispatchBelowADInplaceOrView below;
+    BlockState st;
+    return block_forward(s, x.contiguous().view({s.B * s.T, s.hidden}), w, false, st).view(x.sizes());
+}
+
+// ---------------------------------------------------------------------------------- final norm, head and loss
+
+struct Head : torch::autograd::Function<Head> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& n, const Tensor& w, double eps, at::ScalarType t) {
+        const Tensor x = x_in.contiguous().view({-1, x_in.size(-1)});
+        auto r = rms_norm(x, Tensor(), n, eps, t);
+        const Tensor w16 = cast_to(w, t);
+        Tensor logits = at::mm(r.y, w16.t());
+        ctx->save_for_backward({x, n, r.y, r.rstd, w16});
+        auto sizes = x_in.sizes().vec();
+        sizes.back() = w.size(0);
+        return logits.view(sizes);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        c10::DeviceGuard guard(sv[0].device());
+        const Tensor d = grads[0].contiguous().view({-1, grads[0].size(-1)});
+        const Tensor dy = at::mm(d, sv[4]);
+        const Tensor dw = weight_grads({{d, sv[2]}})[0];
+        auto g = rms_norm_grad(dy, sv[0], sv[1], sv[3], Tensor(), false);
+        auto sizes = grads[0].sizes().vec();
+        sizes.back() = sv[0].size(1);
+        return {g.dx.view(sizes), g.dw, dw, Tensor(), Tensor()};
+    }
+};
+
+Tensor head(const Tensor& x, const Tensor& n, const Tensor& w, double eps, py::object dtype) {
+    const at::ScalarType t = torch::python::detail::py_object_to_dtype(dtype);
+    c10::DeviceGuard guard(x.device());
+    NoAutocast no_autocast;
+    if (at::GradMode::is_enabled() && (x.requires_grad() || n.requires_grad() || w.requires_grad()))
+        return Head::apply(x, n, w, eps, t);
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor rows = x.contiguous().view({-1, x.size(-1)});
+    auto r = rms_norm(rows, Tensor(), n, eps, t);
+    auto sizes = x.sizes().vec();
+    sizes.back() = w.size(0);
+    return at::mm(r.y, cast_to(w, t).t()).view(sizes);
+}
+
+struct LossRows { Tensor mean, count, lse; };
+LossRows loss_rows(const Tensor& logits, const Tensor& labels, int64_t ignore) {
+    const int64_t rows = labels.numel();
+    LossRows r{empty({}, logits, at::kFloat), empty({}, logits, at::kFloat), empty({2, rows}, logits, at::kFloat)};
+    float* lse = r.lse.data_ptr<float>();
+    ok(loss_fwd(logits.data_ptr(), labels.data_ptr<int64_t>(), lse, lse + rows, r.mean.data_ptr<float>(), r.count.data_ptr<float>(),
+                (int)rows, (int)labels.size(-1), (int)logits.size(-1), ignore, is_f16(logits.scalar_type()), stream_of(logits)));
+    return r;
+}
+
+struct Loss : torch::autograd::Function<Loss> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits_in, const Tensor& labels_in, int64_t ignore) {
+        const Tensor logits = logits_in.contiguous(), labels = labels_in.contiguous();
+        auto r = loss_rows(logits, labels, ignore);
+        ctx->save_for_backward({logits, labels, r.lse, r.count});
+        ctx->saved_data["ignore"] = ignore;
+        return r.mean;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &logits = sv[0], &labels = sv[1];
+        c10::DeviceGuard guard(logits.device());
+        const Tensor g = grads[0].contiguous();
+        Tensor d = at::empty_like(logits);
+        ok(loss_bwd(logits.data_ptr(), labels.data_ptr<int64_t>(), sv[2].data_ptr<float>(), sv[3].data_ptr<float>(),
+                    g.data_ptr<float>(), d.data_ptr(), (int)labels.numel(), (int)labels.size(-1), (int)logits.size(-1),
+                    ctx->saved_data["ignore"].toInt(), is_f16(logits.scalar_type()), stream_of(logits)));
+        return {d, Tensor(), Tensor()};
+    }
+};
+
+Tensor next_token_loss(const Tensor& logits, const Tensor& labels, int64_t ignore) {
+    c10::DeviceGuard guard(logits.device());
+    if (at::GradMode::is_enabled() && logits.requires_grad()) return Loss::apply(logits, labels, ignore);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return loss_rows(logits.contiguous(), labels.contiguous(), ignore).mean;
+}
+
+// ---------------------------------------------------------------------------------------------- clip and step
+
+// One pass of gradient clipping and AdamW over all weights; groups[group_of[i]]: {lr, weight_decay, beta1, beta2, eps} of
+// weight i.  Returns the gradients' norm, or nothing, with nothing done, if a tensor is not one the kernels take.
+std::optional<Tensor> clip_and_step(const std::vector<Tensor>& p, const std::vector<Tensor>& g, const std::vector<Tensor>& m,
+                                    const std::vector<Tensor>& v, const std::vector<Tensor>& step,
+                                    const std::vector<int64_t>& group_of, const std::vector<std::vector<double>>& groups,
+                                    double max_norm) {
+    const int64_t n = (int64_t)p.size();
+    if (n == 0) return std::nullopt;
+    const c10::Device device = p[0].device();
+    for (int64_t i = 0; i < n; ++i) {
+        for (const Tensor* t : {&p[i], &g[i], &m[i], &v[i]})
+            if (t->scalar_type() != at::kFloat || t->device() != device || !device.is_cuda() || t->layout() != at::kStrided ||
+                !t->is_contiguous() || t->numel() != p[i].numel())
+                return std::nullopt;
+        if (step[i].scalar_type() != at::kFloat || step[i].device() != device || step[i].numel() != 1) return std::nullopt;
+    }
+    c10::DeviceGuard guard(device);
+    Tensor host = at::empty({n * (int64_t)sizeof(OptTensor)}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+    auto* t = (OptTensor*)host.data_ptr();
+    int64_t chunks = 0;
+    for (int64_t i = 0; i < n; ++i) {
+        const auto& h = groups[group_of[i]];
+        OptTensor o = {};
+        o.p = p[i].data_ptr<float>();
+        o.g = g[i].data_ptr<float>();
+        o.m = m[i].data_ptr<float>();
+        o.v = v[i].data_ptr<float>();
+        o.step = step[i].data_ptr<float>();
+        o.n = p[i].numel();
+        o.first_chunk = chunks;
+        o.lr = h[0];
+        o.decay = (float)(1.0 - h[0] * h[1]);
+        o.beta1 = h[2];
+        o.beta2 = h[3];
+        o.one_minus_beta1 = (float)(1.0 - h[2]);
+        o.beta2_f = (float)h[3];
+        o.one_minus_beta2 = (float)(1.0 - h[3]);
+        o.eps = (float)h[4];
+        t[i] = o;
+        chunks += (o.n + kOptChunk - 1) / kOptChunk;
+    }
+    const Tensor table = host.to(device, /*non_blocking=*/true);
+    const Tensor work = empty({chunks + 1}, p[0], at::kFloat), norm = empty({}, p[0], at::kFloat);
+    ok(clip_and_adamw((OptTensor*)table.data_ptr(), (int)n, chunks, (float)max_norm, work.data_ptr<float>(), norm.data_ptr<float>(),
+                      stream_of(p[0])));
+    for (const auto* list : {&p, &g, &m, &v, &step})       // written in place
+        for (const auto& x : *list) x.unsafeGetTensorImpl()->bump_version();
+    return norm;
+}
+
+}  // namespace
+
+void bind_model(py::module& m) {
+    m.def("block", &block);
+    m.def("head", &head);
+    m.def("next_token_loss", &next_token_loss);
+    m.def("clip_and_step", &clip_and_step);
+    m.attr("max_norm_width") = kMaxNormWidth;
+}
+
+}  // namespace sba_torch

@@ -8,11 +8,10 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 from transformers.modeling_outputs import BaseModelOutputWithPast, CausalLMOutputWithPast
 from transformers.modeling_utils import PreTrainedModel
 
-from ..modeling_sba import SBABlock
+from ..modeling_sba import SBABlock, next_token_loss
 from .configuration_sba import SBAConfig
 
 
@@ -94,8 +93,7 @@ class SBAForCausalLM(SBAPreTrainedModel):
         loss = None
         if labels is not None:
             # modeling_sba.py:391: labels shifted left by one, the last position ignored
-            shifted = torch.cat((labels[..., 1:], torch.full_like(labels[:, :1], -100)), 1)
-            loss = F.cross_entropy(logits.view(shifted.numel(), -1).float(), shifted.view(-1), ignore_index=-100)
+            loss = next_token_loss(logits, labels)
         if return_dict is False:
             return (loss, logits) if loss is not None else (logits,)
         return CausalLMOutputWithPast(loss=loss, logits=logits, past_key_values=None)

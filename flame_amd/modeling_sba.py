@@ -19,6 +19,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import fused
 from .sba_layer import SBA, fused_weight
 
 
@@ -98,6 +99,8 @@ class SBAMLP(nn.Module):
 
 
 class SBABlock(nn.Module):
+    attention_class, mlp_class = SBA, SBAMLP
+
     def __init__(self, cfg: SBAConfig, layer_idx: int):
         super().__init__()
         self.attn_norm = nn.RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
@@ -113,9 +116,21 @@ class SBABlock(nn.Module):
         self.mlp = SBAMLP(cfg)
 
     def forward(self, x, **kwargs):
+        y = fused.block(self, x, kwargs)
+        if y is not None:
+            return y
         h, _, _ = self.attn(_autocast_once(self.attn_norm(x)), **kwargs)
         x = x + h
         return x + self.mlp(_autocast_once(self.mlp_norm(x)))
+
+
+def next_token_loss(logits: torch.Tensor, labels: torch.Tensor) -> torch.Tensor:
+    """Mean cross-entropy against the labels shifted left by one; the last position of a row is ignored."""
+    loss = fused.next_token_loss(logits, labels)
+    if loss is None:
+        shifted = torch.cat((labels[..., 1:], torch.full_like(labels[:, :1], -100)), 1)
+        loss = F.cross_entropy(logits.view(shifted.numel(), -1).float(), shifted.view(-1), ignore_index=-100)
+    return loss
 
 
 class SBAModel(nn.Module):
@@ -125,11 +140,15 @@ class SBAModel(nn.Module):
         self.layers = nn.ModuleList([SBABlock(cfg, i) for i in range(cfg.num_hidden_layers)])
         self.norm = nn.RMSNorm(cfg.hidden_size, eps=cfg.norm_eps)
 
-    def forward(self, input_ids, **kwargs):
+    def residual(self, input_ids, **kwargs):
+        """The residual stream in front of the final norm."""
         x = self.embeddings(input_ids)
         for layer in self.layers:
             x = layer(x, **kwargs)
-        return self.norm(x)
+        return x
+
+    def forward(self, input_ids, **kwargs):
+        return self.norm(self.residual(input_ids, **kwargs))
 
 
 class SBAForCausalLM(nn.Module):
@@ -152,13 +171,15 @@ class SBAForCausalLM(nn.Module):
             nn.init.normal_(m.weight, mean=0.0, std=self.config.initializer_range)
 
     def forward(self, input_ids, labels=None, **kwargs):
-        h = self.model(input_ids, **kwargs)
-        logits = self.lm_head(h)
-        loss = None
-        if labels is not None:
-            shifted = torch.cat((labels[..., 1:], torch.full_like(labels[:, :1], -100)), 1)
-            loss = F.cross_entropy(logits.view(shifted.numel(), -1).float(), shifted.view(-1), ignore_index=-100)
-        return loss, logits
+        logits = None
+        if fused.plain(self.model, SBAModel):
+            x = self.model.residual(input_ids, **kwargs)
+            logits = fused.head(x, self.model.norm, self.lm_head)
+            if logits is None:
+                logits = self.lm_head(self.model.norm(x))
+        else:
+            logits = self.lm_head(self.model(input_ids, **kwargs))
+        return None if labels is None else next_token_loss(logits, labels), logits
 
     def num_parameters(self, exclude_embeddings=False):
         n = sum(p.numel() for p in self.parameters())

@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import torch
 
+from . import fused
 from .modeling_sba import SBAConfig, SBAForCausalLM
 
 
@@ -22,6 +23,8 @@ def train_step(model: SBAForCausalLM, opt, input_ids, labels, cu_seqlens=None, m
     with torch.autocast("cuda", dtype=torch.bfloat16):
         loss, _ = model(input_ids, labels=labels, **kwargs)
     loss.backward()
-    gn = torch.nn.utils.clip_grad_norm_(model.parameters(), clip)
-    opt.step()
+    gn = fused.clip_and_step(model.parameters(), opt, clip)
+    if gn is None:
+        gn = torch.nn.utils.clip_grad_norm_(model.parameters(), clip)
+        opt.step()
     return loss.detach(), gn

@@ -1,0 +1,133 @@
+"""The native nodes of the language model (csrc/sba_torch_model.cpp) against the module-by-module path with the same weights in
+fp32, and clipping with AdamW against torch's own."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from helpers import cu_from_lengths, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+# hidden sizes at and off the 256 columns a wave keeps per register group, one to many rows, both head dims
+@pytest.mark.parametrize("hidden,heads,B,T,lens,dtype", [
+    (64, 1, 1, 1, None, torch.bfloat16),
+    (256, 4, 2, 33, None, torch.bfloat16),
+    (320, 5, 1, 700, [130, 7, 500, 63], torch.bfloat16),
+    (512, 4, 3, 257, None, torch.float16),
+    (1024, 16, 1, 1500, [1, 1499], torch.float16),
+    (2048, 32, 1, 129, None, torch.bfloat16),
+])
+def test_block_and_head_and_loss_match_the_modules(hidden, heads, B, T, lens, dtype, monkeypatch):
+    from flame_amd import fused
+    from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM
+    torch.manual_seed(hidden + T)
+    m = SBAForCausalLM(SBAConfig(hidden_size=hidden, num_heads=heads, num_hidden_layers=2, vocab_size=1000,
+                                 initializer_range=hidden ** -0.5)).cuda()
+    with torch.no_grad():
+        for p in m.parameters():
+            if p.dim() == 1:
+                p.add_(0.1 * torch.randn_like(p))
+    ids = torch.randint(0, 1000, (B, T), device="cuda")
+    labels = ids.clone()
+    labels[:, T // 2] = -100
+    kwargs = {} if lens is None else {"cu_seqlens": cu_from_lengths(lens).cuda(), "max_seqlen": max(lens)}
+
+    def run(grads=True):
+        m.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=dtype):
+            loss, logits = m(ids, labels=labels, **kwargs)
+        if T == 1 or not grads:
+            return loss, logits, {}
+        loss.backward()
+        return loss, logits, {n: p.grad for n, p in m.named_parameters()}
+
+    taken = []
+    block = fused.block
+    with monkeypatch.context() as mp:
+        mp.setattr(fused, "block", lambda *a: taken.append(block(*a)) or taken[-1])
+        loss, logits, grads = run()
+    assert len(taken) == 2 and all(y is not None for y in taken)
+    with torch.no_grad():
+        assert torch.equal(run(False)[1], logits)
+    with monkeypatch.context() as mp:
+        for name in ("block", "head", "next_token_loss"):
+            mp.setattr(fused, name, lambda *a, **k: None)
+        loss_ref, logits_ref, grads_ref = run()
+    tol = 2e-2 if dtype == torch.bfloat16 else 4e-3
+    assert rel_l2(logits.float(), logits_ref.float()) <= tol
+    assert T == 1 or abs(float(loss) - float(loss_ref)) <= tol
+    for n in grads:
+        assert grads[n].dtype == torch.float32 and grads[n].shape == grads_ref[n].shape
+        assert rel_l2(grads[n], grads_ref[n]) <= 2 * tol, n
+
+
+def test_hooks_and_other_modules_keep_the_module_path():
+    from flame_amd import fused
+    from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM
+    m = SBAForCausalLM(SBAConfig(hidden_size=128, num_heads=2, num_hidden_layers=1, vocab_size=64)).cuda()
+    x = torch.randn(1, 5, 128, device="cuda")
+    blk = m.model.layers[0]
+    assert fused.block(blk, x, {}) is None                       # no autocast
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert fused.block(blk, x, {}) is not None
+        seen = []
+        hook = blk.mlp.down_proj.register_forward_hook(lambda *a: seen.append(1))
+        assert fused.block(blk, x, {}) is None
+        blk(x)
+        assert seen == [1]
+        hook.remove()
+        assert fused.block(blk, x.to(torch.bfloat16), {}) is None
+        blk.attn.attn_fn = lambda q, k, v, t: (q, None)
+        assert fused.block(blk, x, {}) is None
+
+
+@pytest.mark.parametrize("rows,len_,classes", [(1, 1, 8), (6, 3, 2048), (7, 7, 2056), (40, 10, 32000)])
+def test_loss_edges_against_torch(rows, len_, classes):
+    from flame_amd import fused
+    torch.manual_seed(classes)
+    logits = (4 * torch.randn(rows // len_, len_, classes, device="cuda")).to(torch.bfloat16)
+    logits[0, 0, : classes // 2] = -float("inf")
+    labels = torch.randint(classes // 2, classes, (rows // len_, len_), device="cuda")
+    a, b = (logits.clone().requires_grad_(True) for _ in range(2))
+    got = fused.next_token_loss(a, labels)
+    shifted = torch.cat((labels[:, 1:], torch.full_like(labels[:, :1], -100)), 1)
+    ref = F.cross_entropy(b.float().view(rows, -1), shifted.view(-1), ignore_index=-100)
+    if len_ == 1:
+        assert torch.isnan(got) and torch.isnan(ref)             # no row counts
+        return
+    (3 * got).backward()
+    (3 * ref).backward()
+    assert abs(float(got) - float(ref)) <= 1e-5 * float(ref)
+    assert rel_l2(a.grad.float(), b.grad.float()) <= 5e-3
+
+
+@pytest.mark.parametrize("max_norm", [1e-2, 1e6])
+def test_clip_and_adamw_in_one_pass_matches_torch(max_norm):
+    # lengths around the four values of a load and the chunk a workgroup takes; two parameter groups, one weight without gradient
+    from flame_amd import fused
+    sizes = [1, 3, 4, 1023, 16383, 16384, 16385, 50000]
+    runs = []
+    for native in (True, False):
+        torch.manual_seed(0)
+        ps = [torch.nn.Parameter(torch.randn(n, device="cuda")) for n in sizes] + [torch.nn.Parameter(torch.ones(5, device="cuda"))]
+        opt = torch.optim.AdamW([{"params": ps[:4], "lr": 1e-2, "weight_decay": 0.3}, {"params": ps[4:]}], lr=1e-3,
+                                betas=(0.9, 0.95), eps=1e-8, fused=True)
+        sched = torch.optim.lr_scheduler.LambdaLR(opt, lambda s: 1.0 / (s + 1))
+        norms = []
+        for step in range(4):
+            for p in ps[:-1]:
+                p.grad = torch.randn_like(p)
+            norm = fused.clip_and_step(ps, opt, max_norm) if native else None
+            assert (norm is not None) == (native and step > 0)   # the first step sets the state up
+            if norm is None:
+                norm = torch.nn.utils.clip_grad_norm_(ps, max_norm)
+                opt.step()
+            sched.step()
+            norms.append(float(norm))
+        runs.append((norms, [p.detach() for p in ps], [p.grad for p in ps[:-1]],
+                     [opt.state[p][k] for p in ps[:-1] for k in ("exp_avg", "exp_avg_sq", "step")]))
+    (na, pa, ga, sa), (nb, pb, gb, sb) = runs
+    assert all(abs(x - y) <= 1e-5 * y for x, y in zip(na, nb))
+    for a, b in zip(pa + ga + sa, pb + gb + sb):
+        assert torch.allclose(a, b, rtol=2e-5, atol=1e-7)
