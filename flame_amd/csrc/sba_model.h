@@ -51,6 +51,24 @@ int loss_fwd(const void* logits, const int64_t* labels, float* lse, float* row_l
 int loss_bwd(const void* logits, const int64_t* labels, const float* lse, const float* count, const float* d_loss,
              void* d_logits, int rows, int len, int classes, int64_t ignore, bool f16, hipStream_t stream);
 
+// Weight gradients c[m][n] = sum over k rows of a[.][m] * b[.][n] (16-bit operands, fp32 results) of up to four products with
+// the same rows, in one launch (sba_gemm.hip).  m, n and the leading dimensions are multiples of 8; the results lie one after
+// the other from `out` on.
+struct WeightGrad {
+    const void* a; const void* b; int64_t lda, ldb; int m, n;
+    int64_t at;                          // first element of the result behind `out`
+};
+struct WeightGrads {
+    WeightGrad one[4];
+    int first_tile[4];
+    int n, tiles, k;
+    float* out; float* partial; int64_t total;
+};
+int weight_grad_splits(WeightGrads& g, int cus);         // fills first_tile, tiles, at, total; partial sums of how many splits
+int weight_grads(const WeightGrads& g, int splits, bool f16, hipStream_t stream);     // partial: [splits][total] if more than one
+int weight_grads_bf16(const WeightGrads& g, int splits, hipStream_t stream);
+int weight_grads_f16(const WeightGrads& g, int splits, hipStream_t stream);
+
 // One weight tensor of a clip + AdamW step.
 struct OptTensor {
     float* p; float* g; float* m; float* v; float* step;

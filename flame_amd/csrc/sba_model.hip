@@ -401,6 +401,14 @@ __global__ __launch_bounds__(kThreads) void adamw_kernel(const OptTensor* tensor
     }
 }
 
+__global__ __launch_bounds__(kThreads) void sum_splits_kernel(const float* part, float* out, int64_t n4, int splits) {
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n4; i += (int64_t)gridDim.x * kThreads) {
+        f32x4 s = *(const f32x4*)(part + i * 4);
+        for (int k = 1; k < splits; ++k) s += *(const f32x4*)(part + (k * n4 + i) * 4);
+        *(f32x4*)(out + i * 4) = s;
+    }
+}
+
 unsigned grid_for(int64_t work_items) {
     const int64_t blocks = (work_items + kThreads - 1) / kThreads;
     return (unsigned)(blocks < 1 ? 1 : blocks > 16384 ? 16384 : blocks);
@@ -471,6 +479,35 @@ int swiglu_bwd(const void* y, const void* d_out, void* dy, int64_t rows, int wid
         hipLaunchKernelGGL(swiglu_bwd_kernel<_Float16>, grid, block, 0, s, (const _Float16*)y, (const _Float16*)d_out, (_Float16*)dy, n8, width / 8);
     else
         hipLaunchKernelGGL(swiglu_bwd_kernel<__bf16>, grid, block, 0, s, (const __bf16*)y, (const __bf16*)d_out, (__bf16*)dy, n8, width / 8);
+    return launched();
+}
+
+// How many workgroups share a tile's contraction.  A launch takes ceil(tiles * splits / CUs) rounds of 1/splits of the rows each
+// (about 0.9 us per 32 rows with the chip full); partial sums are written, read and summed at about 4 TB/s.
+int weight_grad_splits(WeightGrads& g, int cus) {
+    g.tiles = 0;
+    g.total = 0;
+    for (int i = 0; i < g.n; ++i) {
+        g.first_tile[i] = g.tiles;
+        g.one[i].at = g.total;
+        g.tiles += ((g.one[i].m + 255) / 256) * ((g.one[i].n + 255) / 256);
+        g.total += (int64_t)g.one[i].m * g.one[i].n;
+    }
+    const double stages = (g.k + 31) / 32;
+    int best = 1;
+    double best_us = 1e30;
+    for (int s = 1; s <= 16 && s * 4 <= stages + 3; ++s) {
+        const double rounds = (double)((g.tiles * (int64_t)s + cus - 1) / cus);
+        const double us = rounds * (0.9 * stages / s + 4.0) + (s > 1 ? (2 * s + 1) * 4.0 * g.total / 4e6 + 3.0 : 0.0);
+        if (us < best_us) { best_us = us; best = s; }
+    }
+    return best;
+}
+
+int weight_grads(const WeightGrads& g, int splits, bool f16, hipStream_t s) {
+    const int rc = f16 ? weight_grads_f16(g, splits, s) : weight_grads_bf16(g, splits, s);
+    if (rc || splits == 1) return rc;
+    hipLaunchKernelGGL(sum_splits_kernel, dim3(grid_for(g.total / 4)), dim3(kThreads), 0, s, g.partial, g.out, g.total / 4, splits);
     return launched();
 }
 

@@ -51,10 +51,37 @@ std::vector<Tensor> cast_weights(at::ArrayRef<Tensor> w, at::IntArrayRef groups,
     return out;
 }
 
-// d_weight = d_out^T . in, in fp32
+// d_weight = d_out^T . in, in fp32, of several products over the same rows at once
 std::vector<Tensor> weight_grads(std::initializer_list<std::pair<Tensor, Tensor>> pairs) {
+    WeightGrads g = {};
+    for (const auto& [d_out, in] : pairs) {
+        auto& one = g.one[g.n++];
+        one.a = d_out.data_ptr();
+        one.b = in.data_ptr();
+        one.lda = d_out.stride(0);
+        one.ldb = in.stride(0);
+        one.m = (int)d_out.size(1);
+        one.n = (int)in.size(1);
+        g.k = (int)in.size(0);
+    }
+    const Tensor& like = pairs.begin()->first;
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 256;
+        return n > 0 ? n : 256;
+    }();
+    const int splits = weight_grad_splits(g, cus);
+    const Tensor out = empty({g.total}, like, at::kFloat);
+    Tensor partial;
+    g.out = out.data_ptr<float>();
+    if (splits > 1) {
+        partial = empty({splits, g.total}, like, at::kFloat);
+        g.partial = partial.data_ptr<float>();
+    }
+    ok(sba_model::weight_grads(g, splits, is_f16(like.scalar_type()), stream_of(like)));
     std::vector<Tensor> r;
-    for (const auto& [d_out, in] : pairs) r.push_back(at::mm(d_out.t(), in, at::kFloat));
+    for (int i = 0; i < g.n; ++i)
+        r.push_back(out.narrow(0, g.one[i].at, (int64_t)g.one[i].m * g.one[i].n).view({g.one[i].m, g.one[i].n}));
     return r;
 }
 
