@@ -1439,6 +1439,193 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
 }
 
 
+// ---------------------------------------------------------------- short sequences: the whole backward in one kernel
+// A sequence of at most 32 * W tokens fits one workgroup of W waves: its queries (Q and dO) stay in LDS and, as row fragments, in
+// registers, and its key blocks pass by from left to right as in the dQ pass.  Every score is evaluated ONCE: the step's
+// weights and logit gradients go to LDS as 16-bit [query][64 keys] rows, and after a barrier the waves reduce them over all
+// queries into the finished dK and dV rows of the key block (nobody else contributes to them).  q, k, v, dO are read once
+// where the two passes read them twice, no prefix table is written or read, and it is one launch.
+// What bounds it is memory (seven tensors' bytes): two workgroups of four waves (80 KB of LDS) or four of two waves (sequences
+// of at most 64 tokens) share a CU at head_dim 64, so that one's loads and stores run under the other's arithmetic; the next key
+// block's K and V are requested into the tile just used.
+template <int D, int W>
+__global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel(KParams p) {
+    constexpr int kRows = W * 32;
+    constexpr int kTile = 64 * D * 2;
+    constexpr int kQ = 0, kDO = kRows * D * 2, kK = 2 * kDO, kV = kK + kTile, kA = kV + kTile, kZ = kA + kRows * 128;
+    constexpr int kNB = D / 32;                // 32-column blocks of dK or dV that a wave reduces, for
+    constexpr int kKH = W == 2 ? 2 : 1;        // one 32-key half of the block or both
+    constexpr int kCols = 32 * kNB;
+    static_assert(W * kKH * 32 * kCols * 2 <= 2 * kRows * 128, "the waves stage their outputs in the weight tiles");
+    __shared__ __attribute__((aligned(1024))) char lds[kZ + kRows * 128];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 31, h = lane >> 5;
+    const int head = blockIdx.x % p.n_heads;
+    const Job job = decode_job(p, blockIdx.x / p.n_heads);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.gave_up) *p.gave_up = 0;
+    LaneOffsets<D> lo;
+    lo.init(lane);
+    lo.rebase(lds);
+    LaneOffsets<64> lz;
+    lz.init(lane);
+    lz.rebase(lds);
+    const int strict = p.attend_current ? 0 : 1;
+    const int q0w = 32 * wave, qi = q0w + n;
+    const bool row_ok = qi < job.len;
+    auto base_of = [&](const TensorArg& t) { return (int64_t)job.seq * t.sb + (int64_t)head * t.sh + (int64_t)job.tok0 * t.st; };
+    const int64_t qbase = base_of(p.q), kbase = base_of(p.k), vbase = base_of(p.v), dobase = base_of(p.d_o);
+
+    // a tile is four waves' copies: two each where there are only two
+    auto copy = [&](auto natural, const TensorArg& t, int64_t base, int row0, char* tile) {
+#pragma unroll
+        for (int w4 = 0; w4 < 4; w4 += W) {
+            TileDma<D, decltype(natural)::value> c;
+            c.init(lane, wave + w4, t, base);
+            c.issue(row0, job.len, tile);
+        }
+    };
+    constexpr std::true_type kNaturalRows{};
+    constexpr std::false_type kMfmaRows{};
+    copy(kMfmaRows, p.k, kbase, 0, lds + kK);
+    copy(kMfmaRows, p.v, vbase, 0, lds + kV);
+    for (int r = 0; r < job.len; r += 64) {
+        copy(kNaturalRows, p.q, qbase, r, lds + kQ + r * D * 2);
+        copy(kNaturalRows, p.d_o, dobase, r, lds + kDO + r * D * 2);
+    }
+    // the carry that enters this lane's 32 keys of a block; 0 for rows past the end, whose weights are then exactly 0
+    // (and for a block that holds nothing but the invisible last token: the forward has no entry for it)
+    constexpr int kBlocks = W / 2;
+    const int n_kb = (job.len + kKeyBlock - 1) / kKeyBlock;
+    const float* rcur = (h ? p.rtab : p.rmid) + tab_index(p, head, job, 0, 0) + q0w + n;
+    float F[kBlocks];
+#pragma unroll
+    for (int kb = 0; kb < kBlocks; ++kb) F[kb] = row_ok && 64 * kb + strict <= min(q0w + 31, job.len - 1) ? rcur[kb * kRowBlock] : 0.f;
+    float dr = 0.f;
+    if (row_ok && p.d_rem.ptr)
+        dr = Elem16::load(p.d_rem.ptr, (int64_t)job.seq * p.d_rem.sb + (int64_t)head * p.d_rem.sh + job.tok0 + qi);
+    wait_global_memory();
+    __syncthreads();
+    // row fragments from the tiles that the reduction needs anyway (as loads of their own they are 64 cache lines an instruction);
+    // rows past the end repeat the last one, and their weights are zeros
+    h16x8 qf[D / 16], dof[D / 16];
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+        qf[ks] = *(const h16x8*)(lds + kQ + tile_offset<D>(qi, 2 * ks + h));
+        dof[ks] = *(const h16x8*)(lds + kDO + tile_offset<D>(qi, 2 * ks + h));
+    }
+    prescale_frags(qf, p.scale2);
+
+    f32x16 dqacc[D / 32];
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db) dqacc[db] = f32x16{0};
+    float Gc = 0.f;
+    constexpr TileAt ktile{kK}, vtile{kV};
+    const int which = W == 2 ? wave : wave >> 1, kh0 = W == 2 ? 0 : wave & 1;
+
+#pragma unroll
+    for (int kb = 0; kb < kBlocks; ++kb) {
+        if (kb >= n_kb && kb > 0) break;
+        const int key0 = kb * kKeyBlock;
+        // a wave whose queries see nothing of the block has no rows in the reduction below, which starts at the block's first token
+        if (q0w < job.len && key0 + strict <= q0w + 31) {
+            float x[32], beta[32], dp[32];
+            score_tiles_ps<D>(x, ktile, lo, qf);
+            if (key0 + 63 + strict > q0w) mask_step(x, key0 + 32 * h, qi, strict);
+            const float Lend = carried_weights_and_dp<D>(x, beta, dp, F[kb], vtile, lo, dof);
+            if (kb == 0) {
+                float Llo, Lup;
+                half_values(Lend, Llo, Lup);
+                Gc = dr * Llo;                 // what leaves the left half of the leftmost block is rem (see the dQ pass)
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) *(h16x8*)(lds + kA + tile_offset<64>(qi, 4 * h + c)) = pack8(&x[8 * c]);
+            logit_grads<false>(x, beta, dp, Gc, lane);
+            h16x8 zf[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                zf[c] = pack8(&dp[8 * c]);
+                *(h16x8*)(lds + kZ + tile_offset<64>(qi, 4 * h + c)) = zf[c];
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                h16x8 kt[D / 32];
+#pragma unroll
+                for (int db = 0; db < D / 32; ++db) kt[db] = fetch_cols_o<D>(ktile, lo, db, c);
+#pragma unroll
+                for (int db = 0; db < D / 32; ++db) dqacc[db] = mfma(kt[db], zf[c], dqacc[db]);
+            }
+        }
+        __syncthreads();                       // weights complete, K and V free
+        if (kb + 1 < n_kb) {
+            copy(kMfmaRows, p.k, kbase, key0 + kKeyBlock, lds + kK);
+            copy(kMfmaRows, p.v, vbase, key0 + kKeyBlock, lds + kV);
+        }
+        // [32 keys x kCols] of dV (which = 0) or dK: keys 32 kh .. of the block, over the queries from the block on
+        f32x16 acc[kKH][kNB];
+#pragma unroll
+        for (int i = 0; i < kKH; ++i)
+#pragma unroll
+            for (int db = 0; db < kNB; ++db) acc[i][db] = f32x16{0};
+        {
+            const int offw = which ? kZ : kA, offb = which ? kQ : kDO;
+            auto fetch = [&](int x0, int x1, int add) {
+                union { s16x4 v[2]; h16x8 b; } u;
+                u.v[0] = lds_read_tr_at((uint32_t)(x0 + add), 0);
+                u.v[1] = lds_read_tr_at((uint32_t)(x1 + add), 0);
+                return u.b;
+            };
+            for (int r = key0; r < job.len; r += 16) {
+                h16x8 w[kKH];
+#pragma unroll
+                for (int i = 0; i < kKH; ++i)
+                    w[i] = fetch(kh0 + i ? lz.nat[0][1] : lz.nat[0][0], kh0 + i ? lz.nat[1][1] : lz.nat[1][0], offw + r * 128);
+#pragma unroll
+                for (int db = 0; db < kNB; ++db) {
+                    const h16x8 b = fetch(lo.nat[0][db], lo.nat[1][db], offb + r * D * 2);
+#pragma unroll
+                    for (int i = 0; i < kKH; ++i) acc[i][db] = mfma(w[i], b, acc[i][db]);
+                }
+            }
+        }
+        __syncthreads();                       // weight tiles free
+        {
+            char* stage = lds + kA + wave * (kKH * 32 * kCols * 2);
+            const TensorArg& out = which ? p.dk : p.dv;
+            const int64_t ob = base_of(out);
+#pragma unroll
+            for (int i = 0; i < kKH; ++i)
+#pragma unroll
+                for (int db = 0; db < kNB; ++db) stage_acc_tile<kCols>(stage, 32 * i, 32 * db, acc[i][db], which ? p.scale : 1.0f, lane);
+            for (int c = lane; c < kKH * 32 * kCols / 8; c += 64) {
+                const int row = c / (kCols / 8), cc = c % (kCols / 8), key = key0 + 32 * kh0 + row;
+                if (key < job.len)
+                    *(u32x4*)(out.ptr + 2 * (ob + (int64_t)key * out.st + cc * 8)) = *(const u32x4*)(stage + row * (kCols * 2) + cc * 16);
+            }
+        }
+        if (kb + 1 < n_kb) {
+            wait_global_memory();              // the next K and V have landed
+            __syncthreads();
+        }
+    }
+
+    if (row_ok) {
+        const int64_t ob = base_of(p.dq) + (int64_t)qi * p.dq.st;
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                f32x2 a = {dqacc[db][4 * g] * p.scale, dqacc[db][4 * g + 1] * p.scale};
+                f32x2 b = {dqacc[db][4 * g + 2] * p.scale, dqacc[db][4 * g + 3] * p.scale};
+                uint2 w;
+                w.x = __builtin_bit_cast(uint32_t, __builtin_convertvector(a, h16x2));
+                w.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(b, h16x2));
+                *(uint2*)(p.dq.ptr + 2 * (ob + 32 * db + 8 * g + 4 * h)) = w;
+            }
+    }
+}
+
 // ---------------------------------------------------------------- pass 2, two waves per 32 keys
 // What a wave of the own-keys kernel holds for its 32 keys at head_dim 128 - K and V fragments and the
 // [32 keys x 128] accumulators of dK and dV - is 190 registers: one wave per SIMD.  Here TWO waves share
@@ -1745,6 +1932,18 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     const bool stream = kp.head_dim == 64 && !plain && !own;
     if (stream && !kp.q_scaled.ptr) return SBA_ERR_WORKSPACE;
     if (!stream) kp.q_scaled.ptr = nullptr;
+    // Sequences of at most 128 tokens: one kernel for both passes (it all runs in phase 1).  A kernel asked for by name is one of
+    // the two-pass ones.
+    if (kp.seq_len <= kRowBlock && kp.head_dim <= 128 && !which && !getenv("SBA_DQ_KERNEL") && sba_two_step_env() < 0) {
+        if (!p1) return SBA_OK;
+        if (kp.head_dim == 128) {
+            hipLaunchKernelGGL((mfma_bwd_short_kernel<128, 4>), grid, dim3(256), 0, s, kp);
+        } else {
+            if (kp.seq_len <= 64) hipLaunchKernelGGL((mfma_bwd_short_kernel<64, 2>), grid, dim3(128), 0, s, kp);
+            else hipLaunchKernelGGL((mfma_bwd_short_kernel<64, 4>), grid, dim3(256), 0, s, kp);
+        }
+        return hipGetLastError() == hipSuccess ? SBA_OK : SBA_ERR_LAUNCH;
+    }
     if (kp.head_dim == 64) {
         // Small grids that last as long as their longest sweep (tail ratio from 3.7: B=1, H=16 up to T=4096) take the
         // variant that halves it; batches of short sequences on the same number of workgroups do not (B=8, T=512:
