@@ -97,6 +97,8 @@ int check_common(const SbaParams* p) {
     if (p->dtype != SBA_DTYPE_F32 && !is_16bit(p)) return SBA_ERR_DTYPE;
     if (p->n_seq <= 0 || p->n_heads <= 0 || p->seq_len <= 0 || p->total_tokens <= 0) return SBA_ERR_SHAPE;
     if (p->head_dim <= 0 || p->head_dim > sba::kMaxHeadDim) return SBA_ERR_SHAPE;
+    if (p->columns && (p->columns < 72 || p->columns > 96 || (p->columns & 7) || p->head_dim != 128 || !is_16bit(p) || !use_mfma_bwd(p)))
+        return SBA_ERR_SHAPE;
     if (!p->q.ptr || !p->k.ptr || !p->v.ptr) return SBA_ERR_NULL;
     if (p->cu_seqlens) {
         if (!p->schedule || p->n_schedule <= 0 || p->table_cols <= 0) return SBA_ERR_SCHEDULE;
@@ -120,7 +122,9 @@ KParams make_kparams(const SbaParams* p) {
     KParams kp;
     memset(&kp, 0, sizeof(kp));
     kp.n_seq = p->n_seq; kp.n_heads = p->n_heads; kp.seq_len = p->seq_len;
-    kp.total_tokens = p->total_tokens; kp.head_dim = p->head_dim;
+    kp.total_tokens = p->total_tokens;
+    kp.head_dim = p->columns ? 96 : p->head_dim;           // rows of 72 .. 96 columns: the kernels of that width
+    kp.cols = p->columns ? p->columns : p->head_dim;
     kp.attend_current = p->attend_current ? 1 : 0;
     kp.save = p->save_for_backward ? 1 : 0;
     kp.scale = p->scale; kp.scale2 = p->scale * sba::kLog2e;

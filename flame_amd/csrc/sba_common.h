@@ -25,6 +25,7 @@ struct VectorArg { char* ptr; int64_t sb, sh; };
 // Kernel-side copy of SbaParams (by value in the launch).
 struct KParams {
     int n_seq, n_heads, seq_len, total_tokens, head_dim, attend_current, save, n_jobs;
+    int cols;                      // columns of q, k, v, o, dO, dq, dk, dv that exist: head_dim, or less at head_dim 96
     int carry_only;                // forward kernels: write the carry table and nothing else (no P*V, no o / rem)
     float scale2;                  // scale * log2(e): logits in base-2 units
     float scale;                   // natural-unit scale (for dq/dk)

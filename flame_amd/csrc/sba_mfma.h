@@ -96,8 +96,15 @@ template <> __device__ inline int swz<256>(int row) {  // 32 chunks per row: a r
     return swz<128>(row);                               // of a chunk is its index modulo 16 as at head_dim 128
 }
 
+// head_dim 96 (which carries 72 .. 96 columns of the caller's, see KParams::cols) keeps head_dim 128's rows and swizzle in LDS -
+// a power of two for the chunk index - and leaves the last four chunks of a row unused: every loop over columns is a quarter
+// shorter, in matrix products and registers.
+template <> __device__ inline int swz<96>(int row) { return swz<128>(row); }
+template <int D> constexpr int kPitch = D == 96 ? 128 : D;      // elements from one LDS tile row to the next
+template <int D> constexpr bool kWide = D == 96 || D == 128;
+
 template <int D> __device__ inline int tile_offset(int row, int chunk) {   // bytes
-    return row * (D * 2) + ((chunk ^ swz<D>(row)) << 4);
+    return row * (kPitch<D> * 2) + ((chunk ^ swz<D>(row)) << 4);
 }
 
 // Lane-dependent byte offsets of the three fetch patterns, computed once per kernel.  The
@@ -182,10 +189,10 @@ __device__ inline s16x4 lds_read_tr_at(uint32_t base, int imm) {
 //                 tiles of the key-owner pass): lane (m, h) gets column 32*cb + m of rows
 //                 row0 + 8*h + j, j = 0..7.
 template <int D> __device__ inline h16x8 fetch_rows_o(const char* tile, const LaneOffsets<D>& o, int t, int ks) {
-    return *(const h16x8*)(tile + o.rows[ks] + t * 32 * D * 2);
+    return *(const h16x8*)(tile + o.rows[ks] + t * 32 * kPitch<D> * 2);
 }
 template <int D> __device__ inline h16x8 fetch_rows_o(TileAt tile, const LaneOffsets<D>& o, int t, int ks) {
-    return *(const __attribute__((address_space(3))) h16x8*)((__attribute__((address_space(3))) char*)(uintptr_t)(uint32_t)o.rows[ks] + (tile.off + t * 32 * D * 2));
+    return *(const __attribute__((address_space(3))) h16x8*)((__attribute__((address_space(3))) char*)(uintptr_t)(uint32_t)o.rows[ks] + (tile.off + t * 32 * kPitch<D> * 2));
 }
 // kPinBase: the sum `tile + lane offset` is pinned in a register (lds_lane_base) and the fetch's constant goes into
 // the offset field; one vector add per offset register and step instead of one per fetch, at the price of registers
@@ -194,7 +201,7 @@ template <int D> __device__ inline h16x8 fetch_rows_o(TileAt tile, const LaneOff
 template <int D, bool kPinBase = true>
 __device__ inline h16x8 fetch_cols_o(const char* tile, const LaneOffsets<D>& o, int db, int c) {
     union { s16x4 v[2]; h16x8 b; } u;
-    const int add = (32 * (c >> 1) + 16 * (c & 1)) * D * 2;
+    const int add = (32 * (c >> 1) + 16 * (c & 1)) * kPitch<D> * 2;
     if (kPinBase) {
         u.v[0] = lds_read_tr_at(lds_lane_base(tile, o.cols[0][db]), add);
         u.v[1] = lds_read_tr_at(lds_lane_base(tile, o.cols[1][db]), add);
@@ -207,7 +214,7 @@ __device__ inline h16x8 fetch_cols_o(const char* tile, const LaneOffsets<D>& o, 
 template <int D, bool kPinBase = true>
 __device__ inline h16x8 fetch_cols_o(TileAt tile, const LaneOffsets<D>& o, int db, int c) {
     union { s16x4 v[2]; h16x8 b; } u;
-    const int add = tile.off + (32 * (c >> 1) + 16 * (c & 1)) * D * 2;
+    const int add = tile.off + (32 * (c >> 1) + 16 * (c & 1)) * kPitch<D> * 2;
     u.v[0] = lds_read_tr_at((uint32_t)o.cols[0][db], add);
     u.v[1] = lds_read_tr_at((uint32_t)o.cols[1][db], add);
     return u.b;
@@ -215,19 +222,19 @@ __device__ inline h16x8 fetch_cols_o(TileAt tile, const LaneOffsets<D>& o, int d
 template <int D, bool kPinBase = false>
 __device__ inline h16x8 fetch_nat_o(TileAt tile, const LaneOffsets<D>& o, int row0, int cb) {
     union { s16x4 v[2]; h16x8 b; } u;
-    u.v[0] = lds_read_tr_at((uint32_t)o.nat[0][cb], tile.off + row0 * D * 2);
-    u.v[1] = lds_read_tr_at((uint32_t)o.nat[1][cb], tile.off + row0 * D * 2);
+    u.v[0] = lds_read_tr_at((uint32_t)o.nat[0][cb], tile.off + row0 * kPitch<D> * 2);
+    u.v[1] = lds_read_tr_at((uint32_t)o.nat[1][cb], tile.off + row0 * kPitch<D> * 2);
     return u.b;
 }
 template <int D, bool kPinBase = false>
 __device__ inline h16x8 fetch_nat_o(const char* tile, const LaneOffsets<D>& o, int row0, int cb) {
     union { s16x4 v[2]; h16x8 b; } u;
     if (kPinBase) {
-        u.v[0] = lds_read_tr_at(lds_lane_base(tile, o.nat[0][cb]), row0 * D * 2);
-        u.v[1] = lds_read_tr_at(lds_lane_base(tile, o.nat[1][cb]), row0 * D * 2);
+        u.v[0] = lds_read_tr_at(lds_lane_base(tile, o.nat[0][cb]), row0 * kPitch<D> * 2);
+        u.v[1] = lds_read_tr_at(lds_lane_base(tile, o.nat[1][cb]), row0 * kPitch<D> * 2);
     } else {
-        u.v[0] = lds_read_tr(tile + o.nat[0][cb] + row0 * D * 2);
-        u.v[1] = lds_read_tr(tile + o.nat[1][cb] + row0 * D * 2);
+        u.v[0] = lds_read_tr(tile + o.nat[0][cb] + row0 * kPitch<D> * 2);
+        u.v[1] = lds_read_tr(tile + o.nat[1][cb] + row0 * kPitch<D> * 2);
     }
     return u.b;
 }
@@ -236,7 +243,7 @@ template <int D> __device__ inline h16x8 fetch_rows_p(TileAt tile, const LaneOff
     return fetch_rows_o<D>(tile, o, t, ks);
 }
 template <int D> __device__ inline h16x8 fetch_rows_p(const char* tile, const LaneOffsets<D>& o, int t, int ks) {
-    return *(const __attribute__((address_space(3))) h16x8*)((__attribute__((address_space(3))) char*)(uintptr_t)lds_lane_base(tile, o.rows[ks]) + t * 32 * D * 2);
+    return *(const __attribute__((address_space(3))) h16x8*)((__attribute__((address_space(3))) char*)(uintptr_t)lds_lane_base(tile, o.rows[ks]) + t * 32 * kPitch<D> * 2);
 }
 // The same with the two lane offsets already picked (column block chosen at run time:
 // indexing the offset table with a run-time value would push it into scratch memory).
@@ -322,23 +329,33 @@ template <int D> struct TileCopy {
 __device__ inline void dma16(const char* base, uint32_t off, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" : : "s"(base), "v"(off), "s"(lds_addr) : "memory");
 }
+// the same from the lanes of `lanes` only: the others' 16 bytes of LDS stay as they are
+__device__ inline void dma16_lanes(const char* base, uint32_t off, uint32_t lds_addr, uint64_t lanes) {
+    uint64_t all;
+    asm volatile("s_mov_b32 m0, %3\n\ts_and_saveexec_b64 %0, %4\n\tglobal_load_lds_dwordx4 %2, %1\n\ts_mov_b64 exec, %0"
+                 : "=&s"(all) : "s"(base), "v"(off), "s"(lds_addr), "s"(lanes) : "memory", "scc");
+}
 __device__ inline uint32_t lds_address(const char* p) { return (uint32_t)(uintptr_t)p; }   // (low half of the flat address)
 
 template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma {      // kNatural: rows kept in their order (query tiles)
-    static constexpr int kPerWave = 64 * D * 2 / 1024 / 4;    // 2 (D=64) or 4 (D=128)
+    static constexpr int kPerWave = 64 * kPitch<D> * 2 / 1024 / 4;    // 2 (D=64) or 4 (D=128)
     uint32_t off[kPerWave];
     const char* origin;        // row 0 of the (sequence, head) slice: uniform
     int st, w4, lane;          // row stride in elements
+    static constexpr bool kCut = D == 96;      // rows shorter than the tile's: lanes of missing chunks take no part in a copy
+    uint64_t live[kCut ? kPerWave : 1];
+    int chunks;
 
     __device__ static inline void where(int inst, int lane, int& kl, int& c) {
         const int pos = inst * 64 + lane;                  // LDS chunk position
-        const int r = pos / (D / 8), pc = pos % (D / 8);
+        const int r = pos / (kPitch<D> / 8), pc = pos % (kPitch<D> / 8);
         c = pc ^ swz<D>(r);
         kl = kNatural ? r : (((r >> 2) & 1) << 5) | (((r >> 5) & 1) << 4) | (((r >> 3) & 3) << 2) | (r & 3);
     }
     // Only the slice origin and the row stride are kept: holding on to the whole tensor
     // descriptor costs scalar registers that the loops do not have.
-    __device__ inline void init(int lane_, int w4_, const TensorArg& t, int64_t base) {
+    __device__ inline void init(int lane_, int w4_, const TensorArg& t, int64_t base, int cols = D) {
+        chunks = cols / 8;
         lane = lane_; w4 = w4_;
         origin = t.ptr + 2 * base;
         st = (int)t.st;
@@ -356,13 +373,32 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
             int kl, c;
             where(w4 + 4 * i, lane, kl, c);
             off[i] = 2u * (uint32_t)(kl * st + c * 8);
+            if (kCut) {
+                live[i] = __builtin_amdgcn_ballot_w64(c < chunks);
+                asm("" : "+s"(live[i]));
+            }
         }
+    }
+    __device__ inline void copy(int i, const char* tile_base, uint32_t o, char* tile) const {
+        if (kCut) dma16_lanes(tile_base, o, lds_address(tile + (w4 + 4 * i) * 1024), live[i]);
+        else dma16(tile_base, o, lds_address(tile + (w4 + 4 * i) * 1024));
+    }
+    // Zeros where this wave's copies into `tile` write (and, in rows shorter than 96 columns, never will): once per tile buffer,
+    // before its first copy.
+    __device__ inline void clear(char* tile) const {
+        if (!kCut || chunks * 8 == D) return;
+#pragma unroll
+        for (int i = 0; i < kPerWave; ++i) {
+            const u32x4 z = {0u, 0u, 0u, 0u};
+            *(u32x4*)(tile + (w4 + 4 * i) * 1024 + lane * 16) = z;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     // a tile known to lie inside the sequence (every key tile of a sweep but the rightmost)
     __device__ inline void issue_full(int row0, char* tile) const {
         const char* tile_base = origin + (((uint64_t)(uint32_t)row0 * (uint32_t)st) << 1);
 #pragma unroll
-        for (int i = 0; i < kPerWave; ++i) dma16(tile_base, off[i], lds_address(tile + (w4 + 4 * i) * 1024));
+        for (int i = 0; i < kPerWave; ++i) copy(i, tile_base, off[i], tile);
     }
     __device__ inline void issue(int row0, int len, char* tile) const {
         // uniform; row0 and the stride are non-negative: the unsigned product is two scalar instructions, the
@@ -370,7 +406,7 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
         const char* tile_base = origin + (((uint64_t)(uint32_t)row0 * (uint32_t)st) << 1);
         if (row0 + 64 <= len) {
 #pragma unroll
-            for (int i = 0; i < kPerWave; ++i) dma16(tile_base, off[i], lds_address(tile + (w4 + 4 * i) * 1024));
+            for (int i = 0; i < kPerWave; ++i) copy(i, tile_base, off[i], tile);
         } else {
             int lane_here = lane;
             if (kLateRagged) asm volatile("" : "+v"(lane_here));
@@ -379,7 +415,7 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
                 int kl, c;
                 where(w4 + 4 * i, lane_here, kl, c);
                 kl = min(kl, len - 1 - row0);
-                dma16(tile_base, 2u * (uint32_t)(kl * st + c * 8), lds_address(tile + (w4 + 4 * i) * 1024));
+                copy(i, tile_base, 2u * (uint32_t)(kl * st + c * 8), tile);
             }
         }
     }
@@ -419,12 +455,15 @@ __device__ inline void store_staged_rows(const char* staging, const TensorArg& t
 // predicate; the ks fragments are at constant offsets from it.
 template <int D>
 __device__ inline void load_row_frags(h16x8 (&f)[D / 16], const TensorArg& t, int64_t base, int row,
-                                      int len, int lane) {
+                                      int len, int lane, int cols = D) {
     const int h = lane >> 5;
     const char* ptr = t.ptr + 2 * (base + (int64_t)row * t.st + 8 * h);
     if (row < len) {
 #pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) f[ks] = __builtin_bit_cast(h16x8, *(const u32x4*)(ptr + 32 * ks));
+        for (int ks = 0; ks < D / 16; ++ks) {
+            if (D == 96 && 16 * ks + 8 * h >= cols) f[ks] = h16x8{0};
+            else f[ks] = __builtin_bit_cast(h16x8, *(const u32x4*)(ptr + 32 * ks));
+        }
     } else {
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks) f[ks] = h16x8{0};
@@ -453,7 +492,7 @@ __device__ inline f32x16 mfma(h16x8 a, h16x8 b, f32x16 c) {
 // S^T tile pair for one wave, raw MFMA accumulators (no vector-ALU instruction touches
 // them here, so the matrix cores run ahead of whatever vector work follows):
 // raw[t][r] = (K Q^T)[key_local = 32h + 16t + r][query n].
-template <int D, bool kBatch = (D == 128), class Tile>
+template <int D, bool kBatch = kWide<D>, class Tile>
 __device__ inline void score_raw_o(f32x16 (&raw)[2], Tile ktile, const LaneOffsets<D>& o,
                                    const h16x8 (&qf)[D / 16]) {
     // tile 1 first: the product chain starts at its keys (the right half of the lane's 32), and
@@ -481,7 +520,7 @@ __device__ inline void scale_scores(float (&x)[32], const f32x16 (&raw)[2], floa
         for (int r = 0; r < 16; ++r) x[16 * t + r] = raw[t][r] * scale2;
 }
 
-template <int D, bool kBatch = (D == 128), class Tile>
+template <int D, bool kBatch = kWide<D>, class Tile>
 __device__ inline void score_tiles_o(float (&x)[32], Tile ktile, const LaneOffsets<D>& o,
                                      const h16x8 (&qf)[D / 16], float scale2) {
     f32x16 raw[2];
@@ -490,7 +529,7 @@ __device__ inline void score_tiles_o(float (&x)[32], Tile ktile, const LaneOffse
 }
 
 // Score tiles from pre-scaled fragments: x[16*t + r] = raw accumulator, no vector work.
-template <int D, bool kBatch = (D == 128), class Tile>
+template <int D, bool kBatch = kWide<D>, class Tile>
 __device__ inline void score_tiles_ps(float (&x)[32], Tile ktile, const LaneOffsets<D>& o,
                                       const h16x8 (&qf)[D / 16]) {
     f32x16 raw[2];
@@ -683,7 +722,7 @@ template <int D, class Tile>
 __device__ inline void stick_weights_and_dp(float (&x)[32], float (&beta)[32], float (&dp)[32], float& R, int lane,
                                             float* lane_carry, Tile vtile, const LaneOffsets<D>& o,
                                             const h16x8 (&dof)[D / 16]) {
-    constexpr int kPer = D / 64;               // MFMAs per segment: 2 tiles x D/16 slices over 8 segments
+    constexpr int kPer = (D / 8 + 7) / 8;      // MFMAs per segment: 2 tiles x D/16 slices over 8 segments
     f32x16 dacc[2];
     h16x8 nx[kPer];
     // MFMA m (0 .. D/8 - 1): tile t = m & 1, slice ks = m >> 1 (neighbours use different accumulators)
@@ -697,13 +736,13 @@ __device__ inline void stick_weights_and_dp(float (&x)[32], float (&beta)[32], f
 #pragma unroll
             for (int i = 0; i < kPer; ++i) {
                 const int m = kPer * (seg + 1) + i;
-                nx[i] = fetch_rows_o<D>(vtile, o, m & 1, m >> 1);
+                if (m < D / 8) nx[i] = fetch_rows_o<D>(vtile, o, m & 1, m >> 1);
             }
         }
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int m = kPer * seg + i, t = m & 1, ks = m >> 1;
-            dacc[t] = mfma(cur[i], dof[ks], ks == 0 ? f32x16{0} : dacc[t]);
+            if (m < D / 8) dacc[t] = mfma(cur[i], dof[ks], ks == 0 ? f32x16{0} : dacc[t]);
         }
     });
 #pragma unroll
@@ -721,7 +760,7 @@ __device__ inline void stick_weights_and_dp(float (&x)[32], float (&beta)[32], f
 template <int D, bool kPaced = false, class Tile>
 __device__ inline float carried_weights_and_dp(float (&x)[32], float (&beta)[32], float (&dp)[32], float F,
                                                Tile vtile, const LaneOffsets<D>& o, const h16x8 (&dof)[D / 16]) {
-    constexpr int kPer = D / 64;
+    constexpr int kPer = (D / 8 + 7) / 8;
     f32x16 dacc[2];
     h16x8 nx[kPer];
 #pragma unroll
@@ -740,13 +779,13 @@ __device__ inline float carried_weights_and_dp(float (&x)[32], float (&beta)[32]
 #pragma unroll
             for (int i = 0; i < kPer; ++i) {
                 const int m = kPer * (seg + 1) + i;
-                nx[i] = fetch_rows_o<D>(vtile, o, m & 1, m >> 1);
+                if (m < D / 8) nx[i] = fetch_rows_o<D>(vtile, o, m & 1, m >> 1);
             }
         }
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int m = kPer * seg + i, t = m & 1, ks = m >> 1;
-            dacc[t] = mfma(cur[i], dof[ks], ks == 0 ? f32x16{0} : dacc[t]);
+            if (m < D / 8) dacc[t] = mfma(cur[i], dof[ks], ks == 0 ? f32x16{0} : dacc[t]);
         }
     });
 #pragma unroll

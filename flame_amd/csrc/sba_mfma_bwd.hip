@@ -49,7 +49,7 @@ __device__ inline void store_scaled_q(const KParams& p, const Job& job, int head
 // -6 %); on launches that last as long as their longest sweep the plain arrangement's shorter step is ahead.
 template <int D, bool kLean = false>
 __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 1)) void mfma_bwd_dq_kernel(KParams p) {
-    constexpr int kTile = 64 * D * 2;
+    constexpr int kTile = 64 * kPitch<D> * 2;
     __shared__ __attribute__((aligned(16))) char lds[4 * kTile];   // K0 V0 K1 V1
 
     const int lane = threadIdx.x & 63;
@@ -72,9 +72,9 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
 
     if (blockIdx.x == 0 && threadIdx.x == 0 && p.gave_up) *p.gave_up = 0;     // error word of the launch pair, see wait_for_count()
     h16x8 qf[D / 16], dof[D / 16];
-    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane);
+    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane, p.cols);
     prescale_frags(qf, p.scale2);          // the score MFMAs then deliver base-2 logits
-    load_row_frags<D>(dof, p.d_o, dobase, qi, job.len, lane);
+    load_row_frags<D>(dof, p.d_o, dobase, qi, job.len, lane, p.cols);
 
     f32x16 dqacc[D / 32];
 #pragma unroll
@@ -86,8 +86,13 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     const int n_steps = kmax >= 0 ? kmax / kKeyBlock + 1 : 0;
 
     TileDma<D, false, D == 64 && kLean> kc, vc;
-    kc.init(lane, wave, p.k, kbase);
-    vc.init(lane, wave, p.v, vbase);
+    kc.init(lane, wave, p.k, kbase, p.cols);
+    vc.init(lane, wave, p.v, vbase, p.cols);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        kc.clear(lds + b * 2 * kTile);
+        vc.clear(lds + b * 2 * kTile + kTile);
+    }
     if (n_steps > 0) {
         kc.issue(0, job.len, lds);
         vc.issue(0, job.len, lds + kTile);
@@ -135,7 +140,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
         }
         if (!skip) {
             h16x8 zf[4];
-            if constexpr (D == 128 || kLean) {
+            if constexpr (kWide<D> || kLean) {
                 // Register-lean arrangement (two arrays of 32 live instead of four: two waves per SIMD
                 // instead of one): scores and dP first, then the chain over both in place.
                 float x[32], dp[32];
@@ -189,7 +194,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
                 h16x8 kt[D / 32];
 #pragma unroll
                 for (int db = 0; db < D / 32; ++db) kt[db] = fetch_cols_o<D>(ktile, lo, db, c);
-                if (D == 128) __builtin_amdgcn_sched_barrier(0);
+                if (kWide<D>) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int db = 0; db < D / 32; ++db) dqacc[db] = mfma(kt[db], zf[c], dqacc[db]);
             }
@@ -210,6 +215,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
         for (int db = 0; db < D / 32; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                if (D == 96 && 32 * db + 8 * g >= p.cols) continue;
                 f32x2 a = {dqacc[db][4 * g] * p.scale, dqacc[db][4 * g + 1] * p.scale};
                 f32x2 b = {dqacc[db][4 * g + 2] * p.scale, dqacc[db][4 * g + 3] * p.scale};
                 h16x2 pa = __builtin_convertvector(a, h16x2), pb = __builtin_convertvector(b, h16x2);
@@ -1451,8 +1457,8 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
 template <int D, int W>
 __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel(KParams p) {
     constexpr int kRows = W * 32;
-    constexpr int kTile = 64 * D * 2;
-    constexpr int kQ = 0, kDO = kRows * D * 2, kK = 2 * kDO, kV = kK + kTile, kA = kV + kTile, kZ = kA + kRows * 128;
+    constexpr int kTile = 64 * kPitch<D> * 2;
+    constexpr int kQ = 0, kDO = kRows * kPitch<D> * 2, kK = 2 * kDO, kV = kK + kTile, kA = kV + kTile, kZ = kA + kRows * 128;
     constexpr int kNB = D / 32;                // 32-column blocks of dK or dV that a wave reduces, for
     constexpr int kKH = W == 2 ? 2 : 1;        // one 32-key half of the block or both
     constexpr int kCols = 32 * kNB;
@@ -1478,21 +1484,22 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
     const int64_t qbase = base_of(p.q), kbase = base_of(p.k), vbase = base_of(p.v), dobase = base_of(p.d_o);
 
     // a tile is four waves' copies: two each where there are only two
-    auto copy = [&](auto natural, const TensorArg& t, int64_t base, int row0, char* tile) {
+    auto copy = [&](auto natural, const TensorArg& t, int64_t base, int row0, char* tile, bool fresh) {
 #pragma unroll
         for (int w4 = 0; w4 < 4; w4 += W) {
             TileDma<D, decltype(natural)::value> c;
-            c.init(lane, wave + w4, t, base);
+            c.init(lane, wave + w4, t, base, p.cols);
+            if (fresh) c.clear(tile);
             c.issue(row0, job.len, tile);
         }
     };
     constexpr std::true_type kNaturalRows{};
     constexpr std::false_type kMfmaRows{};
-    copy(kMfmaRows, p.k, kbase, 0, lds + kK);
-    copy(kMfmaRows, p.v, vbase, 0, lds + kV);
+    copy(kMfmaRows, p.k, kbase, 0, lds + kK, true);
+    copy(kMfmaRows, p.v, vbase, 0, lds + kV, true);
     for (int r = 0; r < job.len; r += 64) {
-        copy(kNaturalRows, p.q, qbase, r, lds + kQ + r * D * 2);
-        copy(kNaturalRows, p.d_o, dobase, r, lds + kDO + r * D * 2);
+        copy(kNaturalRows, p.q, qbase, r, lds + kQ + r * kPitch<D> * 2, true);
+        copy(kNaturalRows, p.d_o, dobase, r, lds + kDO + r * kPitch<D> * 2, true);
     }
     // the carry that enters this lane's 32 keys of a block; 0 for rows past the end, whose weights are then exactly 0
     // (and for a block that holds nothing but the invisible last token: the forward has no entry for it)
@@ -1559,8 +1566,8 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
         }
         __syncthreads();                       // weights complete, K and V free
         if (kb + 1 < n_kb) {
-            copy(kMfmaRows, p.k, kbase, key0 + kKeyBlock, lds + kK);
-            copy(kMfmaRows, p.v, vbase, key0 + kKeyBlock, lds + kV);
+            copy(kMfmaRows, p.k, kbase, key0 + kKeyBlock, lds + kK, false);
+            copy(kMfmaRows, p.v, vbase, key0 + kKeyBlock, lds + kV, false);
         }
         // [32 keys x kCols] of dV (which = 0) or dK: keys 32 kh .. of the block, over the queries from the block on
         f32x16 acc[kKH][kNB];
@@ -1583,7 +1590,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
                     w[i] = fetch(kh0 + i ? lz.nat[0][1] : lz.nat[0][0], kh0 + i ? lz.nat[1][1] : lz.nat[1][0], offw + r * 128);
 #pragma unroll
                 for (int db = 0; db < kNB; ++db) {
-                    const h16x8 b = fetch(lo.nat[0][db], lo.nat[1][db], offb + r * D * 2);
+                    const h16x8 b = fetch(lo.nat[0][db], lo.nat[1][db], offb + r * kPitch<D> * 2);
 #pragma unroll
                     for (int i = 0; i < kKH; ++i) acc[i][db] = mfma(w[i], b, acc[i][db]);
                 }
@@ -1600,7 +1607,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
                 for (int db = 0; db < kNB; ++db) stage_acc_tile<kCols>(stage, 32 * i, 32 * db, acc[i][db], which ? p.scale : 1.0f, lane);
             for (int c = lane; c < kKH * 32 * kCols / 8; c += 64) {
                 const int row = c / (kCols / 8), cc = c % (kCols / 8), key = key0 + 32 * kh0 + row;
-                if (key < job.len)
+                if (key < job.len && (D != 96 || cc * 8 < p.cols))
                     *(u32x4*)(out.ptr + 2 * (ob + (int64_t)key * out.st + cc * 8)) = *(const u32x4*)(stage + row * (kCols * 2) + cc * 16);
             }
         }
@@ -1616,6 +1623,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
         for (int db = 0; db < D / 32; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                if (D == 96 && 32 * db + 8 * g >= p.cols) continue;
                 f32x2 a = {dqacc[db][4 * g] * p.scale, dqacc[db][4 * g + 1] * p.scale};
                 f32x2 b = {dqacc[db][4 * g + 2] * p.scale, dqacc[db][4 * g + 3] * p.scale};
                 uint2 w;
@@ -1637,17 +1645,21 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
 // SIMD.  Two workgroup barriers per step (weights complete; tiles handed over).
 template <int D>
 __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KParams p) {
-    constexpr int kQTile = 64 * D * 2;           // Q or dO tile of one step (64 queries)
+    constexpr int kQTile = 64 * kPitch<D> * 2;           // Q or dO tile of one step (64 queries)
     constexpr int kZTile = 64 * 64 * 2;          // per pair: [64 queries][32 a | 32 dz] bf16
     constexpr int kStep = 64;
     constexpr bool kPairPin = true;              // LDS fetch bases pinned in registers: 3 % faster here
-    constexpr int kBlocks = D / 64;              // 32-wide column blocks of dK / dV per wave
+    constexpr int kBlocks = (D + 63) / 64;       // 32-wide column blocks of dK / dV per wave (head_dim 96: two or one)
     static_assert(32 * D * 2 <= kZTile, "the pair's tile doubles as the staging of its [32 keys x D] outputs");
     __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + 4 * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = wave >> 1, r = wave & 1;
+    // this wave's column blocks: kBlocks * half ..; at head_dim 96 the second half is one block, and the pairs take turns at which
+    // of their waves (r: which SIMD) has it
+    const int half = D == 96 ? r ^ (grp >> 1) : r;
+    const bool both = D != 96 || half == 0;
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
@@ -1671,8 +1683,8 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
     {
         const int m = lane & 31;
         const int key = kb0 + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
-        load_row_frags<D>(kfr, p.k, kbase, key, job.len, lane);
-        load_row_frags<D>(vfr, p.v, vbase, key, job.len, lane);
+        load_row_frags<D>(kfr, p.k, kbase, key, job.len, lane, p.cols);
+        load_row_frags<D>(vfr, p.v, vbase, key, job.len, lane, p.cols);
         prescale_frags(kfr, p.scale2);
     }
     f32x16 dkacc[kBlocks], dvacc[kBlocks];
@@ -1683,8 +1695,10 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
 
     // waves 0-3 copy the Q tiles, waves 4-7 the dO tiles
     TileDma<D, true> tc;
-    tc.init(lane, wave & 3, wave < 4 ? p.q : p.d_o, wave < 4 ? qbase : dobase);
+    tc.init(lane, wave & 3, wave < 4 ? p.q : p.d_o, wave < 4 ? qbase : dobase, p.cols);
     const int my_tile = wave < 4 ? 0 : kQTile;
+    tc.clear(lds + my_tile);
+    tc.clear(lds + 2 * kQTile + my_tile);
     if (n_steps > 0) tc.issue(q_begin, job.len, lds + my_tile);
 
     // carries of a (query, this pair's 32 keys) pair, see the own-keys kernel
@@ -1714,14 +1728,14 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
     uint32_t row_at[D / 16], nat_at[2][kBlocks], z_at[2][2];
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) row_at[ks] = lds_lane_base(lds + r * 32 * D * 2, lo.rows[ks]);
+    for (int ks = 0; ks < D / 16; ++ks) row_at[ks] = lds_lane_base(lds + r * 32 * kPitch<D> * 2, lo.rows[ks]);
     {
         const int hh = lane >> 5, G1 = (lane >> 4) & 1, sl = lane & 15;
 #pragma unroll
         for (int a2 = 0; a2 < 2; ++a2) {
 #pragma unroll
             for (int j = 0; j < kBlocks; ++j) {
-                const int chunk = 4 * (kBlocks * r + j) + 2 * G1 + ((sl & 3) >> 1);
+                const int chunk = 4 * (kBlocks * half + j) + 2 * G1 + ((sl & 3) >> 1);
                 nat_at[a2][j] = lds_lane_base(lds, tile_offset<D>(8 * hh + 4 * a2 + (sl >> 2), chunk) + ((sl & 1) << 3));
             }
 #pragma unroll
@@ -1785,7 +1799,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
                         if (idx >= nvis) x[idx] = -INFINITY;
                 }
                 // dP = dO V^T between the segments of the chain, its operands fetched one segment ahead
-                constexpr int kPer = D / 64;
+                constexpr int kPer = (D / 16 + 3) / 4;
                 h16x8 nx[kPer];
 #pragma unroll
                 for (int i = 0; i < kPer; ++i) nx[i] = rows_at(row_at[i], kDO);
@@ -1796,12 +1810,13 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
                     for (int i = 0; i < kPer; ++i) cur[i] = nx[i];
                     if (seg < 3) {
 #pragma unroll
-                        for (int i = 0; i < kPer; ++i) nx[i] = rows_at(row_at[kPer * (seg + 1) + i], kDO);
+                        for (int i = 0; i < kPer; ++i)
+                            if (kPer * (seg + 1) + i < D / 16) nx[i] = rows_at(row_at[kPer * (seg + 1) + i], kDO);
                     }
 #pragma unroll
                     for (int i = 0; i < kPer; ++i) {
                         const int ks = kPer * seg + i;
-                        dacc = mfma(vfr[ks], cur[i], ks == 0 ? f32x16{0} : dacc);
+                        if (ks < D / 16) dacc = mfma(vfr[ks], cur[i], ks == 0 ? f32x16{0} : dacc);
                     }
                     if (seg == 1) __builtin_amdgcn_s_setprio(2);
                 });
@@ -1828,8 +1843,9 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
                 ww[1] = nat_pair(z_at, 1, 16 * kk * 64 * 2);
 #pragma unroll
                 for (int j = 0; j < kBlocks; ++j) {
-                    oo[2 * j] = nat_pair(nat_at, j, kDO + 16 * kk * D * 2);
-                    oo[2 * j + 1] = nat_pair(nat_at, j, kQ + 16 * kk * D * 2);
+                    if (j > 0 && !both) break;
+                    oo[2 * j] = nat_pair(nat_at, j, kDO + 16 * kk * kPitch<D> * 2);
+                    oo[2 * j + 1] = nat_pair(nat_at, j, kQ + 16 * kk * kPitch<D> * 2);
                 }
             };
             fetch_kk(0, w[0], o[0]);
@@ -1839,6 +1855,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int j = 0; j < kBlocks; ++j) {
+                    if (j > 0 && !both) break;
                     dvacc[j] = mfma(w[kk & 1][0], o[kk & 1][2 * j], dvacc[j]);
                     dkacc[j] = mfma(w[kk & 1][1], o[kk & 1][2 * j + 1], dkacc[j]);
                 }
@@ -1861,11 +1878,11 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
         const int64_t ob = (int64_t)job.seq * out.sb + (int64_t)head * out.sh + (int64_t)job.tok0 * out.st;
 #pragma unroll
         for (int j = 0; j < kBlocks; ++j)
-            stage_acc_tile<D>(ztile, 0, 32 * (kBlocks * r + j), which == 0 ? dkacc[j] : dvacc[j], which == 0 ? p.scale : 1.0f, lane);
+            if (j == 0 || both) stage_acc_tile<D>(ztile, 0, 32 * (kBlocks * half + j), which == 0 ? dkacc[j] : dvacc[j], which == 0 ? p.scale : 1.0f, lane);
         __syncthreads();
         for (int c = lane + 64 * r; c < 32 * D / 8; c += 128) {
             const int row = c / (D / 8), cc = c % (D / 8);
-            if (kb0 + row < job.len)
+            if (kb0 + row < job.len && (D != 96 || cc * 8 < p.cols))
                 *(u32x4*)(out.ptr + 2 * (ob + (int64_t)(kb0 + row) * out.st + cc * 8)) = *(const u32x4*)(ztile + row * (D * 2) + cc * 16);
         }
         __syncthreads();
@@ -1936,7 +1953,9 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     // the two-pass ones.
     if (kp.seq_len <= kRowBlock && kp.head_dim <= 128 && !which && !getenv("SBA_DQ_KERNEL") && sba_two_step_env() < 0) {
         if (!p1) return SBA_OK;
-        if (kp.head_dim == 128) {
+        if (kp.head_dim == 96) {
+            hipLaunchKernelGGL((mfma_bwd_short_kernel<96, 4>), grid, dim3(256), 0, s, kp);
+        } else if (kp.head_dim == 128) {
             hipLaunchKernelGGL((mfma_bwd_short_kernel<128, 4>), grid, dim3(256), 0, s, kp);
         } else {
             if (kp.seq_len <= 64) hipLaunchKernelGGL((mfma_bwd_short_kernel<64, 2>), grid, dim3(128), 0, s, kp);
@@ -1972,6 +1991,9 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
             if (stream8) hipLaunchKernelGGL((mfma_bwd_dkv_stream_kernel<64, 8>), dim3(n_wg), dim3(12 * 64), 0, s, kp);
             else hipLaunchKernelGGL((mfma_bwd_dkv_stream_kernel<64, 4>), dim3(n_wg), dim3(8 * 64), 0, s, kp);
         }
+    } else if (kp.head_dim == 96) {
+        if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<96>), grid, dim3(kThreads), 0, s, kp);
+        if (p2) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<96>), grid, dim3(2 * kThreads), 0, s, kp);
     } else if (kp.head_dim == 256) {
         // one wave per SIMD in both passes; every wave of the key-owner pass on its own 32 keys, two workgroups per
         // key block that each accumulate one half of the columns of dK and dV - the other key-owner kernels do not

@@ -40,7 +40,7 @@ __device__ inline bool fwd_step(const char* ktile, const char* vtile, const Lane
             for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
                 for (int db = 0; db < D / 32; ++db) vt[cc][db] = fetch_cols_o<D, kPinBase>(vtile, lo, db, 2 * c2 + cc);
-            if (D == 128) __builtin_amdgcn_sched_barrier(0);
+            if (kWide<D>) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
@@ -60,6 +60,7 @@ __device__ inline void store_o_row(const KParams& p, const Job& job, int head, i
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
+            if (D == 96 && 32 * db + 8 * g >= p.cols) continue;
             f32x2 a = {oacc[db][4 * g], oacc[db][4 * g + 1]};
             f32x2 b = {oacc[db][4 * g + 2], oacc[db][4 * g + 3]};
             h16x2 pa = __builtin_convertvector(a, h16x2), pb = __builtin_convertvector(b, h16x2);
@@ -74,7 +75,7 @@ __device__ inline void store_o_row(const KParams& p, const Job& job, int head, i
 // getting the table when the forward kept none.
 template <int D, bool kCarryOnly>
 __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
-    constexpr int kTile = 64 * D * 2;            // bytes per K or V tile
+    constexpr int kTile = 64 * kPitch<D> * 2;            // bytes per K or V tile
     __shared__ __attribute__((aligned(16))) char lds[4 * kTile];   // K0 V0 K1 V1
 
     const int lane = threadIdx.x & 63;
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
 
     h16x8 qf[D / 16];
-    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane);
+    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane, p.cols);
     prescale_frags(qf, p.scale2);
 
     f32x16 oacc[D / 32];
@@ -108,8 +109,13 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     const int64_t tabq = tab_index(p, head, job, job.rb, 0) + 32 * wave + n;   // + step * kRowBlock
 
     TileDma<D> kc, vc;
-    kc.init(lane, wave, p.k, kbase);
-    vc.init(lane, wave, p.v, vbase);
+    kc.init(lane, wave, p.k, kbase, p.cols);
+    vc.init(lane, wave, p.v, vbase, p.cols);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        kc.clear(lds + b * 2 * kTile);
+        vc.clear(lds + b * 2 * kTile + kTile);
+    }
     if (n_steps > 0) {
         kc.issue((n_steps - 1) * kKeyBlock, job.len, lds);
         if (!kCarryOnly) vc.issue((n_steps - 1) * kKeyBlock, job.len, lds + kTile);
@@ -153,7 +159,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
         const bool skip = key0 + strict > q0w + 31 || q0w >= job.len;
         open_step(step, buf, skip);
         if (!skip) {
-            if (!fwd_step<D, kCarryOnly, true, D == 128>(ktile, ktile + kTile, lo, qf, oacc, R, lane, key0, q0w, qi, strict, carry_out)) {
+            if (!fwd_step<D, kCarryOnly, true, kWide<D>>(ktile, ktile + kTile, lo, qf, oacc, R, lane, key0, q0w, qi, strict, carry_out)) {
                 redo = true;
                 break;
             }
@@ -169,7 +175,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
         if (!redo) open_step(step, buf, skip);
         redo = false;
         if (!skip) {
-            fwd_step<D, kCarryOnly, false, D == 128>(ktile, ktile + kTile, lo, qf, oacc, R, lane, key0, q0w, qi, strict, carry_out);
+            fwd_step<D, kCarryOnly, false, kWide<D>>(ktile, ktile + kTile, lo, qf, oacc, R, lane, key0, q0w, qi, strict, carry_out);
             carry_step = step;
         }
         wait_global_memory();
@@ -197,7 +203,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
 // sweep; the groups only share the workgroup barrier that hands over the tiles.
 template <int D, int G, bool kCarryOnly>
 __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
-    constexpr int kTile = 64 * D * 2;
+    constexpr int kTile = 64 * kPitch<D> * 2;
     // tile(grp, buf, kv) = lds + ((grp * 2 + buf) * 2 + kv) * kTile
     __shared__ __attribute__((aligned(16))) char lds[G * 4 * kTile];
     __shared__ float totals[G][kRowBlock];
@@ -220,7 +226,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
 
     h16x8 qf[D / 16];
-    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane);
+    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane, p.cols);
     prescale_frags(qf, p.scale2);
     f32x16 oacc[D / 32];
 #pragma unroll
@@ -237,8 +243,13 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     char* my_tiles = lds + grp * 4 * kTile;                // + buf * 2 * kTile
 
     TileDma<D> kc, vc;
-    kc.init(lane, qs, p.k, kbase);
-    vc.init(lane, qs, p.v, vbase);
+    kc.init(lane, qs, p.k, kbase, p.cols);
+    vc.init(lane, qs, p.v, vbase, p.cols);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        kc.clear(my_tiles + b * 2 * kTile);
+        vc.clear(my_tiles + b * 2 * kTile + kTile);
+    }
     if (hi - 1 >= low) {
         kc.issue((hi - 1) * kKeyBlock, job.len, my_tiles);
         if (!kCarryOnly) vc.issue((hi - 1) * kKeyBlock, job.len, my_tiles + kTile);
@@ -376,7 +387,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
 // the rule by "segments (4, or as forced) up to n workgroups".
 static int forward_segments(const sba::KParams& kp, unsigned grid) {
     if (kp.head_dim == 256) return 0;      // two K / V tile pairs are 128 KB of LDS: one group of waves per workgroup
-    if (kp.head_dim == 128) {
+    if (kp.head_dim == 128 || kp.head_dim == 96) {
         // head_dim 128: the one-sweep kernel holds two workgroups per CU, the two-segment one (8 waves, 129 KB of
         // LDS) one; it pays while the grid is at most two rounds of those and the longest sweep dominates.  B=1,
         // H=16, one sweep / two segments in us: T=1024 29.8 / 26.2, T=2048 50.4 / 41.6, T=3072 77.2 / 60.0, T=4096
@@ -396,7 +407,8 @@ static int forward_segments(const sba::KParams& kp, unsigned grid) {
 template <bool kCarryOnly>
 static void launch_seg(int groups, dim3 grid, hipStream_t s, const sba::KParams& kp) {
     using namespace sba;
-    if (kp.head_dim == 128) hipLaunchKernelGGL((mfma_fwd_seg_kernel<128, 2, kCarryOnly>), grid, dim3(2 * kThreads), 0, s, kp);
+    if (kp.head_dim == 96) hipLaunchKernelGGL((mfma_fwd_seg_kernel<96, 2, kCarryOnly>), grid, dim3(2 * kThreads), 0, s, kp);
+    else if (kp.head_dim == 128) hipLaunchKernelGGL((mfma_fwd_seg_kernel<128, 2, kCarryOnly>), grid, dim3(2 * kThreads), 0, s, kp);
     else if (groups == 2) hipLaunchKernelGGL((mfma_fwd_seg_kernel<64, 2, kCarryOnly>), grid, dim3(2 * kThreads), 0, s, kp);
     else if (groups == 3) hipLaunchKernelGGL((mfma_fwd_seg_kernel<64, 3, kCarryOnly>), grid, dim3(3 * kThreads), 0, s, kp);
     else hipLaunchKernelGGL((mfma_fwd_seg_kernel<64, 4, kCarryOnly>), grid, dim3(4 * kThreads), 0, s, kp);
@@ -416,6 +428,9 @@ int sba_launch_mfma_fwd(const sba::KParams& kp, hipStream_t s) {
     } else if (kp.head_dim == 64) {
         if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<64, true>), grid, dim3(kThreads), 0, s, kp);
         else hipLaunchKernelGGL((mfma_fwd_kernel<64, false>), grid, dim3(kThreads), 0, s, kp);
+    } else if (kp.head_dim == 96) {
+        if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<96, true>), grid, dim3(kThreads), 0, s, kp);
+        else hipLaunchKernelGGL((mfma_fwd_kernel<96, false>), grid, dim3(kThreads), 0, s, kp);
     } else if (kp.head_dim == 128) {
         if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<128, true>), grid, dim3(kThreads), 0, s, kp);
         else hipLaunchKernelGGL((mfma_fwd_kernel<128, false>), grid, dim3(kThreads), 0, s, kp);

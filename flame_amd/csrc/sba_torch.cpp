@@ -60,6 +60,13 @@ int dtype_code(at::ScalarType t) {
     }
 }
 
+// 16-bit rows of 72, 80, 88 or 96 columns go to the matrix-core kernels as they are (SbaParams::columns)
+bool rides_96(const Tensor& t) {
+    const int64_t D = t.size(-1);
+    return D > 64 && D <= 96 && D % 8 == 0 && t.scalar_type() != at::kFloat && !env_is_1("SBA_FORCE_GENERIC") &&
+           !env_is_1("SBA_FORCE_GENERIC_BWD");
+}
+
 SbaTensor describe(const Tensor& t) {
     const auto s = t.strides();
     return t.dim() == 4 ? SbaTensor{t.data_ptr(), s[0], s[1], s[2]} : SbaTensor{t.data_ptr(), 0, s[0], s[1]};
@@ -78,6 +85,10 @@ SbaParams params_of(const Problem& pr) {
     const int64_t lead = pr.q.dim() - 3;                 // 1: dense, 0: packed
     p.n_heads = (int32_t)sz[lead];
     p.head_dim = (int32_t)sz[lead + 2];
+    if (rides_96(pr.q)) {
+        p.columns = p.head_dim;
+        p.head_dim = 128;
+    }
     p.total_tokens = (int32_t)sz[lead + 1];
     if (pr.plan) {
         p.n_seq = pr.plan->n_docs;
@@ -188,11 +199,11 @@ void check_plan(const Plan& plan, int64_t tokens, int64_t max_seqlens) {
                       plan.max_len, ")");
 }
 
-// Head dim that a problem runs with: 64, 128 and (16-bit types) 256 have matrix-core kernels, smaller ones ride them
-// zero-padded; float32 above 128 and everything under SBA_FORCE_GENERIC=1 keeps its own.
+// Head dim that a problem's tensors are handed over with: 64, 128 and (16-bit types) 72 .. 96 and 256 have matrix-core kernels,
+// others ride them zero-padded; float32 above 128 and everything under SBA_FORCE_GENERIC=1 keeps its own.
 int64_t matrix_core_head_dim(const Tensor& t) {
     const int64_t D = t.size(-1);
-    if (D == 64 || D == 128 || D > kMaxHeadDim || env_is_1("SBA_FORCE_GENERIC")) return D;
+    if (D == 64 || D == 128 || D > kMaxHeadDim || rides_96(t) || env_is_1("SBA_FORCE_GENERIC")) return D;
     if (D > 128) return t.scalar_type() == at::kFloat ? D : 256;
     return D < 64 ? 64 : 128;
 }

@@ -91,6 +91,10 @@ typedef struct SbaParams {
     int32_t  bwd_phases;       /* backward only: 0 = whole backward; 1 = first kernel only (dq and the
                                   prefix table), 2 = second kernel only (dk, dv; needs phase 1 done on
                                   the same workspace).  Lets a profiler time the kernels one by one */
+    int32_t  columns;          /* 0: the tensors have head_dim columns.  With head_dim 128 and a 16-bit dtype on the matrix-core
+                                  kernels it may be 72, 80, 88 or 96: the tensors' rows are that long, nothing outside them is
+                                  read or written, and the results are those of rows padded with zeros to 128.  (In the four
+                                  bytes in front of the pointers that were padding before: sizes and offsets are as they were) */
 
     const int32_t* cu_seqlens; /* device, n_seq+1 entries, or NULL for dense */
     const int32_t* schedule;   /* device, from sba_build_schedule(); packed layout only */
