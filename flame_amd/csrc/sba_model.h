@@ -11,10 +11,10 @@ constexpr int kMaxNormWidth = 2048;      // columns of a row that a wave keeps i
 constexpr int kCastTensors = 8;
 constexpr int kOptChunk = 16384;         // weights that one workgroup of the optimizer kernels takes
 
-// y = rms_norm(x + h) * w as 16-bit; h (16-bit) may be null; sum receives x + h when h is given.
+// y = rms_norm(x) * w as 16-bit
 struct NormFwd {
-    const float* x; const void* h; const float* w;
-    float* sum; void* y; float* rstd;
+    const float* x; const float* w;
+    void* y; float* rstd;
     int rows, cols; float eps;
 };
 int norm_fwd(const NormFwd& a, bool f16, hipStream_t stream);
@@ -68,6 +68,25 @@ int weight_grad_splits(WeightGrads& g, int cus);         // fills first_tile, ti
 int weight_grads(const WeightGrads& g, int splits, bool f16, hipStream_t stream);     // partial: [splits][total] if more than one
 int weight_grads_bf16(const WeightGrads& g, int splits, hipStream_t stream);
 int weight_grads_f16(const WeightGrads& g, int splits, hipStream_t stream);
+
+// y[t][n] = sum over k of x[t][k] w[n][k] (rows_w: w[k][n]) for m token rows, k a multiple of 32, n of 8, and what follows:
+//   kStore        out = y                                    16-bit [m][n]
+//   kAddResidual  out = residual + y                         fp32   [m][n]
+//   kSwigluFwd    w = gate rows | up rows: out = silu(gate) * up, 16-bit [m][n/2]; pre = y if given
+//   kSwigluBwd    y = gradient of silu(gate) * up, pre = gate | up [m][2n]: out = their gradients, 16-bit [m][2n]
+// x and w are 16-byte aligned with leading dimensions that are multiples of 8; outputs are dense.
+enum { kStore, kAddResidual, kSwigluFwd, kSwigluBwd };
+struct Projection {
+    const void* x; const void* w; int64_t ldx, ldw; int m, n, k;
+    bool rows_w; int epilogue;
+    const float* residual; void* pre; void* out;
+};
+bool projects(const Projection& p, int cus);             // whether the kernels take it
+enum ProjectionTile { kTile256, kTile128x256, kTile128 };
+ProjectionTile projection_tile(const Projection& p, int cus);
+int project(const Projection& p, bool f16, int cus, hipStream_t stream);
+int project_bf16(const Projection& p, ProjectionTile tile, hipStream_t stream);
+int project_f16(const Projection& p, ProjectionTile tile, hipStream_t stream);
 
 // One weight tensor of a clip + AdamW step.
 struct OptTensor {

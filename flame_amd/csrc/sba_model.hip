@@ -36,7 +36,7 @@ int launched() { return hipGetLastError() == hipSuccess ? 0 : -6; }
 // ------------------------------------------------------------------------------------------------- RMS norm
 // One wave per row, the row in registers (K groups of 256 columns, four columns a lane and group: 16-byte accesses, 1 KB per
 // wave and instruction).
-template <typename E, int K, bool kAdd>
+template <typename E, int K>
 __global__ __launch_bounds__(kThreads) void norm_fwd_kernel(NormFwd a) {
     const int lane = threadIdx.x & 63, row = blockIdx.x * kWaves + (threadIdx.x >> 6);
     if (row >= a.rows) return;
@@ -50,12 +50,6 @@ __global__ __launch_bounds__(kThreads) void norm_fwd_kernel(NormFwd a) {
         x[k] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (c < a.cols) {
             x[k] = *(const f32x4*)(a.x + base + c);
-            if (kAdd) {
-                const e4 h = *(const e4*)((const E*)a.h + base + c);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) x[k][i] += (float)h[i];
-                *(f32x4*)(a.sum + base + c) = x[k];
-            }
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) ss += x[k][i] * x[k][i];
@@ -419,8 +413,7 @@ int norm_fwd_t(const NormFwd& a, hipStream_t s) {
     const dim3 grid((a.rows + kWaves - 1) / kWaves), block(kThreads);
 #define SBA_NORM(K)                                                                                          \
     if (a.cols <= K * 256) {                                                                                 \
-        if (a.h) hipLaunchKernelGGL((norm_fwd_kernel<E, K, true>), grid, block, 0, s, a);                    \
-        else hipLaunchKernelGGL((norm_fwd_kernel<E, K, false>), grid, block, 0, s, a);                       \
+        hipLaunchKernelGGL((norm_fwd_kernel<E, K>), grid, block, 0, s, a);                                   \
         return launched();                                                                                   \
     }
     SBA_NORM(1) SBA_NORM(2) SBA_NORM(4) SBA_NORM(8)
@@ -502,6 +495,47 @@ int weight_grad_splits(WeightGrads& g, int cus) {
         if (us < best_us) { best_us = us; best = s; }
     }
     return best;
+}
+
+bool projects(const Projection& p, int cus) {
+    if (!(p.k % 32 == 0 && p.k > 0 && p.n % (p.epilogue == kSwigluFwd ? 16 : 8) == 0 && p.n > 0 && p.m > 0 && p.ldx % 8 == 0 &&
+          p.ldw % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.w & 15) == 0 && p.ldx < (1 << 22) && p.ldw < (1 << 22) &&
+          (int64_t)(p.rows_w ? p.k : p.n) * p.ldw < (INT64_C(1) << 31)))
+        return false;
+    // where a tile of one workgroup a CU is the better one, the gradient of silu(gate) * up is left to a kernel of its own: it reads
+    // and writes 12 bytes per product, which nothing hides there (8192 x 2816, k = 1024: 103 us against 55 + 36)
+    if (p.epilogue == kSwigluBwd) return projection_tile(p, cus) == kTile128;
+    // plain products of four rounds of the largest tile and more (the language model's head): the library's is ahead there, 417 against
+    // 475 us for 8192 x 32000, k = 1024
+    return p.epilogue != kStore || p.rows_w || (int64_t)p.m * p.n < (int64_t)4 * 256 * 256 * cus;
+}
+
+// Time estimates in us of the three kernels (sba_gemm.hip), from k sweeps of 8192 and 4096 rows times 1024 .. 32000 features:
+// rounds of resident workgroups times (time per 64 k, and the part of a tile that does not depend on k).
+//   256 x 256 tiles, one a CU: 1.42 and 5.5, the best rate; 128 x 256, one a CU: 0.78 and 3; 128 x 128, two a CU: 1.15 for both or
+//   0.58 alone, and 3, for what would leave CUs without work (4096 x 1024, k = 1024: 13 against 17 and 26 us).
+// The residual epilogue of the largest tile does not fit its registers.
+ProjectionTile projection_tile(const Projection& p, int cus) {
+    const bool glu = p.epilogue == kSwigluFwd;
+    const int64_t features = glu ? p.n / 2 : p.n;
+    auto tiles = [&](int tm, int tn) { return (((int64_t)p.m + tm - 1) / tm) * ((features + tn - 1) / tn); };
+    const double k64 = p.k / 64.0;
+    const int64_t t2 = tiles(128, glu ? 64 : 128), full = t2 / (2 * cus), rest = t2 % (2 * cus);
+    ProjectionTile best = kTile128;
+    double best_us = full * (1.15 * k64 + 3) + (rest == 0 ? 0 : rest <= cus ? 0.58 * k64 + 3 : 1.15 * k64 + 3) + 2;
+    if (p.k % 64 == 0) {
+        const int own = glu ? 128 : 256;
+        const double t1 = (double)((tiles(128, own) + cus - 1) / cus) * (0.78 * k64 + 3) + 3;
+        if (t1 < best_us) { best = kTile128x256; best_us = t1; }
+        const double t0 = (double)((tiles(256, own) + cus - 1) / cus) * (1.42 * k64 + 5.5) + 1;
+        if (p.epilogue != kAddResidual && t0 < best_us) { best = kTile256; best_us = t0; }
+    }
+    return best;
+}
+
+int project(const Projection& p, bool f16, int cus, hipStream_t s) {
+    const ProjectionTile tile = projection_tile(p, cus);
+    return f16 ? project_f16(p, tile, s) : project_bf16(p, tile, s);
 }
 
 int weight_grads(const WeightGrads& g, int splits, bool f16, hipStream_t s) {

@@ -51,6 +51,15 @@ std::vector<Tensor> cast_weights(at::ArrayRef<Tensor> w, at::IntArrayRef groups,
     return out;
 }
 
+int compute_units() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 256;
+        return n > 0 ? n : 256;
+    }();
+    return cus;
+}
+
 // d_weight = d_out^T . in, in fp32, of several products over the same rows at once
 std::vector<Tensor> weight_grads(std::initializer_list<std::pair<Tensor, Tensor>> pairs) {
     WeightGrads g = {};
@@ -65,12 +74,7 @@ std::vector<Tensor> weight_grads(std::initializer_list<std::pair<Tensor, Tensor>
         g.k = (int)in.size(0);
     }
     const Tensor& like = pairs.begin()->first;
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 256;
-        return n > 0 ? n : 256;
-    }();
-    const int splits = weight_grad_splits(g, cus);
+    const int splits = weight_grad_splits(g, compute_units());
     const Tensor out = empty({g.total}, like, at::kFloat);
     Tensor partial;
     g.out = out.data_ptr<float>();
@@ -85,19 +89,14 @@ std::vector<Tensor> weight_grads(std::initializer_list<std::pair<Tensor, Tensor>
     return r;
 }
 
-struct Norm { Tensor y, rstd, sum; };
-Norm rms_norm(const Tensor& x, const Tensor& h, const Tensor& w, double eps, at::ScalarType t) {
+struct Norm { Tensor y, rstd; };
+Norm rms_norm(const Tensor& x, const Tensor& w, double eps, at::ScalarType t) {
     Norm r;
     const int64_t rows = x.size(0), cols = x.size(1);
     r.y = empty({rows, cols}, x, t);
     r.rstd = empty({rows}, x, at::kFloat);
     NormFwd a = {};
     a.x = x.data_ptr<float>();
-    if (h.defined()) {
-        r.sum = at::empty_like(x);
-        a.h = h.data_ptr();
-        a.sum = r.sum.data_ptr<float>();
-    }
     a.w = w.data_ptr<float>();
     a.y = r.y.data_ptr();
     a.rstd = r.rstd.data_ptr<float>();
@@ -134,6 +133,65 @@ NormGrad rms_norm_grad(const Tensor& dy, const Tensor& x, const Tensor& w, const
     ok(norm_bwd(a, is_f16(dy.scalar_type()), s));
     ok(sum_parts(part.data_ptr<float>(), r.dw.data_ptr<float>(), parts, (int)cols, s));
     return r;
+}
+
+// y = x w^T (rows_w: x w) into `out`, with what sba_model.h's epilogues do on the way; false where the kernels do not take it
+bool try_project(const Tensor& x, const Tensor& w, bool rows_w, int epilogue, const Tensor& residual, const Tensor& pre, const Tensor& out) {
+    Projection p = {};
+    p.x = x.data_ptr();
+    p.w = w.data_ptr();
+    p.ldx = x.stride(0);
+    p.ldw = w.stride(0);
+    p.m = (int)x.size(0);
+    p.k = (int)x.size(1);
+    p.n = (int)w.size(rows_w ? 1 : 0);
+    p.rows_w = rows_w;
+    p.epilogue = epilogue;
+    if (residual.defined()) p.residual = residual.data_ptr<float>();
+    if (pre.defined()) p.pre = pre.data_ptr();
+    p.out = out.data_ptr();
+    if (!projects(p, compute_units())) return false;
+    ok(sba_model::project(p, is_f16(x.scalar_type()), compute_units(), stream_of(x)));
+    return true;
+}
+
+// x w^T for w [n][k], x w for w [k][n]: 16-bit
+Tensor project(const Tensor& x, const Tensor& w, bool rows_w) {
+    Tensor out = empty({x.size(0), w.size(rows_w ? 1 : 0)}, x, x.scalar_type());
+    if (!try_project(x, w, rows_w, kStore, Tensor(), Tensor(), out)) at::mm_out(out, x, rows_w ? w : w.t());
+    return out;
+}
+
+// residual + x w^T: fp32
+Tensor project_add(const Tensor& x, const Tensor& w, const Tensor& residual) {
+    Tensor out = at::empty_like(residual);
+    if (!try_project(x, w, false, kAddResidual, residual, Tensor(), out)) {
+        const Tensor y = project(x, w, false);
+        ok(add_residual(residual.data_ptr<float>(), y.data_ptr(), out.data_ptr<float>(), out.numel(), is_f16(x.scalar_type()), stream_of(x)));
+    }
+    return out;
+}
+
+// silu(x gate^T) * (x up^T) for w = gate rows | up rows; `pre`, if defined, receives the two products
+Tensor project_swiglu(const Tensor& x, const Tensor& w, Tensor& pre, bool keep) {
+    const int64_t rows = x.size(0), width = w.size(0) / 2;
+    Tensor out = empty({rows, width}, x, x.scalar_type());
+    if (keep) pre = empty({rows, 2 * width}, x, x.scalar_type());
+    if (!try_project(x, w, false, kSwigluFwd, Tensor(), pre, out)) {
+        pre = project(x, w, false);
+        ok(swiglu_fwd(pre.data_ptr(), out.data_ptr(), rows, (int)width, is_f16(x.scalar_type()), stream_of(x)));
+    }
+    return out;
+}
+
+// the gradient of gate | up from d, the gradient of what silu(gate) * up was multiplied with: d w, then through the product
+Tensor project_swiglu_grad(const Tensor& d, const Tensor& w, const Tensor& pre) {
+    Tensor out = at::empty_like(pre);
+    if (!try_project(d, w, true, kSwigluBwd, Tensor(), pre, out)) {
+        const Tensor da = project(d, w, true);
+        ok(swiglu_bwd(pre.data_ptr(), da.data_ptr(), out.data_ptr(), d.size(0), (int)w.size(1), is_f16(d.scalar_type()), stream_of(d)));
+    }
+    return out;
 }
 
 Tensor cast_to(const Tensor& x, at::ScalarType t) {
@@ -182,26 +240,20 @@ Tensor block_forward(const BlockShape& s, const Tensor& x, at::ArrayRef<Tensor> 
     const Tensor cast[] = {weights[1], weights[2], weights[3], weights[4], weights[6], weights[7], weights[8]};
     st.w = cast_weights(cast, {3, 1, 2, 1}, s.t);
     const int64_t N = s.B * s.T;
-    auto n1 = rms_norm(x, Tensor(), weights[0], s.eps1, s.t);
+    auto n1 = rms_norm(x, weights[0], s.eps1, s.t);
     st.y1 = n1.y;
     st.rstd1 = n1.rstd;
-    st.qkv = at::mm(st.y1, st.w[0].t());
+    st.qkv = project(st.y1, st.w[0], false);
     Problem pr = problem_of(s, st.qkv);
     st.o = empty({N, s.hidden}, x, s.t);
     Tensor rem = s.plan ? empty({s.heads, s.T}, x, s.t) : empty({s.B, s.heads, s.T}, x, s.t);
     st.tables = attention_forward(pr, heads_of(s, st.o), rem, train);
-    Tensor h = at::mm(st.o, st.w[1].t());
-    auto n2 = rms_norm(x, h, weights[5], s.eps2, s.t);
-    st.x1 = n2.sum;
+    st.x1 = project_add(st.o, st.w[1], x);
+    auto n2 = rms_norm(st.x1, weights[5], s.eps2, s.t);
     st.y2 = n2.y;
     st.rstd2 = n2.rstd;
-    st.gu = at::mm(st.y2, st.w[2].t());
-    st.a = empty({N, s.width}, x, s.t);
-    ok(swiglu_fwd(st.gu.data_ptr(), st.a.data_ptr(), N, (int)s.width, is_f16(s.t), stream_of(x)));
-    Tensor m = at::mm(st.a, st.w[3].t());
-    Tensor out = at::empty_like(x);
-    ok(add_residual(st.x1.data_ptr<float>(), m.data_ptr(), out.data_ptr<float>(), x.numel(), is_f16(s.t), stream_of(x)));
-    return out;
+    st.a = project_swiglu(st.y2, st.w[2], st.gu, train);
+    return project_add(st.a, st.w[3], st.x1);
 }
 
 struct Block : torch::autograd::Function<Block> {
@@ -234,19 +286,17 @@ struct Block : torch::autograd::Function<Block> {
         const Tensor dx2 = grads[0].contiguous().view({N, s.hidden});
 
         const Tensor dm = cast_to(dx2, s.t);
-        const Tensor da = at::mm(dm, w_d);
-        const Tensor dgu = at::empty_like(gu);
-        ok(swiglu_bwd(gu.data_ptr(), da.data_ptr(), dgu.data_ptr(), N, (int)s.width, is_f16(s.t), stream_of(x)));
-        const Tensor dy2 = at::mm(dgu, w_gu);
+        const Tensor dgu = project_swiglu_grad(dm, w_d, gu);
+        const Tensor dy2 = project(dgu, w_gu, true);
         auto g2 = rms_norm_grad(dy2, x1, n2, rstd2, dx2, true);
-        const Tensor d_o = at::mm(g2.dx16, w_o);
+        const Tensor d_o = project(g2.dx16, w_o, true);
         const Tensor dqkv = at::empty_like(qkv);
         {
             Problem pr = problem_of(s, qkv);
             const Problem g = problem_of(s, dqkv);
             attention_backward(pr, tables, heads_of(s, d_o), Tensor(), g.q, g.k, g.v);
         }
-        const Tensor dy1 = at::mm(dqkv, w_qkv);
+        const Tensor dy1 = project(dqkv, w_qkv, true);
         const auto dw = weight_grads({{dqkv, y1}, {g2.dx16, o}, {dgu, y2}, {dm, a}});
         const Tensor &dwqkv = dw[0], &dwo = dw[1], &dwgu = dw[2], &dwd = dw[3];
         auto g1 = rms_norm_grad(dy1, x, n1, rstd1, g2.dx, false);
@@ -289,9 +339,9 @@ Tensor block(const Tensor& x, const std::vector<Tensor>& w, int64_t heads, doubl
 struct Head : torch::autograd::Function<Head> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& n, const Tensor& w, double eps, at::ScalarType t) {
         const Tensor x = x_in.contiguous().view({-1, x_in.size(-1)});
-        auto r = rms_norm(x, Tensor(), n, eps, t);
+        auto r = rms_norm(x, n, eps, t);
         const Tensor w16 = cast_to(w, t);
-        Tensor logits = at::mm(r.y, w16.t());
+        Tensor logits = project(r.y, w16, false);
         ctx->save_for_backward({x, n, r.y, r.rstd, w16});
         auto sizes = x_in.sizes().vec();
         sizes.back() = w.size(0);
@@ -301,7 +351,7 @@ struct Head : torch::autograd::Function<Head> {
         const auto sv = ctx->get_saved_variables();
         c10::DeviceGuard guard(sv[0].device());
         const Tensor d = grads[0].contiguous().view({-1, grads[0].size(-1)});
-        const Tensor dy = at::mm(d, sv[4]);
+        const Tensor dy = project(d, sv[4], true);
         const Tensor dw = weight_grads({{d, sv[2]}})[0];
         auto g = rms_norm_grad(dy, sv[0], sv[1], sv[3], Tensor(), false);
         auto sizes = grads[0].sizes().vec();
@@ -318,10 +368,10 @@ Tensor head(const Tensor& x, const Tensor& n, const Tensor& w, double eps, py::o
         return Head::apply(x, n, w, eps, t);
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor rows = x.contiguous().view({-1, x.size(-1)});
-    auto r = rms_norm(rows, Tensor(), n, eps, t);
+    auto r = rms_norm(rows, n, eps, t);
     auto sizes = x.sizes().vec();
     sizes.back() = w.size(0);
-    return at::mm(r.y, cast_to(w, t).t()).view(sizes);
+    return project(r.y, cast_to(w, t), false).view(sizes);
 }
 
 struct LossRows { Tensor mean, count, lse; };
@@ -421,6 +471,14 @@ void bind_model(py::module& m) {
     m.def("head", &head);
     m.def("next_token_loss", &next_token_loss);
     m.def("clip_and_step", &clip_and_step);
+    m.def("project", &project);
+    m.def("project_add", &project_add);
+    m.def("project_swiglu", [](const Tensor& x, const Tensor& w) {
+        Tensor pre;
+        const Tensor out = project_swiglu(x, w, pre, true);
+        return std::make_pair(out, pre);
+    });
+    m.def("project_swiglu_grad", &project_swiglu_grad);
     m.attr("max_norm_width") = kMaxNormWidth;
 }
 
