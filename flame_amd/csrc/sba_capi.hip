@@ -65,6 +65,13 @@ size_t generic_acc_bytes(const SbaParams* p) {
     return (b + 255) & ~(size_t)255;
 }
 
+// SBA_FULL_SWEEPS=1: every sweep evaluates all pairs of the causal triangle, also those whose weights are exactly 0 (for
+// measurements that are quoted against the triangle's operations, and to compare results)
+bool full_sweeps() {
+    const char* e = getenv("SBA_FULL_SWEEPS");
+    return e && e[0] == '1';
+}
+
 constexpr size_t kErrorWordBytes = 256;     // tail of the bf16 matrix-core backward's scratch: the error word
 
 // Carry tables of the matrix-core path.  bf16, four in all: the forward writes two - the product of (1 - beta)
@@ -127,6 +134,7 @@ KParams make_kparams(const SbaParams* p) {
     kp.cols = p->columns ? p->columns : p->head_dim;
     kp.attend_current = p->attend_current ? 1 : 0;
     kp.save = p->save_for_backward ? 1 : 0;
+    kp.early_end = full_sweeps() ? 0 : 1;
     kp.scale = p->scale; kp.scale2 = p->scale * sba::kLog2e;
     kp.cu_seqlens = p->cu_seqlens; kp.schedule = p->schedule;
     if (p->cu_seqlens) {

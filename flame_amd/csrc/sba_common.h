@@ -43,6 +43,7 @@ struct KParams {
                                    //   the key-owner stream kernel (ptr NULL: not wanted)
     float* dkv32;                  // generic path: fp32 dk|dv accumulators
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)
+    int early_end;                 // forward sweeps end once nothing is left of any of their rows' sticks
     int* gave_up;                  // backward error word (set if a kernel abandoned a bounded internal wait)
     int64_t tab_head_stride;       // floats per head in each carry table
     int64_t tab_tokens;            // generic path: tokens per head in the fp32 accumulators (n_seq*T dense, sumT packed)
@@ -51,11 +52,19 @@ struct KParams {
 // tab0: first carry-table column of the job's sequence
 struct Job { int tok0, len, rb, seq, tab0; };
 
-// Workgroup -> (job, head).  blockIdx.x = slot * n_heads + head, so that consecutive
-// workgroups (which the dispatcher deals round-robin to the 8 XCDs) are different heads of
-// the same job and a head stays on one XCD's L2.  Jobs are sorted by decreasing sweep
+// Workgroup -> (job, head).  A slot of n_heads consecutive workgroups (which the dispatcher deals round-robin to the 8 XCDs) is
+// one job of every head.  Which head comes first moves on by one from slot to slot in the dense layout and every eighth slot
+// in the packed one: heads differ in how far their sweeps reach, and a head that stayed on one XCD (which is best for the
+// XCD's L2 if all sweeps are full: 6 % at B=1, H=16, T=16384, d=128 with every eighth slot, 12 % with every slot) makes that
+// XCD the last to finish, and the others wait for it, since workgroups are dealt in order.  Mean logits 0 .. -6 over 16 heads,
+// forward + backward: T=16384, d=128 4.92 ms with fixed heads, 4.35 moving every eighth slot, 3.55 every slot; packs of
+// 65536 tokens d=64 1.74 / 1.66 / 1.71, 20011 tokens d=80 472 / 458 / 476 us.  Jobs are sorted by decreasing sweep
 // length (longest first); `longest_last` walks the list from its other end (the key-owner
 // pass, whose work grows as the row-block index falls).
+__device__ inline int head_of_block(const KParams& p, int block) {
+    const int slot = block / p.n_heads;
+    return (block - slot * p.n_heads + (p.cu_seqlens ? slot >> 3 : slot)) % p.n_heads;
+}
 __device__ inline int order_job(int slot, int n_jobs, bool longest_last) {
     return longest_last ? n_jobs - 1 - slot : slot;
 }
@@ -119,6 +128,48 @@ __device__ inline int64_t tab_token(const KParams& p, const Job& j, int local) {
 // Returns the index of (row block qb, key block kb, query 0 of the row block).
 __device__ inline int64_t tab_index(const KParams& p, int head, const Job& j, int qb, int kb) {
     return (int64_t)head * p.tab_head_stride + ((int64_t)j.tab0 + qb * (qb + 1) + kb) * kRowBlock;
+}
+
+// Where a sweep ends.  A row whose product of (1 - beta) has become exactly 0 gives every key further left the weight 0, the
+// logit gradient 0 and leaves no remainder, so a sweep in which that holds for all of its rows ends there: nothing that
+// follows could change a bit of any result.  The forward records the leftmost key block it reached per row block
+// ("first live block"); the dQ pass starts its sweep there, and leaves for every row block of keys the last row block of
+// queries whose sweep reached it ("last live row block"), where the key-owner sweeps end.  Table entries left of a row block's
+// first live block exist only where a key-owner sweep passes over them, as zeros that the dQ pass fills in.
+// Both numbers live in the tables: the first 64 rows of a row block never see its last key block, so that column's first
+// entry belongs to nobody, in rtab as in gtab.
+typedef const __attribute__((address_space(4))) int32_t* UniformInts;       // read-only in the kernel: scalar loads
+__device__ inline int64_t live_index(const KParams& p, int head, const Job& j, int rb) { return tab_index(p, head, j, rb, 2 * rb + 1); }
+__device__ inline void set_first_live(const KParams& p, int head, const Job& j, int kb) {
+    ((int32_t*)p.rtab)[live_index(p, head, j, j.rb)] = kb;
+}
+__device__ inline int first_live_block(const KParams& p, int head, const Job& j) {
+    return ((UniformInts)(uintptr_t)p.rtab)[live_index(p, head, j, j.rb)];
+}
+__device__ inline int last_live_row_block(const KParams& p, int head, const Job& j) {
+    return ((UniformInts)(uintptr_t)p.gtab)[live_index(p, head, j, j.rb)];
+}
+// What one wave of a dQ workgroup does for its row block, whose own sweep starts at key block s0: the last live row block of
+// the keys of the same number, and zeros in the entries that key-owner sweeps read although this row block's sweep did not
+// reach them (those of later row blocks reach further left: between the lowest of their first blocks and s0).
+__device__ inline void close_live_ranges(const KParams& p, int head, const Job& j, int lane, int s0) {
+    const int n_rb = (j.len + kRowBlock - 1) / kRowBlock;
+    int lowest = s0, last = j.rb;
+    for (int at = j.rb + 1; at < n_rb; at += 64) {
+        const int f = at + lane < n_rb ? ((const int32_t*)p.rtab)[live_index(p, head, j, at + lane)] : INT32_MAX;
+        lowest = min(lowest, f);
+        const uint64_t reach = __builtin_amdgcn_ballot_w64((f >> 1) <= j.rb);
+        if (reach) last = at + 63 - __builtin_clzll(reach);
+    }
+    if (lane == 0) ((int32_t*)p.gtab)[live_index(p, head, j, j.rb)] = last;
+    if (s0 == 0) return;
+    for (int d = 32; d; d >>= 1) lowest = min(lowest, __shfl_xor(lowest, d));
+    const int64_t at = tab_index(p, head, j, j.rb, 0);
+    for (int i = (lowest & ~1) * kRowBlock + lane; i < s0 * kRowBlock; i += 64) {       // (pairs of key blocks end their sweeps together)
+        p.rtab[at + i] = 0.f;
+        p.gtab[at + i] = 0.f;
+        if (p.rmid) { p.rmid[at + i] = 0.f; p.gmid[at + i] = 0.f; }
+    }
 }
 
 __device__ inline float bf16_to_f32(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }

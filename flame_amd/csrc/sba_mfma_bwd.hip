@@ -58,7 +58,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     LaneOffsets<D> lo;
     lo.init(lane);
     lo.rebase(lds);                        // absolute addresses: the loop below runs in one copy per tile buffer
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
@@ -84,6 +84,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     const int imax = min(m0 + kRowBlock - 1, job.len - 1);
     const int kmax = imax - strict;
     const int n_steps = kmax >= 0 ? kmax / kKeyBlock + 1 : 0;
+    const int first = first_live_block(p, head, job);      // the sweep's first step, see live_index()
 
     TileDma<D, false, D == 64 && kLean> kc, vc;
     kc.init(lane, wave, p.k, kbase, p.cols);
@@ -94,9 +95,10 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
         vc.clear(lds + b * 2 * kTile + kTile);
     }
     if (n_steps > 0) {
-        kc.issue(0, job.len, lds);
-        vc.issue(0, job.len, lds + kTile);
+        kc.issue(first * kKeyBlock, job.len, lds);
+        vc.issue(first * kKeyBlock, job.len, lds + kTile);
     }
+    if (wave == 3) close_live_ranges(p, head, job, lane, first);
 
     // carry-table traffic is kept off the critical path: the value of the NEXT step is loaded
     // while this one is computed, and this step's prefix is stored before the tile loads are
@@ -106,7 +108,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     // the same 32 keys goes to the same entry of gmid / gtab, which lies the same distance from the cursor for
     // both half-waves (gmid - rtab == gtab - rmid: the library lays the tables out that way).
     constexpr int64_t tstride = kRowBlock;
-    const float* rcur = (h ? p.rtab : p.rmid) + tab_index(p, head, job, job.rb, 0) + 32 * wave + n;
+    const float* rcur = (h ? p.rtab : p.rmid) + tab_index(p, head, job, job.rb, first) + 32 * wave + n;
     const int64_t g_from_r = (const char*)p.gtab - (const char*)p.rmid;
     float Rnext = (row_ok && n_steps > 0) ? *rcur : 1.0f;
     float Gstore = 0.f;
@@ -149,7 +151,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
                 if (key0 + 63 + strict > q0w) mask_step(x, key0 + 32 * h, qi, strict);
                 float gsum;
                 const float Lend = carried_beta_g(x, dp, F, gsum);
-                if (step == 0) {                         // the gradient of rem rides in the prefix, see below
+                if (step == 0) {                         // the gradient of rem rides in the prefix, see below (further right: no remainder)
                     float Llo, Lup;
                     half_values(Lend, Llo, Lup);
                     Gc = dr * Llo;                       // what leaves the left half of the leftmost block is rem
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
         wait_global_memory();                  // the next tiles have landed
         __syncthreads();
     };
-    for (int step = 0; step < n_steps; step += 2) {
+    for (int step = first; step < n_steps; step += 2) {
         do_step(step, std::integral_constant<int, 0>{});
         if (step + 1 < n_steps) do_step(step + 1, std::integral_constant<int, 1>{});
     }
@@ -250,7 +252,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dq2_kernel(KParams p
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
@@ -276,24 +278,28 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dq2_kernel(KParams p
     const int imax = min(m0 + kRowBlock - 1, job.len - 1);
     const int kmax = imax - strict;
     const int n_steps = kmax >= 0 ? kmax / kKeyBlock + 1 : 0;
-    const int n_it = (n_steps + 1) / 2;
+    // the sweep's first step (see live_index()), from the even step on: pairs of steps stay the same pairs wherever a sweep begins
+    const int live = first_live_block(p, head, job), first = live & ~1;
+    const int n_it = (n_steps - first + 1) / 2;
     char* my_tiles = lds + grp * 2 * kTile;          // + buf * 4 * kTile
 
     // each group copies its own tiles (256 threads per tile pair)
     TileDma<D> kc, vc;
     kc.init(lane, qs, p.k, kbase);
     vc.init(lane, qs, p.v, vbase);
-    if (grp < n_steps) {
-        kc.issue(grp * kKeyBlock, job.len, my_tiles);
-        vc.issue(grp * kKeyBlock, job.len, my_tiles + kTile);
+    if (first + grp < n_steps) {
+        kc.issue((first + grp) * kKeyBlock, job.len, my_tiles);
+        vc.issue((first + grp) * kKeyBlock, job.len, my_tiles + kTile);
     }
+    if (wave == 7) close_live_ranges(p, head, job, lane, live);
 
     // the forward's carry for this group's NEXT step is loaded while this one is computed
     constexpr int64_t tstride = kRowBlock;
     // this lane's cursor into the carry tables and the distance to its prefix entry, see the one-step kernel
-    const float* rcur = (h ? p.rtab : p.rmid) + tab_index(p, head, job, job.rb, 0) + 32 * qs + n + grp * tstride;
+    const float* rcur = (h ? p.rtab : p.rmid) + tab_index(p, head, job, job.rb, first) + 32 * qs + n + grp * tstride;
     const int64_t g_from_r = (const char*)p.gtab - (const char*)p.rmid;
-    float Rnext = (row_ok && grp < n_steps) ? *rcur : 1.0f;
+    float Rnext = (row_ok && first + grp < n_steps) ? *rcur : 1.0f;
+    if (first + grp < live) Rnext = 0.f;             // (no entry)
     float Gstore = 0.f;
     bool g_pending = false;
     // (last of the prologue's loads: its conversion waits for it, and with it for everything requested before)
@@ -310,7 +316,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dq2_kernel(KParams p
         constexpr int buf = decltype(buf_c)::value;
         constexpr TileAt ktile = {buf * 4 * kTile};
         constexpr TileAt vtile = {buf * 4 * kTile + kTile};
-        const int step = 2 * it + grp;                   // == n_steps: this group idles in the last iteration
+        const int step = first + 2 * it + grp;           // == n_steps: this group idles in the last iteration
         const bool more = step + 2 < n_steps;
         const int key0 = step * kKeyBlock;
         const bool active = step < n_steps && !(key0 + strict > q0w + 31) && q0w < job.len;
@@ -438,7 +444,7 @@ __global__ __launch_bounds__(kThreads, 2) void mfma_bwd_dkv_kernel(KParams p) {
     lo.init(lane);
     LaneOffsets<64> lz;                        // the weight tiles have 64-key rows whatever D is
     lz.init(lane);
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const int slot = blockIdx.x / p.n_heads;   // two 64-key blocks per scheduled 128-row job
     const Job job = decode_key_job(p, slot >> 1);
     const int kb = 2 * job.rb + (slot & 1);
@@ -449,7 +455,7 @@ __global__ __launch_bounds__(kThreads, 2) void mfma_bwd_dkv_kernel(KParams p) {
     const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
     const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
     const int64_t dobase = (int64_t)job.seq * p.d_o.sb + (int64_t)head * p.d_o.sh + (int64_t)job.tok0 * p.d_o.st;
-    const int n_qb = (job.len + kRowBlock - 1) / kRowBlock;
+    const int n_qb = last_live_row_block(p, head, job) + 1;
     const int kh = wave & 1;                   // which 32 keys this wave reduces
     const int dbw = wave >> 1;                 // and which d-blocks: dbw + 2*i
     // lane offsets of this wave's operand columns, picked once (no run-time table indexing)
@@ -645,12 +651,12 @@ __device__ inline KeyItem decode_item(const KParams& p, int idx) {
     KeyItem r;
     r.valid = idx >= 0;
     if (idx < 0) idx = 0;
-    r.head = idx % p.n_heads;
+    r.head = head_of_block(p, idx);
     const int slot = idx / p.n_heads;          // two 64-key blocks per scheduled 128-row job
     r.job = decode_key_job(p, slot >> 1);
     r.kb = 2 * r.job.rb + (slot & 1);
     r.key0 = r.kb * kKeyBlock;
-    r.n_steps = (r.job.len + kRowBlock - 1) / kRowBlock - r.job.rb;
+    r.n_steps = last_live_row_block(p, r.head, r.job) + 1 - r.job.rb;
     return r;
 }
 
@@ -1189,7 +1195,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
     lo.init(lane);
     LaneOffsets<64> lz;
     lz.init(lane);
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_key_job(p, blockIdx.x / p.n_heads);
     const int strict = p.attend_current ? 0 : 1;
     const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it
@@ -1216,7 +1222,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
 #pragma unroll
     for (int db = 0; db < kNB; ++db) { dkacc[db] = f32x16{0}; dvacc[db] = f32x16{0}; }
 
-    const int n_steps = q_begin < job.len ? (job.len - q_begin + kStep - 1) / kStep : 0;
+    const int n_steps = min((job.len - q_begin + kStep - 1) / kStep, 2 * (last_live_row_block(p, head, job) + 1 - job.rb));
 
     TileDma<D, true> qc, dc;
     qc.init(lane, wave, p.q, qbase);
@@ -1468,7 +1474,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_job(p, blockIdx.x / p.n_heads);
     if (blockIdx.x == 0 && threadIdx.x == 0 && p.gave_up) *p.gave_up = 0;
     LaneOffsets<D> lo;
@@ -1665,7 +1671,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
     lo.init(lane);
     LaneOffsets<64> lz;
     lz.init(lane);
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_key_job(p, blockIdx.x / p.n_heads);
     const int strict = p.attend_current ? 0 : 1;
     const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it
@@ -1691,7 +1697,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
 #pragma unroll
     for (int j = 0; j < kBlocks; ++j) { dkacc[j] = f32x16{0}; dvacc[j] = f32x16{0}; }
 
-    const int n_steps = q_begin < job.len ? (job.len - q_begin + kStep - 1) / kStep : 0;
+    const int n_steps = min((job.len - q_begin + kStep - 1) / kStep, 2 * (last_live_row_block(p, head, job) + 1 - job.rb));
 
     // waves 0-3 copy the Q tiles, waves 4-7 the dO tiles
     TileDma<D, true> tc;

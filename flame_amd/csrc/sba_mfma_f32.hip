@@ -133,10 +133,11 @@ __global__ __launch_bounds__(kThreads) void fwd_kernel(KParams p) {
     constexpr int SD = row_stride<D>();
     __shared__ __attribute__((aligned(16))) float ktile[64 * SD];
     __shared__ __attribute__((aligned(16))) float vT[D * SK];
+    __shared__ int done_waves[4];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock, q0w = m0 + 32 * wave, qi = q0w + n;
@@ -149,30 +150,40 @@ __global__ __launch_bounds__(kThreads) void fwd_kernel(KParams p) {
     f32x16 oacc[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) oacc[db] = f32x16{0};
-    float R = 1.0f;
+    float R = qi < job.len ? 1.0f : 0.0f;
+    bool done = q0w >= job.len;                // nothing (left) of this wave's rows' sticks, see live_index()
+    if (lane == 0) done_waves[wave] = done;
     const int imax = min(m0 + kRowBlock - 1, job.len - 1);
     const int kmax = imax - strict;
     const int n_steps = kmax >= 0 ? kmax / kKeyBlock + 1 : 0;
     const int64_t tabq = tab_index(p, head, job, job.rb, 0) + 32 * wave + n;
 
-    for (int step = n_steps - 1; step >= 0; --step) {
+    int step = n_steps - 1;
+    for (; step >= 0; --step) {
         const int key0 = step * kKeyBlock;
         TileRegs<64, D> kr, vr;
         kr.load(p.k, kbase, key0, job.len);
         if (!kCarryOnly) vr.load(p.v, vbase, key0, job.len);
         __syncthreads();                       // the previous step's tiles have been read
+        if (done && __builtin_amdgcn_readfirstlane(done_waves[0] & done_waves[1] & done_waves[2] & done_waves[3])) break;      // (the same in all waves)
         kr.store_natural(ktile);
         if (!kCarryOnly) vr.store_transposed(vT);
         __syncthreads();
         if (key0 + strict > q0w + 31) continue;           // whole step right of this wave's last query (uniform per wave)
         if (p.save && h == 0 && qi < job.len) p.rtab[tabq + step * kRowBlock] = R;
+        if (done) continue;
         float x[32];
         head_dim_product<D>(x, ktile, qf, lane);
         if (key0 + 63 + strict > q0w) mask_step(x, key0 + 32 * h, qi, strict);
         float dummy[1];
         stick_weights<false>(x, dummy, R, lane);
         if (!kCarryOnly) key_product<D>(oacc, vT, x, lane);
+        if (__builtin_amdgcn_ballot_w64(R != 0.f) == 0 && p.early_end) {
+            done = true;
+            if (lane == 0) done_waves[wave] = 1;
+        }
     }
+    if (p.save && threadIdx.x == 0) set_first_live(p, head, job, step + 1);
     if (qi < job.len && !kCarryOnly) {
         store_query_row<D>(p.o, (int64_t)job.seq * p.o.sb + (int64_t)head * p.o.sh + (int64_t)job.tok0 * p.o.st, qi, lane, oacc, 1.0f);
         if (h == 0) ((float*)p.rem.ptr)[(int64_t)job.seq * p.rem.sb + (int64_t)head * p.rem.sh + job.tok0 + qi] = R;
@@ -189,7 +200,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dq_kernel(KParams p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock, q0w = m0 + 32 * wave, qi = q0w + n;
@@ -213,8 +224,10 @@ __global__ __launch_bounds__(kThreads) void bwd_dq_kernel(KParams p) {
     const int kmax = imax - strict;
     const int n_steps = kmax >= 0 ? kmax / kKeyBlock + 1 : 0;
     const int64_t tix0 = tab_index(p, head, job, job.rb, 0) + 32 * wave + n;
+    const int first = first_live_block(p, head, job);
+    if (wave == 3) close_live_ranges(p, head, job, lane, first);
 
-    for (int step = 0; step < n_steps; ++step) {
+    for (int step = first; step < n_steps; ++step) {
         const int key0 = step * kKeyBlock;
         TileRegs<64, D> kr, vr;
         kr.load(p.k, kbase, key0, job.len);
@@ -263,7 +276,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(KParams p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const int slot = blockIdx.x / p.n_heads;   // two 64-key blocks per scheduled 128-row job
     const Job job = decode_key_job(p, slot >> 1);
     const int kb = 2 * job.rb + (slot & 1);
@@ -287,7 +300,7 @@ __global__ __launch_bounds__(kThreads) void bwd_dkv_kernel(KParams p) {
     f32x16 dkacc[kMine], dvacc[kMine];
 #pragma unroll
     for (int j = 0; j < kMine; ++j) { dkacc[j] = f32x16{0}; dvacc[j] = f32x16{0}; }
-    const int n_qb = (job.len + kRowBlock - 1) / kRowBlock;
+    const int n_qb = last_live_row_block(p, head, job) + 1;
     for (int qb = job.rb; qb < n_qb; ++qb) {
         const int q0w = qb * kRowBlock + 32 * wave, qi = q0w + n;
         float qf[D / 2], dof[D / 2];

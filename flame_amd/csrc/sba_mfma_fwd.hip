@@ -76,14 +76,15 @@ __device__ inline void store_o_row(const KParams& p, const Job& job, int head, i
 template <int D, bool kCarryOnly>
 __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     constexpr int kTile = 64 * kPitch<D> * 2;            // bytes per K or V tile
-    __shared__ __attribute__((aligned(16))) char lds[4 * kTile];   // K0 V0 K1 V1
+    __shared__ __attribute__((aligned(16))) char lds[4 * kTile + (kCarryOnly ? 0 : 32)];   // K0 V0 K1 V1 | words
+    int (*const done_waves)[4] = (int (*)[4])(lds + (kCarryOnly ? kTile : 4 * kTile));     // [parity of the step][wave]
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform, keep it scalar
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
@@ -101,7 +102,10 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     f32x16 oacc[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) oacc[db] = f32x16{0};
-    float R = 1.0f;
+    float R = qi < job.len ? 1.0f : 0.0f;
+    // This wave has no more weights to give: its rows' carries are exactly 0, or it has no rows at all.
+    bool done = q0w >= job.len;
+    if (threadIdx.x < 8) done_waves[threadIdx.x >> 2][threadIdx.x & 3] = 0;
 
     const int imax = min(m0 + kRowBlock - 1, job.len - 1);
     const int kmax = imax - strict;                       // last key any row of the block sees
@@ -139,7 +143,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
         carry_step = -1;
     };
     // what a step does before its arithmetic
-    auto open_step = [&](int step, int buf, bool skip) {
+    auto open_step = [&](int step, int buf) {
         store_carries();
         if (step > 0) {   // next tiles, straight into the other buffer (free since the last barrier);
                           // every tile left of the sweep's first lies inside the sequence
@@ -150,14 +154,35 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     // The sweep runs with the one-reciprocal chain until a step refuses it (logits too large for
     // it); from that step on this wave continues with the reciprocal-per-key chain.  Every wave
     // executes one barrier per step whichever loop it is in.
-    int step = n_steps - 1, buf = 0;
+    // A wave that is done only copies its share of the tiles and enters zero carries; the sweep ends after the step in which the
+    // last of the four is done (live_index() says why).  A wave with work left pays one comparison per step for this: only a
+    // wave that is done looks at what the others have said.  Their words are kept by parity of the step, so that none can
+    // be about a later one; they are never taken back.
+    const float nothing = p.early_end ? 0.f : -1.f;
+    // (the number of iterations is a variable of the loops' only exit: with a break of its own the accumulators would meet copies
+    // of themselves behind the loops, 32 registers more)
+    int it = 0, iterations = n_steps;
+    auto close_step = [&](int step, int buf) {
+        wait_global_memory();                  // the next tiles have landed
+        if (__builtin_amdgcn_ballot_w64(R != nothing) != 0) {
+            __syncthreads();
+            return;
+        }
+        done = true;
+        if (q0w < job.len && carry_step < 0) { carry_out = 0.f; carry_step = step; }
+        if (lane == 0) done_waves[buf][wave] = 1;
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(done_waves[buf][0] & done_waves[buf][1] & done_waves[buf][2] & done_waves[buf][3])) iterations = it + 1;
+    };
+    int buf = 0;
     bool redo = false;
-    for (; step >= 0; --step, buf ^= 1) {
+    for (; it < iterations; ++it, buf ^= 1) {
+        const int step = n_steps - 1 - it;
         const char* ktile = lds + buf * 2 * kTile;
         const int key0 = step * kKeyBlock;
         // whole step right of this wave's last query, or all of this wave's queries past the end of the sequence
-        const bool skip = key0 + strict > q0w + 31 || q0w >= job.len;
-        open_step(step, buf, skip);
+        const bool skip = key0 + strict > q0w + 31 || done;
+        open_step(step, buf);
         if (!skip) {
             if (!fwd_step<D, kCarryOnly, true, kWide<D>>(ktile, ktile + kTile, lo, qf, oacc, R, lane, key0, q0w, qi, strict, carry_out)) {
                 redo = true;
@@ -165,23 +190,23 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
             }
             carry_step = step;
         }
-        wait_global_memory();                  // the next tiles have landed
-        __syncthreads();
+        close_step(step, buf);
     }
-    for (; step >= 0; --step, buf ^= 1) {
+    for (; it < iterations; ++it, buf ^= 1) {
+        const int step = n_steps - 1 - it;
         const char* ktile = lds + buf * 2 * kTile;
         const int key0 = step * kKeyBlock;
-        const bool skip = key0 + strict > q0w + 31 || q0w >= job.len;
-        if (!redo) open_step(step, buf, skip);
+        const bool skip = key0 + strict > q0w + 31 || done;
+        if (!redo) open_step(step, buf);
         redo = false;
         if (!skip) {
             fwd_step<D, kCarryOnly, false, kWide<D>>(ktile, ktile + kTile, lo, qf, oacc, R, lane, key0, q0w, qi, strict, carry_out);
             carry_step = step;
         }
-        wait_global_memory();
-        __syncthreads();
+        close_step(step, buf);
     }
     store_carries();
+    if (p.save && threadIdx.x == 0) set_first_live(p, head, job, n_steps - iterations);
 
     if (qi < job.len && !kCarryOnly) {
         store_o_row<D>(p, job, head, qi, lane, oacc);
@@ -207,6 +232,8 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     // tile(grp, buf, kv) = lds + ((grp * 2 + buf) * 2 + kv) * kTile
     __shared__ __attribute__((aligned(16))) char lds[G * 4 * kTile];
     __shared__ float totals[G][kRowBlock];
+    __shared__ int done_waves[2][4 * G];
+    __shared__ int first_live;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -214,7 +241,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
-    const int head = blockIdx.x % p.n_heads;
+    const int head = head_of_block(p, blockIdx.x);
     const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
@@ -231,7 +258,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     f32x16 oacc[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) oacc[db] = f32x16{0};
-    float R = 1.0f;
+    float R = qi < job.len ? 1.0f : 0.0f;
 
     const int imax = min(m0 + kRowBlock - 1, job.len - 1);
     const int kmax = imax - strict;
@@ -254,6 +281,13 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
         kc.issue((hi - 1) * kKeyBlock, job.len, my_tiles);
         if (!kCarryOnly) vc.issue((hi - 1) * kKeyBlock, job.len, my_tiles + kTile);
     }
+    // A segment ends early as the sweep of mfma_fwd_kernel does, once its own product is exactly 0 for all rows; the workgroup's
+    // loop ends when every wave is done or at the end of its segment.
+    bool done = q0w >= job.len, group_done = false;
+    int reached = low;                                     // leftmost step for which this wave had weights to give
+    const float nothing = p.early_end ? 0.f : -1.f;
+    if (threadIdx.x < 8 * G) done_waves[threadIdx.x / (4 * G)][threadIdx.x % (4 * G)] = 0;
+    if (threadIdx.x == 0) first_live = n_steps;
     wait_global_memory();
     __syncthreads();
 
@@ -269,21 +303,42 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
         }
         carry_step = -1;
     };
-    auto open_step = [&](int step, int buf, bool skip) {
+    auto open_step = [&](int step, int buf) {
         store_carries();
-        if (step - 1 >= low) {
+        if (step - 1 >= low && !group_done) {
             kc.issue_full((step - 1) * kKeyBlock, my_tiles + (buf ^ 1) * 2 * kTile);
             if (!kCarryOnly) vc.issue_full((step - 1) * kKeyBlock, my_tiles + (buf ^ 1) * 2 * kTile + kTile);
         }
     };
-    int it = 0, buf = 0;
+    int it = 0, iterations = chunk;
+    auto close_step = [&](int step, int buf) {
+        wait_global_memory();
+        if (__builtin_amdgcn_ballot_w64(R != nothing) != 0 && step > low) {
+            __syncthreads();
+            return;
+        }
+        // nothing more to come from this wave: at the end of its segment, or done
+        if (__builtin_amdgcn_ballot_w64(R != nothing) == 0) {
+            if (!done) reached = max(step, low);
+            done = true;
+            if (step >= low && q0w < job.len && !group_done && carry_step < 0) { carry_out = 0.f; carry_step = step; }
+        }
+        if (lane == 0) done_waves[buf][wave] = done ? 1 : 2;
+        __syncthreads();
+        // one lane per wave's word
+        const int said = done_waves[buf][lane % (4 * G)];
+        const uint64_t group = UINT64_C(0xf) << (4 * grp);
+        if ((__builtin_amdgcn_ballot_w64(said == 1) & group) == group) group_done = true;
+        if (__builtin_amdgcn_ballot_w64(said == 0) == 0) iterations = it + 1;
+    };
+    int buf = 0;
     bool redo = false;
-    for (; it < chunk; ++it, buf ^= 1) {
+    for (; it < iterations; ++it, buf ^= 1) {
         const int step = hi - 1 - it;
         const char* ktile = my_tiles + buf * 2 * kTile;
         const int key0 = step * kKeyBlock;
-        const bool skip = step < low || key0 + strict > q0w + 31;
-        open_step(step, buf, skip);
+        const bool skip = step < low || key0 + strict > q0w + 31 || done;
+        open_step(step, buf);
         if (!skip) {
             if (!fwd_step<D, kCarryOnly, true, true>(ktile, ktile + kTile, lo, qf, oacc, R, lane, key0, q0w, qi, strict, carry_out)) {
                 redo = true;
@@ -291,22 +346,20 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
             }
             carry_step = step;
         }
-        wait_global_memory();
-        __syncthreads();
+        close_step(step, buf);
     }
-    for (; it < chunk; ++it, buf ^= 1) {       // reciprocal-per-key chain from the refused step on
+    for (; it < iterations; ++it, buf ^= 1) {       // reciprocal-per-key chain from the refused step on
         const int step = hi - 1 - it;
         const char* ktile = my_tiles + buf * 2 * kTile;
         const int key0 = step * kKeyBlock;
-        const bool skip = step < low || key0 + strict > q0w + 31;
-        if (!redo) open_step(step, buf, skip);
+        const bool skip = step < low || key0 + strict > q0w + 31 || done;
+        if (!redo) open_step(step, buf);
         redo = false;
         if (!skip) {
             fwd_step<D, kCarryOnly, false, true>(ktile, ktile + kTile, lo, qf, oacc, R, lane, key0, q0w, qi, strict, carry_out);
             carry_step = step;
         }
-        wait_global_memory();
-        __syncthreads();
+        close_step(step, buf);
     }
     store_carries();
     wait_global_memory();                      // the group's last entries are in memory before they are rescaled below
@@ -321,11 +374,13 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
         if (g < grp) F *= t;
         all *= t;
     }
+    // (rows for which nothing is left of the stick to the right of this segment have all their live entries there)
+    if (__builtin_amdgcn_ballot_w64(F != 0.f && qi < job.len) != 0 && lane == 0) atomicMin(&first_live, reached);
     // carry-table entries of this group, written relative to its own right edge: times F.  Every lane
     // rescales the entries it wrote (the half-waves have a table each); the loads go out in batches so that
     // their latencies overlap.  Its stores have completed (wait above).
     if (p.save && grp > 0 && qi < job.len) {
-        for (int s0 = low; s0 < hi; s0 += 8) {
+        for (int s0 = reached; s0 < hi; s0 += 8) {
             float v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j)
@@ -335,7 +390,11 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
                 if (s0 + j < hi) my_tab[tabq + (s0 + j) * kRowBlock] = v[j] * F;
         }
     }
-    if (kCarryOnly) return;
+    if (kCarryOnly) {
+        __syncthreads();
+        if (p.save && threadIdx.x == 0) set_first_live(p, head, job, p.early_end ? first_live : 0);
+        return;
+    }
 
     // ---- O = sum_g F_g O_g: groups 1.. park their scaled accumulators in LDS (the tiles are free
     // since the last barrier of the sweep), group 0 adds them up
@@ -348,6 +407,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
                 park[((((grp - 1) * 4 + qs) * (D / 32) + db) * 16 + r) * 64 + lane] = oacc[db][r] * F;
     }
     __syncthreads();
+    if (p.save && threadIdx.x == 0) set_first_live(p, head, job, p.early_end ? first_live : 0);
     if (grp == 0 && qi < job.len) {
 #pragma unroll
         for (int g = 1; g < G; ++g)
