@@ -211,22 +211,8 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     }
     if (g_pending && row_ok) *(float*)((char*)(rcur - tstride) + g_from_r) = Gstore;
 
-    if (row_ok) {
-        const int64_t ob = (int64_t)job.seq * p.dq.sb + (int64_t)head * p.dq.sh + (int64_t)(job.tok0 + qi) * p.dq.st;
-#pragma unroll
-        for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                if (D == 96 && 32 * db + 8 * g >= p.cols) continue;
-                f32x2 a = {dqacc[db][4 * g] * p.scale, dqacc[db][4 * g + 1] * p.scale};
-                f32x2 b = {dqacc[db][4 * g + 2] * p.scale, dqacc[db][4 * g + 3] * p.scale};
-                h16x2 pa = __builtin_convertvector(a, h16x2), pb = __builtin_convertvector(b, h16x2);
-                uint2 w;
-                w.x = __builtin_bit_cast(uint32_t, pa);
-                w.y = __builtin_bit_cast(uint32_t, pb);
-                *(uint2*)(p.dq.ptr + 2 * (ob + 32 * db + 8 * g + 4 * h)) = w;
-            }
-    }
+    store_query_rows<D>(lds + wave * kRowStage<D>, dqacc, p.scale, p.dq,                 // (the tiles are free)
+                        (int64_t)job.seq * p.dq.sb + (int64_t)head * p.dq.sh + (int64_t)job.tok0 * p.dq.st, q0w, job.len, lane, p.cols);
 }
 
 // ---------------------------------------------------------------- pass 1, two steps per iteration
@@ -392,23 +378,13 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dq2_kernel(KParams p
             for (int r = 0; r < 16; ++r) park[((qs * (D / 32) + db) * 16 + r) * 64 + lane] = dqacc[db][r];
     }
     __syncthreads();
-    if (grp == 0 && row_ok) {
-        const int64_t ob = (int64_t)job.seq * p.dq.sb + (int64_t)head * p.dq.sh + (int64_t)(job.tok0 + qi) * p.dq.st;
+    if (grp == 0) {
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db) {
+        for (int db = 0; db < D / 32; ++db)
 #pragma unroll
             for (int r = 0; r < 16; ++r) dqacc[db][r] += park[((qs * (D / 32) + db) * 16 + r) * 64 + lane];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                f32x2 a = {dqacc[db][4 * g] * p.scale, dqacc[db][4 * g + 1] * p.scale};
-                f32x2 b = {dqacc[db][4 * g + 2] * p.scale, dqacc[db][4 * g + 3] * p.scale};
-                h16x2 pa = __builtin_convertvector(a, h16x2), pb = __builtin_convertvector(b, h16x2);
-                uint2 w;
-                w.x = __builtin_bit_cast(uint32_t, pa);
-                w.y = __builtin_bit_cast(uint32_t, pb);
-                *(uint2*)(p.dq.ptr + 2 * (ob + 32 * db + 8 * g + 4 * h)) = w;
-            }
-        }
+        store_query_rows<D>((char*)(park + qs * (D / 32) * 16 * 64), dqacc, p.scale, p.dq,      // (over what this wave has just read)
+                            (int64_t)job.seq * p.dq.sb + (int64_t)head * p.dq.sh + (int64_t)job.tok0 * p.dq.st, q0w, job.len, lane, D);
     }
 }
 
@@ -1467,8 +1443,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
     constexpr int kQ = 0, kDO = kRows * kPitch<D> * 2, kK = 2 * kDO, kV = kK + kTile, kA = kV + kTile, kZ = kA + kRows * 128;
     constexpr int kNB = D / 32;                // 32-column blocks of dK or dV that a wave reduces, for
     constexpr int kKH = W == 2 ? 2 : 1;        // one 32-key half of the block or both
-    constexpr int kCols = 32 * kNB;
-    static_assert(W * kKH * 32 * kCols * 2 <= 2 * kRows * 128, "the waves stage their outputs in the weight tiles");
+    static_assert(W * kKH * kRowStage<D> <= 2 * kRows * 128, "the waves stage their outputs in the weight tiles");
     __shared__ __attribute__((aligned(1024))) char lds[kZ + kRows * 128];
 
     const int lane = threadIdx.x & 63;
@@ -1575,7 +1550,8 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
             copy(kMfmaRows, p.k, kbase, key0 + kKeyBlock, lds + kK, false);
             copy(kMfmaRows, p.v, vbase, key0 + kKeyBlock, lds + kV, false);
         }
-        // [32 keys x kCols] of dV (which = 0) or dK: keys 32 kh .. of the block, over the queries from the block on
+        // [32 keys x D] of dV (which = 0) or dK: keys 32 kh .. of the block, over the queries from the block on; transposed tiles
+        // (lane = key), which leave as rows the way dQ does
         f32x16 acc[kKH][kNB];
 #pragma unroll
         for (int i = 0; i < kKH; ++i)
@@ -1598,24 +1574,17 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
                 for (int db = 0; db < kNB; ++db) {
                     const h16x8 b = fetch(lo.nat[0][db], lo.nat[1][db], offb + r * kPitch<D> * 2);
 #pragma unroll
-                    for (int i = 0; i < kKH; ++i) acc[i][db] = mfma(w[i], b, acc[i][db]);
+                    for (int i = 0; i < kKH; ++i) acc[i][db] = mfma(b, w[i], acc[i][db]);
                 }
             }
         }
         __syncthreads();                       // weight tiles free
         {
-            char* stage = lds + kA + wave * (kKH * 32 * kCols * 2);
             const TensorArg& out = which ? p.dk : p.dv;
-            const int64_t ob = base_of(out);
 #pragma unroll
             for (int i = 0; i < kKH; ++i)
-#pragma unroll
-                for (int db = 0; db < kNB; ++db) stage_acc_tile<kCols>(stage, 32 * i, 32 * db, acc[i][db], which ? p.scale : 1.0f, lane);
-            for (int c = lane; c < kKH * 32 * kCols / 8; c += 64) {
-                const int row = c / (kCols / 8), cc = c % (kCols / 8), key = key0 + 32 * kh0 + row;
-                if (key < job.len && (D != 96 || cc * 8 < p.cols))
-                    *(u32x4*)(out.ptr + 2 * (ob + (int64_t)key * out.st + cc * 8)) = *(const u32x4*)(stage + row * (kCols * 2) + cc * 16);
-            }
+                store_query_rows<D>(lds + kA + (wave * kKH + i) * kRowStage<D>, acc[i], which ? p.scale : 1.0f, out, base_of(out),
+                                    key0 + 32 * (kh0 + i), job.len, lane, p.cols);
         }
         if (kb + 1 < n_kb) {
             wait_global_memory();              // the next K and V have landed
@@ -1623,21 +1592,8 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
         }
     }
 
-    if (row_ok) {
-        const int64_t ob = base_of(p.dq) + (int64_t)qi * p.dq.st;
-#pragma unroll
-        for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                if (D == 96 && 32 * db + 8 * g >= p.cols) continue;
-                f32x2 a = {dqacc[db][4 * g] * p.scale, dqacc[db][4 * g + 1] * p.scale};
-                f32x2 b = {dqacc[db][4 * g + 2] * p.scale, dqacc[db][4 * g + 3] * p.scale};
-                uint2 w;
-                w.x = __builtin_bit_cast(uint32_t, __builtin_convertvector(a, h16x2));
-                w.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(b, h16x2));
-                *(uint2*)(p.dq.ptr + 2 * (ob + 32 * db + 8 * g + 4 * h)) = w;
-            }
-    }
+    // (the wave's own Q rows: nobody reads them any more)
+    store_query_rows<D>(lds + kQ + q0w * kPitch<D> * 2, dqacc, p.scale, p.dq, base_of(p.dq), q0w, job.len, lane, p.cols);
 }
 
 // ---------------------------------------------------------------- pass 2, two waves per 32 keys

@@ -50,25 +50,10 @@ __device__ inline bool fwd_step(const char* ktile, const char* vtile, const Lane
     return true;
 }
 
-// rows d = 32*db + 8*g + 4*h + 0..3 of O^T, column = this lane's query
 template <int D>
-__device__ inline void store_o_row(const KParams& p, const Job& job, int head, int qi, int lane,
-                                   const f32x16 (&oacc)[D / 32]) {
-    const int h = lane >> 5;
-    const int64_t obase = (int64_t)job.seq * p.o.sb + (int64_t)head * p.o.sh + (int64_t)(job.tok0 + qi) * p.o.st;
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            if (D == 96 && 32 * db + 8 * g >= p.cols) continue;
-            f32x2 a = {oacc[db][4 * g], oacc[db][4 * g + 1]};
-            f32x2 b = {oacc[db][4 * g + 2], oacc[db][4 * g + 3]};
-            h16x2 pa = __builtin_convertvector(a, h16x2), pb = __builtin_convertvector(b, h16x2);
-            uint2 w;
-            w.x = __builtin_bit_cast(uint32_t, pa);
-            w.y = __builtin_bit_cast(uint32_t, pb);
-            *(uint2*)(p.o.ptr + 2 * (obase + 32 * db + 8 * g + 4 * h)) = w;
-        }
+__device__ inline void store_o_rows(char* stage, const KParams& p, const Job& job, int head, int q0w, int lane, const f32x16 (&oacc)[D / 32]) {
+    store_query_rows<D>(stage, oacc, 1.0f, p.o, (int64_t)job.seq * p.o.sb + (int64_t)head * p.o.sh + (int64_t)job.tok0 * p.o.st,
+                        q0w, job.len, lane, p.cols);
 }
 
 // kCarryOnly: write the carry table and nothing else (no P*V, no o / rem): the backward's way of
@@ -208,9 +193,9 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     store_carries();
     if (p.save && threadIdx.x == 0) set_first_live(p, head, job, n_steps - iterations);
 
-    if (qi < job.len && !kCarryOnly) {
-        store_o_row<D>(p, job, head, qi, lane, oacc);
-        if (h == 0)
+    if (!kCarryOnly) {
+        store_o_rows<D>(lds + wave * kRowStage<D>, p, job, head, q0w, lane, oacc);       // (the tiles are free)
+        if (h == 0 && qi < job.len)
             Elem16::store(p.rem.ptr, (int64_t)job.seq * p.rem.sb + (int64_t)head * p.rem.sh + job.tok0 + qi, R);
     }
 }
@@ -408,7 +393,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     }
     __syncthreads();
     if (p.save && threadIdx.x == 0) set_first_live(p, head, job, p.early_end ? first_live : 0);
-    if (grp == 0 && qi < job.len) {
+    if (grp == 0) {
 #pragma unroll
         for (int g = 1; g < G; ++g)
 #pragma unroll
@@ -416,8 +401,9 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     oacc[db][r] += park[((((g - 1) * 4 + qs) * (D / 32) + db) * 16 + r) * 64 + lane];
-        store_o_row<D>(p, job, head, qi, lane, oacc);
-        if (h == 0)
+        static_assert(kRowStage<D> <= (D / 32) * 16 * 64 * 4, "a wave's own accumulators were parked there");
+        store_o_rows<D>((char*)(park + qs * (D / 32) * 16 * 64), p, job, head, q0w, lane, oacc);
+        if (h == 0 && qi < job.len)
             Elem16::store(p.rem.ptr, (int64_t)job.seq * p.rem.sb + (int64_t)head * p.rem.sh + job.tok0 + qi, all);
     }
 }
