@@ -52,8 +52,8 @@ int loss_bwd(const void* logits, const int64_t* labels, const float* lse, const 
              void* d_logits, int rows, int len, int classes, int64_t ignore, bool f16, hipStream_t stream);
 
 // Weight gradients c[m][n] = sum over k rows of a[.][m] * b[.][n] (16-bit operands, fp32 results) of up to four products with
-// the same rows, in one launch (sba_gemm.hip).  m, n and the leading dimensions are multiples of 8; the results lie one after
-// the other from `out` on.
+// the same rows, in one launch (sba_gemm.hip).  m, n and the leading dimensions are multiples of 8 and the operands 16-byte aligned
+// (the copies move whole 16-byte chunks of a row); others are refused with -2.  The results lie one after the other from `out` on.
 struct WeightGrad {
     const void* a; const void* b; int64_t lda, ldb; int m, n;
     int64_t at;                          // first element of the result behind `out`
@@ -64,6 +64,7 @@ struct WeightGrads {
     int n, tiles, k;
     float* out; float* partial; int64_t total;
 };
+bool weight_grads_fit(const WeightGrads& g);             // whether the kernel takes it
 int weight_grad_splits(WeightGrads& g, int cus);         // fills first_tile, tiles, at, total; partial sums of how many splits
 int weight_grads(const WeightGrads& g, int splits, bool f16, hipStream_t stream);     // partial: [splits][total] if more than one
 int weight_grads_bf16(const WeightGrads& g, int splits, hipStream_t stream);

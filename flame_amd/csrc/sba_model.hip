@@ -475,6 +475,17 @@ int swiglu_bwd(const void* y, const void* d_out, void* dy, int64_t rows, int wid
     return launched();
 }
 
+bool weight_grads_fit(const WeightGrads& g) {
+    if (g.n < 1 || g.n > 4 || g.k < 1) return false;
+    for (int i = 0; i < g.n; ++i) {
+        const WeightGrad& p = g.one[i];
+        if (p.m < 8 || p.n < 8 || ((p.m | p.n) & 7) || ((p.lda | p.ldb) & 7) || (((uintptr_t)p.a | (uintptr_t)p.b) & 15)) return false;
+        // (a stage of 32 rows is addressed with 32-bit byte offsets from its first)
+        if (p.lda < p.m || p.ldb < p.n || p.lda >= (1 << 26) || p.ldb >= (1 << 26)) return false;
+    }
+    return true;
+}
+
 // How many workgroups share a tile's contraction.  A launch takes ceil(tiles * splits / CUs) rounds of 1/splits of the rows each
 // (about 0.9 us per 32 rows with the chip full); partial sums are written, read and summed at about 4 TB/s.
 int weight_grad_splits(WeightGrads& g, int cus) {
@@ -539,6 +550,7 @@ int project(const Projection& p, bool f16, int cus, hipStream_t s) {
 }
 
 int weight_grads(const WeightGrads& g, int splits, bool f16, hipStream_t s) {
+    if (!weight_grads_fit(g)) return -2;
     const int rc = f16 ? weight_grads_f16(g, splits, s) : weight_grads_bf16(g, splits, s);
     if (rc || splits == 1) return rc;
     hipLaunchKernelGGL(sum_splits_kernel, dim3(grid_for(g.total / 4)), dim3(kThreads), 0, s, g.partial, g.out, g.total / 4, splits);

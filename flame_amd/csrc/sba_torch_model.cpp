@@ -67,13 +67,14 @@ std::vector<Tensor> weight_grads(std::initializer_list<std::pair<Tensor, Tensor>
         auto& one = g.one[g.n++];
         one.a = d_out.data_ptr();
         one.b = in.data_ptr();
-        one.lda = d_out.stride(0);
-        one.ldb = in.stride(0);
+        one.lda = d_out.size(0) > 1 ? d_out.stride(0) : d_out.size(1);
+        one.ldb = in.size(0) > 1 ? in.stride(0) : in.size(1);
         one.m = (int)d_out.size(1);
         one.n = (int)in.size(1);
         g.k = (int)in.size(0);
     }
     const Tensor& like = pairs.begin()->first;
+    ok(weight_grads_fit(g) ? 0 : SBA_ERR_SHAPE);
     const int splits = weight_grad_splits(g, compute_units());
     const Tensor out = empty({g.total}, like, at::kFloat);
     Tensor partial;
@@ -350,7 +351,9 @@ struct Head : torch::autograd::Function<Head> {
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto sv = ctx->get_saved_variables();
         c10::DeviceGuard guard(sv[0].device());
-        const Tensor d = grads[0].contiguous().view({-1, grads[0].size(-1)});
+        Tensor d = grads[0].contiguous();
+        if ((uintptr_t)d.data_ptr() & 15) d = d.clone();         // (a caller's own buffer)
+        d = d.view({-1, d.size(-1)});
         const Tensor dy = project(d, sv[4], true);
         const Tensor dw = weight_grads({{d, sv[2]}})[0];
         auto g = rms_norm_grad(dy, sv[0], sv[1], sv[3], Tensor(), false);
@@ -479,6 +482,7 @@ void bind_model(py::module& m) {
         return std::make_pair(out, pre);
     });
     m.def("project_swiglu_grad", &project_swiglu_grad);
+    m.def("weight_grad", [](const Tensor& d_out, const Tensor& in) { return weight_grads({{d_out, in}})[0]; });
     m.attr("max_norm_width") = kMaxNormWidth;
 }
 

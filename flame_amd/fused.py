@@ -86,7 +86,8 @@ def head(x: torch.Tensor, norm: nn.Module, lm_head: nn.Module):
     if t is None or not (_norm_fits(norm) and plain(lm_head, nn.Linear)):
         return None
     n, w = _weight(norm, x), _weight(lm_head, x)
-    if n is None or w is None:
+    # a vocabulary that is no multiple of 8 is not for the kernel of the weight's gradient (weight_grads_fit() in sba_model.h)
+    if n is None or w is None or w.shape[0] % 8:
         return None
     return _lib.native().head(x, n, w, _eps(norm), t)
 

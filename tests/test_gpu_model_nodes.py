@@ -62,6 +62,49 @@ def test_block_and_head_and_loss_match_the_modules(hidden, heads, B, T, lens, dt
         assert rel_l2(grads[n], grads_ref[n]) <= 2 * tol, n
 
 
+# vocabularies off the 8 columns of a 16-byte chunk, also one to seven columns past a tile of 256
+@pytest.mark.parametrize("vocab", [1004, 1009, 1025])
+def test_ragged_vocabularies_match_the_modules(vocab, monkeypatch):
+    from flame_amd import fused
+    from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM
+    torch.manual_seed(vocab)
+    m = SBAForCausalLM(SBAConfig(hidden_size=128, num_heads=2, num_hidden_layers=1, vocab_size=vocab, initializer_range=0.1)).cuda()
+    ids = torch.randint(0, vocab, (2, 65), device="cuda")
+
+    def run():
+        m.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            loss, logits = m(ids, labels=ids)
+        loss.backward()
+        return loss, logits, {n: p.grad for n, p in m.named_parameters()}
+
+    loss, logits, grads = run()
+    with monkeypatch.context() as mp:
+        for name in ("block", "head", "next_token_loss"):
+            mp.setattr(fused, name, lambda *a, **k: None)
+        loss_ref, logits_ref, grads_ref = run()
+    assert rel_l2(logits.float(), logits_ref.float()) <= 2e-2 and abs(float(loss) - float(loss_ref)) <= 2e-2
+    for n in grads:
+        assert rel_l2(grads[n], grads_ref[n]) <= 4e-2, n
+    # every row of the weight's gradient on its own: none may hold another one's
+    assert (grads["lm_head.weight"] - grads_ref["lm_head.weight"]).norm(dim=1).max() <= 4e-2 * grads_ref["lm_head.weight"].norm(dim=1).max()
+
+
+def test_weight_gradient_of_an_unaligned_buffer():
+    # a gradient of the logits that a caller cut out of a larger buffer of its own
+    from flame_amd import fused
+    torch.manual_seed(0)
+    norm, lm_head = torch.nn.RMSNorm(64).cuda(), torch.nn.Linear(64, 264, bias=False).cuda()
+    x = torch.randn(1, 37, 64, device="cuda")
+    buf = torch.randn(37 * 264 + 3, device="cuda").to(torch.bfloat16)
+    d = buf[3:].view(1, 37, 264)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        logits = fused.head(x, norm, lm_head)
+    logits.backward(d)
+    ref = d[0].float().t() @ F.rms_norm(x[0], (64,), norm.weight, torch.finfo(torch.float32).eps).detach().to(torch.bfloat16).float()
+    assert rel_l2(lm_head.weight.grad, ref) <= 1e-2
+
+
 def test_hooks_and_other_modules_keep_the_module_path():
     from flame_amd import fused
     from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM

@@ -1,0 +1,41 @@
+"""Which calls the language model's native nodes take, decided on the host: no GPU needed."""
+import pytest
+import torch
+
+from flame_amd import _lib, fused
+
+
+class _Native:
+    """Stands in for the native module and notes what it is asked for."""
+    max_norm_width = 2048
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        return lambda *a: self.calls.append(name) or name
+
+
+@pytest.fixture
+def native(monkeypatch):
+    n = _Native()
+    monkeypatch.setattr(_lib, "native", lambda: n)
+    return n
+
+
+@pytest.mark.parametrize("vocab,taken", [(1000, True), (1004, False), (1009, False), (32001, False)])
+def test_head_takes_vocabularies_of_whole_chunks(vocab, taken, native, monkeypatch):
+    monkeypatch.setattr(fused, "_compute_dtype", lambda x: torch.bfloat16)
+    x, norm, lm_head = torch.randn(1, 3, 64), torch.nn.RMSNorm(64), torch.nn.Linear(64, vocab, bias=False)
+    assert (fused.head(x, norm, lm_head) is not None) == taken
+    assert native.calls == (["head"] if taken else [])
+
+
+def test_weight_gradients_outside_their_contract_are_refused():
+    grad = _lib.native().weight_grad                  # every one of these is refused before anything is launched
+    rows = lambda cols, off=0: torch.zeros(64 * 2048, dtype=torch.bfloat16)[off:off + 16 * cols].view(16, cols)
+    for d, x in [(rows(1009), rows(64)), (rows(1004), rows(64)), (rows(257), rows(64)), (rows(64), rows(60)),
+                 (rows(64, off=1), rows(64)), (rows(64), rows(64, off=4)), (rows(72)[:, :64][:0], rows(64)[:0]),
+                 (torch.zeros(16, 68, dtype=torch.bfloat16)[:, :64], rows(64))]:
+        with pytest.raises(RuntimeError, match="bad shape"):
+            grad(d, x)
