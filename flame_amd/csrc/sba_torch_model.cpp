@@ -10,6 +10,7 @@
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
 #include <ATen/ops/mm.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/util/SmallVector.h>
 #include <torch/csrc/autograd/custom_function.h>
 
@@ -418,7 +419,9 @@ Tensor next_token_loss(const Tensor& logits, const Tensor& labels, int64_t ignor
 // ---------------------------------------------------------------------------------------------- clip and step
 
 // One pass of gradient clipping and AdamW over all weights; groups[group_of[i]]: {lr, weight_decay, beta1, beta2, eps} of
-// weight i.  Returns the gradients' norm, or nothing, with nothing done, if a tensor is not one the kernels take.
+// weight i.  Returns the gradients' norm, or nothing, with nothing done, if a tensor is not one the kernels take or the stream
+// captures a graph: the table of pointers and the step's settings leave from a host buffer of this call alone, which a replay would
+// read after others have used it (an optimizer that is not `capturable` refuses to be captured for the like reason).
 std::optional<Tensor> clip_and_step(const std::vector<Tensor>& p, const std::vector<Tensor>& g, const std::vector<Tensor>& m,
                                     const std::vector<Tensor>& v, const std::vector<Tensor>& step,
                                     const std::vector<int64_t>& group_of, const std::vector<std::vector<double>>& groups,
@@ -434,6 +437,7 @@ std::optional<Tensor> clip_and_step(const std::vector<Tensor>& p, const std::vec
         if (step[i].scalar_type() != at::kFloat || step[i].device() != device || step[i].numel() != 1) return std::nullopt;
     }
     c10::DeviceGuard guard(device);
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return std::nullopt;
     Tensor host = at::empty({n * (int64_t)sizeof(OptTensor)}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
     auto* t = (OptTensor*)host.data_ptr();
     int64_t chunks = 0;

@@ -174,3 +174,28 @@ def test_clip_and_adamw_in_one_pass_matches_torch(max_norm):
     assert all(abs(x - y) <= 1e-5 * y for x, y in zip(na, nb))
     for a, b in zip(pa + ga + sa, pb + gb + sb):
         assert torch.allclose(a, b, rtol=2e-5, atol=1e-7)
+
+
+def test_clip_and_step_leaves_a_captured_step_to_the_optimizer():
+    # which refuses it without `capturable`: nothing of the step may be in the graph
+    from flame_amd import fused
+    ps = [torch.nn.Parameter(torch.ones(1000, device="cuda"))]
+    opt = torch.optim.AdamW(ps, lr=1e-2, fused=True)
+    ps[0].grad = torch.ones_like(ps[0])
+    opt.step()
+    before = [t.clone() for t in (ps[0], *(opt.state[ps[0]][k] for k in ("exp_avg", "exp_avg_sq", "step")))]
+    x = torch.ones(8, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = x + 1
+        assert fused.clip_and_step(ps, opt, 1.0) is None
+        with pytest.raises(RuntimeError, match="capturable"):
+            opt.step()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, x + 1)
+    after = [ps[0], *(opt.state[ps[0]][k] for k in ("exp_avg", "exp_avg_sq", "step"))]
+    assert all(torch.equal(a, b) for a, b in zip(before, after))
+    assert fused.clip_and_step(ps, opt, 1.0) is not None         # and outside of a capture it is taken again
