@@ -326,6 +326,8 @@ std::tuple<Tensor, Tensor> run(const Tensor& q, const Tensor& k, const Tensor& v
                       cu_seqlens ? "q, k, v must all be [H, total_tokens, D]" : "q, k, v must all be [B, H, T, D]");
     dtype_code(q.scalar_type());
     TORCH_CHECK_VALUE(q.size(-1) <= kMaxHeadDim, "head_dim ", q.size(-1), " is not supported (at most ", kMaxHeadDim, ")");
+    TORCH_CHECK_NOT_IMPLEMENTED(!has_tangent(q) && !has_tangent(k) && !has_tangent(v),
+                                "stick-breaking attention has no forward-mode derivative");
     c10::DeviceGuard guard(q.device());
     c10::intrusive_ptr<Plan> plan;
     if (cu_seqlens) {

@@ -42,6 +42,9 @@ void attention_backward(const Problem& pr, const Tensor& tables, const Tensor& d
 
 void bind_model(py::module& m);          // sba_torch_model.cpp
 
+// A dual tensor of forward-mode differentiation: the nodes here have no such derivative, and the kernels would drop it silently.
+inline bool has_tangent(const Tensor& t) { return t._fw_grad(/*level=*/0).defined(); }
+
 hipStream_t stream_of(const Tensor& t);
 void check_status(int rc, const char* what);
 

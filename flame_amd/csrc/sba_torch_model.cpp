@@ -309,8 +309,12 @@ struct Block : torch::autograd::Function<Block> {
     }
 };
 
-Tensor block(const Tensor& x, const std::vector<Tensor>& w, int64_t heads, double eps1, double eps2, py::object dtype,
-             const std::optional<Tensor>& cu_seqlens, int64_t max_seqlens) {
+// block(), head() and next_token_loss() return nothing where the modules have to be called instead: they differentiate forward, too.
+std::optional<Tensor> block(const Tensor& x, const std::vector<Tensor>& w, int64_t heads, double eps1, double eps2, py::object dtype,
+                            const std::optional<Tensor>& cu_seqlens, int64_t max_seqlens) {
+    bool dual = has_tangent(x);
+    for (const auto& t : w) dual = dual || has_tangent(t);
+    if (dual) return std::nullopt;
     BlockShape s;
     s.B = x.size(0);
     s.T = x.size(1);
@@ -364,7 +368,8 @@ struct Head : torch::autograd::Function<Head> {
     }
 };
 
-Tensor head(const Tensor& x, const Tensor& n, const Tensor& w, double eps, py::object dtype) {
+std::optional<Tensor> head(const Tensor& x, const Tensor& n, const Tensor& w, double eps, py::object dtype) {
+    if (has_tangent(x) || has_tangent(n) || has_tangent(w)) return std::nullopt;
     const at::ScalarType t = torch::python::detail::py_object_to_dtype(dtype);
     c10::DeviceGuard guard(x.device());
     NoAutocast no_autocast;
@@ -409,7 +414,8 @@ struct Loss : torch::autograd::Function<Loss> {
     }
 };
 
-Tensor next_token_loss(const Tensor& logits, const Tensor& labels, int64_t ignore) {
+std::optional<Tensor> next_token_loss(const Tensor& logits, const Tensor& labels, int64_t ignore) {
+    if (has_tangent(logits)) return std::nullopt;
     c10::DeviceGuard guard(logits.device());
     if (at::GradMode::is_enabled() && logits.requires_grad()) return Loss::apply(logits, labels, ignore);
     at::AutoDispatchBelowADInplaceOrView below;

@@ -199,3 +199,38 @@ def test_clip_and_step_leaves_a_captured_step_to_the_optimizer():
     after = [ps[0], *(opt.state[ps[0]][k] for k in ("exp_avg", "exp_avg_sq", "step"))]
     assert all(torch.equal(a, b) for a, b in zip(before, after))
     assert fused.clip_and_step(ps, opt, 1.0) is not None         # and outside of a capture it is taken again
+
+
+def test_forward_mode_tangents_are_kept_or_refused():
+    # a dual input that needs no gradient: the operator says that it has no such derivative, the model's other parts have one
+    from torch.autograd import forward_ad
+    from flame_amd import fused, sb_attn, sb_attn_varlen
+    from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM, next_token_loss
+    torch.manual_seed(0)
+    m = SBAForCausalLM(SBAConfig(hidden_size=128, num_heads=2, num_hidden_layers=1, vocab_size=256)).cuda()
+    m.requires_grad_(False)
+    rand = lambda *s: torch.randn(*s, device="cuda")
+    x, tx, logits, tl = rand(1, 9, 128), rand(1, 9, 128), rand(1, 9, 256), rand(1, 9, 256)
+    ids = torch.randint(0, 256, (1, 9), device="cuda")
+    with forward_ad.dual_level():
+        q = rand(1, 2, 9, 64).to(torch.bfloat16)
+        for i in range(3):
+            args = [q, q, q]
+            args[i] = forward_ad.make_dual(q, torch.ones_like(q))
+            with pytest.raises(NotImplementedError):
+                sb_attn(*args)
+            with pytest.raises(NotImplementedError):
+                sb_attn_varlen(*(a[0] for a in args), torch.tensor([0, 4, 9], dtype=torch.int32), 5)
+        sb_attn(q, q, q)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            dual = forward_ad.make_dual(x, tx)
+            assert fused.block(m.model.layers[0], dual, {}) is None
+            with pytest.raises(NotImplementedError):
+                m.model.layers[0](dual)
+            assert fused.head(dual, m.model.norm, m.lm_head) is None
+            assert fused.head(x, m.model.norm, m.lm_head) is not None
+        half = logits.to(torch.bfloat16)
+        loss, got = forward_ad.unpack_dual(next_token_loss(forward_ad.make_dual(half, tl.to(torch.bfloat16)), ids))
+    leaf = half.float().requires_grad_()
+    want, = torch.autograd.grad(F.cross_entropy(leaf[0, :-1], ids[0, 1:]), leaf)
+    assert got is not None and abs(float(got) - float((want * tl.to(torch.bfloat16).float()).sum())) <= 1e-5 * float(want.norm() * tl.norm())
