@@ -10,6 +10,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 from torch.nn.modules import module as _module
+from torch.optim import optimizer as _optimizer
 
 from . import _lib
 from .stickbreaking_attention import profiling, sb_attn, sb_attn_varlen
@@ -105,7 +106,8 @@ def next_token_loss(logits: torch.Tensor, labels: torch.Tensor, ignore: int = -1
 def clip_and_step(params, opt, max_norm: float):
     """Gradient clipping to `max_norm` over `params` and opt.step(), in one pass over the weights; returns the gradients' norm,
     or None, with nothing done, where that is not what the two calls would do one after the other."""
-    if type(opt) is not torch.optim.AdamW or opt._optimizer_step_pre_hooks or opt._optimizer_step_post_hooks:
+    if type(opt) is not torch.optim.AdamW or opt._optimizer_step_pre_hooks or opt._optimizer_step_post_hooks \
+            or _optimizer._global_optimizer_pre_hooks or _optimizer._global_optimizer_post_hooks:
         return None
     step_fn = opt.__dict__.get("step")           # a learning-rate scheduler's wrapper notes that a step was taken
     if step_fn is not None and not getattr(step_fn, "_wrapped_by_lr_sched", False):

@@ -39,3 +39,22 @@ def test_weight_gradients_outside_their_contract_are_refused():
                  (torch.zeros(16, 68, dtype=torch.bfloat16)[:, :64], rows(64))]:
         with pytest.raises(RuntimeError, match="bad shape"):
             grad(d, x)
+
+
+def _adamw_after_one_step():
+    p = torch.nn.Parameter(torch.ones(4))
+    opt = torch.optim.AdamW([p], lr=1e-3, fused=True)
+    p.grad = torch.ones(4)
+    opt.step()
+    return p, opt
+
+
+def test_clip_and_step_leaves_hooked_optimizers_alone(native):
+    from torch.optim.optimizer import register_optimizer_step_post_hook, register_optimizer_step_pre_hook
+    p, opt = _adamw_after_one_step()
+    for register in (register_optimizer_step_pre_hook, register_optimizer_step_post_hook,
+                     opt.register_step_pre_hook, opt.register_step_post_hook):
+        hook = register(lambda *a: None)
+        assert fused.clip_and_step([p], opt, 1.0) is None and not native.calls
+        hook.remove()
+    assert fused.clip_and_step([p], opt, 1.0) is not None and native.calls == ["clip_and_step"]
