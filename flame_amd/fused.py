@@ -25,16 +25,15 @@ def _compute_dtype(x: torch.Tensor):
     if not torch.is_autocast_enabled("cuda"):
         return None
     t = torch.get_autocast_dtype("cuda")
-    if t not in _HALF or _module._global_forward_hooks or _module._global_forward_pre_hooks \
-            or _module._global_backward_hooks or _module._global_backward_pre_hooks:
-        return None
-    return t
+    return t if t in _HALF else None
 
 
 def plain(m: nn.Module, kind: type) -> bool:
     """A module of exactly this class whose call is its class's forward() and nothing else."""
     return (type(m) is kind and not m._forward_hooks and not m._forward_pre_hooks and not m._backward_hooks
-            and not m._backward_pre_hooks and "forward" not in m.__dict__)
+            and not m._backward_pre_hooks and "forward" not in m.__dict__ and m._compiled_call_impl is None
+            and not (_module._global_forward_hooks or _module._global_forward_pre_hooks
+                     or _module._global_backward_hooks or _module._global_backward_pre_hooks))
 
 
 def _weight(m: nn.Module, like: torch.Tensor):

@@ -58,3 +58,24 @@ def test_clip_and_step_leaves_hooked_optimizers_alone(native):
         assert fused.clip_and_step([p], opt, 1.0) is None and not native.calls
         hook.remove()
     assert fused.clip_and_step([p], opt, 1.0) is not None and native.calls == ["clip_and_step"]
+
+
+def test_the_backbone_is_called_where_a_hook_or_a_compiled_call_would_see_it(monkeypatch):
+    from torch.nn.modules.module import register_module_forward_hook, register_module_full_backward_hook
+    from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM, SBAModel
+    from oracle import sb_oracle as O
+    m = SBAForCausalLM(SBAConfig(hidden_size=64, num_hidden_layers=1, num_heads=1, vocab_size=40))
+    m.model.layers[0].attn.attn_fn = lambda q, k, v, t: O.sb_attn_oracle(q, k, v)
+    ids, seen = torch.randint(0, 40, (1, 6)), []
+    note = lambda mod, *a: seen.append(type(mod)) and None
+    assert fused.plain(m.model, SBAModel)
+    for register in (register_module_forward_hook, register_module_full_backward_hook):
+        hook = register(note)
+        assert not fused.plain(m.model, SBAModel)
+        m(ids, labels=ids)[0].backward()
+        hook.remove()
+        assert seen.count(SBAModel) == 1
+        seen.clear()
+    monkeypatch.setattr(m.model, "_compiled_call_impl", lambda *a, **k: seen.append(SBAModel) or m.model.forward(*a, **k))
+    m(ids)
+    assert seen == [SBAModel]
