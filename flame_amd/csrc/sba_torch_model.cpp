@@ -13,6 +13,8 @@
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/util/SmallVector.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 
 #include <cstring>
 
@@ -202,6 +204,30 @@ Tensor cast_to(const Tensor& x, at::ScalarType t) {
     return out;
 }
 
+// What a backward of these kernels returns under create_graph: its gradients, which say so if they are differentiated again (the
+// kernels leave no graph, so they would pass for constants).
+template <class F>
+variable_list differentiable_once(const variable_list& in, F&& backward) {
+    const bool graph = at::GradMode::is_enabled();
+    variable_list grads;
+    {
+        at::AutoGradMode no_graph(false);
+        grads = backward();
+    }
+    if (!graph) return grads;
+    // they depend on what the node's inputs and its incoming gradients do
+    torch::autograd::edge_list edges = torch::autograd::get_current_node()->next_edges();
+    for (auto& e : torch::autograd::collect_next_edges(in)) edges.push_back(std::move(e));
+    const auto error = std::make_shared<torch::autograd::Error>(
+        "the language model's native nodes differentiate once: their gradients cannot be differentiated again", std::move(edges));
+    for (auto& g : grads) {
+        if (!g.defined()) continue;
+        g = g.detach();
+        torch::autograd::set_history(g, error);
+    }
+    return grads;
+}
+
 // -------------------------------------------------------------------------------------------------------- one block
 
 struct BlockShape {
@@ -275,6 +301,10 @@ struct Block : torch::autograd::Function<Block> {
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        return differentiable_once(grads, [&] { return gradients(ctx, grads); });
+    }
+
+    static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
         const auto sv = ctx->get_saved_variables();
         const Tensor &x = sv[0], &n1 = sv[1], &n2 = sv[2], &x1 = sv[3], &y1 = sv[4], &rstd1 = sv[5], &qkv = sv[6], &o = sv[7],
                      &tables = sv[8], &y2 = sv[9], &rstd2 = sv[10], &gu = sv[11], &a = sv[12], &w_qkv = sv[13], &w_o = sv[14],
@@ -354,6 +384,9 @@ struct Head : torch::autograd::Function<Head> {
         return logits.view(sizes);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        return differentiable_once(grads, [&] { return gradients(ctx, grads); });
+    }
+    static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
         const auto sv = ctx->get_saved_variables();
         c10::DeviceGuard guard(sv[0].device());
         Tensor d = grads[0].contiguous();
@@ -393,19 +426,29 @@ LossRows loss_rows(const Tensor& logits, const Tensor& labels, int64_t ignore) {
     return r;
 }
 
+// The loss's gradient from operators that leave a graph (create_graph).
+Tensor differentiable_loss_grad(const Tensor& logits, const Tensor& labels, const Tensor& count, const Tensor& d_loss, int64_t ignore) {
+    const Tensor target = at::cat({labels.narrow(1, 1, labels.size(1) - 1), at::full_like(labels.narrow(1, 0, 1), ignore)}, 1).unsqueeze(-1);
+    const Tensor hit = target.eq(at::arange(logits.size(-1), labels.options())).to(at::kFloat);
+    const Tensor scale = at::where(target.eq(ignore), at::zeros_like(count), d_loss / count);
+    return ((at::softmax(logits.to(at::kFloat), -1) - hit) * scale).to(logits.scalar_type());
+}
+
 struct Loss : torch::autograd::Function<Loss> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& logits_in, const Tensor& labels_in, int64_t ignore) {
-        const Tensor logits = logits_in.contiguous(), labels = labels_in.contiguous();
-        auto r = loss_rows(logits, labels, ignore);
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& labels_in, int64_t ignore) {
+        const Tensor labels = labels_in.contiguous();
+        auto r = loss_rows(logits.contiguous(), labels, ignore);
         ctx->save_for_backward({logits, labels, r.lse, r.count});
         ctx->saved_data["ignore"] = ignore;
         return r.mean;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto sv = ctx->get_saved_variables();
-        const Tensor &logits = sv[0], &labels = sv[1];
-        c10::DeviceGuard guard(logits.device());
-        const Tensor g = grads[0].contiguous();
+        const Tensor& labels = sv[1];
+        c10::DeviceGuard guard(labels.device());
+        if (at::GradMode::is_enabled())
+            return {differentiable_loss_grad(sv[0], labels, sv[3], grads[0], ctx->saved_data["ignore"].toInt()), Tensor(), Tensor()};
+        const Tensor logits = sv[0].contiguous(), g = grads[0].contiguous();
         Tensor d = at::empty_like(logits);
         ok(loss_bwd(logits.data_ptr(), labels.data_ptr<int64_t>(), sv[2].data_ptr<float>(), sv[3].data_ptr<float>(),
                     g.data_ptr<float>(), d.data_ptr(), (int)labels.numel(), (int)labels.size(-1), (int)logits.size(-1),

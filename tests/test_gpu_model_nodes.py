@@ -234,3 +234,50 @@ def test_forward_mode_tangents_are_kept_or_refused():
     leaf = half.float().requires_grad_()
     want, = torch.autograd.grad(F.cross_entropy(leaf[0, :-1], ids[0, 1:]), leaf)
     assert got is not None and abs(float(got) - float((want * tl.to(torch.bfloat16).float()).sum())) <= 1e-5 * float(want.norm() * tl.norm())
+
+
+def test_gradients_of_gradients_are_right_or_refused():
+    from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM, next_token_loss
+    torch.manual_seed(0)
+    labels = torch.randint(0, 264, (2, 9), device="cuda")
+    labels[0, 3] = -100
+    a = torch.randn(2, 9, 264, device="cuda").to(torch.bfloat16).transpose(0, 1).contiguous().transpose(0, 1).requires_grad_()
+    b = a.detach().float().requires_grad_()
+    w = torch.randn(2, 9, 264, device="cuda")
+    shifted = torch.cat((labels[:, 1:], torch.full_like(labels[:, :1], -100)), 1)
+    first, second = [], []
+    for x, loss in ((a, 3 * next_token_loss(a, labels)),
+                    (b, 3 * F.cross_entropy(b.reshape(18, -1), shifted.view(-1), ignore_index=-100))):
+        g, = torch.autograd.grad(loss, x, create_graph=True)
+        first.append(g.detach().float())
+        second.append(torch.autograd.grad((g.float() * w).sum(), x)[0].float())
+    # bf16 values of both: 2^-9 each, and of the second one's incoming gradient, which is rounded the same way
+    assert rel_l2(first[0], first[1]) <= 5e-3 and rel_l2(second[0], second[1]) <= 1e-2
+
+    m = SBAForCausalLM(SBAConfig(hidden_size=128, num_heads=2, num_hidden_layers=1, vocab_size=264, initializer_range=0.1)).cuda()
+    ids = torch.randint(0, 264, (1, 40), device="cuda")
+    params = list(m.parameters())
+
+    def loss():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return m(ids, labels=ids)[0]
+
+    plain = torch.autograd.grad(loss(), params)
+    kept = torch.autograd.grad(loss(), params, create_graph=True)
+    for p, x, y in zip(params, plain, kept):
+        assert rel_l2(y, x) <= 1e-2                              # (the logits' gradient rounds elsewhere)
+        if p is not m.model.embeddings.weight:
+            with pytest.raises(RuntimeError, match="differentiate once"):
+                torch.autograd.grad(y.square().sum(), params, retain_graph=True, allow_unused=True)
+            with pytest.raises(RuntimeError, match="differentiate once"):
+                y.sum().backward(retain_graph=True)
+
+    # one weight alone, behind gradients that depend on nothing
+    blk = m.model.layers[0].requires_grad_(False)
+    wq = blk.attn.q_proj.weight.requires_grad_()
+    x = torch.randn(1, 40, 128, device="cuda")
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = blk(x)
+    g, = torch.autograd.grad(y, wq, torch.ones_like(y), create_graph=True)
+    with pytest.raises(RuntimeError, match="differentiate once"):
+        torch.autograd.grad(g.sum(), wq)
