@@ -64,7 +64,7 @@ int compute_units() {
 }
 
 // d_weight = d_out^T . in, in fp32, of several products over the same rows at once
-std::vector<Tensor> weight_grads(std::initializer_list<std::pair<Tensor, Tensor>> pairs) {
+std::vector<Tensor> weight_grads(at::ArrayRef<std::pair<Tensor, Tensor>> pairs) {
     WeightGrads g = {};
     for (const auto& [d_out, in] : pairs) {
         auto& one = g.one[g.n++];
@@ -76,7 +76,7 @@ std::vector<Tensor> weight_grads(std::initializer_list<std::pair<Tensor, Tensor>
         one.n = (int)in.size(1);
         g.k = (int)in.size(0);
     }
-    const Tensor& like = pairs.begin()->first;
+    const Tensor& like = pairs[0].first;
     ok(weight_grads_fit(g) ? 0 : SBA_ERR_SHAPE);
     const int splits = weight_grad_splits(g, compute_units());
     const Tensor out = empty({g.total}, like, at::kFloat);
@@ -317,25 +317,57 @@ struct Block : torch::autograd::Function<Block> {
         const int64_t N = s.B * s.T;
         const Tensor dx2 = grads[0].contiguous().view({N, s.hidden});
 
+        // what is asked for - x, norm1, q, k, v, o, norm2, gate, up, down -, and no further back than that leads
+        auto asked = [&](int first, int last) {
+            for (int i = first; i <= last; ++i)
+                if (ctx->needs_input_grad(i)) return true;
+            return false;
+        };
         const Tensor dm = cast_to(dx2, s.t);
-        const Tensor dgu = project_swiglu_grad(dm, w_d, gu);
-        const Tensor dy2 = project(dgu, w_gu, true);
-        auto g2 = rms_norm_grad(dy2, x1, n2, rstd2, dx2, true);
-        const Tensor d_o = project(g2.dx16, w_o, true);
-        const Tensor dqkv = at::empty_like(qkv);
-        {
+        Tensor dgu, dqkv, dy1;
+        NormGrad g1, g2;
+        if (asked(0, 8)) dgu = project_swiglu_grad(dm, w_d, gu);
+        if (asked(0, 6)) g2 = rms_norm_grad(project(dgu, w_gu, true), x1, n2, rstd2, dx2, true);
+        if (asked(0, 4)) {
+            const Tensor d_o = project(g2.dx16, w_o, true);
+            dqkv = at::empty_like(qkv);
             Problem pr = problem_of(s, qkv);
             const Problem g = problem_of(s, dqkv);
             attention_backward(pr, tables, heads_of(s, d_o), Tensor(), g.q, g.k, g.v);
         }
-        const Tensor dy1 = project(dqkv, w_qkv, true);
-        const auto dw = weight_grads({{dqkv, y1}, {g2.dx16, o}, {dgu, y2}, {dm, a}});
-        const Tensor &dwqkv = dw[0], &dwo = dw[1], &dwgu = dw[2], &dwd = dw[3];
-        auto g1 = rms_norm_grad(dy1, x, n1, rstd1, g2.dx, false);
+        if (asked(0, 1)) dy1 = project(dqkv, w_qkv, true);
 
-        const int64_t C = s.hidden, F = s.width;
-        return {g1.dx.view(grads[0].sizes()), g1.dw, dwqkv.narrow(0, 0, C), dwqkv.narrow(0, C, C), dwqkv.narrow(0, 2 * C, C), dwo,
-                g2.dw, dwgu.narrow(0, 0, F), dwgu.narrow(0, F, F), dwd, Tensor(), Tensor()};
+        // weights first .. last lie stacked, `rows` of each: from the first asked one to the last
+        c10::SmallVector<std::pair<Tensor, Tensor>, 4> products;
+        c10::SmallVector<std::array<int64_t, 3>, 4> owners;
+        auto want = [&](int first, int last, int64_t rows, const Tensor& d, const Tensor& in) {
+            const int stacked = first;
+            while (first <= last && !asked(first, first)) ++first;
+            while (first < last && !asked(last, last)) --last;
+            if (first > last) return;
+            products.emplace_back(d.narrow(1, (first - stacked) * rows, (last - first + 1) * rows), in);
+            owners.push_back({first, last, rows});
+        };
+        want(2, 4, s.hidden, dqkv, y1);
+        want(5, 5, s.hidden, g2.dx16, o);
+        want(7, 8, s.width, dgu, y2);
+        want(9, 9, s.hidden, dm, a);
+        variable_list out(12);
+        if (!products.empty()) {
+            const auto dw = weight_grads(products);
+            for (size_t i = 0; i < dw.size(); ++i) {
+                const auto [first, last, rows] = owners[i];
+                for (int64_t w = first; w <= last; ++w)
+                    if (asked(w, w)) out[w] = dw[i].narrow(0, (w - first) * rows, rows);
+            }
+        }
+        if (asked(0, 1)) {
+            g1 = rms_norm_grad(dy1, x, n1, rstd1, g2.dx, false);
+            out[0] = g1.dx.view(grads[0].sizes());
+            out[1] = g1.dw;
+        }
+        out[6] = g2.dw;
+        return out;
     }
 };
 
@@ -392,12 +424,16 @@ struct Head : torch::autograd::Function<Head> {
         Tensor d = grads[0].contiguous();
         if ((uintptr_t)d.data_ptr() & 15) d = d.clone();         // (a caller's own buffer)
         d = d.view({-1, d.size(-1)});
-        const Tensor dy = project(d, sv[4], true);
-        const Tensor dw = weight_grads({{d, sv[2]}})[0];
-        auto g = rms_norm_grad(dy, sv[0], sv[1], sv[3], Tensor(), false);
-        auto sizes = grads[0].sizes().vec();
-        sizes.back() = sv[0].size(1);
-        return {g.dx.view(sizes), g.dw, dw, Tensor(), Tensor()};
+        variable_list out(5);                                    // x, norm, weight
+        if (ctx->needs_input_grad(2)) out[2] = weight_grads({{d, sv[2]}})[0];
+        if (ctx->needs_input_grad(0) || ctx->needs_input_grad(1)) {
+            auto g = rms_norm_grad(project(d, sv[4], true), sv[0], sv[1], sv[3], Tensor(), false);
+            auto sizes = grads[0].sizes().vec();
+            sizes.back() = sv[0].size(1);
+            out[0] = g.dx.view(sizes);
+            out[1] = g.dw;
+        }
+        return out;
     }
 };
 

@@ -281,3 +281,47 @@ def test_gradients_of_gradients_are_right_or_refused():
     g, = torch.autograd.grad(y, wq, torch.ones_like(y), create_graph=True)
     with pytest.raises(RuntimeError, match="differentiate once"):
         torch.autograd.grad(g.sum(), wq)
+
+
+def test_frozen_weights_cost_no_gradients():
+    # every single weight of a block and its head, the norms, a few together, the input alone: the same gradients as when all are
+    # asked for, and no memory for the others'
+    from flame_amd import fused
+    from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM
+    torch.manual_seed(0)
+    m = SBAForCausalLM(SBAConfig(hidden_size=256, num_heads=4, num_hidden_layers=1, vocab_size=512, initializer_range=0.06)).cuda()
+    blk = m.model.layers[0]
+    x = torch.randn(1, 100, 256, device="cuda")
+    dy, dl = torch.randn(1, 100, 256, device="cuda"), torch.randn(1, 100, 512, device="cuda").to(torch.bfloat16)
+
+    def grads(weights, with_x):
+        leaves = dict(weights, x=x.clone()) if with_x else dict(weights)
+        for p in m.parameters():
+            p.requires_grad_(False)
+        for t in leaves.values():
+            t.requires_grad_(True)
+        xin = leaves.get("x", x)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            head = any(n == "norm" or n == "lm_head" for n in weights)
+            out, d = (fused.head(xin, m.model.norm, m.lm_head), dl) if head else (fused.block(blk, xin, {}), dy)
+        before = torch.cuda.memory_stats()["allocated_bytes.all.allocated"]
+        got = torch.autograd.grad(out, list(leaves.values()), d)
+        return dict(zip(leaves, got)), torch.cuda.memory_stats()["allocated_bytes.all.allocated"] - before
+
+    own = dict(blk.named_parameters())
+    names = list(own)
+    for weights, picks in (
+            (own, [[n] for n in names] + [[], ["attn.q_proj.weight", "attn.v_proj.weight"], ["attn.k_proj.weight", "mlp.up_proj.weight"]]),
+            ({"norm": m.model.norm.weight, "lm_head": m.lm_head.weight}, [["norm"], ["lm_head"]])):
+        full, bytes_full = grads(weights, True)
+        for pick in picks:
+            for with_x in (True, False) if pick else (True,):
+                got, used = grads({n: weights[n] for n in pick}, with_x)
+                assert set(got) == set(pick) | ({"x"} if with_x else set())
+                for n, g in got.items():
+                    assert rel_l2(g, full[n]) <= 1e-5, (pick, n)      # fp32 sums, perhaps in another number of splits
+                # (a norm's gradient comes with its input's, k's lies between q's and v's)
+                spared = [n for n in weights if n not in pick and weights[n].dim() == 2]
+                if pick == ["attn.q_proj.weight", "attn.v_proj.weight"]:
+                    spared.remove("attn.k_proj.weight")
+                assert used <= bytes_full - sum(weights[n].numel() * 4 for n in spared), pick
