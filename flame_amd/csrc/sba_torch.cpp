@@ -141,6 +141,9 @@ std::unordered_map<CacheKey, CacheEntry, CacheHash> g_plans;
 int64_t version_of(const Tensor& t) { return t.is_inference() ? 0 : (int64_t)t._version(); }
 
 c10::intrusive_ptr<Plan> build_plan(const Tensor& cu_seqlens, int64_t n_heads, c10::Device device) {
+    // the copy waits for the stream: the program's other threads go on meanwhile
+    std::optional<py::gil_scoped_release> unlocked;
+    if (PyGILState_Check()) unlocked.emplace();
     // one copy to the host per new packing (none for a tensor that lives there)
     const Tensor host = cu_seqlens.detach().to(at::kCPU, at::kInt).contiguous();
     TORCH_CHECK_VALUE(host.dim() == 1 && host.numel() >= 2 && host.data_ptr<int32_t>()[0] == 0,

@@ -235,3 +235,37 @@ def test_hf_auto_model_loss_matches_oracle_attention_packed_and_dense():
         g = getattr(gpu.model.layers[0].attn, name).weight.grad.float().cpu()
         r = getattr(ref.model.layers[0].attn, name).weight.grad
         assert rel_l2(g, r) <= 5e-2, name
+
+
+def test_other_threads_run_while_a_new_packing_is_copied_to_the_host():
+    import threading
+    import time
+    from flame_amd import sb_attn_varlen
+    a = torch.randn(8192, 8192, device="cuda").to(torch.bfloat16)
+    out = torch.empty_like(a)
+    q = torch.randn(2, 256, 64, device="cuda").to(torch.bfloat16)
+    cu = [torch.tensor([0, 100, 256], dtype=torch.int32, device="cuda") for _ in range(2)]
+    sb_attn_varlen(q, q, q, cu[0], 156)                          # everything is loaded
+    torch.mm(a, a, out=out)
+    torch.cuda.synchronize()
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(0.001)
+
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        for _ in range(150):                                     # some 150 ms of work in front of the copy
+            torch.mm(a, a, out=out)
+        begin = time.perf_counter()
+        sb_attn_varlen(q, q, q, cu[1], 156)
+        end = time.perf_counter()
+    finally:
+        stop.set()
+        thread.join()
+    assert end - begin > 0.02                                    # the copy did wait
+    seen = [begin] + [t for t in ticks if begin < t < end] + [end]
+    assert max(b - a for a, b in zip(seen, seen[1:])) < (end - begin) / 2
