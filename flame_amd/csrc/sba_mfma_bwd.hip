@@ -117,6 +117,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     float dr = 0.f;
     if (row_ok && p.d_rem.ptr)
         dr = Elem16::load(p.d_rem.ptr, (int64_t)job.seq * p.d_rem.sb + (int64_t)head * p.d_rem.sh + job.tok0 + qi);
+    if (first > 0) Gc = dr * 0.f;              // nothing left of the stick there: 0, and NaN where dr is no number, as in a full sweep
     wait_global_memory();
     __syncthreads();
     // (behind the prologue's loads: a store in front of them would keep the compiler from issuing them together,
@@ -292,6 +293,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dq2_kernel(KParams p
     float dr = 0.f;
     if (row_ok && p.d_rem.ptr)
         dr = Elem16::load(p.d_rem.ptr, (int64_t)job.seq * p.d_rem.sb + (int64_t)head * p.d_rem.sh + job.tok0 + qi);
+    if (first > 0) Gc = dr * 0.f;              // (see the one-step kernel)
     wait_global_memory();
     __syncthreads();
     if (grp == 0) store_scaled_q<D>(p, job, head, qi, lane, qf);      // (placed as in the one-step kernel)

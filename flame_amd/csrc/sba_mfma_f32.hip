@@ -338,6 +338,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void bwd_dq_kernel(KPara
     const int n_steps = kmax >= 0 ? kmax / kKeyBlock + 1 : 0;
     const int64_t tabq = tab_index(p, grp.head, job, job.rb, 0) + 32 * grp.sub + n;
     const int first = __builtin_amdgcn_readfirstlane(((const int32_t*)p.rtab)[live_index(p, grp.head, job, job.rb) + grp.sub]);
+    if (first > 0) Gc = dr * 0.f;                          // (see the bf16 dQ kernel)
     if (S == 1 || wave == 3) close_group_ranges(p, grp, lane, first);
 
     // (whole fours of steps: every wave keeps its share of them wherever a sweep begins)

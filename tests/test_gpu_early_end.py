@@ -74,3 +74,22 @@ def test_against_the_oracle(D):
     ref = O.sb_attn_grads_oracle(*(t.cpu() for t in x))
     for a, b in zip(got, ref):
         assert rel_l2(a.float().cpu(), b) <= 2e-2
+
+
+@pytest.mark.parametrize("B,T,D,dtype", [
+    (1, 1100, 64, torch.bfloat16),         # two steps an iteration
+    (5, 1100, 64, torch.bfloat16),         # one step
+    (1, 1100, 128, torch.float16),
+    (1, 1100, 64, torch.float32),
+])
+def test_a_gradient_of_rem_that_is_no_number_shows_where_the_stick_is_used_up(B, T, D, dtype, monkeypatch):
+    # the first head (logits near 0) uses its stick up within some 150 keys; inf * 0 and NaN * 0 of a row whose sweep ended are NaN
+    x = list(_inputs(4, (B,), T, D, dtype, 11))
+    dr = x[4]
+    dr[0, 0, 700], dr[0, 0, 901], dr[0, 0, 1099] = float("inf"), float("nan"), -float("inf")
+    dq, dk = _run(x, None, False)[2:4]
+    monkeypatch.setenv("SBA_FULL_SWEEPS", "1")
+    full = _run(x, None, False)[2]
+    assert torch.equal(dq.isnan(), full.isnan()) and torch.equal(dq.nan_to_num(7), full.nan_to_num(7))
+    assert bool(dq[0, 0, [700, 901, 1099]].isnan().all())
+    assert bool(dk[0, 0, [690, 890, 1090]].isnan().all())        # the keys that these rows still reach
