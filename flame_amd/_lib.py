@@ -35,7 +35,6 @@ class SbaParams(C.Structure):
         ("n_heads", C.c_int32), ("seq_len", C.c_int32), ("total_tokens", C.c_int32),
         ("head_dim", C.c_int32), ("attend_current", C.c_int32), ("scale", C.c_float),
         ("save_for_backward", C.c_int32), ("bwd_phases", C.c_int32),
-        ("columns", C.c_int32),
         ("cu_seqlens", C.c_void_p), ("schedule", C.c_void_p), ("n_schedule", C.c_int32),
         ("table_cols", C.c_int64),
         ("q", SbaTensor), ("k", SbaTensor), ("v", SbaTensor), ("o", SbaTensor),
@@ -43,6 +42,7 @@ class SbaParams(C.Structure):
         ("dq", SbaTensor), ("dk", SbaTensor), ("dv", SbaTensor),
         ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t),
         ("bwd_scratch", C.c_void_p), ("bwd_scratch_bytes", C.c_size_t), ("stream", C.c_void_p),
+        ("columns", C.c_int32), ("reserved", C.c_int32 * 3),
     ]
 
 

@@ -98,14 +98,19 @@ sba::VectorArg cvt(const SbaVector& t) { return sba::VectorArg{(char*)t.ptr, t.s
 // element type, stay below 2^31.
 constexpr int64_t kMaxTokenStride = (INT64_C(1) << 31) / (64 * 4) - 1;
 
+// the fields behind SBA_PARAMS_BASE_SIZE exist only where the caller's structure has them
+bool whole_params(const SbaParams* p) { return p->struct_size == sizeof(SbaParams); }
+int columns_field(const SbaParams* p) { return whole_params(p) ? p->columns : 0; }
+
 int check_common(const SbaParams* p) {
     if (!p) return SBA_ERR_NULL;
-    if (p->struct_size != sizeof(SbaParams)) return SBA_ERR_ABI;
+    if (!whole_params(p) && p->struct_size != SBA_PARAMS_BASE_SIZE) return SBA_ERR_ABI;
+    if (whole_params(p) && (p->reserved[0] || p->reserved[1] || p->reserved[2])) return SBA_ERR_ABI;
     if (p->dtype != SBA_DTYPE_F32 && !is_16bit(p)) return SBA_ERR_DTYPE;
     if (p->n_seq <= 0 || p->n_heads <= 0 || p->seq_len <= 0 || p->total_tokens <= 0) return SBA_ERR_SHAPE;
     if (p->head_dim <= 0 || p->head_dim > sba::kMaxHeadDim) return SBA_ERR_SHAPE;
-    if (p->columns && (p->columns < 72 || p->columns > 96 || (p->columns & 7) || p->head_dim != 128 || !is_16bit(p) || !use_mfma_bwd(p)))
-        return SBA_ERR_SHAPE;
+    const int columns = columns_field(p);
+    if (columns && (columns < 72 || columns > 96 || (columns & 7) || p->head_dim != 128 || !is_16bit(p) || !use_mfma_bwd(p))) return SBA_ERR_SHAPE;
     if (!p->q.ptr || !p->k.ptr || !p->v.ptr) return SBA_ERR_NULL;
     if (p->cu_seqlens) {
         if (!p->schedule || p->n_schedule <= 0 || p->table_cols <= 0) return SBA_ERR_SCHEDULE;
@@ -130,8 +135,9 @@ KParams make_kparams(const SbaParams* p) {
     memset(&kp, 0, sizeof(kp));
     kp.n_seq = p->n_seq; kp.n_heads = p->n_heads; kp.seq_len = p->seq_len;
     kp.total_tokens = p->total_tokens;
-    kp.head_dim = p->columns ? 96 : p->head_dim;           // rows of 72 .. 96 columns: the kernels of that width
-    kp.cols = p->columns ? p->columns : p->head_dim;
+    const int columns = columns_field(p);
+    kp.head_dim = columns ? 96 : p->head_dim;              // rows of 72 .. 96 columns: the kernels of that width
+    kp.cols = columns ? columns : p->head_dim;
     kp.attend_current = p->attend_current ? 1 : 0;
     kp.save = p->save_for_backward ? 1 : 0;
     kp.early_end = full_sweeps() ? 0 : 1;
@@ -210,7 +216,7 @@ const char* sba_error_string(int code) {
         case SBA_ERR_WORKSPACE: return "workspace / bwd_scratch missing or smaller than sba_workspace_bytes() / sba_bwd_scratch_bytes()";
         case SBA_ERR_SCHEDULE: return "packed layout needs a row-block schedule from sba_build_schedule()";
         case SBA_ERR_LAUNCH: return "kernel launch failed";
-        case SBA_ERR_ABI: return "SbaParams.struct_size does not match this library";
+        case SBA_ERR_ABI: return "SbaParams.struct_size does not match this library, or a reserved field is not 0";
         case SBA_ERR_STATIC_LIMIT: return "problem needs more backward scratch than sba_bwd_static() holds (SBA_STATIC_SCRATCH_BYTES); use sba_bwd() with a caller-allocated bwd_scratch";
         default: return "unknown error";
     }
@@ -364,7 +370,8 @@ int sba_bwd_static(const SbaParams* p) {
     if (rc) return rc;
     // Nothing in the array has to start at zero: the matrix-core kernels write every table entry
     // before they read it, and the generic path clears its accumulators with a fill kernel.
-    SbaParams q = *p;
+    SbaParams q = {};
+    memcpy(&q, p, p->struct_size);             // (checked: the size of the caller's structure)
     q.bwd_scratch = ptr;
     q.bwd_scratch_bytes = SBA_STATIC_SCRATCH_BYTES;
     return sba_bwd(&q);

@@ -57,7 +57,7 @@ enum {
     SBA_ERR_WORKSPACE = -4,   /* workspace or bwd_scratch missing or too small */
     SBA_ERR_SCHEDULE = -5,    /* packed layout without a row-block schedule */
     SBA_ERR_LAUNCH = -6,      /* hipGetLastError() after a launch was not hipSuccess */
-    SBA_ERR_ABI = -7,         /* struct_size does not match this library */
+    SBA_ERR_ABI = -7,         /* struct_size does not match this library, or a reserved field is not 0 */
     SBA_ERR_STATIC_LIMIT = -8 /* sba_bwd_static(): the problem needs more scratch than the library holds */
 };
 
@@ -77,7 +77,7 @@ typedef struct SbaVector {
 } SbaVector;
 
 typedef struct SbaParams {
-    uint32_t struct_size;      /* = sizeof(SbaParams); checked */
+    uint32_t struct_size;      /* = sizeof(SbaParams), or SBA_PARAMS_BASE_SIZE; checked */
     int32_t  dtype;            /* SBA_DTYPE_*: element type of q,k,v,o,rem,do,drem,dq,dk,dv */
     int32_t  n_seq;            /* B (dense) or number of documents (packed) */
     int32_t  n_heads;
@@ -91,10 +91,6 @@ typedef struct SbaParams {
     int32_t  bwd_phases;       /* backward only: 0 = whole backward; 1 = first kernel only (dq and the
                                   prefix table), 2 = second kernel only (dk, dv; needs phase 1 done on
                                   the same workspace).  Lets a profiler time the kernels one by one */
-    int32_t  columns;          /* 0: the tensors have head_dim columns.  With head_dim 128 and a 16-bit dtype on the matrix-core
-                                  kernels it may be 72, 80, 88 or 96: the tensors' rows are that long, nothing outside them is
-                                  read or written, and the results are those of rows padded with zeros to 128.  (In the four
-                                  bytes in front of the pointers that were padding before: sizes and offsets are as they were) */
 
     const int32_t* cu_seqlens; /* device, n_seq+1 entries, or NULL for dense */
     const int32_t* schedule;   /* device, from sba_build_schedule(); packed layout only */
@@ -113,7 +109,17 @@ typedef struct SbaParams {
     void*    bwd_scratch;      /* backward only: device memory for the call, see sba_bwd_scratch_bytes() */
     size_t   bwd_scratch_bytes;
     void*    stream;           /* hipStream_t */
+
+    /* A structure may end here (struct_size = SBA_PARAMS_BASE_SIZE): it is taken as one with zeros below. */
+
+    int32_t  columns;          /* 0: the tensors have head_dim columns.  With head_dim 128 and a 16-bit dtype on the matrix-core
+                                  kernels it may be 72, 80, 88 or 96: the tensors' rows are that long, nothing outside them is
+                                  read or written, and the results are those of rows padded with zeros to 128 */
+    int32_t  reserved[3];      /* 0 */
 } SbaParams;
+
+/* Size of the structure before `columns`, which callers built against the first headers of this ABI version give. */
+#define SBA_PARAMS_BASE_SIZE ((uint32_t)offsetof(SbaParams, columns))
 
 /* Library identity: SBA_ABI_VERSION it was built with. */
 int sba_abi_version(void);

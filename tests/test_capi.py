@@ -37,6 +37,31 @@ def test_abi_version_and_struct_size(lib):
     assert b"struct_size" in lib.sba_error_string(-7)
 
 
+def test_structure_without_the_later_fields(lib):
+    # a caller built before `columns` existed gives the shorter structure; what lies in its padding and behind it is its own business
+    p = _lib.SbaParams()
+    base = _lib.SbaParams.columns.offset
+    assert base == _lib.SbaParams.stream.offset + 8 and C.sizeof(_lib.SbaParams) == base + 16
+    p.struct_size = base
+    p.dtype = _lib.SBA_DTYPE_BF16
+    p.n_seq, p.n_heads, p.seq_len, p.total_tokens, p.head_dim = 1, 2, 64, 64, 128
+    padding = _lib.SbaParams.bwd_phases.offset + 4
+    assert padding + 4 == _lib.SbaParams.cu_seqlens.offset
+    C.memset(C.addressof(p) + padding, 0xAB, 4)
+    C.memset(C.addressof(p) + base, 0xAB, 16)
+    assert lib.sba_fwd(C.byref(p)) == -1          # NULL q/k/v, behind the checks of size and shape
+    assert lib.sba_bwd_static(C.byref(p)) == -1
+    p.struct_size = C.sizeof(_lib.SbaParams)      # the fields are looked at where the structure has them
+    assert lib.sba_fwd(C.byref(p)) == -7
+    p.reserved[:] = [0, 0, 0]
+    assert lib.sba_fwd(C.byref(p)) == -2          # columns is no number of columns
+    p.columns = 80
+    assert lib.sba_fwd(C.byref(p)) == -1
+    for size in (0, base - 8, base + 8, C.sizeof(_lib.SbaParams) + 8):
+        p.struct_size = size
+        assert lib.sba_fwd(C.byref(p)) == -7
+
+
 def test_argument_checks_without_gpu(lib):
     p = _lib.SbaParams()
     p.struct_size = C.sizeof(_lib.SbaParams)
