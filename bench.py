@@ -396,12 +396,17 @@ def main():
     # row's stick is used up after some 150 keys, and by default a sweep ends there.  The default's time is reported beside it.
     os.environ["SBA_FULL_SWEEPS"] = "1"
     settle_clocks(step)
-    for _ in range(args.warmup):
-        step()
     # Kernel durations come from HIP events on the launch stream inside the timed region, on a
     # few evenly spaced steps: an event record stalls the queue for a few microseconds, and five of
-    # them on every step would cost this workload more than a tenth of its time.
+    # them on every step would cost this workload more than a tenth of its time.  A step with events goes through the Python
+    # layer of the operator (the others through the native one), which the warm-up has to have met as well: its first pass takes the
+    # host 0.3 to 0.6 ms (16 to 28 us of each of 20 steps, which was the difference between the step and its three kernels).
     every = max(1, args.steps // KERNEL_TIMING_SAMPLES)
+    timer = profiling.KernelTimer(every=every)
+    profiling.install(timer)
+    for _ in range(args.warmup):
+        timer.next_step()
+        step()
     timer = profiling.KernelTimer(every=every)
     profiling.install(timer)
     torch.cuda.synchronize()
