@@ -36,10 +36,11 @@ def plain(m: nn.Module, kind: type) -> bool:
                      or _module._global_backward_hooks or _module._global_backward_pre_hooks))
 
 
-def _weight(m: nn.Module, like: torch.Tensor):
-    """The fp32 weight of a plain module without bias, contiguous on x's device; None otherwise."""
+def _weight(m: nn.Module, like: torch.Tensor, *shape: int):
+    """The fp32 weight of this shape of a plain module without bias, contiguous on x's device; None otherwise (the module says what
+    is wrong with another shape)."""
     w = m.weight
-    if type(w) is not nn.Parameter or w.dtype != torch.float32 or w.device != like.device or not w.is_contiguous():
+    if type(w) is not nn.Parameter or w.dtype != torch.float32 or w.device != like.device or not w.is_contiguous() or w.shape != shape:
         return None
     return w if getattr(m, "bias", None) is None else None
 
@@ -48,9 +49,9 @@ def _eps(norm: nn.RMSNorm) -> float:
     return torch.finfo(torch.float32).eps if norm.eps is None else norm.eps
 
 
-def _norm_fits(norm: nn.Module) -> bool:
-    return (plain(norm, nn.RMSNorm) and len(norm.normalized_shape) == 1 and norm.normalized_shape[0] % 8 == 0
-            and norm.normalized_shape[0] <= _lib.native().max_norm_width)
+def _norm_fits(norm: nn.Module, width: int) -> bool:
+    return (plain(norm, nn.RMSNorm) and tuple(norm.normalized_shape) == (width,) and width % 8 == 0
+            and width <= _lib.native().max_norm_width)
 
 
 def block(blk: nn.Module, x: torch.Tensor, kwargs: dict):
@@ -58,23 +59,26 @@ def block(blk: nn.Module, x: torch.Tensor, kwargs: dict):
     t = _compute_dtype(x)
     if t is None:
         return None
-    attn, mlp = blk.attn, blk.mlp
-    if not (plain(attn, blk.attention_class) and plain(mlp, blk.mlp_class) and _norm_fits(blk.attn_norm) and _norm_fits(blk.mlp_norm)):
+    attn, mlp, width = blk.attn, blk.mlp, x.shape[2]
+    if not (plain(attn, blk.attention_class) and plain(mlp, blk.mlp_class) and _norm_fits(blk.attn_norm, width)
+            and _norm_fits(blk.mlp_norm, width)):
         return None
     if attn.attn_fn is not sb_attn or attn.attn_varlen_fn is not sb_attn_varlen or not attn.fuse_qkv or attn.head_dim not in (64, 128) \
-            or attn.head_dim * attn.num_heads != x.shape[2] or kwargs.get("attention_mask") is not None:
+            or attn.head_dim * attn.num_heads != width or kwargs.get("attention_mask") is not None:
         return None
     cu_seqlens = kwargs.get("cu_seqlens")
     if cu_seqlens is not None and x.shape[0] != 1:
         return None                              # the layer says what is wrong with that
-    ws = []
-    for m in (blk.attn_norm, attn.q_proj, attn.k_proj, attn.v_proj, attn.o_proj, blk.mlp_norm, mlp.gate_proj, mlp.up_proj, mlp.down_proj):
-        w = _weight(m, x) if (type(m) is nn.RMSNorm or plain(m, nn.Linear)) else None
+    inner = mlp.gate_proj.weight.shape[0]
+    if inner % 8:
+        return None
+    square, ws = (width, width), []
+    for m, shape in ((blk.attn_norm, (width,)), (attn.q_proj, square), (attn.k_proj, square), (attn.v_proj, square), (attn.o_proj, square),
+                     (blk.mlp_norm, (width,)), (mlp.gate_proj, (inner, width)), (mlp.up_proj, (inner, width)), (mlp.down_proj, (width, inner))):
+        w = _weight(m, x, *shape) if (type(m) is nn.RMSNorm or plain(m, nn.Linear)) else None
         if w is None:
             return None
         ws.append(w)
-    if ws[6].shape[0] % 8 or ws[6].shape != ws[7].shape:
-        return None
     max_len = kwargs.get("max_seqlen")
     return _lib.native().block(x, ws, attn.num_heads, _eps(blk.attn_norm), _eps(blk.mlp_norm), t, cu_seqlens,
                                x.shape[1] if max_len is None else int(max_len))
@@ -83,9 +87,9 @@ def block(blk: nn.Module, x: torch.Tensor, kwargs: dict):
 def head(x: torch.Tensor, norm: nn.Module, lm_head: nn.Module):
     """lm_head(norm(x)) as one node, or None."""
     t = _compute_dtype(x)
-    if t is None or not (_norm_fits(norm) and plain(lm_head, nn.Linear)):
+    if t is None or not (_norm_fits(norm, x.shape[2]) and plain(lm_head, nn.Linear)):
         return None
-    n, w = _weight(norm, x), _weight(lm_head, x)
+    n, w = _weight(norm, x, x.shape[2]), _weight(lm_head, x, lm_head.weight.shape[0], x.shape[2])
     # a vocabulary that is no multiple of 8 is not for the kernel of the weight's gradient (weight_grads_fit() in sba_model.h)
     if n is None or w is None or w.shape[0] % 8:
         return None

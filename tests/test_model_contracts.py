@@ -41,6 +41,32 @@ def test_weight_gradients_outside_their_contract_are_refused():
             grad(d, x)
 
 
+def test_weights_of_other_shapes_are_left_to_the_modules_to_refuse(native, monkeypatch):
+    from flame_amd.modeling_sba import SBABlock, SBAConfig
+    from oracle import sb_oracle as O
+    monkeypatch.setattr(fused, "_compute_dtype", lambda x: torch.bfloat16)
+    cfg = SBAConfig(hidden_size=128, num_heads=2, intermediate_size=192)
+    x = torch.randn(1, 5, 128)
+    assert fused.block(SBABlock(cfg, 0), x, {}) is not None
+    for name, shape in (("attn_norm", (136,)), ("mlp_norm", (64,)), ("attn.q_proj", (136, 128)), ("attn.k_proj", (128, 120)),
+                        ("attn.v_proj", (64, 128)), ("attn.o_proj", (128, 64)), ("mlp.gate_proj", (192, 64)), ("mlp.up_proj", (200, 128)),
+                        ("mlp.down_proj", (128, 184))):
+        blk = SBABlock(cfg, 0)
+        monkeypatch.setattr(blk.attn, "attn_fn", lambda q, k, v, t: O.sb_attn_oracle(q, k, v))
+        with pytest.raises((RuntimeError, ValueError)):
+            m = blk.get_submodule(name)
+            m.weight = torch.nn.Parameter(torch.randn(shape))
+            if "norm" in name:
+                m.normalized_shape = shape
+            blk.attn.attn_fn = fused.sb_attn                      # as far as fused.block() can tell, a usual block
+            assert fused.block(blk, x, {}) is None
+            blk.attn.attn_fn = lambda q, k, v, t: O.sb_attn_oracle(q, k, v)
+            blk(x)
+    norm, wide, head = torch.nn.RMSNorm(128), torch.nn.RMSNorm(136), torch.nn.Linear(128, 64, bias=False)
+    assert fused.head(x, norm, head) is not None
+    assert fused.head(x, wide, head) is None and fused.head(x, norm, torch.nn.Linear(136, 64, bias=False)) is None
+
+
 def _adamw_after_one_step():
     p = torch.nn.Parameter(torch.ones(4))
     opt = torch.optim.AdamW([p], lr=1e-3, fused=True)
