@@ -18,9 +18,22 @@ from .stickbreaking_attention import profiling, sb_attn, sb_attn_varlen
 _HALF = (torch.bfloat16, torch.float16)
 
 
+def _observed() -> bool:
+    """Someone looks at the operators of this thread one by one (a dispatch mode: tracing, counting, selective checkpointing) or
+    transforms them (torch.func); a kernel launched beside them would be missed."""
+    return torch._C._len_torch_dispatch_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None
+
+
+def _tensor(t) -> bool:
+    """A tensor itself, and not of a class that may mean something else by its operators."""
+    return type(t) is torch.Tensor or type(t) is nn.Parameter
+
+
 def _compute_dtype(x: torch.Tensor):
     """The 16-bit type that products run in, or None where the native nodes do not apply."""
     if not x.is_cuda or x.dtype != torch.float32 or x.dim() != 3 or x.numel() == 0 or not profiling.native():
+        return None
+    if not _tensor(x) or _observed():
         return None
     if not torch.is_autocast_enabled("cuda"):
         return None
@@ -101,7 +114,7 @@ def next_token_loss(logits: torch.Tensor, labels: torch.Tensor, ignore: int = -1
     ignored), or None."""
     if not (logits.is_cuda and logits.dtype in _HALF and logits.dim() == 3 and logits.shape[-1] % 8 == 0 and labels.numel() > 0
             and labels.dtype == torch.int64 and labels.device == logits.device and labels.shape == logits.shape[:2]
-            and profiling.native()):
+            and _tensor(logits) and _tensor(labels) and profiling.native() and not _observed()):
         return None
     return _lib.native().next_token_loss(logits, labels, ignore)
 

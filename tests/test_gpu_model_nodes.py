@@ -325,3 +325,34 @@ def test_frozen_weights_cost_no_gradients():
                 if pick == ["attn.q_proj.weight", "attn.v_proj.weight"]:
                     spared.remove("attn.k_proj.weight")
                 assert used <= bytes_full - sum(weights[n].numel() * 4 for n in spared), pick
+
+
+def test_observed_and_transformed_operators_keep_the_module_path():
+    from torch.utils.flop_counter import FlopCounterMode
+    from flame_amd import fused
+    from flame_amd.modeling_sba import SBAConfig, SBAForCausalLM, next_token_loss
+
+    class Other(torch.Tensor):
+        pass
+
+    torch.manual_seed(0)
+    m = SBAForCausalLM(SBAConfig(hidden_size=128, num_heads=2, num_hidden_layers=1, vocab_size=64)).cuda()
+    ids = torch.randint(0, 64, (1, 20), device="cuda")
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16), FlopCounterMode(display=False) as counter:
+        m(ids)
+    block = 4 * 128 ** 2 + 3 * 128 * m.model.layers[0].mlp.gate_proj.weight.shape[0]
+    assert counter.get_total_flops() == 2 * 20 * (block + 128 * 64)
+    logits = torch.randn(3, 1, 20, 64, device="cuda").to(torch.bfloat16)
+    each = torch.func.vmap(lambda x: next_token_loss(x, ids))(logits)
+    grads = torch.func.grad(lambda x: next_token_loss(x, ids))(logits[0])
+    leaf = logits.clone().requires_grad_()
+    want = [next_token_loss(x, ids) for x in leaf]
+    want[0].backward()
+    for a, b in zip(each, want):
+        assert abs(float(a) - float(b.detach())) <= 1e-5 * float(b.detach())
+    assert rel_l2(grads.float(), leaf.grad[0].float()) <= 5e-3
+    assert fused.next_token_loss(logits[0].as_subclass(Other), ids) is None
+    x = torch.randn(1, 20, 128, device="cuda")
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert fused.head(x, m.model.norm, m.lm_head) is not None
+        assert fused.head(x.as_subclass(Other), m.model.norm, m.lm_head) is None
