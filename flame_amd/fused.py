@@ -128,7 +128,7 @@ def clip_and_step(params, opt, max_norm: float):
     step_fn = opt.__dict__.get("step")           # a learning-rate scheduler's wrapper notes that a step was taken
     if step_fn is not None and not getattr(step_fn, "_wrapped_by_lr_sched", False):
         return None
-    if getattr(opt, "grad_scale", None) is not None or getattr(opt, "found_inf", None) is not None:
+    if getattr(opt, "grad_scale", None) is not None or getattr(opt, "found_inf", None) is not None or _observed():
         return None
     params = list(params)
     ids = {id(p) for p in params}
@@ -144,6 +144,8 @@ def clip_and_step(params, opt, max_norm: float):
                 continue
             state = opt.state.get(p)
             if id(p) not in ids or not state:    # a first step sets up its state
+                return None
+            if not (_tensor(p) and _tensor(p.grad) and _tensor(state["exp_avg"])):       # (sharded weights, say)
                 return None
             ps.append(p)
             gs.append(p.grad)

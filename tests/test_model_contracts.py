@@ -105,3 +105,24 @@ def test_the_backbone_is_called_where_a_hook_or_a_compiled_call_would_see_it(mon
     monkeypatch.setattr(m.model, "_compiled_call_impl", lambda *a, **k: seen.append(SBAModel) or m.model.forward(*a, **k))
     m(ids)
     assert seen == [SBAModel]
+
+
+def test_clip_and_step_leaves_other_tensor_classes_and_observed_steps_alone(native):
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Other(torch.Tensor):
+        pass
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    p, opt = _adamw_after_one_step()
+    with Mode():
+        assert fused.clip_and_step([p], opt, 1.0) is None
+    plain = p.grad
+    p.grad = plain.as_subclass(Other)
+    assert fused.clip_and_step([p], opt, 1.0) is None
+    p.grad = plain
+    opt.state[p]["exp_avg"] = opt.state[p]["exp_avg"].as_subclass(Other)
+    assert fused.clip_and_step([p], opt, 1.0) is None and not native.calls
