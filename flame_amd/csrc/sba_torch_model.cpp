@@ -28,6 +28,12 @@ using namespace sba_model;
 void ok(int rc) { check_status(rc, "model kernel"); }
 bool is_f16(at::ScalarType t) { return t == at::kHalf; }
 
+// a 16-bit tensor of a caller's: dense, and from a 16-byte boundary on, as the kernels' loads of eight elements are meant to be
+Tensor aligned(const Tensor& t) {
+    const Tensor c = t.contiguous();
+    return (uintptr_t)c.data_ptr() & 15 ? c.clone() : c;
+}
+
 Tensor empty(at::IntArrayRef sizes, const Tensor& like, at::ScalarType t) { return at::empty(sizes, like.options().dtype(t)); }
 
 // fp32 weights as 16-bit ones, stacked along their rows in one buffer each; `groups` says how many weights share a buffer
@@ -421,9 +427,7 @@ struct Head : torch::autograd::Function<Head> {
     static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
         const auto sv = ctx->get_saved_variables();
         c10::DeviceGuard guard(sv[0].device());
-        Tensor d = grads[0].contiguous();
-        if ((uintptr_t)d.data_ptr() & 15) d = d.clone();         // (a caller's own buffer)
-        d = d.view({-1, d.size(-1)});
+        const Tensor d = aligned(grads[0]).view({-1, grads[0].size(-1)});
         variable_list out(5);                                    // x, norm, weight
         if (ctx->needs_input_grad(2)) out[2] = weight_grads({{d, sv[2]}})[0];
         if (ctx->needs_input_grad(0) || ctx->needs_input_grad(1)) {
@@ -473,7 +477,7 @@ Tensor differentiable_loss_grad(const Tensor& logits, const Tensor& labels, cons
 struct Loss : torch::autograd::Function<Loss> {
     static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& labels_in, int64_t ignore) {
         const Tensor labels = labels_in.contiguous();
-        auto r = loss_rows(logits.contiguous(), labels, ignore);
+        auto r = loss_rows(aligned(logits), labels, ignore);
         ctx->save_for_backward({logits, labels, r.lse, r.count});
         ctx->saved_data["ignore"] = ignore;
         return r.mean;
@@ -484,7 +488,7 @@ struct Loss : torch::autograd::Function<Loss> {
         c10::DeviceGuard guard(labels.device());
         if (at::GradMode::is_enabled())
             return {differentiable_loss_grad(sv[0], labels, sv[3], grads[0], ctx->saved_data["ignore"].toInt()), Tensor(), Tensor()};
-        const Tensor logits = sv[0].contiguous(), g = grads[0].contiguous();
+        const Tensor logits = aligned(sv[0]), g = grads[0].contiguous();
         Tensor d = at::empty_like(logits);
         ok(loss_bwd(logits.data_ptr(), labels.data_ptr<int64_t>(), sv[2].data_ptr<float>(), sv[3].data_ptr<float>(),
                     g.data_ptr<float>(), d.data_ptr(), (int)labels.numel(), (int)labels.size(-1), (int)logits.size(-1),
@@ -498,7 +502,7 @@ std::optional<Tensor> next_token_loss(const Tensor& logits, const Tensor& labels
     c10::DeviceGuard guard(logits.device());
     if (at::GradMode::is_enabled() && logits.requires_grad()) return Loss::apply(logits, labels, ignore);
     at::AutoDispatchBelowADInplaceOrView below;
-    return loss_rows(logits.contiguous(), labels.contiguous(), ignore).mean;
+    return loss_rows(aligned(logits), labels.contiguous(), ignore).mean;
 }
 
 // ---------------------------------------------------------------------------------------------- clip and step

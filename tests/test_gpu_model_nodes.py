@@ -145,6 +145,21 @@ def test_loss_edges_against_torch(rows, len_, classes):
     assert rel_l2(a.grad.float(), b.grad.float()) <= 5e-3
 
 
+def test_loss_of_logits_off_a_16_byte_boundary():
+    from flame_amd import fused
+    torch.manual_seed(0)
+    buf = torch.randn(2 * 9 * 264 + 3, device="cuda").to(torch.bfloat16)
+    labels = torch.randint(0, 264, (2, 9), device="cuda")
+    a = buf[3:].view(2, 9, 264).requires_grad_()
+    b = a.detach().clone().requires_grad_()
+    assert a.data_ptr() % 16 and b.data_ptr() % 16 == 0
+    with torch.no_grad():
+        assert torch.equal(fused.next_token_loss(a, labels), fused.next_token_loss(b, labels))
+    for x in (a, b):
+        fused.next_token_loss(x, labels).backward()
+    assert torch.equal(a.grad, b.grad)
+
+
 @pytest.mark.parametrize("max_norm", [1e-2, 1e6])
 def test_clip_and_adamw_in_one_pass_matches_torch(max_norm):
     # lengths around the four values of a load and the chunk a workgroup takes; two parameter groups, one weight without gradient
