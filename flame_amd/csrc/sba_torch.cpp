@@ -10,6 +10,7 @@
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
 #include <ATen/ops/zeros_like.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <torch/csrc/autograd/custom_function.h>
 
@@ -95,6 +96,9 @@ SbaParams params_of(const Problem& pr) {
         // the library chooses its kernels from the longest sweep of the launch: the real longest document
         p.seq_len = std::max(pr.plan->max_len, 1);
         const int32_t* base = pr.plan->buffer.data_ptr<int32_t>();
+        // a packing can leave the cache while a launch on a stream that did not build it still reads it
+        const auto stream = c10::hip::getCurrentHIPStream(pr.q.device().index());
+        if (stream.stream() != pr.plan->built_on) c10::hip::HIPCachingAllocator::recordStream(pr.plan->buffer.storage().data_ptr(), stream);
         p.cu_seqlens = base;
         p.schedule = base + pr.plan->schedule_at;
         p.n_schedule = pr.plan->n_jobs;
@@ -166,6 +170,7 @@ c10::intrusive_ptr<Plan> build_plan(const Tensor& cu_seqlens, int64_t n_heads, c
     const int got = sba_build_schedule(cu, plan->n_docs, (int)n_heads, out + plan->schedule_at, plan->n_jobs);
     TORCH_INTERNAL_ASSERT(got == plan->n_jobs);
     plan->buffer = all.to(device);
+    if (device.is_cuda()) plan->built_on = stream_of(plan->buffer);
     return plan;
 }
 

@@ -14,6 +14,7 @@ using at::Tensor;
 // kept by plan_for(); a backward holds the one its forward used.
 struct Plan : torch::CustomClassHolder {
     Tensor buffer;                       // int32 on the device: cu_seqlens (leading 0), then the schedule
+    hipStream_t built_on = nullptr;      // the stream that `buffer` belongs to
     int64_t schedule_at = 0;             // first schedule int in `buffer`
     int n_docs = 0, n_jobs = 0, max_len = 0, total = 0;
     int64_t table_cols = 0;

@@ -27,7 +27,7 @@ _SCHEDULES: dict = {}
 
 def _schedule_for(cu_seqlens: torch.Tensor, n_heads: int, device: torch.device):
     """(cu int32 on `device` with leading 0, schedule on `device`, n_jobs, max_len, total, table
-    columns).  `cu_seqlens` itself may live anywhere (a CPU tensor spares the host sync); what the
+    columns, the stream that built them).  `cu_seqlens` itself may live anywhere (a CPU tensor spares the host sync); what the
     kernels read is placed on the device of q.  The job order depends on the launch size
     (jobs x heads): one entry per cu_seqlens tensor, device and order."""
     key = (id(cu_seqlens), device)
@@ -44,7 +44,7 @@ def _schedule_for(cu_seqlens: torch.Tensor, n_heads: int, device: torch.device):
         raise ValueError("cu_seqlens must be non-decreasing")
     sched = _lib.build_schedule(cu_host, n_heads)
     entry = (cu_host.to(device), sched.to(device), sched.shape[0], int(lens.max()), int(cu_host[-1]),
-             _lib.table_columns(cu_host))
+             _lib.table_columns(cu_host), _lib.current_stream_handle(device) if device.type == "cuda" else None)
     ref = weakref.ref(cu_seqlens, lambda _r, key=key: _SCHEDULES.pop(key, None))
     _SCHEDULES[key] = (ref, cu_seqlens._version, entry, sched.shape[0] * n_heads >= _lib.DOC_MAJOR_GRID)
     return entry
@@ -64,7 +64,11 @@ def _params(q, k, v, n_docs, max_seqlens, inv_temp, attend_current):
 
 
 def _bind_schedule(p, q, cu_seqlens, max_seqlens):
-    cu_dev, sched, n_jobs, max_len, total, cols = _schedule_for(cu_seqlens, q.shape[0], q.device)
+    cu_dev, sched, n_jobs, max_len, total, cols, built_on = _schedule_for(cu_seqlens, q.shape[0], q.device)
+    if built_on is not None and (p.stream or 0) != built_on:      # (the default stream's handle is 0)
+        # a packing can leave the cache while a launch on a stream that did not build it still reads it
+        for t in (cu_dev, sched):
+            t.record_stream(torch.cuda.current_stream(q.device))
     if total != q.shape[1]:
         raise ValueError(f"cu_seqlens ends at {total} but q has {q.shape[1]} tokens")
     if max_len > max_seqlens:

@@ -269,3 +269,34 @@ def test_other_threads_run_while_a_new_packing_is_copied_to_the_host():
     assert end - begin > 0.02                                    # the copy did wait
     seen = [begin] + [t for t in ticks if begin < t < end] + [end]
     assert max(b - a for a, b in zip(seen, seen[1:])) < (end - begin) / 2
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_packing_that_goes_away_while_another_stream_works_on_it(native, monkeypatch):
+    # the cache drops a packing whose tensor is gone when the next one is built; its schedule has to stay whole until a stream that
+    # did not build it is through
+    from flame_amd import sb_attn_varlen
+    from flame_amd.stickbreaking_attention import profiling
+    if not native:
+        monkeypatch.setattr(profiling, "native", lambda: False)
+    a = torch.randn(8192, 8192, device="cuda").to(torch.bfloat16)
+    out = torch.empty_like(a)
+    lens = [40, 300, 1, 129, 64, 200, 7, 283]
+    q = torch.randn(2, sum(lens), 64, device="cuda").to(torch.bfloat16)
+    attend = lambda cu: sb_attn_varlen(q, q, q, cu, 1024)[0]
+    want = attend(cu_from_lengths(lens).cuda())
+    cu, side = cu_from_lengths(lens).cuda(), torch.cuda.Stream()
+    attend(cu)                                                   # built on this stream
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(100):                                     # some 100 ms in front of the call
+            torch.mm(a, a, out=out)
+        got = attend(cu)
+    del cu
+    others = []
+    for shift in range(1, 6):
+        others.append(cu_from_lengths(lens[shift:] + lens[:shift]).cuda())
+        attend(others[-1])
+    assert not side.query()                                      # the other packings were built before the call ran
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
