@@ -142,8 +142,6 @@ struct CacheEntry {
 std::mutex g_plans_mutex;
 std::unordered_map<CacheKey, CacheEntry, CacheHash> g_plans;
 
-int64_t version_of(const Tensor& t) { return t.is_inference() ? 0 : (int64_t)t._version(); }
-
 c10::intrusive_ptr<Plan> build_plan(const Tensor& cu_seqlens, int64_t n_heads, c10::Device device) {
     // the copy waits for the stream: the program's other threads go on meanwhile
     std::optional<py::gil_scoped_release> unlocked;
@@ -183,8 +181,10 @@ void check_status(int rc, const char* what) {
 }
 
 c10::intrusive_ptr<Plan> plan_for(const Tensor& cu_seqlens, int64_t n_heads, c10::Device device) {
+    // an inference tensor does not say whether it was written to since: nothing is kept for it
+    if (cu_seqlens.is_inference()) return build_plan(cu_seqlens, n_heads, device);
     const CacheKey key{cu_seqlens.unsafeGetTensorImpl(), device.index()};
-    const int64_t version = version_of(cu_seqlens);
+    const int64_t version = (int64_t)cu_seqlens._version();
     {
         std::lock_guard<std::mutex> lock(g_plans_mutex);
         auto it = g_plans.find(key);

@@ -300,3 +300,19 @@ def test_packing_that_goes_away_while_another_stream_works_on_it(native, monkeyp
     assert not side.query()                                      # the other packings were built before the call ran
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+def test_cu_seqlens_written_to_in_place():
+    # also under inference mode, whose tensors have no version to tell by
+    import contextlib
+    from flame_amd import sb_attn_varlen
+    q = torch.randn(2, 300, 64, device="cuda").to(torch.bfloat16)
+    packs = [cu_from_lengths(lens).cuda() for lens in ([100, 200], [170, 130])]
+    want = [sb_attn_varlen(q, q, q, cu, 200)[0] for cu in packs]
+    for mode in (contextlib.nullcontext, torch.inference_mode):
+        with mode():
+            cu = torch.empty_like(packs[0])
+            for _ in range(2):
+                for pack, o in zip(packs, want):
+                    cu.copy_(pack)
+                    assert torch.equal(sb_attn_varlen(q, q, q, cu, 200)[0], o)
