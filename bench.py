@@ -431,6 +431,8 @@ def main():
     f_fb = 12.0 * D * pairs
     tflops = f_fb / (ms * 1e-3) / 1e12
     kern = {name: sum(v_) / len(v_) for name, v_ in timer.durations_ms().items()}
+    if args.workload == "short":
+        kern["bwd"] = kern.pop("bwd_dq") + kern.pop("bwd_dkv")       # sequences of at most 128 tokens: one kernel does both passes
     # algorithmic FLOPs per launch: each of the three kernels carries two of the six
     # counted products (4*d*P); recomputed products are not counted
     per_kernel_flops = 4.0 * D * pairs
@@ -458,14 +460,14 @@ def main():
     }
     if args.workload == "short":
         # algorithmic bytes per launch: q, k, v (+ dO) read once, the outputs written once (bf16), rem and the
-        # carries not counted: forward 4 tensors, dQ pass 5, dK/dV pass 6
+        # carries not counted: forward 4 tensors, backward 7
         unit = tokens * H * D * 2
-        nbytes = {"fwd": 4 * unit, "bwd_dq": 5 * unit, "bwd_dkv": 6 * unit}
+        nbytes = {"fwd": 4 * unit, "bwd": 7 * unit}
         gbs = {n: nbytes[n] / (kern[n] * 1e-3) / 1e9 for n in kern if n in nbytes}
         out["roofline"] = {"bound": "hbm", "kernel": dom, "achieved": round(gbs[dom], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                            "frac": round(gbs[dom] / HBM_PEAK_GBS, 4), "traffic": None,
                            "per_kernel_GBps": {n: round(x, 1) for n, x in gbs.items()},
-                           "step_GBps": round(15 * unit / (ms * 1e-3) / 1e9, 1)}
+                           "step_GBps": round(11 * unit / (ms * 1e-3) / 1e9, 1)}
     fl = issue_floors(args.workload, dom, pairs) if dom in KERNEL_COLUMN else None
     if fl is not None:
         # what the dominant kernel could reach if only instruction issue limited it (MFMA time + vector time): with
