@@ -117,7 +117,7 @@ def make_workload(name, device, dtype_name="bf16"):
         return (torch.randn(shape, generator=g) * scale).to(dtype).to(device)
 
     if name == "d256":
-        # head_dim 256 (no configuration of BASELINE.json; the size the reference would run with BLOCK_D = 256)
+        # head_dim 256 (the size the reference would run with BLOCK_D = 256)
         B, H, T, D = 1, 8, 8192, 256
         q, k, v = rn((B, H, T, D), 0.5), rn((B, H, T, D), 0.5), rn((B, H, T, D), 0.5)
         do = rn((B, H, T, D), 1.0)
@@ -190,7 +190,7 @@ def cpu_baseline(name, reps=3):
     head needs a 1 GiB score matrix per temporary)."""
     import torch
     from oracle import sb_oracle as O
-    # the GPU box gives one GPU's job 16 cores, whatever os.cpu_count() shows there
+    # a job with one GPU is meant to use 16 cores, whatever os.cpu_count() shows
     torch.set_num_threads(min(os.cpu_count() or 1, 16))
     g = torch.Generator().manual_seed(1)
 
@@ -239,7 +239,7 @@ def cpu_baseline(name, reps=3):
 
 
 def parity_sample(name, q, k, v, do, cu, o, rem):
-    """One head of the TIMED tensors against the oracle (the checker of the test-suite, here on a sample small
+    """One head of the TIMED tensors against the oracle (as in the test-suite, here on a sample small
     enough for a few seconds of CPU): cfg2 head 0 whole, forward and all gradients; cfg3 head 0, the first
     documents of the pack (up to 4096 tokens), forward and all gradients; cfg4 head 0, the first 2048 tokens -
     causality makes o, rem and dq of a prefix depend on the prefix alone (dk, dv do not: not compared there).
@@ -339,7 +339,7 @@ def main():
     ap.add_argument("--workload", default="cfg2", choices=["cfg2", "cfg3", "cfg4", "cfg5", "short", "copy", "d256"])
     ap.add_argument("--dtype", default="bf16", choices=["bf16", "f16"],
                     help="element type of the operator workloads (f16: the same kernels compiled for float16; "
-                         "BASELINE.json's configurations are bf16, the default)")
+                         "the configurations cfg2 to cfg5 are bf16, the default)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--carries", default="kept", choices=["kept", "default"],
                     help="kept: the forward keeps its carry tables whatever their size (the kernels as such); default: the "
@@ -362,7 +362,7 @@ def main():
     dev = torch.device("cuda:0")
     if args.autograd_thread == "off":
         # The backward runs in the calling thread instead of autograd's per-device worker: a forward + backward of the
-        # operator then costs the host about 80 us instead of 160-200, which on a box with a slow host is the
+        # operator then costs the host about 80 us instead of 160-200, which with a slow host is the
         # difference between timing the kernels and timing Python.  Same graph, same kernels, same results.
         torch.autograd.set_multithreading_enabled(False)
     if args.workload == "cfg5":
@@ -489,7 +489,7 @@ def main():
                 total = sum(f[which] for f in every_kernel)
                 out["issue_floor"][f"step_pct_of_mfma_peak_at_{which}"] = round(
                     100 * f_fb / (total * 1e-3) / 1e12 / BF16_MFMA_PEAK_TFLOPS, 1)
-    # (the CPU leg is defined for BASELINE's configurations, which are bf16)
+    # (the CPU leg is defined for cfg2 to cfg4, which are bf16)
     if not args.no_cpu_baseline and args.workload not in ("short", "d256") and args.dtype == "bf16":
         out["cpu_baseline"] = cpu_baseline(args.workload)
         o, rem = step()          # the timed tensors once more, for the check below

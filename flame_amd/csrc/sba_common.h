@@ -54,11 +54,18 @@ struct Job { int tok0, len, rb, seq, tab0; };
 
 // Workgroup -> (job, head).  A slot of n_heads consecutive workgroups (which the dispatcher deals round-robin to the 8 XCDs) is
 // one job of every head.  Which head comes first moves on by one from slot to slot in the dense layout and every eighth slot
-// in the packed one: heads differ in how far their sweeps reach, and a head that stayed on one XCD (which is best for the
-// XCD's L2 if all sweeps are full: 6 % at B=1, H=16, T=16384, d=128 with every eighth slot, 12 % with every slot) makes that
-// XCD the last to finish, and the others wait for it, since workgroups are dealt in order.  Mean logits 0 .. -6 over 16 heads,
-// forward + backward: T=16384, d=128 4.92 ms with fixed heads, 4.35 moving every eighth slot, 3.55 every slot; packs of
-// 65536 tokens d=64 1.74 / 1.66 / 1.71, 20011 tokens d=80 472 / 458 / 476 us.  Jobs are sorted by decreasing sweep
+// in the packed one.  A head that stays on one XCD is best for the XCD's L2 if all sweeps are equally long; heads that differ in how far
+// their sweeps reach make one XCD the last to finish, and the others wait for it, since workgroups are dealt in order.  Neither
+// turn is ahead everywhere; forward + backward in us, every slot / every eighth / fixed heads:
+//     mean logits 0 .. -6 over the heads      B=2 H=8 T=16384 d=128 3604 / 3314 / 5497     B=1 H=16 T=8192 d=128 1029 / 1170 / 1207
+//         B=4 H=16 T=4096 d=64 644 / 698 / 758     B=1 H=16 T=8192 d=64 726 / 700 / 756     B=1 H=32 T=4096 d=128 635 / 624 / 627
+//         packs d=64: 65536 tokens, documents up to 16384 1548 / 1502 / 1554     131072 tokens H=8 1567 / 1417 / 1561     32768 tokens
+//         659 / 661 / 657     8192 tokens 212 / 214 / 221     d=128 32768 tokens 1178 / 1193 / 1187
+//     all heads at -6 (sweeps nearly full)     B=2 H=8 T=16384 d=128 6053 / 5968 / 5680     B=1 H=16 T=8192 d=128 1429 / 1355 / 1348
+//         packs d=64: 65536 tokens 1800 / 1740 / 1716     131072 tokens 1775 / 1706 / 1685
+// So turning wins up to 40 % where heads differ and costs up to 7 % where they do not, which no launch can know beforehand (an
+// order by the lengths that the forward leaves behind would be a criterion for the backward); packs, whose documents mix the lengths of
+// a slot already, turn rarely.  Jobs are sorted by decreasing sweep
 // length (longest first); `longest_last` walks the list from its other end (the key-owner
 // pass, whose work grows as the row-block index falls).
 __device__ inline int head_of_block(const KParams& p, int block) {

@@ -1433,7 +1433,8 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
 // A sequence of at most 32 * W tokens fits one workgroup of W waves: its queries (Q and dO) stay in LDS and, as row fragments, in
 // registers, and its key blocks pass by from left to right as in the dQ pass.  Every score is evaluated ONCE: the step's
 // weights and logit gradients go to LDS as 16-bit [query][64 keys] rows, and after a barrier the waves reduce them over all
-// queries into the finished dK and dV rows of the key block (nobody else contributes to them).  q, k, v, dO are read once
+// queries into the finished dK and dV rows of the key block (nobody else contributes to them).  Its weights for dK and dV are the
+// dQ pass's, from Q scaled and rounded to 16 bits as in the forward (the own-keys and paired kernels round scaled K instead).  q, k, v, dO are read once
 // where the two passes read them twice, no prefix table is written or read, and it is one launch.
 // What bounds it is memory (seven tensors' bytes): two workgroups of four waves (80 KB of LDS) or four of two waves (sequences
 // of at most 64 tokens) share a CU at head_dim 64, so that one's loads and stores run under the other's arithmetic; the next key

@@ -2,8 +2,8 @@
 
 The nodes compute what the modules' own forward() does under autocast (fp32 weights and residual stream, 16-bit products, fp32
 normalisation) with the modules' parameters, in one autograd node per block.  They are taken when nothing outside could tell:
-plain modules without hooks, fp32 parameters on the GPU, autocast to a 16-bit type, no tracing.  Everything else runs module by
-module.
+plain modules without hooks, fp32 parameters on the GPU of the shapes that belong together, autocast to a 16-bit type, no tracing, and
+nobody who observes or transforms the operators.  Everything else runs module by module.
 """
 from __future__ import annotations
 

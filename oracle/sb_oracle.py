@@ -1,7 +1,7 @@
 """CPU oracle for stick-breaking attention.  TEST INFRASTRUCTURE ONLY.
 
 This file restates, in plain PyTorch on the CPU, the algorithm of the reference
-operator.  It is the checker that the HIP kernels are compared against; nothing in
+operator.  It is what the HIP kernels are compared against; nothing in
 the shipped package imports it.  Only tests, the smoke check and the benchmark's
 ``cpu_baseline`` leg may call it.
 
