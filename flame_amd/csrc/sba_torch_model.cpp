@@ -222,7 +222,8 @@ variable_list differentiable_once(const variable_list& in, F&& backward) {
     }
     if (!graph) return grads;
     // they depend on what the node's inputs and its incoming gradients do
-    torch::autograd::edge_list edges = torch::autograd::get_current_node()->next_edges();
+    torch::autograd::edge_list edges;
+    if (const auto node = torch::autograd::get_current_node()) edges = node->next_edges();
     for (auto& e : torch::autograd::collect_next_edges(in)) edges.push_back(std::move(e));
     const auto error = std::make_shared<torch::autograd::Error>(
         "the language model's native nodes differentiate once: their gradients cannot be differentiated again", std::move(edges));
