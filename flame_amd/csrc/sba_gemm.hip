@@ -11,15 +11,14 @@
 namespace sba {
 inline namespace SBA_ELEM_NS {
 
-// A workgroup of four waves, one per SIMD, owns a 256 x 256 tile of C; a wave holds 128 x 128 of it (sixteen 32 x 32
-// accumulators, 256 registers).  That is the shape at which the LDS keeps up: per 16 rows of the contraction a wave reads eight
-// operand fragments for sixteen MFMAs, so the four waves' reads (32 KB) and the arriving tiles (16 KB) take 384 of the 544
-// cycles that the MFMAs do; eight waves of 128 x 64 would ask for 48 + 16 KB.
+// A workgroup of four waves, one per SIMD, owns a TM x 256 tile of C; a wave holds TM/2 x 128 of it (with TM = 256 sixty-four 16 x 16
+// accumulators, 256 registers).  That is the shape at which the LDS keeps up: per 32 rows of the contraction a wave reads sixteen
+// operand fragments for sixty-four MFMAs, so the four waves' reads (64 KB) and the arriving tiles (32 KB) take 768 of the 1088 cycles
+// that the MFMAs do; eight waves of 128 x 64 would ask for 96 + 32 KB.
 // Both operands have the contracted index in rows, so every fragment is a transposing fetch (ds_read_b64_tr_b16).
-// Stages of 32 rows, four tile buffers.  In a stage's first half the second half's operands are fetched, then the waves meet
-// once: the buffer is free for stage s + 4 (requested at once, three and a half stages ahead of its use) and stage s + 1 is
-// known to have landed, whose first operands are fetched under the second half's MFMAs.
-constexpr int kTileM = 256, kTileN = 256, kStageRows = 32, kBuffers = 4;
+// Stages of 32 rows, four tile buffers.  The operands of a stage are fetched under the MFMAs of the one before; then the waves meet: the
+// buffer that was read is free for the stage four ahead (requested at once), and the next stage but one is known to have landed.
+constexpr int kTileN = 256, kStageRows = 32, kBuffers = 4;
 constexpr int kTileBytes = kStageRows * 256 * 2;             // one operand's stage: 16 KB
 constexpr int kBBase = kBuffers * kTileBytes;                // A's buffers, then B's
 
@@ -54,7 +53,38 @@ __device__ inline h16x8 fragment(uint32_t a0, uint32_t a1, int imm) {
     return u.b;
 }
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// 16 x 16 x 32: lane l holds row l % 16 (a) or column l % 16 (b), contracted indices 8 * (l / 16) .. + 7; of the result column l % 16,
+// rows 4 * (l / 16) .. + 3.
+__device__ inline f32x4 mfma16(h16x8 a, h16x8 b, f32x4 c) {
+#ifdef SBA_ELEM_F16
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+#else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+#endif
+}
+
+// The same with the sums kept where they are.  The compiler's own instruction may write its result elsewhere, and with 224 of the 256
+// accumulation registers in use it does: 360 moves per four stages.  It does not see the instruction's latency either: settled()
+// before the sums are read.
+__device__ inline void mfma16_in_place(h16x8 a, h16x8 b, f32x4& c) {
+#ifdef SBA_ELEM_F16
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+#else
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+#endif
+}
+template <int N, int M> __device__ inline void settled(f32x4 (&acc)[N][M]) {
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int j = 0; j < M; ++j) asm volatile("" : "+a"(acc[i][j]));
+}
+
+template <int TM>
 __global__ __launch_bounds__(256, 1) void weight_grad_kernel(sba_model::WeightGrads g) {
+    constexpr int TI = TM / 32, TJ = 8;                          // 16-wide blocks of a wave: rows and columns of C
     __shared__ __attribute__((aligned(1024))) char lds[2 * kBuffers * kTileBytes];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
@@ -64,10 +94,10 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(sba_model::WeightGr
     int which = 0;
     while (which + 1 < g.n && t >= g.first_tile[which + 1]) ++which;
     const sba_model::WeightGrad& pr = g.one[which];
-    const int tiles_m = (pr.m + kTileM - 1) / kTileM, tiles_n = (pr.n + kTileN - 1) / kTileN, local = t - g.first_tile[which];
+    const int tiles_m = (pr.m + TM - 1) / TM, tiles_n = (pr.n + kTileN - 1) / kTileN, local = t - g.first_tile[which];
     // bands of four tile rows, walked column by column
     const int band = local / (4 * tiles_n), rows = min(4, tiles_m - 4 * band), in = local - band * 4 * tiles_n;
-    const int m0 = (4 * band + in % rows) * kTileM, n0 = (in / rows) * kTileN;
+    const int m0 = (4 * band + in % rows) * TM, n0 = (in / rows) * kTileN;
 
     // this split's stages of the contraction
     const int all = (g.k + kStageRows - 1) / kStageRows, share = (all + (int)gridDim.y - 1) / (int)gridDim.y;
@@ -75,7 +105,7 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(sba_model::WeightGr
     const int ragged = g.k - (first + nk - 1) * kStageRows;          // rows of the last stage (32 unless it is the end)
 
     TileSource sa, sb;
-    sa.init(pr.a, pr.lda, m0, pr.m, w, lane);
+    sa.init(pr.a, pr.lda, m0, min(pr.m, m0 + TM), w, lane);
     sb.init(pr.b, pr.ldb, n0, pr.n, w, lane);
     sa.at += first * sa.step;
     sb.at += first * sb.step;
@@ -111,30 +141,48 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(sba_model::WeightGr
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     };
 
-    // fetch addresses: [half of the eight rows][column block]; the wave's quarter of the tile is in the base
-    uint32_t fa[2][4], fb[2][4];
+    // fetch addresses: [half of the eight rows][column block]
+    uint32_t fa[2][TI], fb[2][TJ];
     {
-        const int h = lane >> 5, G1 = (lane >> 4) & 1, s = lane & 15;
+        const int h = lane >> 4, s = lane & 15;
+        auto fetch_at = [&](int a, int col) {
+            return lds0 + (uint32_t)tile_offset<256>(8 * h + 4 * a + (s >> 2), col / 8 + ((s & 3) >> 1)) + ((s & 1) << 3);
+        };
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int a = 0; a < 2; ++a) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const uint32_t o = (uint32_t)tile_offset<256>(8 * h + 4 * a + (s >> 2), 4 * c + 2 * G1 + ((s & 3) >> 1)) + ((s & 1) << 3);
-                fa[a][c] = lds0 + (w & 1) * 256 + o;
-                fb[a][c] = lds0 + kBBase + (w >> 1) * 256 + o;
-                asm("" : "+v"(fa[a][c]), "+v"(fb[a][c]));
+            for (int c = 0; c < TI; ++c) {
+                fa[a][c] = fetch_at(a, (w & 1) * (TM / 2) + 16 * c);
+                asm("" : "+v"(fa[a][c]));
             }
+#pragma unroll
+            for (int c = 0; c < TJ; ++c) {
+                fb[a][c] = kBBase + fetch_at(a, (w >> 1) * 128 + 16 * c);
+                asm("" : "+v"(fb[a][c]));
+            }
+        }
     }
 
-    f32x16 acc[4][4];
+    // (formed transposed: a lane then holds four neighbouring columns of a row of C)
+    f32x4 acc[TI][TJ];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    h16x8 va[2][4], vb[2][4];
+        for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    h16x8 va[2][TI], vb[2][TJ];
+    auto fetch = [&](int set, int n, int buf) {
+        if (n < TJ) vb[set][n] = fragment(fb[0][n], fb[1][n], buf * kTileBytes);
+        else va[set][n - TJ] = fragment(fa[0][n - TJ], fa[1][n - TJ], buf * kTileBytes);
+    };
+    constexpr int kFetchEvery = TI * TJ / (TI + TJ) - (TM == 256);       // (in time for the next stage)
+    // behind the MFMAs of stage s: the next but one has landed, and the buffer of the next, which the operand registers now hold, is
+    // free for the stage four behind that one
+    auto turn = [&](int s, int b) __attribute__((always_inline)) {
+        if (s + kBuffers < nk) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (rows_of(s + 2) < kStageRows) clear_from(rows_of(s + 2), (b + 2) % kBuffers);
+        if (s + 1 + kBuffers < nk) request(s + 1 + kBuffers, (b + 1) % kBuffers);
+    };
     if (nk > 0) {
 #pragma unroll
         for (int s = 0; s < kBuffers; ++s)
@@ -143,53 +191,39 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(sba_model::WeightGr
         else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         if (rows_of(0) < kStageRows) clear_from(rows_of(0), 0);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            va[0][c] = fragment(fa[0][c], fa[1][c], 0);
-            vb[0][c] = fragment(fb[0][c], fb[1][c], 0);
-        }
-    }
-    // sixteen MFMAs of one half stage, one fetch of the next half's operands under every second one
-    auto half = [&](int cur, int buf, int row0) {
+        for (int n = 0; n < TI + TJ; ++n) fetch(0, n, 0);
+        turn(-1, kBuffers - 1);
+        // whole groups of four stages, so that the loop has one exit (several cost the compiler copies of the accumulators, 128
+        // spilled registers); a last group is filled up with stages of zeros
+        int s0 = 0;
+        settled(acc);
+        do {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int b = 0; b < kBuffers; ++b) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                acc[i][j] = mfma(va[cur][i], vb[cur][j], acc[i][j]);
-                const int n = i * 4 + j, imm = buf * kTileBytes + row0 * 512;
-                if (n < 4) va[cur ^ 1][n] = fragment(fa[0][n], fa[1][n], imm);
-                else if (n < 8) vb[cur ^ 1][n - 4] = fragment(fb[0][n - 4], fb[1][n - 4], imm);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int n = 0; n < TI * TJ; ++n) {
+                    mfma16_in_place(vb[b & 1][n % TJ], va[b & 1][n / TJ], acc[n / TJ][n % TJ]);
+                    if (n % kFetchEvery == 0 && n / kFetchEvery < TI + TJ) fetch(~b & 1, n / kFetchEvery, (b + 1) % kBuffers);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                turn(s0 + b, b);
             }
-    };
-    // whole groups of four stages, so that the loop has one exit (several cost the compiler copies of the accumulators, 128
-    // spilled registers); a last group is filled up with stages of zeros
-    for (int s0 = 0; s0 < nk; s0 += kBuffers) {
-#pragma unroll
-        for (int b = 0; b < kBuffers; ++b) {
-            const int s = s0 + b;
-            half(0, b, 16);
-            if (s + 3 < nk) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (rows_of(s + 1) < kStageRows) clear_from(rows_of(s + 1), (b + 1) & 3);
-            if (s + kBuffers < nk) request(s + kBuffers, b);
-            half(1, (b + 1) & 3, 0);
-        }
+            s0 += kBuffers;
+        } while (s0 < nk);
+        settled(acc);
     }
 
-    // lane (column lane % 32, h), register r: row 8 * (r / 4) + 4 * h + r % 4
+    // columns 4 * (lane / 16) .. + 3 of a block, row lane % 16 of it
     float* out = (gridDim.y == 1 ? g.out : g.partial + (int64_t)blockIdx.y * g.total) + pr.at;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < TI; ++i) {
+        const int row = m0 + (w & 1) * (TM / 2) + i * 16 + (lane & 15);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int col = n0 + (w >> 1) * 128 + j * 32 + (lane & 31);
-            const int row0 = m0 + (w & 1) * 128 + i * 32 + 4 * (lane >> 5);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = row0 + 8 * (r >> 2) + (r & 3);
-                if (row < pr.m && col < pr.n) out[(int64_t)row * pr.n + col] = acc[i][j][r];
-            }
+        for (int j = 0; j < TJ; ++j) {
+            const int col = n0 + (w >> 1) * 128 + j * 16 + 4 * (lane >> 4);
+            if (row < pr.m && col < pr.n) *(f32x4*)(out + (int64_t)row * pr.n + col) = acc[i][j];
         }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------- projections
@@ -204,15 +238,102 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(sba_model::WeightGr
 // four features of one token, which leave through LDS as whole rows.  4096 x 1024, k = 1024: 13 us.
 using sba_model::Projection;
 
+// What becomes of a wave's products: blocks of 16 features (TI of them; with swiglu TI/2 of gates, then their ups) by 16 tokens
+// (TJ), lane l holding features 4 * (l / 16) .. + 3 of token l % 16 of each.  Rows leave straight from the registers: two blocks'
+// 16-bit halves trade places between neighbouring sixteenths of the wave (v_permlane16_swap), after which a lane holds eight
+// consecutive features of one block and four lanes 64 bytes of a token's row; in fp32 they do so as they are.  (Through LDS, in whole
+// 128-byte lines, the stores of a 128 x 256 tile took 3 us with nothing beside them.)
+// The residual, or gate and up of the backward, can be asked for ahead (`request`, TI loads per 16 tokens, every lane's within the
+// tensor whatever the tile's edge, so that their number is known to the waits of the caller).
+template <int kEpi, int TI, int TJ> struct Results {
+    static constexpr bool kAdd = kEpi == sba_model::kAddResidual, kGlu = kEpi == sba_model::kSwigluFwd, kGluBwd = kEpi == sba_model::kSwigluBwd;
+    static constexpr int kAhead = kAdd || kGluBwd ? TI : 0;        // loads per 16 tokens
+    static constexpr int kStores = kAdd || kGluBwd ? TI : kGlu ? TI / 4 : TI / 2;      // stores per 16 tokens (at least)
+    u32x4 ahead[TJ][kAhead ? kAhead : 1];
+    int tok0, f0, h;               // this lane's first token; its features of block or pair 0
+
+    // (the lane's indices from a copy that the compiler cannot see through: what is made of them would otherwise be worked out ahead of
+    // the caller's loops and kept, 70 spilled registers)
+    __device__ inline void aim(int lane, int tw, int nw) {
+        asm volatile("" : "+v"(lane));
+        h = lane >> 4;
+        tok0 = tw + (lane & 15);
+        f0 = nw + (kAdd ? 4 * h : (h & 1) * 16 + (h >> 1) * 8);
+    }
+    __device__ inline void request(const Projection& p, int j) {
+        const int64_t tok = min(tok0 + 16 * j, p.m - 1);
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            if (kAdd) ahead[j][i] = *(const u32x4*)(p.residual + tok * p.n + min(f0 + 16 * i, p.n - 4));
+            else ahead[j][i] = *(const u32x4*)((const elem16*)p.pre + tok * 2 * p.n + min(f0 + 32 * (i / 2), p.n - 8) + (i & 1) * p.n);
+        }
+    }
+    // features of block a and the block behind it, as 16-bit: eight consecutive ones a lane
+    __device__ static inline h16x8 rows_of(const f32x4& a, const f32x4& b) {
+        auto two = [](float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, y}), h16x2)); };
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        const u32x2 lo = __builtin_amdgcn_permlane16_swap(two(a[0], a[1]), two(b[0], b[1]), false, false);
+        const u32x2 hi = __builtin_amdgcn_permlane16_swap(two(a[2], a[3]), two(b[2], b[3]), false, false);
+        return __builtin_bit_cast(h16x8, (u32x4{lo[0], hi[0], lo[1], hi[1]}));
+    }
+    __device__ inline void store(const Projection& p, const f32x4 (&acc)[TI][TJ], int j) const {
+        const int tok = tok0 + 16 * j, width = kGlu ? p.n / 2 : p.n;
+        const int64_t row = (int64_t)tok * width;
+        if (kAdd) {
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+                if (tok < p.m && f0 + 16 * i < p.n)
+                    *(f32x4*)((float*)p.out + row + f0 + 16 * i) = __builtin_bit_cast(f32x4, ahead[j][i]) + acc[i][j];
+            return;
+        }
+#pragma unroll
+        for (int q = 0; q < (kGlu ? TI / 4 : TI / 2); ++q) {
+            const int n = f0 + 32 * q;
+            const h16x8 y = rows_of(acc[2 * q][j], acc[2 * q + 1][j]);
+            if (kGlu) {
+                const h16x8 u = rows_of(acc[TI / 2 + 2 * q][j], acc[TI / 2 + 2 * q + 1][j]);
+                if (tok >= p.m || n >= width) continue;
+                h16x8 o;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float g = (float)y[e];
+                    o[e] = (elem16)((float)(elem16)(g / (1.f + __expf(-g))) * (float)u[e]);
+                }
+                *(h16x8*)((elem16*)p.out + row + n) = o;
+                if (p.pre) {
+                    *(h16x8*)((elem16*)p.pre + 2 * row + n) = y;
+                    *(h16x8*)((elem16*)p.pre + 2 * row + width + n) = u;
+                }
+            } else if (kGluBwd) {
+                // y is the gradient of silu(gate) * up
+                if (tok >= p.m || n >= width) continue;
+                const h16x8 g = __builtin_bit_cast(h16x8, ahead[j][2 * q]), u = __builtin_bit_cast(h16x8, ahead[j][2 * q + 1]);
+                h16x8 dg, du;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float gf = (float)g[e], df = (float)y[e], sg = 1.f / (1.f + __expf(-gf));
+                    du[e] = (elem16)(df * (float)(elem16)(gf * sg));
+                    dg[e] = (elem16)((float)(elem16)(df * (float)u[e]) * sg * (1.f + gf * (1.f - sg)));
+                }
+                *(h16x8*)((elem16*)p.out + 2 * row + n) = dg;
+                *(h16x8*)((elem16*)p.out + 2 * row + width + n) = du;
+            } else if (tok < p.m && n < width) {
+                *(h16x8*)((elem16*)p.out + row + n) = y;
+            }
+        }
+    }
+};
+
+
 template <bool kRowsW, int kEpi>
 __global__ __launch_bounds__(256, 2) void projection_kernel(Projection p) {
     constexpr int TM = 128, TN = 128, NB = 4;
     constexpr int kX = TM * 64, kW = TN * 64, kStage = kX + kW;        // bytes
     constexpr int PX = TM / 64, PW = TN / 64, P = PX + PW;             // copies per wave and stage
-    constexpr int TI = TN / 64, TJ = TM / 64;                          // 32-wide blocks of a wave: features, tokens
+    constexpr int TI = TN / 32, TJ = TM / 32;                          // 16-wide blocks of a wave: features, tokens
     __shared__ __attribute__((aligned(1024))) char lds[NB * kStage];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m = lane & 31, h = lane >> 5;
+    const int m = lane & 15, h = lane >> 4;
 
     // a swiglu tile's features are TN/2 gates and the TN/2 ups that go with them
     constexpr bool kGlu = kEpi == sba_model::kSwigluFwd;
@@ -260,22 +381,20 @@ __global__ __launch_bounds__(256, 2) void projection_kernel(Projection p) {
         wat += kRowsW ? 64 * p.ldw : (int64_t)64;
     };
 
-    // fetch addresses: X rows and, k contiguous, W rows [k slice]; W columns [half of the eight rows][column block]
-    uint32_t fx[2], fw[2], fc[2][TI];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int c = (2 * s + h) ^ ((m >> 2) & 3);
-        fx[s] = lds0 + (w & 1) * (TM / 2) * 64 + m * 64 + c * 16;
-        fw[s] = lds0 + kX + (w >> 1) * (TN / 2) * 64 + m * 64 + c * 16;
-        asm("" : "+v"(fx[s]), "+v"(fw[s]));
+    // fetch addresses: X rows and, k contiguous, W rows; W columns [half of the eight rows][column block]
+    uint32_t fx, fw, fc[2][TI];
+    {
+        const int c = h ^ ((m >> 2) & 3);
+        fx = lds0 + (w & 1) * (TM / 2) * 64 + m * 64 + c * 16;
+        fw = lds0 + kX + (w >> 1) * (TN / 2) * 64 + m * 64 + c * 16;
+        asm("" : "+v"(fx), "+v"(fw));
     }
     if (kRowsW) {
-        const int G1 = (lane >> 4) & 1, s = lane & 15;
 #pragma unroll
         for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int c = 0; c < TI; ++c) {
-                fc[a][c] = lds0 + kX + (uint32_t)tile_offset<TN>(8 * h + 4 * a + (s >> 2), (w >> 1) * (TN / 16) + 4 * c + 2 * G1 + ((s & 3) >> 1)) + ((s & 1) << 3);
+                fc[a][c] = lds0 + kX + (uint32_t)tile_offset<TN>(8 * h + 4 * a + (m >> 2), (w >> 1) * (TN / 16) + 2 * c + ((m & 3) >> 1)) + ((m & 1) << 3);
                 asm("" : "+v"(fc[a][c]));
             }
     }
@@ -283,151 +402,72 @@ __global__ __launch_bounds__(256, 2) void projection_kernel(Projection p) {
         return *(const __attribute__((address_space(3))) h16x8*)((__attribute__((address_space(3))) char*)(uintptr_t)base + imm);
     };
 
-    f32x16 acc[TI][TJ];
+    f32x4 acc[TI][TJ];
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j < TJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     h16x8 vx[2][TJ], vw[2][TI];
-    // the n-th of the operands of k slice s of buffer `buf`
-    auto fetch = [&](int set, int n, int buf, int s) {
-        if (n < TJ) vx[set][n] = at(fx[s], buf * kStage + n * 2048);
-        else if (n < TJ + TI) {
-            if (kRowsW) vw[set][n - TJ] = fragment(fc[0][n - TJ], fc[1][n - TJ], buf * kStage + s * 16 * TN * 2);
-            else vw[set][n - TJ] = at(fw[s], buf * kStage + (n - TJ) * 2048);
-        }
+    // the n-th of the operands of buffer `buf`
+    auto fetch = [&](int set, int n, int buf) {
+        if (n < TJ) vx[set][n] = at(fx, buf * kStage + n * 1024);
+        else if (kRowsW) vw[set][n - TJ] = fragment(fc[0][n - TJ], fc[1][n - TJ], buf * kStage);
+        else vw[set][n - TJ] = at(fw, buf * kStage + (n - TJ) * 1024);
     };
-    auto half = [&](int cur, int buf, int s) {
-#pragma unroll
-        for (int n = 0; n < TI * TJ; ++n) {
-            const int i = n / TJ, j = n % TJ;
-            acc[i][j] = mfma(vw[cur][i], vx[cur][j], acc[i][j]);
-            fetch(cur ^ 1, n, buf, s);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    static_assert(TI + TJ <= TI * TJ, "one fetch per MFMA");
+    static_assert(TI + TJ <= TI * TJ / 2, "a fetch per two MFMAs");
     auto clear = [&](int buf) {
         for (int c = threadIdx.x; c < kStage / 16; c += 256) *(u32x4*)(lds + buf * kStage + c * 16) = u32x4{0u, 0u, 0u, 0u};
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     };
 
+    Results<kEpi, TI, TJ> res;
+    constexpr int R = Results<kEpi, TI, TJ>::kAhead * TJ;              // loads of the epilogue, asked for in the last four stages, behind all copies
+    auto request_ahead = [&]() __attribute__((always_inline)) {
+        if (R) {
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) res.request(p, j);
+        }
+    };
+    // behind the MFMAs of stage s: the next but one has landed, and the buffer of the next, which the operand registers now hold, is
+    // free for stage s + 1 + NB
+    auto turn = [&](int s, int b, bool asked) __attribute__((always_inline)) {
+        const int behind = nk - 3 - s;                                 // stages behind the one that has to land
+        if (behind >= NB - 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((NB - 2) * P) : "memory");
+        else if (asked && R) {
+            if (behind == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(P + R) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(R) : "memory");
+        } else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(P) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 2 >= nk) clear((b + 2) % NB);
+        if (s + 1 + NB < nk) request((b + 1) % NB);
+    };
+    static_assert(NB == 4, "turn() counts the stages behind by hand");
+
+    res.aim(lane, t0 + (w & 1) * (TM / 2), n0 + (w >> 1) * (kOwn / 2));
 #pragma unroll
     for (int s = 0; s < NB; ++s)
         if (s < nk) request(s);
     if (nk >= NB) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NB - 1) * P) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-    for (int n = 0; n < TI + TJ; ++n) fetch(0, n, 0, 0);
+    for (int n = 0; n < TI + TJ; ++n) fetch(0, n, 0);
+    turn(-1, NB - 1, false);
     for (int s0 = 0; s0 < nk; s0 += NB) {      // whole groups, filled up with stages of zeros (see the weight-gradient kernel)
+        const bool last = s0 + NB >= nk;       // (all copies are on their way by then)
+        if (last) request_ahead();
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const int s = s0 + b;
-            half(0, b, 1);
-            if (s + NB - 1 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((NB - 2) * P) : "memory");
-            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (s + 1 >= nk) clear((b + 1) % NB);
-            if (s + NB < nk) request(b);
-            half(1, (b + 1) % NB, 0);
+#pragma unroll
+            for (int n = 0; n < TI * TJ; ++n) {
+                acc[n / TJ][n % TJ] = mfma16(vw[b & 1][n / TJ], vx[b & 1][n % TJ], acc[n / TJ][n % TJ]);
+                if (n % 2 == 0 && n / 2 < TI + TJ) fetch(~b & 1, n / 2, (b + 1) % NB);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            turn(s0 + b, b, last);
         }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the tiles become the waves' staging
-
-    // 32 tokens at a time: through the wave's own part of LDS into rows
-    char* const stage = lds + w * (NB * kStage / 4);
-    static_assert(NB * kStage / 4 >= 32 * (TN / 2) * 4, "a wave stages 32 tokens' features in fp32");
-    constexpr int F = TN / 2;                                          // features of a wave
-    const int tw = t0 + (w & 1) * (TM / 2), nw = n0 + (w >> 1) * (kOwn / 2);
 #pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-        const int tok0 = tw + 32 * j;
-        if (tok0 >= p.m) break;
-        if (kEpi == sba_model::kAddResidual) {
-            // out = residual + y (rounded to 16 bits, as a tensor of its own would be): 16-byte chunks of four features
-#pragma unroll
-            for (int i = 0; i < TI; ++i)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    typedef float f32x4 __attribute__((ext_vector_type(4)));
-                    f32x4 v;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = (float)(elem16)acc[i][j][4 * g + e];
-                    *(f32x4*)(stage + m * (F * 4) + (((i * 8 + 2 * g + h) ^ m) & (F / 4 - 1)) * 16) = v;
-                }
-            for (int c = lane; c < 32 * F / 4; c += 64) {
-                typedef float f32x4 __attribute__((ext_vector_type(4)));
-                const int row = c / (F / 4), cc = c % (F / 4), tok = tok0 + row, n = nw + 4 * cc;
-                if (tok < p.m && n < p.n) {
-                    const f32x4 v = *(const f32x4*)(stage + row * (F * 4) + ((cc ^ row) & (F / 4 - 1)) * 16);
-                    const f32x4 r = *(const f32x4*)(p.residual + (int64_t)tok * p.n + n);
-                    *(f32x4*)((float*)p.out + (int64_t)tok * p.n + n) = v + r;
-                }
-            }
-        } else {
-            // 16-bit rows of F features, chunks of eight: chunk c of token r at c ^ r
-            constexpr int kChunks = F / 8;
-            auto put = [&](int chunk, const float* v) {
-                const f32x2 a = {v[0], v[1]}, b = {v[2], v[3]};
-                uint2 u;
-                u.x = __builtin_bit_cast(uint32_t, __builtin_convertvector(a, h16x2));
-                u.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(b, h16x2));
-                *(uint2*)(stage + m * (F * 2) + ((chunk ^ m) & (kChunks - 1)) * 16 + h * 8) = u;
-            };
-#pragma unroll
-            for (int i = 0; i < TI; ++i)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const float v[4] = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-                    put(i * 4 + g, v);
-                }
-            auto chunk_of = [&](int row, int cc) { return *(const h16x8*)(stage + row * (F * 2) + ((cc ^ row) & (kChunks - 1)) * 16); };
-            if (kGlu) {
-                // gates are chunks 0 .. kChunks/2 - 1 of a row, their ups the rest
-                for (int c = lane; c < 32 * kChunks / 2; c += 64) {
-                    const int row = c / (kChunks / 2), cc = c % (kChunks / 2), tok = tok0 + row, n = nw + 8 * cc;
-                    if (tok < p.m && n < features) {
-                        const h16x8 g = chunk_of(row, cc), u = chunk_of(row, cc + kChunks / 2);
-                        h16x8 a;
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const float gf = (float)g[e];
-                            a[e] = (elem16)((float)(elem16)(gf / (1.f + __expf(-gf))) * (float)u[e]);
-                        }
-                        *(h16x8*)((elem16*)p.out + (int64_t)tok * features + n) = a;
-                        if (p.pre) {
-                            *(h16x8*)((elem16*)p.pre + (int64_t)tok * p.n + n) = g;
-                            *(h16x8*)((elem16*)p.pre + (int64_t)tok * p.n + features + n) = u;
-                        }
-                    }
-                }
-            } else {
-                for (int c = lane; c < 32 * kChunks; c += 64) {
-                    const int row = c / kChunks, cc = c % kChunks, tok = tok0 + row, n = nw + 8 * cc;
-                    if (tok >= p.m || n >= p.n) continue;
-                    const h16x8 v = chunk_of(row, cc);
-                    if (kEpi == sba_model::kSwigluBwd) {
-                        // y is the gradient of silu(gate) * up: gate and up from `pre`, their gradients to `out`
-                        const elem16* gu = (const elem16*)p.pre + (int64_t)tok * 2 * p.n + n;
-                        elem16* o = (elem16*)p.out + (int64_t)tok * 2 * p.n + n;
-                        const h16x8 g = *(const h16x8*)gu, u = *(const h16x8*)(gu + p.n);
-                        h16x8 dg, du;
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const float gf = (float)g[e], df = (float)v[e], sg = 1.f / (1.f + __expf(-gf));
-                            du[e] = (elem16)(df * (float)(elem16)(gf * sg));
-                            dg[e] = (elem16)((float)(elem16)(df * (float)u[e]) * sg * (1.f + gf * (1.f - sg)));
-                        }
-                        *(h16x8*)o = dg;
-                        *(h16x8*)(o + p.n) = du;
-                    } else {
-                        *(h16x8*)((elem16*)p.out + (int64_t)tok * p.n + n) = v;
-                    }
-                }
-            }
-        }
-    }
+    for (int j = 0; j < TJ; ++j) res.store(p, acc, j);
 }
 
 // Large products: TM x 256 tiles, one resident workgroup a CU that walks tiles, one wave per SIMD with TM/2 x 128 of a tile.
@@ -445,10 +485,10 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
     constexpr int NB = TM == 256 ? 2 : 3;
     constexpr int kX = TM * 128, kStage = kX + 256 * 128;
     constexpr int PX = TM / 32, P = PX + 8;                    // copies per wave and stage
-    constexpr int TJ = TM / 64, kSlots = 4 * TJ;               // blocks of 32 tokens of a wave; MFMAs of a slice
-    __shared__ __attribute__((aligned(1024))) char lds[NB * kStage + 4 * 4096];
+    constexpr int TI = 8, TJ = TM / 32, kSlots = TI * TJ;       // blocks of 16 features and tokens of a wave; MFMAs of a slice
+    __shared__ __attribute__((aligned(1024))) char lds[NB * kStage];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m = lane & 31, h = lane >> 5;
+    const int m = lane & 15, h = lane >> 4;
     constexpr bool kGlu = kEpi == sba_model::kSwigluFwd;
     const int features = kGlu ? p.n / 2 : p.n;
     constexpr int kOwn = kGlu ? 128 : 256;
@@ -513,22 +553,21 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
     };
 
     // ---- operand fetches: X rows and, k contiguous, W rows [slice]; W columns [half of the eight rows][column block]
-    uint32_t fx[4], fw[4], fc[2][4];
+    uint32_t fx[2], fw[2], fc[2][TI];
     const uint32_t lds0 = lds_address(lds);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int c = (2 * q + h) ^ ((m >> 1) & 7);
+    for (int q = 0; q < 2; ++q) {
+        const int c = (4 * q + h) ^ ((m >> 1) & 7);
         fx[q] = lds0 + (w & 1) * (TM / 2) * 128 + m * 128 + c * 16;
         fw[q] = lds0 + kX + (w >> 1) * 128 * 128 + m * 128 + c * 16;
         asm("" : "+v"(fx[q]), "+v"(fw[q]));
     }
     if (kRowsW) {
-        const int G1 = (lane >> 4) & 1, s = lane & 15;
 #pragma unroll
         for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                fc[a][c] = lds0 + kX + (uint32_t)tile_offset<256>(8 * h + 4 * a + (s >> 2), (w >> 1) * 16 + 4 * c + 2 * G1 + ((s & 3) >> 1)) + ((s & 1) << 3);
+            for (int c = 0; c < TI; ++c) {
+                fc[a][c] = lds0 + kX + (uint32_t)tile_offset<256>(8 * h + 4 * a + (m >> 2), (w >> 1) * 16 + 2 * c + ((m & 3) >> 1)) + ((m & 1) << 3);
                 asm("" : "+v"(fc[a][c]));
             }
     }
@@ -538,7 +577,7 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
         uint32_t by = f_buf == 0 ? (uint32_t)-((NB - 1) * kStage) : (uint32_t)kStage;
         asm("" : "+s"(by));
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < 2; ++q) {
             fx[q] += by;
             if (!kRowsW) fw[q] += by;
         }
@@ -546,126 +585,48 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
 #pragma unroll
             for (int a = 0; a < 2; ++a)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) fc[a][c] += by;
+                for (int c = 0; c < TI; ++c) fc[a][c] += by;
         }
     };
     auto at = [](uint32_t base, int imm) {
         return *(const __attribute__((address_space(3))) h16x8*)((__attribute__((address_space(3))) char*)(uintptr_t)base + imm);
     };
-    h16x8 vx[2][TJ], vw[2][4];
+    h16x8 vx[2][TJ], vw[2][TI];
     auto fetch = [&](int set, int n, int q) {
-        if (n < TJ) vx[set][n] = at(fx[q], n * 4096);
-        else if (n < TJ + 4) {
+        if (n < TJ) vx[set][n] = at(fx[q], n * 2048);
+        else if (n < TJ + TI) {
             const int i = n - TJ;
-            if (kRowsW) vw[set][i] = fragment(fc[0][i], fc[1][i], q * 16 * 512);
-            else vw[set][i] = at(fw[q], i * 4096);
+            if (kRowsW) vw[set][i] = fragment(fc[0][i], fc[1][i], q * 32 * 512);
+            else vw[set][i] = at(fw[q], i * 2048);
         }
     };
-    f32x16 acc[4][TJ];
+    f32x4 acc[TI][TJ];
     // MFMAs of one slice; under them the fetches of slice q and copies first .. first + count - 1
+    constexpr int kFetchEvery = TM == 256 ? 3 : 2, kCopyEvery = 4;
+    static_assert((TJ + TI) * kFetchEvery <= kSlots, "the fetches of a slice under the MFMAs of the one before");
     auto slice = [&](int cur, int q, int first, int count, bool fresh = false) __attribute__((always_inline)) {
 #pragma unroll
         for (int n = 0; n < kSlots; ++n) {
-            acc[n / TJ][n % TJ] = mfma(vw[cur][n / TJ], vx[cur][n % TJ], fresh ? f32x16{0} : acc[n / TJ][n % TJ]);
-            fetch(cur ^ 1, n, q);
-            if ((n & 1) && n / 2 < count) copy(first + n / 2);
+            acc[n / TJ][n % TJ] = mfma16(vw[cur][n / TJ], vx[cur][n % TJ], fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[n / TJ][n % TJ]);
+            if (n % kFetchEvery == 0) fetch(cur ^ 1, n / kFetchEvery, q);
+            if (n % kCopyEvery == kCopyEvery - 1 && n / kCopyEvery < count) copy(first + n / kCopyEvery);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // which slices the copies of a stage go under: TM = 256 the fourth and the first, 128 all of them
-    constexpr int C3 = TM == 256 ? 8 : 3, C0 = TM == 256 ? 8 : 3, C1 = TM == 256 ? 0 : 3, C2 = P - C3 - C0 - C1;
-    static_assert(C2 >= 0 && C3 <= kSlots / 2 && C2 <= kSlots / 2, "a copy under every second MFMA");
+    // which slices the copies of a stage go under: TM = 256 the second, 128 both
+    constexpr int C1 = TM == 256 ? 16 : 6, C0 = P - C1;
+    static_assert(C1 <= kSlots / kCopyEvery && C0 <= kSlots / kCopyEvery, "copies of a slice");
 
-    // ---- results: 32 tokens at a time through the wave's 4 KB of staging, 128 bytes of a row: chunk c of token r at c ^ r / 2
-    char* const stage = lds + NB * kStage + w * 4096;
-    auto spot = [&](int row, int c) { return stage + row * 128 + ((c ^ (row >> 1)) & 7) * 16; };
-    // The residual is requested a block of 32 features ahead (block 0 before the tile's last copies): with one wave per SIMD nobody
-    // else has work meanwhile.
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    constexpr bool kAdd = kEpi == sba_model::kAddResidual;
-    constexpr int kChunkBlocks = kAdd ? 1 : 2;                 // blocks of 32 features that are stored together
-    constexpr int kChunks = TJ * 4 / kChunkBlocks;
-    f32x4 ahead[kAdd ? 2 : 1][4];
-    auto read_ahead = [&](int chunk, int t0, int n0) __attribute__((always_inline)) {
-        if (!kAdd || chunk >= kChunks) return;
-        int lane_here = lane;
-        asm volatile("" : "+v"(lane_here));
-        const int tok0 = t0 + (w & 1) * (TM / 2) + 32 * (chunk / 4) + (lane_here >> 3);
-        const int col = n0 + (w >> 1) * 128 + 32 * (chunk % 4) + 4 * (lane_here & 7);
+    // ---- results
+    // With one wave per SIMD nobody else has work while a load is on its way: what the epilogue reads is asked for before the tile's
+    // last slice.
+    Results<kEpi, TI, TJ> res;
+    constexpr int kAhead = Results<kEpi, TI, TJ>::kAhead;
+    auto request = [&](int t0, int n0) __attribute__((always_inline)) {
+        res.aim(lane, t0 + (w & 1) * (TM / 2), n0 + (w >> 1) * (kOwn / 2));
+        if (kAhead) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int tok = tok0 + 8 * c;
-            ahead[chunk & 1][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (tok < p.m && col < p.n) ahead[chunk & 1][c] = *(const f32x4*)(p.residual + (int64_t)tok * p.n + col);
-        }
-    };
-    auto store_tile = [&](int t0, int n0) {
-        const int tw = t0 + (w & 1) * (TM / 2), nw = n0 + (w >> 1) * (kOwn / 2);
-#pragma unroll
-        for (int chunk = 0; chunk < kChunks; ++chunk) {
-            // (this lane's indices from a copy that the compiler cannot see through: the addresses made from them would otherwise be
-            // worked out ahead of the tile loop and kept, 70 spilled registers)
-            int lane_here = lane;
-            asm volatile("" : "+v"(lane_here));
-            const int m = lane_here & 31, h = lane_here >> 5, row8 = lane_here >> 3, cc = lane_here & 7;
-            const int j = chunk * kChunkBlocks / 4, i = chunk * kChunkBlocks % 4, tok0 = tw + 32 * j;
-            read_ahead(chunk + 1, t0, n0);
-            if (kAdd) {                                        // fp32; y rounded to 16 bits as a tensor of its own would be
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    f32x4 v;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = (float)(elem16)acc[i][j][4 * g + e];
-                    *(f32x4*)spot(m, 2 * g + h) = v;
-                }
-                const int n = nw + 32 * i + 4 * cc;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const int tok = tok0 + c * 8 + row8;
-                    const f32x4 v = *(const f32x4*)spot(c * 8 + row8, cc);
-                    if (tok < p.m && n < p.n) *(f32x4*)((float*)p.out + (int64_t)tok * p.n + n) = v + ahead[chunk & 1][c];
-                }
-            } else {                                           // 64 features: two blocks, with swiglu the gates and their ups
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const f32x16& v = acc[kGlu ? i / 2 + 2 * b : i + b][j];
-                        const f32x2 lo = {v[4 * g], v[4 * g + 1]}, hi = {v[4 * g + 2], v[4 * g + 3]};
-                        uint2 u;
-                        u.x = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, h16x2));
-                        u.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, h16x2));
-                        *(uint2*)(spot(m, 4 * b + g) + h * 8) = u;
-                    }
-                if (kGlu) {
-#pragma unroll
-                    for (int c = 0; c < 2; ++c) {
-                        const int row = c * 16 + (lane_here >> 2), tok = tok0 + row, n = nw + 16 * i + 8 * (lane_here & 3);
-                        const h16x8 g = *(const h16x8*)spot(row, lane_here & 3), u = *(const h16x8*)spot(row, 4 + (lane_here & 3));
-                        if (tok < p.m && n < features) {
-                            h16x8 a;
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) {
-                                const float gf = (float)g[e];
-                                a[e] = (elem16)((float)(elem16)(gf / (1.f + __expf(-gf))) * (float)u[e]);
-                            }
-                            *(h16x8*)((elem16*)p.out + (int64_t)tok * features + n) = a;
-                            if (p.pre) {
-                                *(h16x8*)((elem16*)p.pre + (int64_t)tok * p.n + n) = g;
-                                *(h16x8*)((elem16*)p.pre + (int64_t)tok * p.n + features + n) = u;
-                            }
-                        }
-                    }
-                    continue;
-                }
-                const int n = nw + 32 * i + 8 * cc;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const int tok = tok0 + c * 8 + row8;
-                    const h16x8 v = *(const h16x8*)spot(c * 8 + row8, cc);
-                    if (tok < p.m && n < p.n) *(h16x8*)((elem16*)p.out + (int64_t)tok * p.n + n) = v;
-                }
-            }
+            for (int j = 0; j < TJ; ++j) res.request(p, j);
         }
     };
 
@@ -678,36 +639,33 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
     }
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NB - 1) * P) : "memory");
 #pragma unroll
-    for (int n = 0; n < TJ + 4; ++n) fetch(0, n, 0);
+    for (int n = 0; n < TJ + TI; ++n) fetch(0, n, 0);
     // The stores of a tile lie in the queue behind the copies of the next tile's first NB stages, so its first wait can leave them
     // there - if the tile was a whole one, which is sure to have issued all of them.
-    constexpr int kStores = kAdd ? 16 * TJ : kGlu ? 4 * TJ : 8 * TJ;     // (swiglu: 8 * TJ more where `pre` is kept)
+    constexpr int kStores = Results<kEpi, TI, TJ>::kStores * TJ;
     constexpr int kLeave = (NB - 2) * P + kStores < 63 ? (NB - 2) * P + kStores : 63;           // (63: the most a wait can leave)
     bool stores_behind = false;
     for (; local < run; local += stride) {
         int t0, n0;
         tile_at(local, t0, n0);
         slice(0, 1, 0, 0, true);
-        slice(1, 2, 0, 0);
-        slice(0, 3, 0, 0);
         if (stores_behind) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(kLeave) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((NB - 2) * P) : "memory");
         next_buffer();
-        slice(1, 0, 0, C3);
         for (int s = 1; s < nk; ++s) {
-            slice(0, 1, C3, C0);
-            slice(1, 2, C3 + C0, C1);
-            slice(0, 3, C3 + C0 + C1, C2);
+            slice(1, 0, 0, C1);
+            slice(0, 1, C1, C0);
             next_stage();
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((NB - 2) * P) : "memory");
             next_buffer();
-            slice(1, 0, 0, C3);
         }
-        read_ahead(0, t0, n0);
+        request(t0, n0);
+        slice(1, 0, 0, C1);
 #pragma unroll
-        for (int i = C3; i < P; ++i) copy(i);
+        for (int i = C1; i < P; ++i) copy(i);
         next_stage();
-        store_tile(t0, n0);
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) res.store(p, acc, j);
         stores_behind = t0 + TM <= p.m && n0 + kOwn <= features;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // the last copies, unread, have landed before the LDS is given back
@@ -765,7 +723,9 @@ int SBA_PROJECT(const Projection& p, ProjectionTile tile, hipStream_t s) {
     return launch_projection(p, s);
 }
 int SBA_WEIGHT_GRADS(const WeightGrads& g, int splits, hipStream_t stream) {
-    hipLaunchKernelGGL(sba::SBA_ELEM_NS::weight_grad_kernel, dim3((unsigned)((g.tiles + 7) / 8 * 8), (unsigned)splits), dim3(256), 0, stream, g);
+    const dim3 grid((unsigned)((g.tiles + 7) / 8 * 8), (unsigned)splits), block(256);
+    if (g.tile_rows == 256) hipLaunchKernelGGL(sba::SBA_ELEM_NS::weight_grad_kernel<256>, grid, block, 0, stream, g);
+    else hipLaunchKernelGGL(sba::SBA_ELEM_NS::weight_grad_kernel<224>, grid, block, 0, stream, g);
     return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 }  // namespace sba_model

@@ -62,10 +62,11 @@ struct WeightGrads {
     WeightGrad one[4];
     int first_tile[4];
     int n, tiles, k;
+    int tile_rows;                       // 256 or 224: rows of C in a workgroup's tile
     float* out; float* partial; int64_t total;
 };
 bool weight_grads_fit(const WeightGrads& g);             // whether the kernel takes it
-int weight_grad_splits(WeightGrads& g, int cus);         // fills first_tile, tiles, at, total; partial sums of how many splits
+int weight_grad_splits(WeightGrads& g, int cus);         // fills first_tile, tiles, tile_rows, at, total; partial sums of how many splits
 int weight_grads(const WeightGrads& g, int splits, bool f16, hipStream_t stream);     // partial: [splits][total] if more than one
 int weight_grads_bf16(const WeightGrads& g, int splits, hipStream_t stream);
 int weight_grads_f16(const WeightGrads& g, int splits, hipStream_t stream);

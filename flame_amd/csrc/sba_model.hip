@@ -488,24 +488,33 @@ bool weight_grads_fit(const WeightGrads& g) {
     return true;
 }
 
-// How many workgroups share a tile's contraction.  A launch takes ceil(tiles * splits / CUs) rounds of 1/splits of the rows each
-// (about 0.9 us per 32 rows with the chip full); partial sums are written, read and summed at about 4 TB/s.
+// Tile height, and how many workgroups share a tile's contraction.  A launch takes ceil(tiles * splits / CUs) rounds of 1/splits of the
+// rows each (about 0.9 us per 32 rows with the chip full and 256 x 256 tiles, in proportion for 224 x 256 ones, which leave fewer
+// CUs without work where the taller ones do not fill a round: the 340M model's block, 232 tiles instead of 196); partial sums are
+// written, read and summed at about 4 TB/s.
 int weight_grad_splits(WeightGrads& g, int cus) {
-    g.tiles = 0;
+    auto tiles_of = [&](int i, int rows) { return ((g.one[i].m + rows - 1) / rows) * ((g.one[i].n + 255) / 256); };
     g.total = 0;
     for (int i = 0; i < g.n; ++i) {
-        g.first_tile[i] = g.tiles;
         g.one[i].at = g.total;
-        g.tiles += ((g.one[i].m + 255) / 256) * ((g.one[i].n + 255) / 256);
         g.total += (int64_t)g.one[i].m * g.one[i].n;
     }
     const double stages = (g.k + 31) / 32;
     int best = 1;
     double best_us = 1e30;
-    for (int s = 1; s <= 16 && s * 4 <= stages + 3; ++s) {
-        const double rounds = (double)((g.tiles * (int64_t)s + cus - 1) / cus);
-        const double us = rounds * (0.9 * stages / s + 4.0) + (s > 1 ? (2 * s + 1) * 4.0 * g.total / 4e6 + 3.0 : 0.0);
-        if (us < best_us) { best_us = us; best = s; }
+    for (int rows : {256, 224}) {
+        int64_t tiles = 0;
+        for (int i = 0; i < g.n; ++i) tiles += tiles_of(i, rows);
+        for (int s = 1; s <= 16 && s * 4 <= stages + 3; ++s) {
+            const double rounds = (double)((tiles * s + cus - 1) / cus);
+            const double us = rounds * (0.9 * rows / 256 * stages / s + 4.0) + (s > 1 ? (2 * s + 1) * 4.0 * g.total / 4e6 + 3.0 : 0.0);
+            if (us < best_us) { best_us = us; best = s; g.tile_rows = rows; }
+        }
+    }
+    g.tiles = 0;
+    for (int i = 0; i < g.n; ++i) {
+        g.first_tile[i] = g.tiles;
+        g.tiles += tiles_of(i, g.tile_rows);
     }
     return best;
 }
