@@ -230,12 +230,6 @@ __global__ __launch_bounds__(256, 1) void weight_grad_kernel(sba_model::WeightGr
 // Y[t][n] = sum over k of X[t][k] * W[n][k] for token rows t, or W[k][n] (kRowsW: the product of a backward), 16-bit operands,
 // fp32 sums, and what the model does with Y in the same pass (Epilogue).
 //
-// Small products: 128 x 128 tiles, two workgroups a CU, k a multiple of 32.  Such launches are short of workgroups and of time to
-// fill a pipeline; two resident ones hide each other's start and stores.  Four waves, two by two, each 64 tokens x 64 features.
-// Stages of 32 k and four tile buffers, requested, awaited and walked as in the weight-gradient kernel.  A tile row of 32 k is 64
-// bytes, four 16-byte chunks; chunk c of row r lies at c ^ (r / 4 % 4), so that sixteen consecutive rows' chunks of one index fall on
-// sixteen different bank groups.  The products are formed transposed (rows: features, columns: tokens): a lane then holds runs of
-// four features of one token, which leave through LDS as whole rows.  4096 x 1024, k = 1024: 13 us.
 using sba_model::Projection;
 
 // What becomes of a wave's products: blocks of 16 features (TI of them; with swiglu TI/2 of gates, then their ups) by 16 tokens
@@ -325,76 +319,113 @@ template <int kEpi, int TI, int TJ> struct Results {
 };
 
 
-template <bool kRowsW, int kEpi>
-__global__ __launch_bounds__(256, 2) void projection_kernel(Projection p) {
-    constexpr int TM = 128, TN = 128, NB = 4;
-    constexpr int kX = TM * 64, kW = TN * 64, kStage = kX + kW;        // bytes
-    constexpr int PX = TM / 64, PW = TN / 64, P = PX + PW;             // copies per wave and stage
-    constexpr int TI = TN / 32, TJ = TM / 32;                          // 16-wide blocks of a wave: features, tokens
-    __shared__ __attribute__((aligned(1024))) char lds[NB * kStage];
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// Launches that are short of tiles: T x T tiles, kPerCu workgroups a CU, each of G groups of four waves (two by two, T/2 tokens x T/2
+// features each) that share out the contraction: group g takes stages g, g + G, ...  The groups' fp32 sums meet in LDS, in the order of
+// the groups, and as many groups as there are blocks of tokens write the results.  k a multiple of 32.
+// Stages of 64 k, two buffers a group, walked slice by slice as in the kernel for large products below.  Rows of 64 k are whole 128-byte
+// lines: with 32 k the CU's memory pipe takes 16 lines for a kilobyte instead of 8, and 4096 x 1024, k = 2816, with the residual took 34 us (31
+// now; four buffers of 32 k and one group, the shape before this: 37).  What bounds them: LDS, 128 bytes a cycle for the operands of 64 x 64
+// products a wave and the arriving tiles (T = 128), a round trip to memory per stage and group (T = 64).
+// A tile row of 64 k is eight 16-byte chunks; chunk c of row r lies at c ^ (r / 2 % 8), so that sixteen consecutive rows' chunks of one index
+// fall on sixteen different bank groups.  The products are formed transposed (rows: features, columns: tokens).
+template <int T, int G, int kPerCu, bool kRowsW, int kEpi>
+__global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Projection p) {
+    constexpr int KS = 64, NB = 2;                                     // k of a stage, buffers of a group
+    constexpr int kX = T * KS * 2, kStage = 2 * kX;                    // bytes
+    constexpr int PX = T / 32;                                         // copies of one operand per wave and stage
+    constexpr int C = KS / 8;                                          // 16-byte chunks of a row of k
+    constexpr int TI = T / 32, TJ = T / 32;                            // 16-wide blocks of a wave: features, tokens
+    static_assert(kEpi != sba_model::kSwigluFwd || T == 128, "pairs of gate blocks");
+    __shared__ __attribute__((aligned(1024))) char lds[G * NB * kStage];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     const int m = lane & 15, h = lane >> 4;
 
-    // a swiglu tile's features are TN/2 gates and the TN/2 ups that go with them
+    // a swiglu tile's features are T/2 gates and the T/2 ups that go with them
     constexpr bool kGlu = kEpi == sba_model::kSwigluFwd;
     const int features = kGlu ? p.n / 2 : p.n;
-    constexpr int kOwn = kGlu ? TN / 2 : TN;
-    const int tiles_m = (p.m + TM - 1) / TM, tiles_n = (features + kOwn - 1) / kOwn, tiles = tiles_m * tiles_n;
+    constexpr int kOwn = kGlu ? T / 2 : T;
+    const int tiles_m = (p.m + T - 1) / T, tiles_n = (features + kOwn - 1) / kOwn, tiles = tiles_m * tiles_n;
     const int per = (tiles + 7) / 8, t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || t >= tiles) return;
-    constexpr int kBand = 1024 / TM;
+    constexpr int kBand = 1024 / T;
     const int band = t / (kBand * tiles_n), rows = min(kBand, tiles_m - kBand * band), in = t - band * kBand * tiles_n;
-    const int t0 = (kBand * band + in % rows) * TM, n0 = (in / rows) * kOwn;
-    const int nk = p.k / 32;
+    const int t0 = (kBand * band + in % rows) * T, n0 = (in / rows) * kOwn;
+    const int stages = (p.k + KS - 1) / KS, turns = (stages + G - 1) / G, padded = (turns + NB - 1) / NB * NB;
+    const int nk = (stages + G - 1 - group) / G;                       // this group's stages: group, group + G, ...
+    const bool odd = p.k % KS != 0;                                    // the last stage is half a one ...
+    const int half_stage = odd && (stages - 1) % G == group ? nk - 1 : -1;      // ... and this group's, this turn's
 
-    const char* xat = (const char*)p.x + 2 * (int64_t)t0 * p.ldx;
-    const char* wat = (const char*)p.w + (kRowsW ? 2 * (int64_t)n0 : (int64_t)0);
-    uint32_t xoff[PX], woff[PW];
+    const char* xat = (const char*)p.x + 2 * (int64_t)t0 * p.ldx + 2 * KS * group;
+    const char* wat = (const char*)p.w + (kRowsW ? 2 * (int64_t)n0 + 2 * KS * group * p.ldw : (int64_t)2 * KS * group);
+    // chunk swizzle of W's rows of T columns: the transposing fetch of half a wave reads rows r .. r + 3 and r + 8 .. r + 11, two
+    // neighbouring chunks of each, from 64 banks
+    auto col_swz = [](int row) { return T == 64 ? (row & 2) | ((row >> 1) & 4) : swz<128>(row); };
+    // and of rows of k: sixteen consecutive rows' chunks of one index fall on sixteen different bank groups
+    auto row_swz = [](int row) { return row / (16 / C) % C; };
+    uint32_t xoff[PX], woff[PX];
+    auto aim = [&](int lane, bool half) {      // half: the second half of a stage does not exist and reads the first once more
+        const int last_c = half ? C / 2 - 1 : C - 1;
 #pragma unroll
-    for (int i = 0; i < PX; ++i) {
-        const int row = 16 * (w + 4 * i) + (lane >> 2), c = (lane & 3) ^ ((row >> 2) & 3);
-        xoff[i] = (uint32_t)min(row, p.m - 1 - t0) * (uint32_t)(2 * p.ldx) + 16u * c;
-    }
-#pragma unroll
-    for (int i = 0; i < PW; ++i) {
-        if (kRowsW) {
-            constexpr int kPer = 512 / TN;                     // rows of TN columns per copy
-            const int row = kPer * (w + 4 * i) + lane / (TN / 8), c = (lane & (TN / 8 - 1)) ^ swz<TN>(row);
-            woff[i] = (uint32_t)row * (uint32_t)(2 * p.ldw) + 16u * (uint32_t)min(c, (features - n0) / 8 - 1);
-        } else {
-            const int row = 16 * (w + 4 * i) + (lane >> 2), c = (lane & 3) ^ ((row >> 2) & 3);
-            int feature = n0 + row, up = 0;
-            if (kGlu) {                                        // a wave's half of the tile: TN/4 gates, then their ups
-                feature = n0 + (row / (TN / 2)) * (TN / 4) + row % (TN / 4);
-                up = (row % (TN / 2)) / (TN / 4) * features;
+        for (int i = 0; i < PX; ++i) {
+            const int row = 64 / C * (w + 4 * i) + lane / C, c = (lane % C ^ row_swz(row)) & last_c;
+            xoff[i] = (uint32_t)min(row, p.m - 1 - t0) * (uint32_t)(2 * p.ldx) + 16u * c;
+            if (kRowsW) {
+                constexpr int kPer = 512 / T;                  // rows of T columns per copy
+                const int k = kPer * (w + 4 * i) + lane / (T / 8), cc = (lane & (T / 8 - 1)) ^ col_swz(k);
+                woff[i] = (uint32_t)(half ? k & 31 : k) * (uint32_t)(2 * p.ldw) + 16u * (uint32_t)min(cc, (features - n0) / 8 - 1);
+            } else {
+                int feature = n0 + row, up = 0;
+                if (kGlu) {                                    // a wave's half of the tile: T/4 gates, then their ups
+                    feature = n0 + (row / (T / 2)) * (T / 4) + row % (T / 4);
+                    up = (row % (T / 2)) / (T / 4) * features;
+                }
+                woff[i] = (uint32_t)(min(feature, features - 1) + up) * (uint32_t)(2 * p.ldw) + 16u * c;
             }
-            woff[i] = (uint32_t)(min(feature, features - 1) + up) * (uint32_t)(2 * p.ldw) + 16u * c;
         }
-    }
-    const uint32_t lds0 = lds_address(lds);
-    auto request = [&](int buf) {
+    };
+    aim(lane, half_stage == 0);
+    const uint32_t lds0 = lds_address(lds) + group * NB * kStage;
+    auto request = [&](int stage, int buf) {
+        if (stage == half_stage && stage > 0) {                // (the last one: nothing is aimed at after it)
+            int lane_here = lane;
+            asm volatile("" : "+v"(lane_here));
+            aim(lane_here, true);
+        }
 #pragma unroll
         for (int i = 0; i < PX; ++i) dma16(xat, xoff[i], lds0 + buf * kStage + (w + 4 * i) * 1024);
 #pragma unroll
-        for (int i = 0; i < PW; ++i) dma16(wat, woff[i], lds0 + buf * kStage + kX + (w + 4 * i) * 1024);
-        xat += 64;
-        wat += kRowsW ? 64 * p.ldw : (int64_t)64;
+        for (int i = 0; i < PX; ++i) dma16(wat, woff[i], lds0 + buf * kStage + kX + (w + 4 * i) * 1024);
+        xat += 2 * KS * G;
+        wat += kRowsW ? 2 * KS * G * p.ldw : (int64_t)2 * KS * G;
+    };
+    // zeros in place of a stage, or of its second half, that does not exist
+    auto clear = [&](int stage, int buf) {
+        if (stage < nk && stage != half_stage) return;
+        char* at = lds + (group * NB + buf) * kStage;
+        for (int c = threadIdx.x & 255; c < kStage / 16; c += 256) {
+            const int row = c % (kX / 16) / C;
+            const bool second = kRowsW && c >= kX / 16 ? c - kX / 16 >= kX / 32 : (c % C ^ row_swz(row)) >= C / 2;
+            if (stage >= nk || second) *(u32x4*)(at + c * 16) = u32x4{0u, 0u, 0u, 0u};
+        }
     };
 
-    // fetch addresses: X rows and, k contiguous, W rows; W columns [half of the eight rows][column block]
-    uint32_t fx, fw, fc[2][TI];
-    {
-        const int c = h ^ ((m >> 2) & 3);
-        fx = lds0 + (w & 1) * (TM / 2) * 64 + m * 64 + c * 16;
-        fw = lds0 + kX + (w >> 1) * (TN / 2) * 64 + m * 64 + c * 16;
-        asm("" : "+v"(fx), "+v"(fw));
+    // fetch addresses: X rows and, k contiguous, W rows [slice]; W columns [half of the eight rows][column block]
+    uint32_t fx[2], fw[2], fc[2][TI];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int c = (4 * q + h) ^ row_swz(m);
+        fx[q] = lds0 + ((w & 1) * (T / 2) + m) * (KS * 2) + c * 16;
+        fw[q] = lds0 + kX + ((w >> 1) * (T / 2) + m) * (KS * 2) + c * 16;
+        asm("" : "+v"(fx[q]), "+v"(fw[q]));
     }
     if (kRowsW) {
 #pragma unroll
         for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int c = 0; c < TI; ++c) {
-                fc[a][c] = lds0 + kX + (uint32_t)tile_offset<TN>(8 * h + 4 * a + (m >> 2), (w >> 1) * (TN / 16) + 2 * c + ((m & 3) >> 1)) + ((m & 1) << 3);
+                const int row = 8 * h + 4 * a + (m >> 2), chunk = (w >> 1) * (T / 16) + 2 * c + ((m & 3) >> 1);
+                fc[a][c] = lds0 + kX + row * (T * 2) + ((chunk ^ col_swz(row)) << 4) + ((m & 1) << 3);
                 asm("" : "+v"(fc[a][c]));
             }
     }
@@ -408,66 +439,97 @@ __global__ __launch_bounds__(256, 2) void projection_kernel(Projection p) {
 #pragma unroll
         for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     h16x8 vx[2][TJ], vw[2][TI];
-    // the n-th of the operands of buffer `buf`
-    auto fetch = [&](int set, int n, int buf) {
-        if (n < TJ) vx[set][n] = at(fx, buf * kStage + n * 1024);
-        else if (kRowsW) vw[set][n - TJ] = fragment(fc[0][n - TJ], fc[1][n - TJ], buf * kStage);
-        else vw[set][n - TJ] = at(fw, buf * kStage + (n - TJ) * 1024);
+    // the n-th of the operands of slice q (32 k) of buffer `buf`, into one of the two sets of registers
+    auto fetch = [&](int set, int n, int buf, int q) {
+        if (n < TJ) vx[set][n] = at(fx[q], buf * kStage + n * 16 * KS * 2);
+        else if (kRowsW) vw[set][n - TJ] = fragment(fc[0][n - TJ], fc[1][n - TJ], buf * kStage + q * 32 * T * 2);
+        else vw[set][n - TJ] = at(fw[q], buf * kStage + (n - TJ) * 16 * KS * 2);
     };
-    static_assert(TI + TJ <= TI * TJ / 2, "a fetch per two MFMAs");
-    auto clear = [&](int buf) {
-        for (int c = threadIdx.x; c < kStage / 16; c += 256) *(u32x4*)(lds + buf * kStage + c * 16) = u32x4{0u, 0u, 0u, 0u};
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    };
-
-    Results<kEpi, TI, TJ> res;
-    constexpr int R = Results<kEpi, TI, TJ>::kAhead * TJ;              // loads of the epilogue, asked for in the last four stages, behind all copies
-    auto request_ahead = [&]() __attribute__((always_inline)) {
-        if (R) {
+    constexpr int kFetchEvery = TI * TJ / (TI + TJ);
+    // MFMAs of the slice in register set `set`; under them the fetches of slice q of buffer `buf`, which is the one behind it
+    auto slice = [&](int set, int buf, int q) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < TJ; ++j) res.request(p, j);
+        for (int n = 0; n < TI * TJ; ++n) {
+            acc[n / TJ][n % TJ] = mfma16(vw[set][n / TJ], vx[set][n % TJ], acc[n / TJ][n % TJ]);
+            if (n % kFetchEvery == 0 && n / kFetchEvery < TI + TJ) fetch(set ^ 1, n / kFetchEvery, buf, q);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // behind the MFMAs of stage s: the next but one has landed, and the buffer of the next, which the operand registers now hold, is
-    // free for stage s + 1 + NB
-    auto turn = [&](int s, int b, bool asked) __attribute__((always_inline)) {
-        const int behind = nk - 3 - s;                                 // stages behind the one that has to land
-        if (behind >= NB - 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((NB - 2) * P) : "memory");
-        else if (asked && R) {
-            if (behind == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(P + R) : "memory");
-            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(R) : "memory");
-        } else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(P) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (s + 2 >= nk) clear((b + 2) % NB);
-        if (s + 1 + NB < nk) request((b + 1) % NB);
-    };
-    static_assert(NB == 4, "turn() counts the stages behind by hand");
 
-    res.aim(lane, t0 + (w & 1) * (TM / 2), n0 + (w >> 1) * (kOwn / 2));
+    // Token blocks whose results this group finishes, summed over the groups: the first E groups, TJ / E blocks each.
+    constexpr int E = G < TJ ? G : TJ, J = TJ / E;
+    // What the epilogue reads is asked for in the last group of turns, behind all copies; where registers are short, half of it.
+    constexpr int kEarly = G == 1 ? J / 2 : J;
+    Results<kEpi, TI, J> res;
+    constexpr int R = Results<kEpi, TI, J>::kAhead * kEarly;
+    // Stage s is all in operand registers: its buffer b is free for stage s + NB, and the next stage has landed.  Stages that a group
+    // does not have are made with zeros.
+    auto turn = [&](int s, int b, bool asked) __attribute__((always_inline)) {
+        if (asked && R) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(R) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 1 < padded && s + 1 >= stages / G - odd) {             // (some group may lack it: the same for all of them)
+            clear(s + 1, (b + 1) % NB);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+        if (s + NB < nk) request(s + NB, b);
+    };
+    static_assert(NB == 2, "turn() waits for all copies: those of the next stage");
+
+    res.aim(lane, t0 + (w & 1) * (T / 2) + 16 * J * (group % E), n0 + (w >> 1) * (kOwn / 2));
 #pragma unroll
     for (int s = 0; s < NB; ++s)
-        if (s < nk) request(s);
-    if (nk >= NB) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NB - 1) * P) : "memory");
+        if (s < nk) request(s, s);
+    if (nk >= NB) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((NB - 1) * 2 * PX) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-    for (int n = 0; n < TI + TJ; ++n) fetch(0, n, 0);
-    turn(-1, NB - 1, false);
-    for (int s0 = 0; s0 < nk; s0 += NB) {      // whole groups, filled up with stages of zeros (see the weight-gradient kernel)
-        const bool last = s0 + NB >= nk;       // (all copies are on their way by then)
-        if (last) request_ahead();
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-#pragma unroll
-            for (int n = 0; n < TI * TJ; ++n) {
-                acc[n / TJ][n % TJ] = mfma16(vw[b & 1][n / TJ], vx[b & 1][n % TJ], acc[n / TJ][n % TJ]);
-                if (n % 2 == 0 && n / 2 < TI + TJ) fetch(~b & 1, n / 2, (b + 1) % NB);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            turn(s0 + b, b, last);
-        }
+    if (stages < G + odd) {
+        clear(0, 0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
 #pragma unroll
-    for (int j = 0; j < TJ; ++j) res.store(p, acc, j);
+    for (int n = 0; n < TI + TJ; ++n) fetch(0, n, 0, 0);
+    for (int s0 = 0; s0 < turns; s0 += NB) {   // whole groups of stages, filled up with zeros (see the weight-gradient kernel)
+        const bool asked = s0 + NB >= turns && group < E;      // (all copies are on their way by then)
+        if (R && asked) {
+#pragma unroll
+            for (int j = 0; j < kEarly; ++j) res.request(p, j);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            slice(0, b, 1);
+            turn(s0 + b, b, asked);
+            slice(1, (b + 1) % NB, 0);
+        }
+    }
+    if constexpr (G == 1) {
+        if (R) {
+#pragma unroll
+            for (int j = kEarly; j < J; ++j) res.request(p, j);
+        }
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) res.store(p, acc, j);
+        return;
+    }
+    // the groups' sums meet in LDS: [group][wave][block][lane]
+    auto part = [&](int g, int i, int j) { return (f32x4*)(lds + (((g * 4 + w) * TI + i) * TJ + j) * 1024 + lane * 16); };
+    static_assert(G * 4 * TI * TJ * 1024 <= G * NB * kStage, "partial sums in the tiles' place");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (the last slice's fetches)
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) *part(group, i, j) = acc[i][j];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (group >= E) return;
+    f32x4 sum[TI][J];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            sum[i][j] = *part(0, i, group * J + j);
+#pragma unroll
+            for (int g = 1; g < G; ++g) sum[i][j] += *part(g, i, group * J + j);
+        }
+#pragma unroll
+    for (int j = 0; j < J; ++j) res.store(p, sum, j);
 }
 
 // Large products: TM x 256 tiles, one resident workgroup a CU that walks tiles, one wave per SIMD with TM/2 x 128 of a tile.
@@ -671,18 +733,21 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // the last copies, unread, have landed before the LDS is given back
 }
 
+template <int T, int G, int kPerCu>
 int launch_projection(const Projection& p, hipStream_t s) {
-    const int own = p.epilogue == sba_model::kSwigluFwd ? 64 : 128, features = p.epilogue == sba_model::kSwigluFwd ? p.n / 2 : p.n;
-    const int tiles = ((p.m + 127) / 128) * ((features + own - 1) / own);
-    const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256);
+    const int own = p.epilogue == sba_model::kSwigluFwd ? T / 2 : T, features = p.epilogue == sba_model::kSwigluFwd ? p.n / 2 : p.n;
+    const int tiles = ((p.m + T - 1) / T) * ((features + own - 1) / own);
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256 * G);
     if (p.rows_w) {
-        if (p.epilogue == sba_model::kSwigluBwd) hipLaunchKernelGGL((projection_kernel<true, sba_model::kSwigluBwd>), grid, block, 0, s, p);
-        else if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((projection_kernel<true, sba_model::kStore>), grid, block, 0, s, p);
+        if (p.epilogue == sba_model::kSwigluBwd) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, true, sba_model::kSwigluBwd>), grid, block, 0, s, p);
+        else if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, true, sba_model::kStore>), grid, block, 0, s, p);
         else return -2;
     } else {
-        if (p.epilogue == sba_model::kSwigluFwd) hipLaunchKernelGGL((projection_kernel<false, sba_model::kSwigluFwd>), grid, block, 0, s, p);
-        else if (p.epilogue == sba_model::kAddResidual) hipLaunchKernelGGL((projection_kernel<false, sba_model::kAddResidual>), grid, block, 0, s, p);
-        else if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((projection_kernel<false, sba_model::kStore>), grid, block, 0, s, p);
+        if (p.epilogue == sba_model::kSwigluFwd) {
+            if constexpr (T == 128) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, false, sba_model::kSwigluFwd>), grid, block, 0, s, p);
+            else return -2;                    // (swiglu pairs two blocks of gates)
+        } else if (p.epilogue == sba_model::kAddResidual) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, false, sba_model::kAddResidual>), grid, block, 0, s, p);
+        else if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, false, sba_model::kStore>), grid, block, 0, s, p);
         else return -2;
     }
     return hipGetLastError() == hipSuccess ? 0 : -6;
@@ -720,7 +785,10 @@ int SBA_PROJECT(const Projection& p, ProjectionTile tile, hipStream_t s) {
     using namespace sba::SBA_ELEM_NS;
     if (tile == kTile256) return launch_large_projection<256>(p, s);
     if (tile == kTile128x256) return launch_large_projection<128>(p, s);
-    return launch_projection(p, s);
+    if (tile == kTile128Halves) return launch_projection<128, 2, 1>(p, s);
+    if (tile == kTile64Halves) return launch_projection<64, 2, 2>(p, s);
+    if (tile == kTile64Quarters) return launch_projection<64, 4, 1>(p, s);
+    return launch_projection<128, 1, 2>(p, s);
 }
 int SBA_WEIGHT_GRADS(const WeightGrads& g, int splits, hipStream_t stream) {
     const dim3 grid((unsigned)((g.tiles + 7) / 8 * 8), (unsigned)splits), block(256);

@@ -84,9 +84,11 @@ struct Projection {
     const float* residual; void* pre; void* out;
 };
 bool projects(const Projection& p, int cus);             // whether the kernels take it
-enum ProjectionTile { kTile256, kTile128x256, kTile128 };
+enum ProjectionTile { kTile256, kTile128x256, kTile128, kTile128Halves, kTile64Halves, kTile64Quarters };
 ProjectionTile projection_tile(const Projection& p, int cus);
+double tile_time(const Projection& p, ProjectionTile tile, int cus);    // an estimate, us; 1e30 where its kernel does not take it
 int project(const Projection& p, bool f16, int cus, hipStream_t stream);
+int project_tile(const Projection& p, ProjectionTile tile, bool f16, hipStream_t stream);
 int project_bf16(const Projection& p, ProjectionTile tile, hipStream_t stream);
 int project_f16(const Projection& p, ProjectionTile tile, hipStream_t stream);
 

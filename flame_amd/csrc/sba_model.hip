@@ -488,10 +488,11 @@ bool weight_grads_fit(const WeightGrads& g) {
     return true;
 }
 
-// Tile height, and how many workgroups share a tile's contraction.  A launch takes ceil(tiles * splits / CUs) rounds of 1/splits of the
-// rows each (about 0.9 us per 32 rows with the chip full and 256 x 256 tiles, in proportion for 224 x 256 ones, which leave fewer
-// CUs without work where the taller ones do not fill a round: the 340M model's block, 232 tiles instead of 196); partial sums are
-// written, read and summed at about 4 TB/s.
+// Tile height, and how many workgroups share a tile's contraction.  A launch takes rounds of 1/splits of the rows each, 0.7 us per 32
+// rows with 256 x 256 tiles and in proportion for 224 x 256 ones, which leave fewer CUs without work where the taller ones do not
+// fill a round (the 340M model's block over 8192 rows, 235 tiles instead of 196: 184 against 196 us); tiles are dealt to the XCDs
+// in eight equal parts, the last of them short, so that a round is full when the first XCD's CUs are.  Results are written, partial
+// sums written, read and summed at about 5.5 TB/s.
 int weight_grad_splits(WeightGrads& g, int cus) {
     auto tiles_of = [&](int i, int rows) { return ((g.one[i].m + rows - 1) / rows) * ((g.one[i].n + 255) / 256); };
     g.total = 0;
@@ -506,8 +507,9 @@ int weight_grad_splits(WeightGrads& g, int cus) {
         int64_t tiles = 0;
         for (int i = 0; i < g.n; ++i) tiles += tiles_of(i, rows);
         for (int s = 1; s <= 16 && s * 4 <= stages + 3; ++s) {
-            const double rounds = (double)((tiles * s + cus - 1) / cus);
-            const double us = rounds * (0.9 * rows / 256 * stages / s + 4.0) + (s > 1 ? (2 * s + 1) * 4.0 * g.total / 4e6 + 3.0 : 0.0);
+            const int64_t on_xcd = (tiles + 7) / 8 * s, slots = cus > 8 ? cus / 8 : 1;
+            const double rounds = (double)((on_xcd + slots - 1) / slots);
+            const double us = rounds * (0.7 * rows / 256 * stages / s + 3.0) + (s > 1 ? 2 * s + 1 : 1) * 4.0 * g.total / 5.5e6 + (s > 1 ? 3.0 : 0.0);
             if (us < best_us) { best_us = us; best = s; g.tile_rows = rows; }
         }
     }
@@ -519,44 +521,68 @@ int weight_grad_splits(WeightGrads& g, int cus) {
     return best;
 }
 
+// Time estimates in us of the projection kernels (sba_gemm.hip), from sweeps of 512 .. 8192 rows, 512 .. 5632 features and k of 512 .. 5632:
+// rounds of resident workgroups, each k / 64 times `full` (a last round that fills half of the chip or less: `part`, what lies
+// between in proportion) and `round` (in proportion to its fill), and `launch`.
+// Where each is ahead (us): 256 x 256 8192 x 5632 of swiglu, k = 1024 (92, next 101); 128 x 256 8192 x 3072, k = 1024 (49; 52);
+// 128 x 128 two a CU 4096 x 1024, k = 1024 (12; 15); by halves 4096 x 1024, k = 5632 (49; 59); 64 x 64 by halves 2048 x 1024, k = 1024
+// (9; 11); by quarters 1024 x 1024, k = 5632 (27; 32).
+double tile_time(const Projection& p, ProjectionTile tile, int cus) {
+    struct { int rows, features, per_cu; double part, full, round, launch; } static const cost[] = {
+        {256, 256, 1, 1.14, 1.32, 8.7, 2.6},    // kTile256
+        {128, 256, 1, 0.57, 0.78, 3.9, 5.0},    // kTile128x256
+        {128, 128, 2, 0.60, 0.89, 3.5, 2.5},    // kTile128
+        {128, 128, 1, 0.47, 0.475, 3.8, 3.0},   // kTile128Halves
+        {64, 64, 2, 0.32, 0.38, 1.5, 1.6},      // kTile64Halves
+        {64, 64, 1, 0.25, 0.22, 1.5, 2.6},      // kTile64Quarters
+    };
+    const auto& c = cost[tile];
+    const bool glu = p.epilogue == kSwigluFwd;
+    if (tile <= kTile128x256 && (p.k % 64 || p.epilogue == kSwigluBwd)) return 1e30;
+    if (tile == kTile256 && p.epilogue == kAddResidual) return 1e30;       // its registers
+    if (tile >= kTile64Halves && glu) return 1e30;
+    const int64_t own = glu ? c.features / 2 : c.features, features = glu ? p.n / 2 : p.n;
+    const int64_t tiles = ((int64_t)p.m + c.rows - 1) / c.rows * ((features + own - 1) / own), slots = (int64_t)cus * c.per_cu;
+    // bytes of the epilogue that nothing hides: gate and up of the backward with their gradients, the residual, swiglu's second and third tensor
+    const double round = c.round + (p.epilogue == kSwigluBwd ? 10.0 * c.per_cu * c.rows * c.features / 32768 :
+                                    p.epilogue == kAddResidual ? (tile == kTile128x256 ? 9.5 : tile == kTile128 ? 7.0 : 1.5) : glu ? (tile == kTile256 ? 3.0 : 1.0) : 0.0);
+    const double k64 = (p.k + 63) / 64, fill = (double)(tiles % slots) / slots;
+    const double rate = fill <= 0.5 ? c.part : c.part + (c.full - c.part) * (2 * fill - 1);
+    return tiles / slots * (c.full * k64 + round) + (fill > 0 ? rate * k64 + round * fill : 0.0) + c.launch;
+}
+
 bool projects(const Projection& p, int cus) {
     if (!(p.k % 32 == 0 && p.k > 0 && p.n % (p.epilogue == kSwigluFwd ? 16 : 8) == 0 && p.n > 0 && p.m > 0 && p.ldx % 8 == 0 &&
           p.ldw % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.w & 15) == 0 && p.ldx < (1 << 22) && p.ldw < (1 << 22) &&
           (int64_t)(p.rows_w ? p.k : p.n) * p.ldw < (INT64_C(1) << 31)))
         return false;
-    // where a tile of one workgroup a CU is the better one, the gradient of silu(gate) * up is left to a kernel of its own: it reads
-    // and writes 12 bytes per product, which nothing hides there (8192 x 2816, k = 1024: 103 us against 55 + 36)
-    if (p.epilogue == kSwigluBwd) return projection_tile(p, cus) == kTile128;
-    // plain products of four rounds of the largest tile and more (the language model's head): the library's is ahead there, 417 against
-    // 475 us for 8192 x 32000, k = 1024
+    if (p.epilogue == kSwigluBwd) {
+        // against the plain product and a pass of its own, which reads and writes 12 bytes per product at 7.7 TB/s (much of it still in
+        // the last-level cache): 8192 x 2816, k = 1024 76 against 48 + 36 us
+        Projection plain = p;
+        plain.epilogue = kStore;
+        return tile_time(p, projection_tile(p, cus), cus) < tile_time(plain, projection_tile(plain, cus), cus) + 12e-6 * p.m * p.n / 7.7 + 1.5;
+    }
+    // plain products of four rounds of the largest tile and more (the language model's head): the library's is ahead there, 436 against
+    // 466 us for 8192 x 32000, k = 1024
     return p.epilogue != kStore || p.rows_w || (int64_t)p.m * p.n < (int64_t)4 * 256 * 256 * cus;
 }
 
-// Time estimates in us of the three kernels (sba_gemm.hip), from k sweeps of 8192 and 4096 rows times 1024 .. 32000 features:
-// rounds of resident workgroups times (time per 64 k, and the part of a tile that does not depend on k).
-//   256 x 256 tiles, one a CU: 1.42 and 5.5, the best rate; 128 x 256, one a CU: 0.78 and 3; 128 x 128, two a CU: 1.15 for both or
-//   0.58 alone, and 3, for what would leave CUs without work (4096 x 1024, k = 1024: 13 against 17 and 26 us).
-// The residual epilogue of the largest tile does not fit its registers.
 ProjectionTile projection_tile(const Projection& p, int cus) {
-    const bool glu = p.epilogue == kSwigluFwd;
-    const int64_t features = glu ? p.n / 2 : p.n;
-    auto tiles = [&](int tm, int tn) { return (((int64_t)p.m + tm - 1) / tm) * ((features + tn - 1) / tn); };
-    const double k64 = p.k / 64.0;
-    const int64_t t2 = tiles(128, glu ? 64 : 128), full = t2 / (2 * cus), rest = t2 % (2 * cus);
     ProjectionTile best = kTile128;
-    double best_us = full * (1.15 * k64 + 3) + (rest == 0 ? 0 : rest <= cus ? 0.58 * k64 + 3 : 1.15 * k64 + 3) + 2;
-    if (p.k % 64 == 0) {
-        const int own = glu ? 128 : 256;
-        const double t1 = (double)((tiles(128, own) + cus - 1) / cus) * (0.78 * k64 + 3) + 3;
-        if (t1 < best_us) { best = kTile128x256; best_us = t1; }
-        const double t0 = (double)((tiles(256, own) + cus - 1) / cus) * (1.42 * k64 + 5.5) + 1;
-        if (p.epilogue != kAddResidual && t0 < best_us) { best = kTile256; best_us = t0; }
+    double best_us = 1e30;
+    for (int t = kTile256; t <= kTile64Quarters; ++t) {
+        const double us = tile_time(p, (ProjectionTile)t, cus);
+        if (us < best_us) { best = (ProjectionTile)t; best_us = us; }
     }
     return best;
 }
 
 int project(const Projection& p, bool f16, int cus, hipStream_t s) {
-    const ProjectionTile tile = projection_tile(p, cus);
+    return project_tile(p, projection_tile(p, cus), f16, s);
+}
+
+int project_tile(const Projection& p, ProjectionTile tile, bool f16, hipStream_t s) {
     return f16 ? project_f16(p, tile, s) : project_bf16(p, tile, s);
 }
 

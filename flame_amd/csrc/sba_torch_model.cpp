@@ -145,8 +145,7 @@ NormGrad rms_norm_grad(const Tensor& dy, const Tensor& x, const Tensor& w, const
     return r;
 }
 
-// y = x w^T (rows_w: x w) into `out`, with what sba_model.h's epilogues do on the way; false where the kernels do not take it
-bool try_project(const Tensor& x, const Tensor& w, bool rows_w, int epilogue, const Tensor& residual, const Tensor& pre, const Tensor& out) {
+Projection projection_of(const Tensor& x, const Tensor& w, bool rows_w, int epilogue, const Tensor& residual, const Tensor& pre, const Tensor& out) {
     Projection p = {};
     p.x = x.data_ptr();
     p.w = w.data_ptr();
@@ -160,8 +159,25 @@ bool try_project(const Tensor& x, const Tensor& w, bool rows_w, int epilogue, co
     if (residual.defined()) p.residual = residual.data_ptr<float>();
     if (pre.defined()) p.pre = pre.data_ptr();
     p.out = out.data_ptr();
+    return p;
+}
+
+// y = x w^T (rows_w: x w) into `out`, with what sba_model.h's epilogues do on the way; false where the kernels do not take it
+bool try_project(const Tensor& x, const Tensor& w, bool rows_w, int epilogue, const Tensor& residual, const Tensor& pre, const Tensor& out) {
+    const Projection p = projection_of(x, w, rows_w, epilogue, residual, pre, out);
     if (!projects(p, compute_units())) return false;
     ok(sba_model::project(p, is_f16(x.scalar_type()), compute_units(), stream_of(x)));
+    return true;
+}
+
+// The same with the tile of a caller's choice, where that tile's kernel takes the problem (tests of kernels that the rule picks elsewhere).
+bool project_with(int64_t tile, const Tensor& x, const Tensor& w, bool rows_w, int64_t epilogue, const std::optional<Tensor>& residual,
+                  const std::optional<Tensor>& pre, const Tensor& out) {
+    const Projection p = projection_of(x, w, rows_w, (int)epilogue, residual.value_or(Tensor()), pre.value_or(Tensor()), out);
+    TORCH_CHECK(tile >= kTile256 && tile <= kTile64Quarters && p.k % 32 == 0 && p.n % 16 == 0 && p.ldx % 8 == 0 && p.ldw % 8 == 0 && p.m > 0,
+                "project_with: sizes that no tile takes");
+    if (tile_time(p, (ProjectionTile)tile, compute_units()) >= 1e30) return false;
+    ok(project_tile(p, (ProjectionTile)tile, is_f16(x.scalar_type()), stream_of(x)));
     return true;
 }
 
@@ -569,6 +585,8 @@ void bind_model(py::module& m) {
     m.def("next_token_loss", &next_token_loss);
     m.def("clip_and_step", &clip_and_step);
     m.def("project", &project);
+    m.def("project_with", &project_with);
+    m.attr("projection_tiles") = (int)kTile64Quarters + 1;
     m.def("project_add", &project_add);
     m.def("project_swiglu", [](const Tensor& x, const Tensor& w) {
         Tensor pre;
