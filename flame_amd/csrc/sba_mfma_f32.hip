@@ -537,8 +537,9 @@ using namespace sba;
 template <int D, int S>
 void launch_f32_fwd(const KParams& kp, hipStream_t s) {
     const dim3 grid(S * (unsigned)kp.n_jobs * kp.n_heads);
-    if (kp.carry_only) hipLaunchKernelGGL((f32::fwd_kernel<D, true, S>), grid, dim3(kThreads), 0, s, kp);
-    else hipLaunchKernelGGL((f32::fwd_kernel<D, false, S>), grid, dim3(kThreads), 0, s, kp);
+    const KParams turning = sba_turning(kp, D == 64 ? 3 : 2, S);
+    if (kp.carry_only) hipLaunchKernelGGL((f32::fwd_kernel<D, true, S>), grid, dim3(kThreads), 0, s, turning);
+    else hipLaunchKernelGGL((f32::fwd_kernel<D, false, S>), grid, dim3(kThreads), 0, s, turning);
 }
 template <int D>
 void launch_f32_bwd(const KParams& kp, int phases, hipStream_t s) {
@@ -548,7 +549,7 @@ void launch_f32_bwd(const KParams& kp, int phases, hipStream_t s) {
     // waves per workgroup in the key-owner pass.
     const bool one_block = kp.seq_len <= kRowBlock;
     if (phases != 2 && one_block) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 1>), dim3(jobs), dim3(kThreads), 0, s, kp);
-    else if (phases != 2) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 4>), dim3(4 * jobs), dim3(kThreads), 0, s, kp);
+    else if (phases != 2) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 4>), dim3(4 * jobs), dim3(kThreads), 0, s, sba_turning(kp, D == 64 ? 2 : 1, 4));
     if (phases != 1 && one_block) hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 4>), dim3(2 * jobs), dim3(4 * 64), 0, s, kp);
     else if (phases != 1) hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 8>), dim3(2 * jobs), dim3(8 * 64), 0, s, kp);
 }

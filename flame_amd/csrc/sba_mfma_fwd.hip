@@ -455,7 +455,7 @@ static void launch_seg(int groups, dim3 grid, hipStream_t s, const sba::KParams&
     using namespace sba;
     if (kp.head_dim == 96) hipLaunchKernelGGL((mfma_fwd_seg_kernel<96, 2, kCarryOnly>), grid, dim3(2 * kThreads), 0, s, kp);
     else if (kp.head_dim == 128) hipLaunchKernelGGL((mfma_fwd_seg_kernel<128, 2, kCarryOnly>), grid, dim3(2 * kThreads), 0, s, kp);
-    else if (groups == 2) hipLaunchKernelGGL((mfma_fwd_seg_kernel<64, 2, kCarryOnly>), grid, dim3(2 * kThreads), 0, s, kp);
+    else if (groups == 2) hipLaunchKernelGGL((mfma_fwd_seg_kernel<64, 2, kCarryOnly>), grid, dim3(2 * kThreads), 0, s, sba_turning(kp, 2));
     else if (groups == 3) hipLaunchKernelGGL((mfma_fwd_seg_kernel<64, 3, kCarryOnly>), grid, dim3(3 * kThreads), 0, s, kp);
     else hipLaunchKernelGGL((mfma_fwd_seg_kernel<64, 4, kCarryOnly>), grid, dim3(4 * kThreads), 0, s, kp);
 }
@@ -472,8 +472,8 @@ int sba_launch_mfma_fwd(const sba::KParams& kp, hipStream_t s) {
         if (kp.carry_only) launch_seg<true>(segments, grid, s, kp);
         else launch_seg<false>(segments, grid, s, kp);
     } else if (kp.head_dim == 64) {
-        if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<64, true>), grid, dim3(kThreads), 0, s, kp);
-        else hipLaunchKernelGGL((mfma_fwd_kernel<64, false>), grid, dim3(kThreads), 0, s, kp);
+        if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<64, true>), grid, dim3(kThreads), 0, s, sba_turning(kp, 4));
+        else hipLaunchKernelGGL((mfma_fwd_kernel<64, false>), grid, dim3(kThreads), 0, s, sba_turning(kp, 4));
     } else if (kp.head_dim == 96) {
         if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<96, true>), grid, dim3(kThreads), 0, s, kp);
         else hipLaunchKernelGGL((mfma_fwd_kernel<96, false>), grid, dim3(kThreads), 0, s, kp);

@@ -697,3 +697,13 @@ def test_fp32_config1_in_memory_lean_mode(monkeypatch):
     # benchmark configuration 1 once more with the backward recomputing the carry table (fp32 MFMA kernels)
     monkeypatch.setenv("SBA_RECOMPUTE_CARRIES", "1")
     _check_dense(2, 4, 512, 64, torch.float32, seed=0)
+
+
+@pytest.mark.parametrize("B,H,T,D,dtype,grads", [
+    (2, 32, 1000, 64, torch.bfloat16, True),       # 512 workgroups: two rounds of the CUs, four row blocks of two sequences to a round
+    (1, 64, 1409, 64, torch.float16, False),       # 768 of the forward: three rounds
+    (2, 16, 500, 64, torch.float32, True),         # 512 with four workgroups to a sweep
+    (1, 4, 2040, 128, torch.float32, False),       # 256 of the forward: one round, as they come
+    (2, 16, 500, 128, torch.float32, True)])
+def test_launches_whose_order_turns_round_by_round(B, H, T, D, dtype, grads):
+    _check_dense(B, H, T, D, dtype, seed=B + H + T, grads=grads)
