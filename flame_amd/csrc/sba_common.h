@@ -93,7 +93,8 @@ __device__ inline ScheduleRow schedule_row(const KParams& p, int i, int offset) 
 
 // The order of a launch whose workgroups are all resident at once (KParams::turn jobs to a round of the CUs, 0: as they come): the
 // list, longest sweeps first, is walked forwards and backwards in turn, so that the CUs with the longest sweep of one round get
-// the shortest of the next.
+// the shortest of the next.  Only the kernels that are launched with it ask for it (kTurns): the division and what it keeps in scalar
+// registers cost the resident stream 1.4 %.
 __device__ inline int turned(const KParams& p, int i) {
     if (p.turn == 0) return i;
     const int round = i / p.turn;
@@ -111,8 +112,9 @@ __device__ inline Job dense_job(const KParams& p, int job) {
     return j;
 }
 
+template <bool kTurns = false>
 __device__ inline Job decode_job(const KParams& p, int job) {
-    if (p.cu_seqlens == nullptr) return dense_job(p, turned(p, job));
+    if (p.cu_seqlens == nullptr) return dense_job(p, kTurns ? turned(p, job) : job);
     const ScheduleRow s = schedule_row(p, job, 0);
     Job j;
     j.tok0 = s[0]; j.len = s[1]; j.rb = s[2]; j.seq = 0; j.tab0 = s[3];
@@ -123,8 +125,9 @@ __device__ inline Job decode_job(const KParams& p, int job) {
 // their longest sweeps are the FIRST row-blocks of the longest sequences.  i-th job in that
 // order: arithmetic for the dense layout, the second half of row i of the host-built schedule
 // for the packed.
+template <bool kTurns = false>
 __device__ inline Job decode_key_job(const KParams& p, int i) {
-    if (p.cu_seqlens == nullptr) return dense_job(p, p.n_jobs - 1 - turned(p, i));
+    if (p.cu_seqlens == nullptr) return dense_job(p, p.n_jobs - 1 - (kTurns ? turned(p, i) : i));
     const ScheduleRow s = schedule_row(p, i, 4);
     Job j;
     j.tok0 = s[0]; j.len = s[1]; j.rb = s[2]; j.seq = 0; j.tab0 = s[3];

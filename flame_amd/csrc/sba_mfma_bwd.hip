@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     lo.init(lane);
     lo.rebase(lds);                        // absolute addresses: the loop below runs in one copy per tile buffer
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
+    const Job job = decode_job<D == 64>(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * wave;
@@ -1174,7 +1174,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
     LaneOffsets<64> lz;
     lz.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_key_job(p, blockIdx.x / p.n_heads);
+    const Job job = decode_key_job<D == 64>(p, blockIdx.x / p.n_heads);
     const int strict = p.attend_current ? 0 : 1;
     const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it
     const int kb0 = q_begin + 32 * wave;               // first key of this wave

@@ -191,7 +191,7 @@ template <int S> struct RowGroup {
     __device__ inline RowGroup(const KParams& p, int wave) {
         const int slot = blockIdx.x / p.n_heads;
         head = (blockIdx.x - slot * p.n_heads + slot / S) % p.n_heads;
-        job = decode_job(p, slot / S);
+        job = decode_job<true>(p, slot / S);
         sub = S == 4 ? 3 - (slot & 3) : wave;
         lane_of_sweep = S == 4 ? wave : 0;
         q0 = job.rb * kRowBlock + 32 * sub;

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     LaneOffsets<D> lo;
     lo.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
+    const Job job = decode_job<D == 64>(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * wave;              // first query of this wave
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     LaneOffsets<D> lo;
     lo.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
+    const Job job = decode_job<D == 64 && G == 2>(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * qs;
