@@ -707,3 +707,9 @@ def test_fp32_config1_in_memory_lean_mode(monkeypatch):
     (2, 16, 500, 128, torch.float32, True)])
 def test_launches_whose_order_turns_round_by_round(B, H, T, D, dtype, grads):
     _check_dense(B, H, T, D, dtype, seed=B + H + T, grads=grads)
+
+
+@pytest.mark.parametrize("B,H,T", [(4, 16, 1400), (2, 16, 2600), (2, 16, 2300), (1, 8, 4200)])
+def test_key_owner_kernel_of_long_and_short_tails(B, H, T):
+    # tail ratios 2.67, 2.91 (own-keys kernel), 3.37 and 7.5 (stream)
+    _check_dense(B, H, T, 64, torch.bfloat16, seed=B + H + T)
