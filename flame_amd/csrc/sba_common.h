@@ -44,6 +44,7 @@ struct KParams {
     float* dkv32;                  // generic path: fp32 dk|dv accumulators
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)
     int turn;                      // jobs after which the order of a dense launch turns round (0: never), see turned()
+    int cut_keys;                  // fp32 dQ pass: clear the rows of dK and dV that two workgroups will add to
     int early_end;                 // forward sweeps end once nothing is left of any of their rows' sticks
     int* gave_up;                  // backward error word (set if a kernel abandoned a bounded internal wait)
     int64_t tab_head_stride;       // floats per head in each carry table

@@ -309,6 +309,28 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void fwd_kernel(KParams 
     }
 }
 
+// queries of the first half of the steps of the job's key blocks (W = 8)
+__device__ inline int first_half(const Job& job) {
+    return ((job.len - job.rb * kRowBlock + 511) >> 9) << 8;
+}
+// zeros in rows row0 .. row0 + kRows - 1 of dK and dV where two workgroups add to them
+template <int D, int kRows>
+__device__ inline void clear_cut_rows(const KParams& p, const Job& job, int head, int row0) {
+    if (job.len <= job.rb * kRowBlock + first_half(job)) return;
+    const Slice dk(p.dk, job, head), dv(p.dv, job, head);
+    for (int c = threadIdx.x; c < kRows * D / 4; c += kThreads) {
+        const int row = row0 + c / (D / 4), at = 16 * (c % (D / 4));
+        if (row >= job.len) return;
+        *(f32x4*)(const_cast<char*>(dk.row(row)) + at) = f32x4{0};
+        *(f32x4*)(const_cast<char*>(dv.row(row)) + at) = f32x4{0};
+    }
+}
+template <int D>
+__global__ __launch_bounds__(kThreads) void clear_cut_kernel(KParams p) {
+    const Job job = decode_job(p, blockIdx.x / p.n_heads);
+    clear_cut_rows<D, kRowBlock>(p, job, head_of_block(p, blockIdx.x), job.rb * kRowBlock);
+}
+
 // ---------------------------------------------------------------- backward pass 1: dQ + prefix table
 template <int D, int S>
 __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void bwd_dq_kernel(KParams p) {
@@ -320,6 +342,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void bwd_dq_kernel(KPara
     const RowGroup<S> grp(p, wave);
     const Job& job = grp.job;
     if (grp.q0 >= job.len) return;                         // (S = 4: the whole workgroup)
+    if (S == 4 && p.cut_keys) clear_cut_rows<D, 32>(p, job, grp.head, grp.q0);
     const int strict = p.attend_current ? 0 : 1;
     const int qi = grp.q0 + n;
     const bool row_ok = qi < job.len;
@@ -396,7 +419,9 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void bwd_dq_kernel(KPara
 // weights and logit gradients (carries from the two tables) and leaves them in LDS as [query][key] rows; after a barrier
 // it reduces [32 keys x 32 d] tiles of dV (W = 8: waves 0-3) and dK (waves 4-7) over all queries of the step: key half
 // w & 1, column blocks (w >> 1 & 1) + 2*j.
-template <int D, int W>
+// kCut: two workgroups per (64-key block, head), one for each half of its steps, that add their sums to zeroed dK and dV.  Of two
+// addends the order makes no difference; the cut lies at a step that the sequence's length alone decides.
+template <int D, int W, bool kCut = false>
 __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
     constexpr int kMine = D / 64;              // output tiles per wave and tensor
     constexpr int kBoth = 8 / W;               // tensors per wave
@@ -406,7 +431,8 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int head = head_of_block(p, blockIdx.x);
-    const int slot = blockIdx.x / p.n_heads;   // two 64-key blocks per scheduled 128-row job
+    const int slot = blockIdx.x / (kCut ? 2 * p.n_heads : p.n_heads);   // two 64-key blocks per scheduled 128-row job
+    const int part = kCut ? blockIdx.x / p.n_heads & 1 : 0;
     const Job job = decode_key_job(p, slot >> 1);
     const int kb = 2 * job.rb + (slot & 1);
     const int key0 = kb * kKeyBlock;
@@ -420,16 +446,19 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
     for (int t = 0; t < kBoth; ++t)
 #pragma unroll
         for (int j = 0; j < kMine; ++j) acc[t][j] = f32x16{0};
-    const int q_end = min(job.len, (last_live_row_block(p, head, job) + 1) * kRowBlock);
+    const int q_live = min(job.len, (last_live_row_block(p, head, job) + 1) * kRowBlock);
+    const int cut = kCut ? first_half(job) : 0;
+    const int q_start = job.rb * kRowBlock + part * cut, q_end = kCut && part == 0 ? min(q_live, q_start + cut) : q_live;
+    if (kCut && part == 1 && q_start >= q_end) return;         // uniform over the workgroup
     // the step's Q and dO rows, for head_dim 64 requested as soon as the step before has used its own
     constexpr bool kAhead = D == 64;
     float qf[D / 2], dof[D / 2];
     if (kAhead) {
-        const int qi0 = job.rb * kRowBlock + 32 * wave + n;
+        const int qi0 = q_start + 32 * wave + n;
         load_row_share<D>(qf, q, qi0, job.len, h, p.scale2);
         load_row_share<D>(dof, d_o, qi0, job.len, h, 1.0f);
     }
-    for (int q_begin = job.rb * kRowBlock; q_begin < q_end; q_begin += kStep) {
+    for (int q_begin = q_start; q_begin < q_end; q_begin += kStep) {
         const int q0w = q_begin + 32 * wave, qi = q0w + n;
         {
             float x[32], dp[32];
@@ -511,6 +540,7 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
         }
         __syncthreads();                       // the weight tiles are free
     }
+    const bool adds = kCut && job.len > job.rb * kRowBlock + cut;
     // accumulator rows are keys 32*kh + 8*(r/4) + 4*h + r%4, columns d = 32*(dbw + 2j) + n: dk = scale * dZ^T Q
 #pragma unroll
     for (int t = 0; t < kBoth; ++t) {
@@ -522,8 +552,11 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
             const int key = key0 + 32 * kh + 8 * (r >> 2) + 4 * h + (r & 3);
             if (key < job.len)
 #pragma unroll
-                for (int j = 0; j < kMine; ++j)
-                    *(float*)(const_cast<char*>(out.row(key)) + 4 * (32 * (dbw + 2 * j) + n)) = acc[t][j][r] * s;
+                for (int j = 0; j < kMine; ++j) {
+                    float* at = (float*)(const_cast<char*>(out.row(key)) + 4 * (32 * (dbw + 2 * j) + n));
+                    if (adds) unsafeAtomicAdd(at, acc[t][j][r] * s);
+                    else *at = acc[t][j][r] * s;
+                }
         }
     }
 }
@@ -548,10 +581,21 @@ void launch_f32_bwd(const KParams& kp, int phases, hipStream_t s) {
     // 16 .. 128 take 193 us forward + backward this way, 276 with S = 4 and W = 8.  Longer ones are 4-15 % ahead with eight
     // waves per workgroup in the key-owner pass.
     const bool one_block = kp.seq_len <= kRowBlock;
+    // A key-owner workgroup has its CU to itself, so a launch of few lasts as long as the one with the most steps.  Where that is more
+    // than 1.6 times the average share of a CU (an eighth of the tail ratio), two workgroups take half of the steps each.  Both
+    // passes and the forward, with against without, by that measure: 8.0 0.90, 6.1-7.1 0.69-0.77, 3.2-3.6 0.70-0.78, 2.3 0.85-0.88,
+    // 1.8-1.9 0.74-0.92 (H=16, T=1024: 168 -> 155 us, D=128 304 -> 267), 1.7 0.85-0.92;  1.6 0.90 (a pack) ... 1.09 (B=4, T=512, whose
+    // sweeps have two steps), 1.4 1.01-1.05, 1.2 1.00-1.04, 0.9 1.05-1.10: the second workgroup's prologue and the additions in memory.
+    const bool cut = !one_block && sba_tail_ratio(kp, jobs) >= 13.0;
+    KParams dq = sba_turning(kp, D == 64 ? 2 : 1, 4);
+    dq.cut_keys = cut && phases == 0;
     if (phases != 2 && one_block) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 1>), dim3(jobs), dim3(kThreads), 0, s, kp);
-    else if (phases != 2) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 4>), dim3(4 * jobs), dim3(kThreads), 0, s, sba_turning(kp, D == 64 ? 2 : 1, 4));
+    else if (phases != 2) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 4>), dim3(4 * jobs), dim3(kThreads), 0, s, dq);
     if (phases != 1 && one_block) hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 4>), dim3(2 * jobs), dim3(4 * 64), 0, s, kp);
-    else if (phases != 1) hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 8>), dim3(2 * jobs), dim3(8 * 64), 0, s, kp);
+    else if (phases != 1 && cut) {
+        if (phases == 2) hipLaunchKernelGGL((f32::clear_cut_kernel<D>), dim3(jobs), dim3(kThreads), 0, s, kp);
+        hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 8, true>), dim3(4 * jobs), dim3(8 * 64), 0, s, kp);
+    } else if (phases != 1) hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 8>), dim3(2 * jobs), dim3(8 * 64), 0, s, kp);
 }
 }  // namespace
 
