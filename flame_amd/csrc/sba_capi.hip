@@ -135,6 +135,7 @@ KParams make_kparams(const SbaParams* p) {
     memset(&kp, 0, sizeof(kp));
     kp.n_seq = p->n_seq; kp.n_heads = p->n_heads; kp.seq_len = p->seq_len;
     kp.total_tokens = p->total_tokens;
+    kp.heads = sba::divisor(p->n_heads); kp.seqs = sba::divisor(p->n_seq);
     const int columns = columns_field(p);
     kp.head_dim = columns ? 96 : p->head_dim;              // rows of 72 .. 96 columns: the kernels of that width
     kp.cols = columns ? columns : p->head_dim;

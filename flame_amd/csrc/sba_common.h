@@ -22,6 +22,20 @@ constexpr float kLog2e = 1.4426950408889634f;
 struct TensorArg { char* ptr; int64_t sb, sh, st; };
 struct VectorArg { char* ptr; int64_t sb, sh; };
 
+// Division by a number that the host knows, in three scalar instructions where the compiler's takes twenty and two transfers to
+// the vector unit: n / d = n * ceil(2^(31 + l) / d) >> (31 + l) with 2^l >= d, exact for 0 <= n < 2^31 (the product exceeds n / d by
+// less than n 2^l / (d 2^(31 + l)) < 1 / d).  The multiplier is at most 2^32 - 1 from d = 2 on; 2^31 at d = 1.
+struct Divisor {
+    uint32_t mul;
+    int shift;
+};
+inline Divisor divisor(int d) {
+    int l = 0;
+    while ((INT64_C(1) << l) < d) ++l;
+    return Divisor{(uint32_t)(((UINT64_C(1) << (31 + l)) + d - 1) / d), 31 + l};
+}
+__device__ inline int divided(int n, const Divisor& d) { return (int)(((uint64_t)(uint32_t)n * d.mul) >> d.shift); }
+
 // Kernel-side copy of SbaParams (by value in the launch).
 struct KParams {
     int n_seq, n_heads, seq_len, total_tokens, head_dim, attend_current, save, n_jobs;
@@ -43,6 +57,7 @@ struct KParams {
                                    //   the key-owner stream kernel (ptr NULL: not wanted)
     float* dkv32;                  // generic path: fp32 dk|dv accumulators
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)
+    Divisor heads, seqs;           // n_heads and n_seq, for the way from a workgroup's index to its job
     int turn;                      // jobs after which the order of a dense launch turns round (0: never), see turned()
     int cut_keys;                  // fp32 dQ pass: clear the rows of dK and dV that two workgroups will add to
     int early_end;                 // forward sweeps end once nothing is left of any of their rows' sticks
@@ -71,8 +86,15 @@ struct Job { int tok0, len, rb, seq, tab0; };
 // length (longest first); `longest_last` walks the list from its other end (the key-owner
 // pass, whose work grows as the row-block index falls).
 __device__ inline int head_of_block(const KParams& p, int block) {
-    const int slot = block / p.n_heads;
-    return (block - slot * p.n_heads + (p.cu_seqlens ? slot >> 3 : slot)) % p.n_heads;
+    const int slot = divided(block, p.heads);
+    const int i = block - slot * p.n_heads + (p.cu_seqlens ? slot >> 3 : slot);
+    return i - divided(i, p.heads) * p.n_heads;
+}
+__device__ inline int slot_of_block(const KParams& p, int block) { return divided(block, p.heads); }
+// offset of a (sequence, head)'s first row in a tensor, in elements (products of non-negative indices: their high halves need no
+// sign correction)
+__device__ inline int64_t slice_offset(const TensorArg& t, int seq, int head, int tok0) {
+    return (int64_t)((uint64_t)(uint32_t)seq * (uint64_t)t.sb + (uint64_t)(uint32_t)head * (uint64_t)t.sh + (uint64_t)(uint32_t)tok0 * (uint64_t)t.st);
 }
 __device__ inline int order_job(int slot, int n_jobs, bool longest_last) {
     return longest_last ? n_jobs - 1 - slot : slot;
@@ -105,8 +127,9 @@ __device__ inline int turned(const KParams& p, int i) {
 __device__ inline Job dense_job(const KParams& p, int job) {
     Job j;
     int n_rb = (p.seq_len + kRowBlock - 1) / kRowBlock;
-    j.rb = n_rb - 1 - job / p.n_seq;
-    j.seq = job % p.n_seq;
+    const int from_end = divided(job, p.seqs);
+    j.rb = n_rb - 1 - from_end;
+    j.seq = job - from_end * p.n_seq;
     j.tok0 = 0;
     j.len = p.seq_len;
     j.tab0 = j.seq * n_rb * (n_rb + 1);

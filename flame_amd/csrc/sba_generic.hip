@@ -36,14 +36,14 @@ __global__ __launch_bounds__(kGenThreads) void generic_fwd_kernel(KParams p) {
     __shared__ float Ks[kGenChunk * DP];
     __shared__ float Vs[kGenChunk * DP];
     const int head = blockIdx.x % p.n_heads;
-    const Job job = decode_job(p, blockIdx.x / p.n_heads);
+    const Job job = decode_job(p, slot_of_block(p, blockIdx.x));
     const int D = p.head_dim;
     const int i = job.rb * kRowBlock + threadIdx.x;
     const bool active = i < job.len;
     const int strict = p.attend_current ? 0 : 1;
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
 
     float q[DP], acc[DP];
 #pragma unroll
@@ -92,13 +92,13 @@ template <typename T, int DP>
 __global__ __launch_bounds__(kGenThreads) void generic_weights_kernel(KParams p) {
     __shared__ float Ks[kGenChunk * DP];
     const int head = blockIdx.x % p.n_heads;
-    const Job job = decode_job(p, blockIdx.x / p.n_heads);
+    const Job job = decode_job(p, slot_of_block(p, blockIdx.x));
     const int D = p.head_dim;
     const int i = job.rb * kRowBlock + threadIdx.x;
     const bool active = i < job.len;
     const int strict = p.attend_current ? 0 : 1;
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
     // row (token i) of this head's [tokens x tokens] matrix, first column of the sequence
     const int64_t side = p.cu_seqlens ? (int64_t)p.total_tokens : (int64_t)p.seq_len;
     const int64_t plane = p.cu_seqlens ? (int64_t)head : (int64_t)job.seq * p.n_heads + head;
@@ -146,15 +146,15 @@ __global__ __launch_bounds__(kGenThreads) void generic_bwd_kernel(KParams p) {
     __shared__ float Ks[kGenChunk * DP];
     __shared__ float Vs[kGenChunk * DP];
     const int head = blockIdx.x % p.n_heads;
-    const Job job = decode_job(p, blockIdx.x / p.n_heads);
+    const Job job = decode_job(p, slot_of_block(p, blockIdx.x));
     const int D = p.head_dim;
     const int i = job.rb * kRowBlock + threadIdx.x;
     const bool active = i < job.len;
     const int strict = p.attend_current ? 0 : 1;
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
-    const int64_t dobase = (int64_t)job.seq * p.d_o.sb + (int64_t)head * p.d_o.sh + (int64_t)job.tok0 * p.d_o.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
+    const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
 
     float q[DP], dO[DP], dq[DP];
 #pragma unroll

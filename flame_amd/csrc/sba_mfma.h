@@ -338,7 +338,7 @@ __device__ inline void dma16_lanes(const char* base, uint32_t off, uint32_t lds_
 __device__ inline uint32_t lds_address(const char* p) { return (uint32_t)(uintptr_t)p; }   // (low half of the flat address)
 
 template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma {      // kNatural: rows kept in their order (query tiles)
-    static constexpr int kPerWave = 64 * kPitch<D> * 2 / 1024 / 4;    // 2 (D=64) or 4 (D=128)
+    static constexpr int kPerWave = 64 * kPitch<D> * 2 / 1024 / 4;    // 2 (D=64), 4 (D=128) or 8
     uint32_t off[kPerWave];
     const char* origin;        // row 0 of the (sequence, head) slice: uniform
     int st, w4, lane;          // row stride in elements
@@ -348,10 +348,18 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
 
     __device__ static inline void where(int inst, int lane, int& kl, int& c) {
         const int pos = inst * 64 + lane;                  // LDS chunk position
-        const int r = pos / (kPitch<D> / 8), pc = pos % (kPitch<D> / 8);
+        const int r = (unsigned)pos / (kPitch<D> / 8), pc = (unsigned)pos % (kPitch<D> / 8);
         c = pc ^ swz<D>(r);
         kl = kNatural ? r : (((r >> 2) & 1) << 5) | (((r >> 5) & 1) << 4) | (((r >> 3) & 3) << 2) | (r & 3);
     }
+    // Up to head_dim 128 a wave's i-th copy is the same chunk of a row that many rows further on: the copies are 32 or 16
+    // LDS rows apart and the swizzle looks at the low four bits of a row.
+    static constexpr bool kSameChunk = D <= 128;
+    __device__ static constexpr int rows_on(int i) {
+        return kPitch<D> == 64 ? (kNatural ? 32 : 16) * i : kNatural ? 16 * i : 8 * (i & 1) + 16 * (i >> 1);
+    }
+    // bytes from the tile's first row to chunk c of row kl (a row index and twice a token stride have at most 24 bits)
+    __device__ static inline uint32_t offset(int kl, int c, int st) { return __umul24((uint32_t)kl, 2u * (uint32_t)st) + 16u * c; }
     // Only the slice origin and the row stride are kept: holding on to the whole tensor
     // descriptor costs scalar registers that the loops do not have.
     __device__ inline void init(int lane_, int w4_, const TensorArg& t, int64_t base, int cols = D) {
@@ -368,11 +376,16 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
         asm volatile("s_mov_b64 %0, %1" : "=s"(origin_own) : "s"(origin));
         st = st_own;
         origin = origin_own;
+        int kl, c;
+        where(w4, lane, kl, c);
 #pragma unroll
         for (int i = 0; i < kPerWave; ++i) {
-            int kl, c;
-            where(w4 + 4 * i, lane, kl, c);
-            off[i] = 2u * (uint32_t)(kl * st + c * 8);
+            if (kSameChunk) {
+                off[i] = i == 0 ? offset(kl, c, st) : off[0] + 2u * (uint32_t)(rows_on(i) * st);
+            } else {
+                where(w4 + 4 * i, lane, kl, c);
+                off[i] = offset(kl, c, st);
+            }
             if (kCut) {
                 live[i] = __builtin_amdgcn_ballot_w64(c < chunks);
                 asm("" : "+s"(live[i]));
@@ -410,12 +423,12 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
         } else {
             int lane_here = lane;
             if (kLateRagged) asm volatile("" : "+v"(lane_here));
+            int kl, c;
+            where(w4, lane_here, kl, c);
 #pragma unroll
             for (int i = 0; i < kPerWave; ++i) {
-                int kl, c;
-                where(w4 + 4 * i, lane_here, kl, c);
-                kl = min(kl, len - 1 - row0);
-                copy(i, tile_base, 2u * (uint32_t)(kl * st + c * 8), tile);
+                if (!kSameChunk) where(w4 + 4 * i, lane_here, kl, c);
+                copy(i, tile_base, offset(min(kl + (kSameChunk ? rows_on(i) : 0), len - 1 - row0), c, st), tile);
             }
         }
     }
@@ -472,28 +485,31 @@ __device__ inline void store_query_rows(char* stage, const f32x16 (&acc)[D / 32]
             w.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(b, h16x2));
             *(uint2*)(stage + n * (kPitch<D> * 2) + (((4 * db + g) ^ (n & kMask)) << 4) + 8 * h) = w;
         }
+    char* const rows = t.ptr + 2 * (base + (int64_t)((uint64_t)(uint32_t)q0 * (uint64_t)t.st));     // uniform
+    const uint32_t st = 2u * (uint32_t)t.st;                                    // (at most 24 bits)
 #pragma unroll
     for (int i = 0; i < kPitch<D> / 16; ++i) {
-        const int c = lane + 64 * i, row = c / (kPitch<D> / 8), cc = c % (kPitch<D> / 8);
-        if (q0 + row < len && (kPitch<D> == D || cc * 8 < cols))
-            *(u32x4*)(t.ptr + 2 * (base + (int64_t)(q0 + row) * t.st + cc * 8)) =
+        const unsigned c = lane + 64 * i, row = c / (kPitch<D> / 8), cc = c % (kPitch<D> / 8);
+        if (q0 + (int)row < len && (kPitch<D> == D || (int)cc * 8 < cols))
+            *(u32x4*)(rows + (size_t)(__umul24(row, st) + 16 * cc)) =
                 *(const u32x4*)(stage + row * (kPitch<D> * 2) + ((cc ^ (row & kMask)) << 4));
     }
 }
 
-// B operand kept in registers for the whole sweep: row `row` of a [rows, D] tensor,
-// columns 16*ks + 8*h .. +7 for every ks.  Rows >= len read as zero.  One address, one
+// B operand kept in registers for the whole sweep: row row0 + lane_row (row0 uniform, lane_row < 64) of a [rows, D] tensor,
+// columns 16*ks + 8*h .. +7 for every ks.  Rows >= len read as zero.  One uniform address with one 32-bit lane offset, one
 // predicate; the ks fragments are at constant offsets from it.
 template <int D>
-__device__ inline void load_row_frags(h16x8 (&f)[D / 16], const TensorArg& t, int64_t base, int row,
+__device__ inline void load_row_frags(h16x8 (&f)[D / 16], const TensorArg& t, int64_t base, int row0, int lane_row,
                                       int len, int lane, int cols = D) {
     const int h = lane >> 5;
-    const char* ptr = t.ptr + 2 * (base + (int64_t)row * t.st + 8 * h);
-    if (row < len) {
+    const char* const rows = t.ptr + 2 * (base + (int64_t)((uint64_t)(uint32_t)row0 * (uint64_t)t.st));
+    const uint32_t off = __umul24((uint32_t)lane_row, 2u * (uint32_t)t.st) + 16u * h;      // (at most 24 bits each)
+    if (row0 + lane_row < len) {
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks) {
             if (D == 96 && 16 * ks + 8 * h >= cols) f[ks] = h16x8{0};
-            else f[ks] = __builtin_bit_cast(h16x8, *(const u32x4*)(ptr + 32 * ks));
+            else f[ks] = __builtin_bit_cast(h16x8, *(const u32x4*)(rows + 32 * ks + (size_t)off));
         }
     } else {
 #pragma unroll

@@ -59,22 +59,22 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     lo.init(lane);
     lo.rebase(lds);                        // absolute addresses: the loop below runs in one copy per tile buffer
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_job<D == 64>(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
+    const Job job = decode_job<D == 64>(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * wave;
     const int qi = q0w + n;
     const bool row_ok = qi < job.len;
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
-    const int64_t dobase = (int64_t)job.seq * p.d_o.sb + (int64_t)head * p.d_o.sh + (int64_t)job.tok0 * p.d_o.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
+    const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
 
     if (blockIdx.x == 0 && threadIdx.x == 0 && p.gave_up) *p.gave_up = 0;     // error word of the launch pair, see wait_for_count()
     h16x8 qf[D / 16], dof[D / 16];
-    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane, p.cols);
+    load_row_frags<D>(qf, p.q, qbase, q0w, n, job.len, lane, p.cols);
     prescale_frags(qf, p.scale2);          // the score MFMAs then deliver base-2 logits
-    load_row_frags<D>(dof, p.d_o, dobase, qi, job.len, lane, p.cols);
+    load_row_frags<D>(dof, p.d_o, dobase, q0w, n, job.len, lane, p.cols);
 
     f32x16 dqacc[D / 32];
 #pragma unroll
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     if (g_pending && row_ok) *(float*)((char*)(rcur - tstride) + g_from_r) = Gstore;
 
     store_query_rows<D>(lds + wave * kRowStage<D>, dqacc, p.scale, p.dq,                 // (the tiles are free)
-                        (int64_t)job.seq * p.dq.sb + (int64_t)head * p.dq.sh + (int64_t)job.tok0 * p.dq.st, q0w, job.len, lane, p.cols);
+                        slice_offset(p.dq, job.seq, head, job.tok0), q0w, job.len, lane, p.cols);
 }
 
 // ---------------------------------------------------------------- pass 1, two steps per iteration
@@ -240,22 +240,22 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dq2_kernel(KParams p
     LaneOffsets<D> lo;
     lo.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_job(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
+    const Job job = decode_job(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * qs;
     const int qi = q0w + n;
     const bool row_ok = qi < job.len;
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
-    const int64_t dobase = (int64_t)job.seq * p.d_o.sb + (int64_t)head * p.d_o.sh + (int64_t)job.tok0 * p.d_o.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
+    const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
 
     if (blockIdx.x == 0 && threadIdx.x == 0 && p.gave_up) *p.gave_up = 0;     // error word of the launch pair, see wait_for_count()
     h16x8 qf[D / 16], dof[D / 16];
-    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane);
+    load_row_frags<D>(qf, p.q, qbase, q0w, n, job.len, lane);
     prescale_frags(qf, p.scale2);          // the score MFMAs then deliver base-2 logits
-    load_row_frags<D>(dof, p.d_o, dobase, qi, job.len, lane);
+    load_row_frags<D>(dof, p.d_o, dobase, q0w, n, job.len, lane);
 
     f32x16 dqacc[D / 32];
 #pragma unroll
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dq2_kernel(KParams p
 #pragma unroll
             for (int r = 0; r < 16; ++r) dqacc[db][r] += park[((qs * (D / 32) + db) * 16 + r) * 64 + lane];
         store_query_rows<D>((char*)(park + qs * (D / 32) * 16 * 64), dqacc, p.scale, p.dq,      // (over what this wave has just read)
-                            (int64_t)job.seq * p.dq.sb + (int64_t)head * p.dq.sh + (int64_t)job.tok0 * p.dq.st, q0w, job.len, lane, D);
+                            slice_offset(p.dq, job.seq, head, job.tok0), q0w, job.len, lane, D);
     }
 }
 
@@ -423,16 +423,16 @@ __global__ __launch_bounds__(kThreads, 2) void mfma_bwd_dkv_kernel(KParams p) {
     LaneOffsets<64> lz;                        // the weight tiles have 64-key rows whatever D is
     lz.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const int slot = blockIdx.x / p.n_heads;   // two 64-key blocks per scheduled 128-row job
+    const int slot = slot_of_block(p, blockIdx.x);   // two 64-key blocks per scheduled 128-row job
     const Job job = decode_key_job(p, slot >> 1);
     const int kb = 2 * job.rb + (slot & 1);
     const int key0 = kb * kKeyBlock;
     if (key0 >= job.len) return;               // uniform over the workgroup
     const int strict = p.attend_current ? 0 : 1;
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
-    const int64_t dobase = (int64_t)job.seq * p.d_o.sb + (int64_t)head * p.d_o.sh + (int64_t)job.tok0 * p.d_o.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
+    const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
     const int n_qb = last_live_row_block(p, head, job) + 1;
     const int kh = wave & 1;                   // which 32 keys this wave reduces
     const int dbw = wave >> 1;                 // and which d-blocks: dbw + 2*i
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(kThreads, 2) void mfma_bwd_dkv_kernel(KParams p) {
     h16x8 qfn[D / 16];
     {
         const int qi0 = qb0 * kRowBlock + 32 * wave + n;
-        load_row_frags<D>(qfn, p.q, qbase, qi0, job.len, lane);
+        load_row_frags<D>(qfn, p.q, qbase, qb0 * kRowBlock + 32 * wave, n, job.len, lane);
         if (qi0 < job.len) {
             const int64_t t = tab_index(p, head, job, qb0, kb) + 32 * wave + n;
             Rn = p.rtab[t]; Gn = p.gtab[t];
@@ -480,11 +480,11 @@ __global__ __launch_bounds__(kThreads, 2) void mfma_bwd_dkv_kernel(KParams p) {
         h16x8 qf[D / 16], dof[D / 16];
 #pragma unroll
         for (int ks = 0; ks < D / 16; ++ks) qf[ks] = qfn[ks];
-        load_row_frags<D>(dof, p.d_o, dobase, qi, job.len, lane);
+        load_row_frags<D>(dof, p.d_o, dobase, q0w, n, job.len, lane);
         float R = Rn, Gc = Gn;
         if (qb + 1 < n_qb) {
             const int qin = qi + kRowBlock;
-            load_row_frags<D>(qfn, p.q, qbase, qin, job.len, lane);
+            load_row_frags<D>(qfn, p.q, qbase, q0w + kRowBlock, n, job.len, lane);
             Rn = 1.0f; Gn = 0.0f;
             if (qin < job.len) {
                 const int64_t t = tab_index(p, head, job, qb + 1, kb) + 32 * wave + n;
@@ -546,8 +546,8 @@ __global__ __launch_bounds__(kThreads, 2) void mfma_bwd_dkv_kernel(KParams p) {
         stage_acc_tile<D>(stage_v, 32 * kh, 32 * (dbw + 2 * i), dvacc[i], 1.0f, lane);
     }
     __syncthreads();
-    const int64_t dkbase = (int64_t)job.seq * p.dk.sb + (int64_t)head * p.dk.sh + (int64_t)job.tok0 * p.dk.st;
-    const int64_t dvbase = (int64_t)job.seq * p.dv.sb + (int64_t)head * p.dv.sh + (int64_t)job.tok0 * p.dv.st;
+    const int64_t dkbase = slice_offset(p.dk, job.seq, head, job.tok0);
+    const int64_t dvbase = slice_offset(p.dv, job.seq, head, job.tok0);
     store_staged_rows<D>(stage_k, p.dk, dkbase, key0, job.len, threadIdx.x, kThreads);
     store_staged_rows<D>(stage_v, p.dv, dvbase, key0, job.len, threadIdx.x, kThreads);
 }
@@ -630,7 +630,7 @@ __device__ inline KeyItem decode_item(const KParams& p, int idx) {
     r.valid = idx >= 0;
     if (idx < 0) idx = 0;
     r.head = head_of_block(p, idx);
-    const int slot = idx / p.n_heads;          // two 64-key blocks per scheduled 128-row job
+    const int slot = slot_of_block(p, idx);          // two 64-key blocks per scheduled 128-row job
     r.job = decode_key_job(p, slot >> 1);
     r.kb = 2 * r.job.rb + (slot & 1);
     r.key0 = r.kb * kKeyBlock;
@@ -1174,25 +1174,25 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
     LaneOffsets<64> lz;
     lz.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_key_job<D == 64>(p, blockIdx.x / p.n_heads);
+    const Job job = decode_key_job<D == 64>(p, slot_of_block(p, blockIdx.x));
     const int strict = p.attend_current ? 0 : 1;
     const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it
     const int kb0 = q_begin + 32 * wave;               // first key of this wave
     char* ztile = lds + 2 * kNBuf * kQTile + wave * kZTile;
 
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
-    const int64_t dobase = (int64_t)job.seq * p.d_o.sb + (int64_t)head * p.d_o.sh + (int64_t)job.tok0 * p.d_o.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
+    const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
 
     // A operands of the score tiles: MFMA row m holds key 16*((m>>2)&1) + 4*(m>>3) + (m&3) of
     // the wave, so that the accumulator registers of a lane are 16 consecutive keys
     h16x8 kfr[D / 16], vfr[D / 16];
     {
         const int m = lane & 31;
-        const int key = kb0 + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
-        load_row_frags<D>(kfr, p.k, kbase, key, job.len, lane);
-        load_row_frags<D>(vfr, p.v, vbase, key, job.len, lane);
+        const int key = 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
+        load_row_frags<D>(kfr, p.k, kbase, kb0, key, job.len, lane);
+        load_row_frags<D>(vfr, p.v, vbase, kb0, key, job.len, lane);
         prescale_frags(kfr, p.scale2);         // K times the logit scale: the score MFMAs deliver base-2 logits
     }
 
@@ -1415,7 +1415,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
         const TensorArg& out = which == 0 ? p.dk : p.dv;
-        const int64_t ob = (int64_t)job.seq * out.sb + (int64_t)head * out.sh + (int64_t)job.tok0 * out.st;
+        const int64_t ob = slice_offset(out, job.seq, head, job.tok0);
         constexpr int kCols = D / kSplit;          // columns part * kCols .. of the rows
 #pragma unroll
         for (int db = 0; db < kNB; ++db)
@@ -1438,7 +1438,10 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
 // where the two passes read them twice, no prefix table is written or read, and it is one launch.
 // What bounds it is memory (seven tensors' bytes): two workgroups of four waves (80 KB of LDS) or four of two waves (sequences
 // of at most 64 tokens) share a CU at head_dim 64, so that one's loads and stores run under the other's arithmetic; the next key
-// block's K and V are requested into the tile just used.
+// block's K and V are requested into the tile just used.  On 65536 tokens in documents of 16 .. 128 (H=16, d=64) it takes 256 us where
+// its copies and stores alone take 200 and its arithmetic, on rows that the caches hold, about 230: 1650 instructions per wave of
+// which the two chains are 600.  (Two documents in turn per workgroup, the next one's rows requested into registers meanwhile, are
+// behind at every size: 64 registers and the second document's scalars spill, and the loads were not what was waited for.)
 template <int D, int W>
 __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel(KParams p) {
     constexpr int kRows = W * 32;
@@ -1453,7 +1456,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_job(p, blockIdx.x / p.n_heads);
+    const Job job = decode_job(p, slot_of_block(p, blockIdx.x));
     if (blockIdx.x == 0 && threadIdx.x == 0 && p.gave_up) *p.gave_up = 0;
     LaneOffsets<D> lo;
     lo.init(lane);
@@ -1464,7 +1467,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
     const int strict = p.attend_current ? 0 : 1;
     const int q0w = 32 * wave, qi = q0w + n;
     const bool row_ok = qi < job.len;
-    auto base_of = [&](const TensorArg& t) { return (int64_t)job.seq * t.sb + (int64_t)head * t.sh + (int64_t)job.tok0 * t.st; };
+    auto base_of = [&](const TensorArg& t) { return slice_offset(t, job.seq, head, job.tok0); };
     const int64_t qbase = base_of(p.q), kbase = base_of(p.k), vbase = base_of(p.v), dobase = base_of(p.d_o);
 
     // a tile is four waves' copies: two each where there are only two
@@ -1508,9 +1511,7 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
     }
     prescale_frags(qf, p.scale2);
 
-    f32x16 dqacc[D / 32];
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db) dqacc[db] = f32x16{0};
+    f32x16 dqacc[D / 32];                      // (started by the first block, which every wave with rows sees)
     float Gc = 0.f;
     constexpr TileAt ktile{kK}, vtile{kV};
     const int which = W == 2 ? wave : wave >> 1, kh0 = W == 2 ? 0 : wave & 1;
@@ -1545,8 +1546,11 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
 #pragma unroll
                 for (int db = 0; db < D / 32; ++db) kt[db] = fetch_cols_o<D>(ktile, lo, db, c);
 #pragma unroll
-                for (int db = 0; db < D / 32; ++db) dqacc[db] = mfma(kt[db], zf[c], dqacc[db]);
+                for (int db = 0; db < D / 32; ++db) dqacc[db] = mfma(kt[db], zf[c], kb == 0 && c == 0 ? f32x16{0} : dqacc[db]);
             }
+        } else if (kb == 0) {
+#pragma unroll
+            for (int db = 0; db < D / 32; ++db) dqacc[db] = f32x16{0};
         }
         __syncthreads();                       // weights complete, K and V free
         if (kb + 1 < n_kb) {
@@ -1556,10 +1560,6 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
         // [32 keys x D] of dV (which = 0) or dK: keys 32 kh .. of the block, over the queries from the block on; transposed tiles
         // (lane = key), which leave as rows the way dQ does
         f32x16 acc[kKH][kNB];
-#pragma unroll
-        for (int i = 0; i < kKH; ++i)
-#pragma unroll
-            for (int db = 0; db < kNB; ++db) acc[i][db] = f32x16{0};
         {
             const int offw = which ? kZ : kA, offb = which ? kQ : kDO;
             auto fetch = [&](int x0, int x1, int add) {
@@ -1568,26 +1568,44 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
                 u.v[1] = lds_read_tr_at((uint32_t)(x1 + add), 0);
                 return u.b;
             };
-            for (int r = key0; r < job.len; r += 16) {
-                h16x8 w[kKH];
+            // 32 queries at a time, all their operands requested before the first product (a wave writes whole 32-row tiles of
+            // weights, zeros past the end); the first ones start the sums
+            auto reduce = [&](int r, auto first) {
+                h16x8 w[2][kKH], b[2][kNB];
 #pragma unroll
-                for (int i = 0; i < kKH; ++i)
-                    w[i] = fetch(kh0 + i ? lz.nat[0][1] : lz.nat[0][0], kh0 + i ? lz.nat[1][1] : lz.nat[1][0], offw + r * 128);
+                for (int half = 0; half < 2; ++half) {
 #pragma unroll
-                for (int db = 0; db < kNB; ++db) {
-                    const h16x8 b = fetch(lo.nat[0][db], lo.nat[1][db], offb + r * kPitch<D> * 2);
+                    for (int i = 0; i < kKH; ++i)
+                        w[half][i] = fetch(kh0 + i ? lz.nat[0][1] : lz.nat[0][0], kh0 + i ? lz.nat[1][1] : lz.nat[1][0], offw + (r + 16 * half) * 128);
 #pragma unroll
-                    for (int i = 0; i < kKH; ++i) acc[i][db] = mfma(b, w[i], acc[i][db]);
+                    for (int db = 0; db < kNB; ++db) b[half][db] = fetch(lo.nat[0][db], lo.nat[1][db], offb + (r + 16 * half) * kPitch<D> * 2);
                 }
-            }
+#pragma unroll
+                for (int half = 0; half < 2; ++half)
+#pragma unroll
+                    for (int db = 0; db < kNB; ++db)
+#pragma unroll
+                        for (int i = 0; i < kKH; ++i)
+                            acc[i][db] = mfma(b[half][db], w[half][i], decltype(first)::value && half == 0 ? f32x16{0} : acc[i][db]);
+            };
+            reduce(key0, std::true_type{});
+            for (int r = key0 + 32; r < job.len; r += 32) reduce(r, std::false_type{});
+        }
+        if (which) {
+#pragma unroll
+            for (int i = 0; i < kKH; ++i)
+#pragma unroll
+                for (int db = 0; db < kNB; ++db)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[i][db][e] *= p.scale;
         }
         __syncthreads();                       // weight tiles free
         {
             const TensorArg& out = which ? p.dk : p.dv;
 #pragma unroll
             for (int i = 0; i < kKH; ++i)
-                store_query_rows<D>(lds + kA + (wave * kKH + i) * kRowStage<D>, acc[i], which ? p.scale : 1.0f, out, base_of(out),
-                                    key0 + 32 * (kh0 + i), job.len, lane, p.cols);
+                store_query_rows<D>(lds + kA + (wave * kKH + i) * kRowStage<D>, acc[i], 1.0f, out, base_of(out), key0 + 32 * (kh0 + i),
+                                    job.len, lane, p.cols);
         }
         if (kb + 1 < n_kb) {
             wait_global_memory();              // the next K and V have landed
@@ -1631,25 +1649,25 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
     LaneOffsets<64> lz;
     lz.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_key_job(p, blockIdx.x / p.n_heads);
+    const Job job = decode_key_job(p, slot_of_block(p, blockIdx.x));
     const int strict = p.attend_current ? 0 : 1;
     const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it
     const int kb0 = q_begin + 32 * grp;                // first key of this pair
     char* ztile = lds + 4 * kQTile + grp * kZTile;
 
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
-    const int64_t dobase = (int64_t)job.seq * p.d_o.sb + (int64_t)head * p.d_o.sh + (int64_t)job.tok0 * p.d_o.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
+    const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
 
     // A operands of the score tile: MFMA row m holds key 16*((m>>2)&1) + 4*(m>>3) + (m&3) of the pair,
     // so that the accumulator registers of a lane are 16 consecutive keys (as in the own-keys kernel)
     h16x8 kfr[D / 16], vfr[D / 16];
     {
         const int m = lane & 31;
-        const int key = kb0 + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
-        load_row_frags<D>(kfr, p.k, kbase, key, job.len, lane, p.cols);
-        load_row_frags<D>(vfr, p.v, vbase, key, job.len, lane, p.cols);
+        const int key = 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
+        load_row_frags<D>(kfr, p.k, kbase, kb0, key, job.len, lane, p.cols);
+        load_row_frags<D>(vfr, p.v, vbase, kb0, key, job.len, lane, p.cols);
         prescale_frags(kfr, p.scale2);
     }
     f32x16 dkacc[kBlocks], dvacc[kBlocks];
@@ -1840,7 +1858,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
         const TensorArg& out = which == 0 ? p.dk : p.dv;
-        const int64_t ob = (int64_t)job.seq * out.sb + (int64_t)head * out.sh + (int64_t)job.tok0 * out.st;
+        const int64_t ob = slice_offset(out, job.seq, head, job.tok0);
 #pragma unroll
         for (int j = 0; j < kBlocks; ++j)
             if (j == 0 || both) stage_acc_tile<D>(ztile, 0, 32 * (kBlocks * half + j), which == 0 ? dkacc[j] : dvacc[j], which == 0 ? p.scale : 1.0f, lane);

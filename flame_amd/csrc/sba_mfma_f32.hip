@@ -43,7 +43,7 @@ struct Slice {
     const char* origin;
     uint32_t st;
     __device__ inline Slice(const TensorArg& t, const Job& job, int head)
-        : origin(t.ptr + 4 * ((int64_t)job.seq * t.sb + (int64_t)head * t.sh + (int64_t)job.tok0 * t.st)), st(4u * (uint32_t)t.st) {}
+        : origin(t.ptr + 4 * (slice_offset(t, job.seq, head, job.tok0))), st(4u * (uint32_t)t.st) {}
     __device__ inline const char* row(int r) const { return origin + (uint64_t)(uint32_t)r * st; }
 };
 
@@ -189,8 +189,9 @@ template <int S> struct RowGroup {
     Job job;
     int head, sub, q0, lane_of_sweep;
     __device__ inline RowGroup(const KParams& p, int wave) {
-        const int slot = blockIdx.x / p.n_heads;
-        head = (blockIdx.x - slot * p.n_heads + slot / S) % p.n_heads;
+        const int slot = slot_of_block(p, blockIdx.x);
+        head = blockIdx.x - slot * p.n_heads + slot / S;
+        head -= divided(head, p.heads) * p.n_heads;
         job = decode_job<true>(p, slot / S);
         sub = S == 4 ? 3 - (slot & 3) : wave;
         lane_of_sweep = S == 4 ? wave : 0;
@@ -327,7 +328,7 @@ __device__ inline void clear_cut_rows(const KParams& p, const Job& job, int head
 }
 template <int D>
 __global__ __launch_bounds__(kThreads) void clear_cut_kernel(KParams p) {
-    const Job job = decode_job(p, blockIdx.x / p.n_heads);
+    const Job job = decode_job(p, slot_of_block(p, blockIdx.x));
     clear_cut_rows<D, kRowBlock>(p, job, head_of_block(p, blockIdx.x), job.rb * kRowBlock);
 }
 
@@ -431,8 +432,9 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int head = head_of_block(p, blockIdx.x);
-    const int slot = blockIdx.x / (kCut ? 2 * p.n_heads : p.n_heads);   // two 64-key blocks per scheduled 128-row job
-    const int part = kCut ? blockIdx.x / p.n_heads & 1 : 0;
+    const int unit = slot_of_block(p, blockIdx.x);
+    const int slot = kCut ? unit >> 1 : unit;  // two 64-key blocks per scheduled 128-row job
+    const int part = kCut ? unit & 1 : 0;
     const Job job = decode_key_job(p, slot >> 1);
     const int kb = 2 * job.rb + (slot & 1);
     const int key0 = kb * kKeyBlock;

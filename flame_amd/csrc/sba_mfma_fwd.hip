@@ -52,7 +52,7 @@ __device__ inline bool fwd_step(const char* ktile, const char* vtile, const Lane
 
 template <int D>
 __device__ inline void store_o_rows(char* stage, const KParams& p, const Job& job, int head, int q0w, int lane, const f32x16 (&oacc)[D / 32]) {
-    store_query_rows<D>(stage, oacc, 1.0f, p.o, (int64_t)job.seq * p.o.sb + (int64_t)head * p.o.sh + (int64_t)job.tok0 * p.o.st,
+    store_query_rows<D>(stage, oacc, 1.0f, p.o, slice_offset(p.o, job.seq, head, job.tok0),
                         q0w, job.len, lane, p.cols);
 }
 
@@ -70,18 +70,18 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     LaneOffsets<D> lo;
     lo.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_job<D == 64>(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
+    const Job job = decode_job<D == 64>(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * wave;              // first query of this wave
     const int qi = q0w + n;                      // this lane's query
     const bool rows_full = q0w + 31 < job.len;   // wave-uniform
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
 
     h16x8 qf[D / 16];
-    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane, p.cols);
+    load_row_frags<D>(qf, p.q, qbase, q0w, n, job.len, lane, p.cols);
     prescale_frags(qf, p.scale2);
 
     f32x16 oacc[D / 32];
@@ -227,18 +227,18 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     LaneOffsets<D> lo;
     lo.init(lane);
     const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_job<D == 64 && G == 2>(p, order_job(blockIdx.x / p.n_heads, p.n_jobs, false));
+    const Job job = decode_job<D == 64 && G == 2>(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * qs;
     const int qi = q0w + n;
     const bool rows_full = q0w + 31 < job.len;      // wave-uniform
-    const int64_t qbase = (int64_t)job.seq * p.q.sb + (int64_t)head * p.q.sh + (int64_t)job.tok0 * p.q.st;
-    const int64_t kbase = (int64_t)job.seq * p.k.sb + (int64_t)head * p.k.sh + (int64_t)job.tok0 * p.k.st;
-    const int64_t vbase = (int64_t)job.seq * p.v.sb + (int64_t)head * p.v.sh + (int64_t)job.tok0 * p.v.st;
+    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
+    const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
 
     h16x8 qf[D / 16];
-    load_row_frags<D>(qf, p.q, qbase, qi, job.len, lane, p.cols);
+    load_row_frags<D>(qf, p.q, qbase, q0w, n, job.len, lane, p.cols);
     prescale_frags(qf, p.scale2);
     f32x16 oacc[D / 32];
 #pragma unroll
