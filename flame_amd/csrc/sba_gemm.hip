@@ -322,15 +322,18 @@ template <int kEpi, int TI, int TJ> struct Results {
 // Launches that are short of tiles: T x T tiles, kPerCu workgroups a CU, each of G groups of four waves (two by two, T/2 tokens x T/2
 // features each) that share out the contraction: group g takes stages g, g + G, ...  The groups' fp32 sums meet in LDS, in the order of
 // the groups, and as many groups as there are blocks of tokens write the results.  k a multiple of 32.
-// Stages of 64 k, two buffers a group, walked slice by slice as in the kernel for large products below.  Rows of 64 k are whole 128-byte
+// Stages of 64 k, NB buffers a group, walked slice by slice as in the kernel for large products below.  Rows of 64 k are whole 128-byte
 // lines: with 32 k the CU's memory pipe takes 16 lines for a kilobyte instead of 8, and 4096 x 1024, k = 2816, with the residual took 34 us (31
 // now; four buffers of 32 k and one group, the shape before this: 37).  What bounds them: LDS, 128 bytes a cycle for the operands of 64 x 64
-// products a wave and the arriving tiles (T = 128), a round trip to memory per stage and group (T = 64).
+// products a wave and the arriving tiles (T = 128); the round trip to memory, 1.5 us with every CU asking (T = 64), which is what two
+// stages more on their way are for: 1024 x 768, k = 4096, with four groups of two buffers 27 us inside a training step, with two groups of
+// four 21; 2048 x 1024 with the residual, k = 1024, with two workgroups of two groups a CU 9.7, with three of one group and three buffers 9.3.
 // A tile row of 64 k is eight 16-byte chunks; chunk c of row r lies at c ^ (r / 2 % 8), so that sixteen consecutive rows' chunks of one index
 // fall on sixteen different bank groups.  The products are formed transposed (rows: features, columns: tokens).
-template <int T, int G, int kPerCu, bool kRowsW, int kEpi>
+template <int T, int G, int NB, int kPerCu, bool kRowsW, int kEpi>
 __global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Projection p) {
-    constexpr int KS = 64, NB = 2;                                     // k of a stage, buffers of a group
+    constexpr int KS = 64;                                             // k of a stage
+    constexpr bool kPadded = NB == 2;                                  // whole groups of turns, filled up with zeros
     constexpr int kX = T * KS * 2, kStage = 2 * kX;                    // bytes
     constexpr int PX = T / 32;                                         // copies of one operand per wave and stage
     constexpr int C = KS / 8;                                          // 16-byte chunks of a row of k
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Project
     constexpr int kBand = 1024 / T;
     const int band = t / (kBand * tiles_n), rows = min(kBand, tiles_m - kBand * band), in = t - band * kBand * tiles_n;
     const int t0 = (kBand * band + in % rows) * T, n0 = (in / rows) * kOwn;
-    const int stages = (p.k + KS - 1) / KS, turns = (stages + G - 1) / G, padded = (turns + NB - 1) / NB * NB;
+    const int stages = (p.k + KS - 1) / KS, turns = (stages + G - 1) / G, padded = kPadded ? (turns + NB - 1) / NB * NB : turns;
     const int nk = (stages + G - 1 - group) / G;                       // this group's stages: group, group + G, ...
     const bool odd = p.k % KS != 0;                                    // the last stage is half a one ...
     const int half_stage = odd && (stages - 1) % G == group ? nk - 1 : -1;      // ... and this group's, this turn's
@@ -466,6 +469,7 @@ __global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Project
     // does not have are made with zeros.
     auto turn = [&](int s, int b, bool asked) __attribute__((always_inline)) {
         if (asked && R) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(R) : "memory");
+        else if (s + NB <= nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((NB - 2) * 2 * PX) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (s + 1 < padded && s + 1 >= stages / G - odd) {             // (some group may lack it: the same for all of them)
             clear(s + 1, (b + 1) % NB);
@@ -473,7 +477,6 @@ __global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Project
         }
         if (s + NB < nk) request(s + NB, b);
     };
-    static_assert(NB == 2, "turn() waits for all copies: those of the next stage");
 
     res.aim(lane, t0 + (w & 1) * (T / 2) + 16 * J * (group % E), n0 + (w >> 1) * (kOwn / 2));
 #pragma unroll
@@ -487,7 +490,7 @@ __global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Project
     }
 #pragma unroll
     for (int n = 0; n < TI + TJ; ++n) fetch(0, n, 0, 0);
-    for (int s0 = 0; s0 < turns; s0 += NB) {   // whole groups of stages, filled up with zeros (see the weight-gradient kernel)
+    for (int s0 = 0; s0 < turns; s0 += NB) {   // (filled up with zeros where an exit in between would cost copies of the sums)
         const bool asked = s0 + NB >= turns && group < E;      // (all copies are on their way by then)
         if (R && asked) {
 #pragma unroll
@@ -495,6 +498,7 @@ __global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Project
         }
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
+            if (!kPadded && b > 0 && s0 + b >= turns) break;
             slice(0, b, 1);
             turn(s0 + b, b, asked);
             slice(1, (b + 1) % NB, 0);
@@ -733,21 +737,21 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // the last copies, unread, have landed before the LDS is given back
 }
 
-template <int T, int G, int kPerCu>
+template <int T, int G, int NB, int kPerCu>
 int launch_projection(const Projection& p, hipStream_t s) {
     const int own = p.epilogue == sba_model::kSwigluFwd ? T / 2 : T, features = p.epilogue == sba_model::kSwigluFwd ? p.n / 2 : p.n;
     const int tiles = ((p.m + T - 1) / T) * ((features + own - 1) / own);
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256 * G);
     if (p.rows_w) {
-        if (p.epilogue == sba_model::kSwigluBwd) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, true, sba_model::kSwigluBwd>), grid, block, 0, s, p);
-        else if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, true, sba_model::kStore>), grid, block, 0, s, p);
+        if (p.epilogue == sba_model::kSwigluBwd) hipLaunchKernelGGL((projection_kernel<T, G, NB, kPerCu, true, sba_model::kSwigluBwd>), grid, block, 0, s, p);
+        else if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((projection_kernel<T, G, NB, kPerCu, true, sba_model::kStore>), grid, block, 0, s, p);
         else return -2;
     } else {
         if (p.epilogue == sba_model::kSwigluFwd) {
-            if constexpr (T == 128) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, false, sba_model::kSwigluFwd>), grid, block, 0, s, p);
+            if constexpr (T == 128) hipLaunchKernelGGL((projection_kernel<T, G, NB, kPerCu, false, sba_model::kSwigluFwd>), grid, block, 0, s, p);
             else return -2;                    // (swiglu pairs two blocks of gates)
-        } else if (p.epilogue == sba_model::kAddResidual) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, false, sba_model::kAddResidual>), grid, block, 0, s, p);
-        else if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((projection_kernel<T, G, kPerCu, false, sba_model::kStore>), grid, block, 0, s, p);
+        } else if (p.epilogue == sba_model::kAddResidual) hipLaunchKernelGGL((projection_kernel<T, G, NB, kPerCu, false, sba_model::kAddResidual>), grid, block, 0, s, p);
+        else if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((projection_kernel<T, G, NB, kPerCu, false, sba_model::kStore>), grid, block, 0, s, p);
         else return -2;
     }
     return hipGetLastError() == hipSuccess ? 0 : -6;
@@ -785,10 +789,10 @@ int SBA_PROJECT(const Projection& p, ProjectionTile tile, hipStream_t s) {
     using namespace sba::SBA_ELEM_NS;
     if (tile == kTile256) return launch_large_projection<256>(p, s);
     if (tile == kTile128x256) return launch_large_projection<128>(p, s);
-    if (tile == kTile128Halves) return launch_projection<128, 2, 1>(p, s);
-    if (tile == kTile64Halves) return launch_projection<64, 2, 2>(p, s);
-    if (tile == kTile64Quarters) return launch_projection<64, 4, 1>(p, s);
-    return launch_projection<128, 1, 2>(p, s);
+    if (tile == kTile128Halves) return launch_projection<128, 2, 2, 1>(p, s);
+    if (tile == kTile64) return launch_projection<64, 1, 3, 3>(p, s);
+    if (tile == kTile64Halves) return launch_projection<64, 2, 4, 1>(p, s);
+    return launch_projection<128, 1, 2, 2>(p, s);
 }
 int SBA_WEIGHT_GRADS(const WeightGrads& g, int splits, hipStream_t stream) {
     const dim3 grid((unsigned)((g.tiles + 7) / 8 * 8), (unsigned)splits), block(256);

@@ -84,7 +84,7 @@ struct Projection {
     const float* residual; void* pre; void* out;
 };
 bool projects(const Projection& p, int cus);             // whether the kernels take it
-enum ProjectionTile { kTile256, kTile128x256, kTile128, kTile128Halves, kTile64Halves, kTile64Quarters };
+enum ProjectionTile { kTile256, kTile128x256, kTile128, kTile128Halves, kTile64, kTile64Halves };
 ProjectionTile projection_tile(const Projection& p, int cus);
 double tile_time(const Projection& p, ProjectionTile tile, int cus);    // an estimate, us; 1e30 where its kernel does not take it
 int project(const Projection& p, bool f16, int cus, hipStream_t stream);

@@ -521,31 +521,30 @@ int weight_grad_splits(WeightGrads& g, int cus) {
     return best;
 }
 
-// Time estimates in us of the projection kernels (sba_gemm.hip), from sweeps of 512 .. 8192 rows, 512 .. 5632 features and k of 512 .. 5632:
-// rounds of resident workgroups, each k / 64 times `full` (a last round that fills half of the chip or less: `part`, what lies
-// between in proportion) and `round` (in proportion to its fill), and `launch`.
+// Time estimates in us of the projection kernels (sba_gemm.hip), fitted to sweeps of 300 .. 8192 rows, 512 .. 5632 features and k of 512
+// .. 5632 with every epilogue (270 products; the tile chosen takes 1 % more than the best on the average, 16 % at most): rounds of
+// resident workgroups, each k / 64 times `full` (a last round that fills half of the chip or less: `part`, what lies between in
+// proportion) and `round` with what the epilogue adds that nothing hides (in proportion to its fill), and `launch`.
 // Where each is ahead (us): 256 x 256 8192 x 5632 of swiglu, k = 1024 (92, next 101); 128 x 256 8192 x 3072, k = 1024 (49; 52);
-// 128 x 128 two a CU 4096 x 1024, k = 1024 (12; 15); by halves 4096 x 1024, k = 5632 (49; 59); 64 x 64 by halves 2048 x 1024, k = 1024
-// (9; 11); by quarters 1024 x 1024, k = 5632 (27; 32).
+// 128 x 128 two a CU 4096 x 1024, k = 1024 (12; 15); by halves 4096 x 1024, k = 5632 (49; 59); 64 x 64 three a CU 2048 x 2304,
+// k = 768 (13.0; 14.0), 1500 x 2816 with the swiglu gradient, k = 1024 (21; 24); by halves 1024 x 768, k = 4096 (15.8; 19.8).
 double tile_time(const Projection& p, ProjectionTile tile, int cus) {
-    struct { int rows, features, per_cu; double part, full, round, launch; } static const cost[] = {
-        {256, 256, 1, 1.14, 1.32, 8.7, 2.6},    // kTile256
-        {128, 256, 1, 0.57, 0.78, 3.9, 5.0},    // kTile128x256
-        {128, 128, 2, 0.60, 0.89, 3.5, 2.5},    // kTile128
-        {128, 128, 1, 0.47, 0.475, 3.8, 3.0},   // kTile128Halves
-        {64, 64, 2, 0.32, 0.38, 1.5, 1.6},      // kTile64Halves
-        {64, 64, 1, 0.25, 0.22, 1.5, 2.6},      // kTile64Quarters
+    struct { int rows, features, per_cu; double part, full, round, launch, add, swiglu_fwd, swiglu_bwd; } static const cost[] = {
+        {256, 256, 1, 1.07, 1.25, 3.6, 7.1, 0.0, 2.5, 0.0},     // kTile256
+        {128, 256, 1, 0.665, 0.751, 1.4, 5.8, 10.8, 1.1, 0.0},  // kTile128x256
+        {128, 128, 2, 0.608, 0.803, 3.5, 2.5, 8.3, 0.0, 10.4},  // kTile128
+        {128, 128, 1, 0.49, 0.495, 2.1, 3.2, 3.9, 0.6, 7.4},    // kTile128Halves
+        {64, 64, 3, 0.253, 0.509, 0.9, 2.6, 2.4, 0.0, 3.1},     // kTile64
+        {64, 64, 1, 0.187, 0.198, 1.3, 2.6, 0.5, 0.0, 1.5},     // kTile64Halves
     };
     const auto& c = cost[tile];
     const bool glu = p.epilogue == kSwigluFwd;
     if (tile <= kTile128x256 && (p.k % 64 || p.epilogue == kSwigluBwd)) return 1e30;
     if (tile == kTile256 && p.epilogue == kAddResidual) return 1e30;       // its registers
-    if (tile >= kTile64Halves && glu) return 1e30;
+    if (tile >= kTile64 && glu) return 1e30;
     const int64_t own = glu ? c.features / 2 : c.features, features = glu ? p.n / 2 : p.n;
     const int64_t tiles = ((int64_t)p.m + c.rows - 1) / c.rows * ((features + own - 1) / own), slots = (int64_t)cus * c.per_cu;
-    // bytes of the epilogue that nothing hides: gate and up of the backward with their gradients, the residual, swiglu's second and third tensor
-    const double round = c.round + (p.epilogue == kSwigluBwd ? 10.0 * c.per_cu * c.rows * c.features / 32768 :
-                                    p.epilogue == kAddResidual ? (tile == kTile128x256 ? 9.5 : tile == kTile128 ? 7.0 : 1.5) : glu ? (tile == kTile256 ? 3.0 : 1.0) : 0.0);
+    const double round = c.round + (p.epilogue == kAddResidual ? c.add : glu ? c.swiglu_fwd : p.epilogue == kSwigluBwd ? c.swiglu_bwd : 0.0);
     const double k64 = (p.k + 63) / 64, fill = (double)(tiles % slots) / slots;
     const double rate = fill <= 0.5 ? c.part : c.part + (c.full - c.part) * (2 * fill - 1);
     return tiles / slots * (c.full * k64 + round) + (fill > 0 ? rate * k64 + round * fill : 0.0) + c.launch;
@@ -571,7 +570,7 @@ bool projects(const Projection& p, int cus) {
 ProjectionTile projection_tile(const Projection& p, int cus) {
     ProjectionTile best = kTile128;
     double best_us = 1e30;
-    for (int t = kTile256; t <= kTile64Quarters; ++t) {
+    for (int t = kTile256; t <= kTile64Halves; ++t) {
         const double us = tile_time(p, (ProjectionTile)t, cus);
         if (us < best_us) { best = (ProjectionTile)t; best_us = us; }
     }

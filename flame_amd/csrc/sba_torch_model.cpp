@@ -174,7 +174,7 @@ bool try_project(const Tensor& x, const Tensor& w, bool rows_w, int epilogue, co
 bool project_with(int64_t tile, const Tensor& x, const Tensor& w, bool rows_w, int64_t epilogue, const std::optional<Tensor>& residual,
                   const std::optional<Tensor>& pre, const Tensor& out) {
     const Projection p = projection_of(x, w, rows_w, (int)epilogue, residual.value_or(Tensor()), pre.value_or(Tensor()), out);
-    TORCH_CHECK(tile >= kTile256 && tile <= kTile64Quarters && p.k % 32 == 0 && p.n % 16 == 0 && p.ldx % 8 == 0 && p.ldw % 8 == 0 && p.m > 0,
+    TORCH_CHECK(tile >= kTile256 && tile <= kTile64Halves && p.k % 32 == 0 && p.n % 16 == 0 && p.ldx % 8 == 0 && p.ldw % 8 == 0 && p.m > 0,
                 "project_with: sizes that no tile takes");
     if (tile_time(p, (ProjectionTile)tile, compute_units()) >= 1e30) return false;
     ok(project_tile(p, (ProjectionTile)tile, is_f16(x.scalar_type()), stream_of(x)));
@@ -586,7 +586,7 @@ void bind_model(py::module& m) {
     m.def("clip_and_step", &clip_and_step);
     m.def("project", &project);
     m.def("project_with", &project_with);
-    m.attr("projection_tiles") = (int)kTile64Quarters + 1;
+    m.attr("projection_tiles") = (int)kTile64Halves + 1;
     m.def("project_add", &project_add);
     m.def("project_swiglu", [](const Tensor& x, const Tensor& w) {
         Tensor pre;
