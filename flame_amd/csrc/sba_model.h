@@ -27,7 +27,8 @@ struct NormBwd {
 };
 int norm_bwd_parts(int rows);
 int norm_bwd(const NormBwd& a, bool f16, hipStream_t stream);
-int sum_parts(const float* part, float* out, int parts, int cols, hipStream_t stream);
+// out[i][c] = sum over the parts of part[i], for one or two of them in a launch
+int sum_parts(const float* const (&part)[2], float* const (&out)[2], int n, int parts, int cols, hipStream_t stream);
 
 int add_residual(const float* x, const void* h, float* out, int64_t n, bool f16, hipStream_t stream);
 
