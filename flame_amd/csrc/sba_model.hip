@@ -525,20 +525,22 @@ int weight_grad_splits(WeightGrads& g, int cus) {
 }
 
 // Time estimates in us of the projection kernels (sba_gemm.hip), fitted to sweeps of 300 .. 8192 rows, 512 .. 5632 features and k of 512
-// .. 5632 with every epilogue (270 products; the tile chosen takes 1 % more than the best on the average, 16 % at most): rounds of
-// resident workgroups, each k / 64 times `full` (a last round that fills half of the chip or less: `part`, what lies between in
-// proportion) and `round` with what the epilogue adds that nothing hides (in proportion to its fill), and `launch`.
+// .. 5632 with every epilogue and of plain products of k up to 32000 (333 products: the tile chosen takes 0.5 % more than the best on the
+// average, 15 % at most).  Tiles are dealt to the XCDs in equal parts, so the fullest one's count: whole rounds of its resident workgroups,
+// each k / 64 times `rate` of a full CU, then a last one at the rate of as many workgroups a CU as are left (one on half of the CUs or
+// less: `half` of that rate, what lies between in proportion); `round` and what the epilogue adds that nothing hides, per round
+// and in proportion to its fill; `launch`.
 // Where each is ahead (us): 256 x 256 8192 x 5632 of swiglu, k = 1024 (92, next 101); 128 x 256 8192 x 3072, k = 1024 (49; 52);
 // 128 x 128 two a CU 4096 x 1024, k = 1024 (12; 15); by halves 4096 x 1024, k = 5632 (49; 59); 64 x 64 three a CU 2048 x 2304,
 // k = 768 (13.0; 14.0), 1500 x 2816 with the swiglu gradient, k = 1024 (21; 24); by halves 1024 x 768, k = 4096 (15.8; 19.8).
 double tile_time(const Projection& p, ProjectionTile tile, int cus) {
-    struct { int rows, features, per_cu; double part, full, round, launch, add, swiglu_fwd, swiglu_bwd; } static const cost[] = {
-        {256, 256, 1, 1.07, 1.25, 3.6, 7.1, 0.0, 2.5, 0.0},     // kTile256
-        {128, 256, 1, 0.665, 0.751, 1.4, 5.8, 10.8, 1.1, 0.0},  // kTile128x256
-        {128, 128, 2, 0.608, 0.803, 3.5, 2.5, 8.3, 0.0, 10.4},  // kTile128
-        {128, 128, 1, 0.49, 0.495, 2.1, 3.2, 3.9, 0.6, 7.4},    // kTile128Halves
-        {64, 64, 3, 0.253, 0.509, 0.9, 2.6, 2.4, 0.0, 3.1},     // kTile64
-        {64, 64, 1, 0.187, 0.198, 1.3, 2.6, 0.5, 0.0, 1.5},     // kTile64Halves
+    struct { int rows, features, per_cu; double rate[3], half, round, launch, add, swiglu_fwd, swiglu_bwd; } static const cost[] = {
+        {256, 256, 1, {1.24}, 0.87, 3.8, 7.0, 0.0, 2.4, 0.0},                   // kTile256
+        {128, 256, 1, {0.786}, 0.86, 1.0, 5.8, 10.5, 1.2, 0.0},                 // kTile128x256
+        {128, 128, 2, {0.647, 0.813}, 0.95, 2.9, 2.2, 7.7, 0.3, 10.5},          // kTile128
+        {128, 128, 1, {0.542}, 0.89, 1.3, 3.5, 3.8, 0.7, 7.5},                  // kTile128Halves
+        {64, 64, 3, {0.256, 0.365, 0.551}, 0.90, 0.0, 2.7, 2.1, 0.0, 3.1},      // kTile64
+        {64, 64, 1, {0.211}, 0.88, 1.0, 2.6, 0.5, 0.0, 1.6},                    // kTile64Halves
     };
     const auto& c = cost[tile];
     const bool glu = p.epilogue == kSwigluFwd;
@@ -546,11 +548,13 @@ double tile_time(const Projection& p, ProjectionTile tile, int cus) {
     if (tile == kTile256 && p.epilogue == kAddResidual) return 1e30;       // its registers
     if (tile >= kTile64 && glu) return 1e30;
     const int64_t own = glu ? c.features / 2 : c.features, features = glu ? p.n / 2 : p.n;
-    const int64_t tiles = ((int64_t)p.m + c.rows - 1) / c.rows * ((features + own - 1) / own), slots = (int64_t)cus * c.per_cu;
+    const int64_t tiles = (((int64_t)p.m + c.rows - 1) / c.rows * ((features + own - 1) / own) + 7) / 8, wide = std::max(cus / 8, 1);
+    const int64_t rounds = tiles / (wide * c.per_cu), left = tiles % (wide * c.per_cu), deep = (left + wide - 1) / wide;
     const double round = c.round + (p.epilogue == kAddResidual ? c.add : glu ? c.swiglu_fwd : p.epilogue == kSwigluBwd ? c.swiglu_bwd : 0.0);
-    const double k64 = (p.k + 63) / 64, fill = (double)(tiles % slots) / slots;
-    const double rate = fill <= 0.5 ? c.part : c.part + (c.full - c.part) * (2 * fill - 1);
-    return tiles / slots * (c.full * k64 + round) + (fill > 0 ? rate * k64 + round * fill : 0.0) + c.launch;
+    const double k64 = (p.k + 63) / 64, fill = (double)left / wide;
+    double us = rounds * (c.rate[c.per_cu - 1] * k64 + round) + c.launch;
+    if (left) us += c.rate[deep - 1] * (deep > 1 ? 1.0 : c.half + (1.0 - c.half) * std::max(2.0 * fill - 1.0, 0.0)) * k64 + round * fill / c.per_cu;
+    return us;
 }
 
 bool projects(const Projection& p, int cus) {
