@@ -240,9 +240,10 @@ using sba_model::Projection;
 // The residual, or gate and up of the backward, can be asked for ahead (`request`, TI loads per 16 tokens, every lane's within the
 // tensor whatever the tile's edge, so that their number is known to the waits of the caller).
 template <int kEpi, int TI, int TJ> struct Results {
+    static constexpr bool kPart = kEpi == sba_model::kPartialSums;
     static constexpr bool kAdd = kEpi == sba_model::kAddResidual, kGlu = kEpi == sba_model::kSwigluFwd, kGluBwd = kEpi == sba_model::kSwigluBwd;
     static constexpr int kAhead = kAdd || kGluBwd ? TI : 0;        // loads per 16 tokens
-    static constexpr int kStores = kAdd || kGluBwd ? TI : kGlu ? TI / 4 : TI / 2;      // stores per 16 tokens (at least)
+    static constexpr int kStores = kAdd || kPart || kGluBwd ? TI : kGlu ? TI / 4 : TI / 2;      // stores per 16 tokens (at least)
     u32x4 ahead[TJ][kAhead ? kAhead : 1];
     int tok0, f0, h;               // this lane's first token; its features of block or pair 0
 
@@ -252,7 +253,7 @@ template <int kEpi, int TI, int TJ> struct Results {
         asm volatile("" : "+v"(lane));
         h = lane >> 4;
         tok0 = tw + (lane & 15);
-        f0 = nw + (kAdd ? 4 * h : (h & 1) * 16 + (h >> 1) * 8);
+        f0 = nw + (kAdd || kPart ? 4 * h : (h & 1) * 16 + (h >> 1) * 8);
     }
     __device__ inline void request(const Projection& p, int j) {
         const int64_t tok = min(tok0 + 16 * j, p.m - 1);
@@ -273,11 +274,12 @@ template <int kEpi, int TI, int TJ> struct Results {
     __device__ inline void store(const Projection& p, const f32x4 (&acc)[TI][TJ], int j) const {
         const int tok = tok0 + 16 * j, width = kGlu ? p.n / 2 : p.n;
         const int64_t row = (int64_t)tok * width;
-        if (kAdd) {
+        if (kAdd || kPart) {
+            float* const out = kPart ? p.partial + (int64_t)blockIdx.y * p.m * p.n : (float*)p.out;
 #pragma unroll
             for (int i = 0; i < TI; ++i)
                 if (tok < p.m && f0 + 16 * i < p.n)
-                    *(f32x4*)((float*)p.out + row + f0 + 16 * i) = __builtin_bit_cast(f32x4, ahead[j][i]) + acc[i][j];
+                    *(f32x4*)(out + row + f0 + 16 * i) = kPart ? acc[i][j] : __builtin_bit_cast(f32x4, ahead[j][i]) + acc[i][j];
             return;
         }
 #pragma unroll
@@ -571,18 +573,21 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
         t0 = (kBand * band + in % rows) * TM;
         n0 = (in / rows) * kOwn;
     };
-    const int nk = p.k / 64;
+    // kPartialSums: blockIdx.y's share of the stages
+    const int share = kEpi == sba_model::kPartialSums ? (p.k / 64 + p.splits - 1) / p.splits : 0, first = share * (int)blockIdx.y;
+    const int nk = share ? min(share, p.k / 64 - first) : p.k / 64;
 
     // ---- the stream of copies
     const char *xat, *wat;
+    const int64_t wstep = kRowsW ? 128 * p.ldw : (int64_t)128;
     uint32_t xoff[PX], woff[8];
     int d_local = local, d_stage = 0;
     uint32_t d_lds = lds_address(lds) + w * 1024;
     auto aim = [&](int l) {
         int t0, n0;
         tile_at(l, t0, n0);
-        xat = (const char*)p.x + 2 * (int64_t)t0 * p.ldx;
-        wat = (const char*)p.w + (kRowsW ? 2 * (int64_t)n0 : (int64_t)0);
+        xat = (const char*)p.x + 2 * (int64_t)t0 * p.ldx + 128 * (int64_t)first;
+        wat = (const char*)p.w + (kRowsW ? 2 * (int64_t)n0 + first * wstep : (int64_t)0);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int row = 8 * (w + 4 * i) + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
@@ -600,7 +605,6 @@ __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) 
             }
         }
     };
-    const int64_t wstep = kRowsW ? 128 * p.ldw : (int64_t)128;
     const uint32_t lds_end = lds_address(lds) + w * 1024 + NB * kStage;
     auto next_stage = [&]() {
         xat += 128;
@@ -762,7 +766,10 @@ int launch_large_projection(const Projection& p, hipStream_t s) {
     const int own = p.epilogue == sba_model::kSwigluFwd ? 128 : 256, features = p.epilogue == sba_model::kSwigluFwd ? p.n / 2 : p.n;
     const int tiles = ((p.m + TM - 1) / TM) * ((features + own - 1) / own), cus = sba_cu_count() & ~7;
     const dim3 grid((unsigned)(((tiles < cus ? tiles : cus) + 7) & ~7)), block(256);
-    if (p.rows_w) {
+    if (p.splits > 1) {
+        if (!p.rows_w || p.epilogue != sba_model::kStore) return -2;
+        hipLaunchKernelGGL((large_projection_kernel<TM, true, sba_model::kPartialSums>), dim3(grid.x, (unsigned)p.splits), block, 0, s, p);
+    } else if (p.rows_w) {
         if (p.epilogue == sba_model::kStore) hipLaunchKernelGGL((large_projection_kernel<TM, true, sba_model::kStore>), grid, block, 0, s, p);
         else return -2;
     } else {

@@ -78,17 +78,19 @@ int weight_grads_f16(const WeightGrads& g, int splits, hipStream_t stream);
 //   kSwigluFwd    w = gate rows | up rows: out = silu(gate) * up, 16-bit [m][n/2]; pre = y if given
 //   kSwigluBwd    y = gradient of silu(gate) * up, pre = gate | up [m][2n]: out = their gradients, 16-bit [m][2n]
 // x and w are 16-byte aligned with leading dimensions that are multiples of 8; outputs are dense.
-enum { kStore, kAddResidual, kSwigluFwd, kSwigluBwd };
+enum { kStore, kAddResidual, kSwigluFwd, kSwigluBwd, kPartialSums };      // (kPartialSums: within the kernels, fp32 [splits][m][n])
 struct Projection {
     const void* x; const void* w; int64_t ldx, ldw; int m, n, k;
     bool rows_w; int epilogue;
     const float* residual; void* pre; void* out;
+    int splits; float* partial;          // kStore, rows_w: so many workgroups share a tile's contraction (0, 1: none); [splits][m][n]
 };
 bool projects(const Projection& p, int cus);             // whether the kernels take it
 enum ProjectionTile { kTile256, kTile128x256, kTile128, kTile128Halves, kTile64, kTile64Halves };
 ProjectionTile projection_tile(const Projection& p, int cus);
 double tile_time(const Projection& p, ProjectionTile tile, int cus);    // an estimate, us; 1e30 where its kernel does not take it
-int project(const Projection& p, bool f16, int cus, hipStream_t stream);
+// how many workgroups had better share the contraction of a tile, and of which tile; 1: as projection_tile() says
+int projection_splits(const Projection& p, int cus, ProjectionTile& tile);
 int project_tile(const Projection& p, ProjectionTile tile, bool f16, hipStream_t stream);
 int project_bf16(const Projection& p, ProjectionTile tile, hipStream_t stream);
 int project_f16(const Projection& p, ProjectionTile tile, hipStream_t stream);

@@ -407,6 +407,27 @@ __global__ __launch_bounds__(kThreads) void sum_splits_kernel(const float* part,
     }
 }
 
+template <typename E>
+__global__ __launch_bounds__(kThreads) void sum_splits_to_kernel(const float* part, E* out, int64_t n8, int splits) {
+    typedef typename Vec<E>::x8 e8;
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n8; i += (int64_t)gridDim.x * kThreads) {
+        f32x4 a = *(const f32x4*)(part + i * 8), b = *(const f32x4*)(part + i * 8 + 4);
+#pragma unroll 4
+        for (int k = 1; k < splits; ++k) {
+            const float* more = part + (k * n8 + i) * 8;
+            a += *(const f32x4*)more;
+            b += *(const f32x4*)(more + 4);
+        }
+        e8 y;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            y[j] = (E)a[j];
+            y[4 + j] = (E)b[j];
+        }
+        *(e8*)(out + i * 8) = y;
+    }
+}
+
 unsigned grid_for(int64_t work_items) {
     const int64_t blocks = (work_items + kThreads - 1) / kThreads;
     return (unsigned)(blocks < 1 ? 1 : blocks > 16384 ? 16384 : blocks);
@@ -537,7 +558,7 @@ double tile_time(const Projection& p, ProjectionTile tile, int cus) {
     struct { int rows, features, per_cu; double rate[3], half, round, launch, add, swiglu_fwd, swiglu_bwd; } static const cost[] = {
         {256, 256, 1, {1.24}, 0.87, 3.8, 7.0, 0.0, 2.4, 0.0},                   // kTile256
         {128, 256, 1, {0.786}, 0.86, 1.0, 5.8, 10.5, 1.2, 0.0},                 // kTile128x256
-        {128, 128, 2, {0.647, 0.813}, 0.95, 2.9, 2.2, 7.7, 0.3, 10.5},          // kTile128
+        {128, 128, 2, {0.647, 0.85}, 0.95, 2.9, 2.2, 7.7, 0.3, 10.5},          // kTile128
         {128, 128, 1, {0.542}, 0.89, 1.3, 3.5, 3.8, 0.7, 7.5},                  // kTile128Halves
         {64, 64, 3, {0.256, 0.365, 0.551}, 0.90, 0.0, 2.7, 2.1, 0.0, 3.1},      // kTile64
         {64, 64, 1, {0.211}, 0.88, 1.0, 2.6, 0.5, 0.0, 1.6},                    // kTile64Halves
@@ -584,12 +605,38 @@ ProjectionTile projection_tile(const Projection& p, int cus) {
     return best;
 }
 
-int project(const Projection& p, bool f16, int cus, hipStream_t s) {
-    return project_tile(p, projection_tile(p, cus), f16, s);
+// Long contractions over few tiles (the input gradient of a language model's head): the large tiles' kernels with as many workgroups to a
+// tile as the CUs allow, their fp32 sums written, read and added at 5.5 TB/s.  k = 32000, one workgroup a tile against several (us): 300 x 768
+// 94, 57;  1024 x 1024 121, 76;  2048 x 1024 208, 120;  3000 x 768 244, 150;  4096 x 1024 355, 237;  8192 x 1024 436, 423;  k = 8192:
+// 2048 x 1024 52, 43;  4096 x 1024 68 either way;  k = 5632: 3000 x 768 48, 39.
+int projection_splits(const Projection& p, int cus, ProjectionTile& tile) {
+    tile = projection_tile(p, cus);
+    if (!p.rows_w || p.epilogue != kStore || p.k % 64 || p.k < 4096) return 1;
+    double best_us = tile_time(p, tile, cus);
+    int best = 1;
+    const int stages = p.k / 64;
+    for (ProjectionTile t : {kTile256, kTile128x256}) {
+        const int rows = t == kTile256 ? 256 : 128;
+        const int tiles = (int)((((int64_t)p.m + rows - 1) / rows * ((p.n + 255) / 256) + 7) / 8 * 8);
+        for (int splits = 2; splits <= 16 && tiles * splits <= cus; ++splits) {
+            const int per = (stages + splits - 1) / splits;
+            if ((stages + per - 1) / per != splits) continue;          // (the last one would have nothing)
+            const double fill = (double)tiles * splits / cus, rate = (t == kTile256 ? 1.4 : 0.786) * (0.87 + 0.13 * std::max(2.0 * fill - 1.0, 0.0));
+            const double us = (t == kTile256 ? 11.0 : 9.0) + rate * per + (8.0 * splits + 2.0) * p.m * p.n / 5.5e6;
+            if (us < 0.9 * best_us) { best_us = us / 0.9; best = splits; tile = t; }
+        }
+    }
+    return best;
 }
 
 int project_tile(const Projection& p, ProjectionTile tile, bool f16, hipStream_t s) {
-    return f16 ? project_f16(p, tile, s) : project_bf16(p, tile, s);
+    const int rc = f16 ? project_f16(p, tile, s) : project_bf16(p, tile, s);
+    if (rc || p.splits < 2) return rc;
+    const int64_t n8 = (int64_t)p.m * p.n / 8;
+    const dim3 grid(grid_for(n8)), block(kThreads);
+    if (f16) hipLaunchKernelGGL(sum_splits_to_kernel<_Float16>, grid, block, 0, s, p.partial, (_Float16*)p.out, n8, p.splits);
+    else hipLaunchKernelGGL(sum_splits_to_kernel<__bf16>, grid, block, 0, s, p.partial, (__bf16*)p.out, n8, p.splits);
+    return launched();
 }
 
 int weight_grads(const WeightGrads& g, int splits, bool f16, hipStream_t s) {

@@ -177,19 +177,34 @@ Projection projection_of(const Tensor& x, const Tensor& w, bool rows_w, int epil
 
 // y = x w^T (rows_w: x w) into `out`, with what sba_model.h's epilogues do on the way; false where the kernels do not take it
 bool try_project(const Tensor& x, const Tensor& w, bool rows_w, int epilogue, const Tensor& residual, const Tensor& pre, const Tensor& out) {
-    const Projection p = projection_of(x, w, rows_w, epilogue, residual, pre, out);
+    Projection p = projection_of(x, w, rows_w, epilogue, residual, pre, out);
     if (!projects(p, compute_units())) return false;
-    ok(sba_model::project(p, is_f16(x.scalar_type()), compute_units(), stream_of(x)));
+    ProjectionTile tile;
+    p.splits = projection_splits(p, compute_units(), tile);
+    Tensor partial;
+    if (p.splits > 1) {
+        partial = empty({p.splits, p.m, p.n}, x, at::kFloat);
+        p.partial = partial.data_ptr<float>();
+    }
+    ok(project_tile(p, tile, is_f16(x.scalar_type()), stream_of(x)));
     return true;
 }
 
 // The same with the tile of a caller's choice, where that tile's kernel takes the problem (tests of kernels that the rule picks elsewhere).
 bool project_with(int64_t tile, const Tensor& x, const Tensor& w, bool rows_w, int64_t epilogue, const std::optional<Tensor>& residual,
-                  const std::optional<Tensor>& pre, const Tensor& out) {
-    const Projection p = projection_of(x, w, rows_w, (int)epilogue, residual.value_or(Tensor()), pre.value_or(Tensor()), out);
+                  const std::optional<Tensor>& pre, const Tensor& out, int64_t splits) {
+    Projection p = projection_of(x, w, rows_w, (int)epilogue, residual.value_or(Tensor()), pre.value_or(Tensor()), out);
     TORCH_CHECK(tile >= kTile256 && tile <= kTile64Halves && p.k % 32 == 0 && p.n % 16 == 0 && p.ldx % 8 == 0 && p.ldw % 8 == 0 && p.m > 0,
                 "project_with: sizes that no tile takes");
     if (tile_time(p, (ProjectionTile)tile, compute_units()) >= 1e30) return false;
+    Tensor partial;
+    if (splits > 1) {
+        const int64_t stages = p.k / 64, per = (stages + splits - 1) / splits;
+        TORCH_CHECK(tile <= kTile128x256 && rows_w && epilogue == kStore && (splits - 1) * per < stages, "project_with: not shared out");
+        partial = empty({splits, p.m, p.n}, x, at::kFloat);
+        p.splits = (int)splits;
+        p.partial = partial.data_ptr<float>();
+    }
     ok(project_tile(p, (ProjectionTile)tile, is_f16(x.scalar_type()), stream_of(x)));
     return true;
 }
@@ -597,7 +612,8 @@ void bind_model(py::module& m) {
     m.def("next_token_loss", &next_token_loss);
     m.def("clip_and_step", &clip_and_step);
     m.def("project", &project);
-    m.def("project_with", &project_with);
+    m.def("project_with", &project_with, py::arg("tile"), py::arg("x"), py::arg("w"), py::arg("rows_w"), py::arg("epilogue"), py::arg("residual"),
+          py::arg("pre"), py::arg("out"), py::arg("splits") = 1);
     m.attr("projection_tiles") = (int)kTile64Halves + 1;
     m.def("project_add", &project_add);
     m.def("project_swiglu", [](const Tensor& x, const Tensor& w) {

@@ -117,3 +117,30 @@ def test_weight_gradients(m, n, k, dtype):
     assert got.dtype == torch.float32
     # products of 16-bit values are exact in fp32, their sums carry at most k roundings of 2^-24
     assert rel_l2(got.double(), a.double().t() @ b.double()) <= 1e-5
+
+
+# workgroups that share a tile's contraction: one token, edges of 128 and 256, shares of one stage, a last share that is shorter
+@pytest.mark.parametrize("tile", [0, 1])
+@pytest.mark.parametrize("m,n,k,splits,dtype", [
+    (1, 16, 128, 2, torch.bfloat16),
+    (257, 272, 448, 7, torch.float16),
+    (300, 528, 640, 3, torch.bfloat16),
+    (1030, 1008, 4096, 5, torch.bfloat16),
+])
+def test_shared_contractions(m, n, k, splits, dtype, tile):
+    from flame_amd import _lib
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k + 8, generator=g, device="cuda").to(dtype)[:, :k]
+    w = (torch.randn(k, n, generator=g, device="cuda") / k ** 0.5).to(dtype)
+    out = torch.full((m, n), float("nan"), device="cuda", dtype=dtype)
+    assert _lib.native().project_with(tile, x, w, True, 0, None, None, out, splits)
+    # fp32 sums: what is left is the rounding of the result, half a unit in the last place
+    assert rel_l2(out.float(), x.float() @ w.float()) <= (4e-3 if dtype == torch.bfloat16 else 6e-4)
+
+
+def test_the_input_gradient_of_a_head_is_shared_out():
+    from flame_amd import _lib
+    g = torch.Generator("cuda").manual_seed(5)
+    x = torch.randn(700, 16000, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(16000, 512, generator=g, device="cuda") / 126).bfloat16()
+    assert rel_l2(_lib.native().project(x, w, True).float(), x.float() @ w.float()) <= 4e-3
