@@ -79,8 +79,12 @@ constexpr size_t kErrorWordBytes = 256;     // tail of the bf16 matrix-core back
 // that every lane of the backward starts its chain from its own carry - and the dQ pass the two prefix tables
 // (`gtab`, `gmid`).  fp32, two in all: the forward writes `rtab`, the dQ pass `gtab`.
 int forward_tables(const SbaParams* p) { return is_16bit(p) ? 2 : 1; }
-// tables in the backward's scratch: the dQ pass's own, plus the forward's when no workspace brings them
-int scratch_tables(const SbaParams* p) { return forward_tables(p) * (p->workspace ? 1 : 2); }
+// save_for_backward = 2: the forward keeps `rtab` alone, and the dQ pass, whose chains cross a step from right to left as the forward's,
+// makes `rmid` itself
+bool one_table(const SbaParams* p) { return p->save_for_backward == 2 && is_16bit(p) && p->head_dim == 128 && use_mfma_bwd(p); }
+int kept_tables(const SbaParams* p) { return one_table(p) ? 1 : forward_tables(p); }
+// tables in the backward's scratch: the dQ pass's own, plus the forward's that no workspace brings
+int scratch_tables(const SbaParams* p) { return 2 * forward_tables(p) - (p->workspace ? kept_tables(p) : 0); }
 // the bounded waits (and with them the error word) exist in the bf16 matrix-core backward only
 bool has_error_word(const SbaParams* p) { return use_mfma_bwd(p) && is_16bit(p); }
 // bf16 at head_dim 64: the dQ pass leaves a copy of q times the logit scale (bf16, [sequence][head][token][64], dense)
@@ -159,7 +163,8 @@ KParams make_kparams(const SbaParams* p) {
     // Layout rule that the dQ kernels rely on: gmid - rtab == gtab - rmid (one table size both times), so that a
     // lane finds its prefix entry at one uniform distance from its carry entry whichever half-wave it is in.
     if (p->workspace && use_mfma(p)) {
-        if (two) { kp.rmid = (float*)p->workspace; kp.rtab = (float*)((char*)p->workspace + tb); }
+        if (one_table(p)) kp.rtab = (float*)p->workspace;
+        else if (two) { kp.rmid = (float*)p->workspace; kp.rtab = (float*)((char*)p->workspace + tb); }
         else kp.rtab = (float*)p->workspace;
     }
     char* bs = (char*)p->bwd_scratch;
@@ -170,6 +175,9 @@ KParams make_kparams(const SbaParams* p) {
         if (!p->workspace) {                       // the forward's tables, recomputed by sba_bwd
             if (two) kp.rmid = (float*)(bs + tb * slot++);
             kp.rtab = (float*)(bs + tb * slot++);
+        } else if (one_table(p)) {
+            kp.rmid = (float*)(bs + tb * slot++);
+            kp.makes_mid = 1;
         }
         char* tail = bs + tb * slot;
         if (scaled_q_bytes(p)) {
@@ -226,7 +234,7 @@ const char* sba_error_string(int code) {
 size_t sba_workspace_bytes(const SbaParams* p) {
     if (!p || p->n_heads <= 0 || p->seq_len <= 0 || p->head_dim <= 0 || p->head_dim > sba::kMaxHeadDim) return 0;
     if (p->cu_seqlens && p->table_cols <= 0) return 0;
-    return use_mfma(p) ? forward_tables(p) * table_bytes(p) : 0;
+    return use_mfma(p) ? kept_tables(p) * table_bytes(p) : 0;
 }
 
 size_t sba_bwd_scratch_bytes(const SbaParams* p) {

@@ -59,6 +59,7 @@ struct KParams {
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)
     Divisor heads, seqs;           // n_heads and n_seq, for the way from a workgroup's index to its job
     int turn;                      // jobs after which the order of a dense launch turns round (0: never), see turned()
+    int makes_mid;                 // dQ pass: rmid is not there yet (SbaParams::save_for_backward = 2)
     int cut_keys;                  // fp32 dQ pass: clear the rows of dK and dV that two workgroups will add to
     int early_end;                 // forward sweeps end once nothing is left of any of their rows' sticks
     int* gave_up;                  // backward error word (set if a kernel abandoned a bounded internal wait)

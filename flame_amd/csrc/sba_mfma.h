@@ -974,6 +974,12 @@ __device__ inline float carried_beta_g(float (&x)[32], float (&dp)[32], float F,
     gsum = c;
     return clamp01(L);
 }
+// (not to be fused with the running sum below: see there)
+__device__ inline void scale_all(float (&g)[32], float by) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int i = 0; i < 32; ++i) g[i] *= by;
+}
 // dz from beta, g and the prefix G entering the lane's keys
 // (The running sum must stay a plain add: fused with the product that made g - which the compiler does across
 // function boundaries when allowed to - it would need the two factors of every g alive instead of g itself,

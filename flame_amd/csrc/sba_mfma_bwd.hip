@@ -47,8 +47,11 @@ __device__ inline void store_scaled_q(const KParams& p, const Job& job, int head
 // kLean (head_dim 64): the register-lean arrangement of the step that head_dim 128 always uses, held to three waves
 // per SIMD.  Ahead on large launches, whose SIMDs it fills better (the packed benchmark's dQ -5.6 %, short documents
 // -6 %); on launches that last as long as their longest sweep the plain arrangement's shorter step is ahead.
-template <int D, bool kLean = false>
+// kMid: the forward kept `rtab` alone (KParams::makes_mid).  The left half-wave starts its chain from 1, the right half-wave's product
+// completes it, and is the entry of `rmid`: 32 multiplications a step.
+template <int D, bool kLean = false, bool kMid = false>
 __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 1)) void mfma_bwd_dq_kernel(KParams p) {
+    static_assert(!kMid || kWide<D>, "the arrangement that takes the carry into g alone");
     constexpr int kTile = 64 * kPitch<D> * 2;
     __shared__ __attribute__((aligned(16))) char lds[4 * kTile];   // K0 V0 K1 V1
 
@@ -109,10 +112,16 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     // both half-waves (gmid - rtab == gtab - rmid: the library lays the tables out that way).
     constexpr int64_t tstride = kRowBlock;
     const float* rcur = (h ? p.rtab : p.rmid) + tab_index(p, head, job, job.rb, first) + 32 * wave + n;
-    const int64_t g_from_r = (const char*)p.gtab - (const char*)p.rmid;
-    float Rnext = (row_ok && n_steps > 0) ? *rcur : 1.0f;
-    float Gstore = 0.f;
+    // (kMid: rtab is the caller's, so that the distances differ)
+    const int64_t g_from_r = kMid && h ? (const char*)p.gmid - (const char*)p.rtab : (const char*)p.gtab - (const char*)p.rmid;
+    float Rnext = (row_ok && n_steps > 0 && (!kMid || h)) ? *rcur : 1.0f;
+    float Gstore = 0.f, Mstore = 0.f;
     bool g_pending = false;
+    auto store_prefixes = [&]() __attribute__((always_inline)) {
+        if (!g_pending || !row_ok) return;
+        *(float*)((char*)(rcur - tstride) + g_from_r) = Gstore;
+        if (kMid && !h) *const_cast<float*>(rcur - tstride) = Mstore;
+    };
     // (last of the prologue's loads: its conversion waits for it, and with it for everything requested before)
     float dr = 0.f;
     if (row_ok && p.d_rem.ptr)
@@ -132,11 +141,11 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
         const bool skip = key0 + strict > q0w + 31 || q0w >= job.len;     // nothing visible, or no query of this wave inside the sequence
         // the prefixes that entered the previous step (the first block's are only known once that
         // block's weights are: they start at d_rem * rem, see below)
-        if (g_pending && row_ok) *(float*)((char*)(rcur - tstride) + g_from_r) = Gstore;
+        store_prefixes();
         g_pending = false;
         const float F = Rnext;
         if (more) {
-            if (row_ok) Rnext = rcur[tstride];
+            if (row_ok && (!kMid || h)) Rnext = rcur[tstride];
             // next tiles, straight into the other buffer (free since the last barrier)
             kc.issue((step + 1) * kKeyBlock, job.len, lds + (buf ^ 1) * 2 * kTile);
             vc.issue((step + 1) * kKeyBlock, job.len, lds + (buf ^ 1) * 2 * kTile + kTile);
@@ -151,7 +160,19 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
                 dp_tiles_o<D>(dp, vtile, lo, dof);
                 if (key0 + 63 + strict > q0w) mask_step(x, key0 + 32 * h, qi, strict);
                 float gsum;
-                const float Lend = carried_beta_g(x, dp, F, gsum);
+                float Lend = carried_beta_g(x, dp, F, gsum);
+                if constexpr (kMid) {
+                    float Llo, Lup;
+                    half_values(Lend, Llo, Lup);
+                    float carry = h ? 1.0f : Lup;
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm("" : "+v"(carry));
+                    scale_all(dp, carry);
+                    __builtin_amdgcn_sched_barrier(0);
+                    gsum *= carry;
+                    Lend *= carry;
+                    Mstore = Lup;
+                }
                 if (step == 0) {                         // the gradient of rem rides in the prefix, see below (further right: no remainder)
                     float Llo, Lup;
                     half_values(Lend, Llo, Lup);
@@ -210,7 +231,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
         do_step(step, std::integral_constant<int, 0>{});
         if (step + 1 < n_steps) do_step(step + 1, std::integral_constant<int, 1>{});
     }
-    if (g_pending && row_ok) *(float*)((char*)(rcur - tstride) + g_from_r) = Gstore;
+    store_prefixes();
 
     store_query_rows<D>(lds + wave * kRowStage<D>, dqacc, p.scale, p.dq,                 // (the tiles are free)
                         slice_offset(p.dq, job.seq, head, job.tok0), q0w, job.len, lane, p.cols);
@@ -1907,8 +1928,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     dim3 grid((unsigned)kp.n_jobs * kp.n_heads);
     const bool p1 = phases != 2, p2 = phases != 1;
     // the dQ kernels reach a lane's prefix entry from its carry entry by one uniform distance (see there)
-    if (!kp.rtab || !kp.rmid || !kp.gtab || !kp.gmid ||
-        (const char*)kp.gmid - (const char*)kp.rtab != (const char*)kp.gtab - (const char*)kp.rmid) return SBA_ERR_WORKSPACE;
+    if (!kp.rtab || !kp.rmid || !kp.gtab || !kp.gmid) return SBA_ERR_WORKSPACE;
+    if (!kp.makes_mid && (const char*)kp.gmid - (const char*)kp.rtab != (const char*)kp.gtab - (const char*)kp.rmid) return SBA_ERR_WORKSPACE;
     // Key-owner pass.  head_dim 64: the kernel whose waves own their keys outright, one sweep per workgroup, unless the launch hangs
     // on its longest sweeps; then the resident producer/consumer stream, which splits the work into twice as many items and deals
     // them out itself.  Own-keys time over the stream's by tail ratio r, both passes, dense and packed alike:  longest sequence up
@@ -1973,7 +1994,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
             else hipLaunchKernelGGL((mfma_bwd_dkv_stream_kernel<64, 4>), dim3(n_wg), dim3(8 * 64), 0, s, kp);
         }
     } else if (kp.head_dim == 96) {
-        if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<96>), grid, dim3(kThreads), 0, s, kp);
+        if (p1 && kp.makes_mid) hipLaunchKernelGGL((mfma_bwd_dq_kernel<96, false, true>), grid, dim3(kThreads), 0, s, kp);
+        else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<96>), grid, dim3(kThreads), 0, s, kp);
         if (p2) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<96>), grid, dim3(2 * kThreads), 0, s, kp);
     } else if (kp.head_dim == 256) {
         // one wave per SIMD in both passes; every wave of the key-owner pass on its own 32 keys, two workgroups per
@@ -1984,7 +2006,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
             hipLaunchKernelGGL((mfma_bwd_dkv_own_kernel<256, 2>), dim3(grid.x, 2), dim3(kThreads), 0, s, kp);
         }
     } else {
-        if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<128>), grid, dim3(kThreads), 0, s, kp);
+        if (p1 && kp.makes_mid) hipLaunchKernelGGL((mfma_bwd_dq_kernel<128, false, true>), grid, dim3(kThreads), 0, s, kp);
+        else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<128>), grid, dim3(kThreads), 0, s, kp);
         // key owners at head_dim 128: two waves per 32 keys (6-9 % faster than one wave per 32 keys,
         // which SBA_DKV_KERNEL=own still selects)
         const bool pair = !(which && !strcmp(which, "own"));

@@ -118,12 +118,13 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     // operations retire in order, so the wait for those loads at the end of that step also covers the store,
     // long after it has completed, and no wait ever falls on a fresh store.
     float* const my_tab = h ? p.rtab : p.rmid;
+    const bool both_tables = !kWide<D> || p.rmid;          // (without rmid the backward makes it)
     float carry_out = 1.0f;
     int carry_step = -1;                       // wave-uniform: the step whose carries wait to be stored
     auto store_carries = [&]() {
         if (carry_step >= 0 && p.save) {
-            if (rows_full) my_tab[tabq + carry_step * kRowBlock] = carry_out;      // no lane mask
-            else if (qi < job.len) my_tab[tabq + carry_step * kRowBlock] = carry_out;
+            if (rows_full && both_tables) my_tab[tabq + carry_step * kRowBlock] = carry_out;      // no lane mask
+            else if (qi < job.len && (both_tables || h)) my_tab[tabq + carry_step * kRowBlock] = carry_out;
         }
         carry_step = -1;
     };
@@ -279,12 +280,13 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     // carry tables as in mfma_fwd_kernel (right half-wave -> rtab, left -> rmid, stored a step late), here
     // relative to the segment's right edge
     float* const my_tab = h ? p.rtab : p.rmid;
+    const bool both_tables = !kWide<D> || p.rmid;          // (without rmid the backward makes it)
     float carry_out = 1.0f;
     int carry_step = -1;
     auto store_carries = [&]() {
         if (carry_step >= 0 && p.save) {
-            if (rows_full) my_tab[tabq + carry_step * kRowBlock] = carry_out;
-            else if (qi < job.len) my_tab[tabq + carry_step * kRowBlock] = carry_out;
+            if (rows_full && both_tables) my_tab[tabq + carry_step * kRowBlock] = carry_out;
+            else if (qi < job.len && (both_tables || h)) my_tab[tabq + carry_step * kRowBlock] = carry_out;
         }
         carry_step = -1;
     };
@@ -364,7 +366,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     // carry-table entries of this group, written relative to its own right edge: times F.  Every lane
     // rescales the entries it wrote (the half-waves have a table each); the loads go out in batches so that
     // their latencies overlap.  Its stores have completed (wait above).
-    if (p.save && grp > 0 && qi < job.len) {
+    if (p.save && grp > 0 && qi < job.len && (both_tables || h)) {
         for (int s0 = reached; s0 < hi; s0 += 8) {
             float v[8];
 #pragma unroll

@@ -87,7 +87,9 @@ typedef struct SbaParams {
     int32_t  head_dim;         /* D <= 256 */
     int32_t  attend_current;   /* 0: keys j < i;  1: keys j <= i */
     float    scale;            /* logit scale ("inv_temp") in natural-log units */
-    int32_t  save_for_backward;/* forward only: also fill the carry table in workspace */
+    int32_t  save_for_backward;/* 1 (forward): also fill the carry tables in workspace.  2 (forward and backward, 16-bit dtypes at
+                                  head_dim 128, 1 elsewhere): only the first of the two, half the bytes between the calls; the
+                                  backward makes the second on its way, into one table more of its scratch */
     int32_t  bwd_phases;       /* backward only: 0 = whole backward; 1 = first kernel only (dq and the
                                   prefix table), 2 = second kernel only (dk, dv; needs phase 1 done on
                                   the same workspace).  Lets a profiler time the kernels one by one */
@@ -133,7 +135,7 @@ const char* sba_error_string(int code);
  * entering the right and the left half of every 64-key block; fp32: one) and the backward
  * reads them back, so the SAME buffer, untouched in between, must be given to both calls
  * (the Python layer keeps it in the autograd context the way the reference keeps
- * neg_log_acc, sb_attn/__init__.py:30).  Only the size fields of `p` are read.
+ * neg_log_acc, sb_attn/__init__.py:30).  Only the size fields of `p` and save_for_backward are read.
  */
 size_t sba_workspace_bytes(const SbaParams* p);
 
