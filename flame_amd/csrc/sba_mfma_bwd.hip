@@ -51,7 +51,7 @@ __device__ inline void store_scaled_q(const KParams& p, const Job& job, int head
 // completes it, and is the entry of `rmid`: 32 multiplications a step.
 template <int D, bool kLean = false, bool kMid = false>
 __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 1)) void mfma_bwd_dq_kernel(KParams p) {
-    static_assert(!kMid || kWide<D>, "the arrangement that takes the carry into g alone");
+    static_assert(!kMid || kWide<D> || kLean, "the arrangement that takes the carry into g alone");
     constexpr int kTile = 64 * kPitch<D> * 2;
     __shared__ __attribute__((aligned(16))) char lds[4 * kTile];   // K0 V0 K1 V1
 
@@ -1971,7 +1971,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         // 23.8 us with one step per iteration against 27.4, B=4, T=1024 36.0 against 37.7).
         const bool two_steps = sba_two_step_env() >= 0 ? grid.x <= (unsigned)sba_two_step_env()
                                                        : grid.x <= kTwoStepDqMaxGrid && sba_tail_ratio(kp, grid.x) >= 3.7;
-        if (p1 && two_steps) hipLaunchKernelGGL((mfma_bwd_dq2_kernel<64>), grid, dim3(2 * kThreads), 0, s, kp);
+        if (p1 && kp.makes_mid) hipLaunchKernelGGL((mfma_bwd_dq_kernel<64, true, true>), grid, dim3(kThreads), 0, s, sba_turning(kp, 3));
+        else if (p1 && two_steps) hipLaunchKernelGGL((mfma_bwd_dq2_kernel<64>), grid, dim3(2 * kThreads), 0, s, kp);
         // The register-lean arrangement (three waves per SIMD) from five workgroups per CU on, unless the launch hangs on
         // one long sweep (tail ratio above 2.5: there the plain arrangement's shorter step is ahead, e.g. 111 against 118 us
         // on an 8192-token pack with a 4096-token document); from eight workgroups per CU on always.  On 1280-3232

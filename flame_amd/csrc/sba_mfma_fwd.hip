@@ -118,7 +118,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     // operations retire in order, so the wait for those loads at the end of that step also covers the store,
     // long after it has completed, and no wait ever falls on a fresh store.
     float* const my_tab = h ? p.rtab : p.rmid;
-    const bool both_tables = !kWide<D> || p.rmid;          // (without rmid the backward makes it)
+    const bool both_tables = D == 256 || p.rmid;          // (without rmid the backward makes it)
     float carry_out = 1.0f;
     int carry_step = -1;                       // wave-uniform: the step whose carries wait to be stored
     auto store_carries = [&]() {
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     // carry tables as in mfma_fwd_kernel (right half-wave -> rtab, left -> rmid, stored a step late), here
     // relative to the segment's right edge
     float* const my_tab = h ? p.rtab : p.rmid;
-    const bool both_tables = !kWide<D> || p.rmid;          // (without rmid the backward makes it)
+    const bool both_tables = D == 256 || p.rmid;          // (without rmid the backward makes it)
     float carry_out = 1.0f;
     int carry_step = -1;
     auto store_carries = [&]() {

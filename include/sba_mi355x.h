@@ -88,8 +88,9 @@ typedef struct SbaParams {
     int32_t  attend_current;   /* 0: keys j < i;  1: keys j <= i */
     float    scale;            /* logit scale ("inv_temp") in natural-log units */
     int32_t  save_for_backward;/* 1 (forward): also fill the carry tables in workspace.  2 (forward and backward, 16-bit dtypes at
-                                  head_dim 128, 1 elsewhere): only the first of the two, half the bytes between the calls; the
-                                  backward makes the second on its way, into one table more of its scratch */
+                                  head_dim 64 and 128 with sequences of more than 128 tokens, 1 elsewhere): only the first of the
+                                  two, half the bytes between the calls; the backward makes the second on its way, into one table
+                                  more of its scratch */
     int32_t  bwd_phases;       /* backward only: 0 = whole backward; 1 = first kernel only (dq and the
                                   prefix table), 2 = second kernel only (dk, dv; needs phase 1 done on
                                   the same workspace).  Lets a profiler time the kernels one by one */

@@ -1,5 +1,5 @@
 """A budget that holds one of the forward's two carry tables: the forward keeps that one and the dQ pass makes the other
-(16-bit types at head dims 72 to 128)."""
+(16-bit types at head dims up to 128, sequences of more than 128 tokens; shorter ones repeat the forward's sweep)."""
 import pytest
 import torch
 
@@ -29,13 +29,17 @@ def _table_bytes(lens, H):
     ([193], 2, 96, torch.float16, True),
     ([1000], 4, 128, torch.bfloat16, False),
     ([1000], 4, 80, torch.bfloat16, False),
+    ([100, 128, 3], 2, 128, torch.bfloat16, False),
+    ([1000], 4, 64, torch.bfloat16, True),
+    ([500] * 16, 16, 64, torch.float16, False),
+    ([130, 1, 64, 700, 257], 3, 40, torch.bfloat16, False),
     ([500] * 16, 16, 128, torch.bfloat16, False),
     ([500] * 16, 16, 72, torch.float16, True),
     ([130, 1, 64, 700, 257], 3, 128, torch.float16, False),
     ([130, 1, 64, 700, 257], 3, 88, torch.bfloat16, True)])
 def test_one_kept_table_against_the_oracle_and_both(lens, H, D, dtype, current, budget):
     N, dense = sum(lens), len(set(lens)) == 1
-    scale = 1.0 if D == 128 else 0.5                             # (sweeps that end, and that do not)
+    scale = 1.0 if D in (64, 128) else 0.5                             # (sweeps that end, and that do not)
     q, k, v, do = (randn((H, N, D), 740 + i, scale if i < 3 else 1.0, dtype) for i in range(4))
     dr = randn((H, N), 745, 1.0, dtype)
     cu = cu_from_lengths(lens)
