@@ -155,6 +155,9 @@ KParams make_kparams(const SbaParams* p) {
     } else {
         kp.n_jobs = p->n_seq * ((p->seq_len + sba::kRowBlock - 1) / sba::kRowBlock);
     }
+    kp.n_cus = sba_cu_count();
+    kp.cus = sba::divisor(kp.n_cus);
+    kp.spread = p->cu_seqlens ? (int64_t)kp.n_jobs * kp.n_heads >= (int64_t)8 * kp.n_cus : p->seq_len > 24 * sba::kRowBlock;
     kp.q = cvt(p->q); kp.k = cvt(p->k); kp.v = cvt(p->v); kp.o = cvt(p->o);
     kp.d_o = cvt(p->d_o); kp.dq = cvt(p->dq); kp.dk = cvt(p->dk); kp.dv = cvt(p->dv);
     kp.rem = cvt(p->rem); kp.d_rem = cvt(p->d_rem);

@@ -57,7 +57,9 @@ struct KParams {
                                    //   the key-owner stream kernel (ptr NULL: not wanted)
     float* dkv32;                  // generic path: fp32 dk|dv accumulators
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)
-    Divisor heads, seqs;           // n_heads and n_seq, for the way from a workgroup's index to its job
+    Divisor heads, seqs, cus;      // n_heads, n_seq and n_cus, for the way from a workgroup's index to its job
+    int n_cus;
+    int spread;                    // heads change their place from round to round of the CUs, see head_of_block()
     int turn;                      // jobs after which the order of a dense launch turns round (0: never), see turned()
     int makes_mid;                 // dQ pass: rmid is not there yet (SbaParams::save_for_backward = 2)
     int cut_keys;                  // fp32 dQ pass: clear the rows of dK and dV that two workgroups will add to
@@ -86,9 +88,23 @@ struct Job { int tok0, len, rb, seq, tab0; };
 // a slot already, turn rarely.  Jobs are sorted by decreasing sweep
 // length (longest first); `longest_last` walks the list from its other end (the key-owner
 // pass, whose work grows as the row-block index falls).
+//
+// kShared: kernels of which a CU holds several workgroups.  The CU that gets a round's i-th workgroup gets the next round's i-th, too, so
+// by the turn above a head's longest sweeps meet on the same CUs where a round is a multiple of the heads' cycle (2 ... 16 heads on 256
+// CUs).  With KParams::spread the heads of round r start the binary fractions' bit-reversed r-th on instead (0, 1/2, 1/4, 3/4, ... of
+// them).  Forward + backward against the plain turn, mean logits 0 .. -6 over the heads: B=2 H=4 T=16384 d=64 0.73, d=128 0.86; B=4 H=4 T=8192
+// 0.77, 0.87; B=1 H=8 T=16384 0.90, 0.95; B=1 H=16 T=8192 0.92, 0.95; B=8 H=4 T=4096 0.88, 0.92; B=1 H=32 T=4096 0.92, 0.98; packs of 30000 and
+// 65536 tokens 0.97 ... 0.99.  Up to 3000 tokens, whose sweeps end near their starts in no head, and on packs of fewer rounds 0.98 ... 1.02:
+// not there.  Kernels with one workgroup a CU lose by it (key owners at d=128 223 -> 237 us, 566 -> 617).
+template <bool kShared = false>
 __device__ inline int head_of_block(const KParams& p, int block) {
     const int slot = divided(block, p.heads);
-    const int i = block - slot * p.n_heads + (p.cu_seqlens ? slot >> 3 : slot);
+    int turn = p.cu_seqlens ? slot >> 3 : slot;
+    if (kShared && p.spread) {
+        const int round = divided(slot * p.n_heads, p.cus), of_round = slot - divided(round * p.n_cus + p.n_heads - 1, p.heads);
+        turn = (p.cu_seqlens ? of_round >> 3 : of_round) + (int)__umulhi(__builtin_bitreverse32((uint32_t)round), (uint32_t)p.n_heads);
+    }
+    const int i = block - slot * p.n_heads + turn;
     return i - divided(i, p.heads) * p.n_heads;
 }
 __device__ inline int slot_of_block(const KParams& p, int block) { return divided(block, p.heads); }
