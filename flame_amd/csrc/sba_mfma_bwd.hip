@@ -1934,14 +1934,16 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     // on its longest sweeps; then the resident producer/consumer stream, which splits the work into twice as many items and deals
     // them out itself.  Own-keys time over the stream's by tail ratio r, both passes, dense and packed alike:  longest sequence up
     // to 4096 tokens  r 2.5 0.94, 2.7 0.90, 2.9 0.92-0.97, 3.1 0.92, 3.2 0.90-0.95, 3.4 0.99-1.02, 3.6 1.04, 3.9 1.13;  longer ones
-    // r 2.0 0.91, 2.2 0.93, 2.6 0.985, 2.7-2.8 1.00, 3.05 1.02, 3.2 1.05.
+    // r 2.0 0.87, 2.2 0.93, 2.6 0.985, 2.7-2.8 1.00, 3.05 1.02, 3.2 1.04-1.06; with fewer heads, of which one that looks far is a larger
+    // part, B=2 H=4 T=16384 (2.0) 1.02, H=4 T=34000 (1.9) 1.03, T=26000 (2.5) 1.09, H=6 T=20000 (2.2) 1.01, H=2 T=50000 (2.6) 0.96.
     // Batches of short sequences (sweeps of at most 16 steps) also take the own-keys kernel at any size: on 512 workgroups B=8,
     // T=512 takes 27.3 us against the stream's 33.0, B=4, T=1024 44.0 against 45.3.
     // head_dim 128: the paired kernel at every size (on 64 ... 256 workgroups of B=1, H=16 it takes 27 / 44 / 62 / 81 us where the
     // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103); SBA_DKV_KERNEL=other still selects that one.
     const unsigned cus = (unsigned)sba_cu_count();
     const bool short_sweeps = kp.seq_len <= 8 * kRowBlock && grid.x >= 2u * cus;
-    const bool own = own_keys_kernel(kp.head_dim == 64 ? short_sweeps || sba_tail_ratio(kp, grid.x) <= (kp.seq_len <= 32 * kRowBlock ? 3.35 : 2.75) : true);
+    const double own_up_to = kp.seq_len <= 32 * kRowBlock ? 3.35 : kp.n_heads < 8 ? 1.9 : 2.75;
+    const bool own = own_keys_kernel(kp.head_dim == 64 ? short_sweeps || sba_tail_ratio(kp, grid.x) <= own_up_to : true);
     const char* which = getenv("SBA_DKV_KERNEL");
     const bool plain = which && !strcmp(which, "plain");
     // the stream with eight half-block producers (12 waves): behind the one with four full-block producers

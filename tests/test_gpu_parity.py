@@ -713,3 +713,22 @@ def test_launches_whose_order_turns_round_by_round(B, H, T, D, dtype, grads):
 def test_key_owner_kernel_of_long_and_short_tails(B, H, T):
     # tail ratios 2.67, 2.91 (own-keys kernel), 3.37 and 7.5 (stream)
     _check_dense(B, H, T, 64, torch.bfloat16, seed=B + H + T)
+
+
+@pytest.mark.parametrize("B,H,T,D", [(1, 8, 3200, 64), (1, 12, 3300, 64), (1, 5, 3080, 128)])
+def test_heads_spread_over_the_rounds(B, H, T, D):
+    # heads whose cycle divides a round of the CUs and heads whose does not, a single round; keys without queries' help: forward and
+    # gradients against those of one head alone, which has other neighbours
+    sb_attn, _ = _ops()
+    q, k, v, do = (randn((B, H, T, D), 90 + i, 0.5 if i < 3 else 1.0, torch.bfloat16).cuda() for i in range(4))
+
+    def run(h):
+        x = [t[:, h].contiguous().requires_grad_() for t in (q, k, v)]
+        o, rem = sb_attn(*x)
+        return (o, rem, *torch.autograd.grad(o, x, do[:, h].contiguous()))
+
+    whole = run(slice(None))
+    for h in (0, H // 2, H - 1):
+        for x, y in zip(whole, run(slice(h, h + 1))):
+            # (the kernels of a small launch sum the segments of a sweep in another order: single roundings to bf16)
+            assert rel_l2(x[:, h:h + 1].float(), y.float()) <= 1e-2
