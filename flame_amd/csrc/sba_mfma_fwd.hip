@@ -440,8 +440,13 @@ static int forward_segments(const sba::KParams& kp, unsigned grid) {
         // LDS) one; it pays while the grid is at most two rounds of those and the longest sweep dominates.  B=1,
         // H=16, one sweep / two segments in us: T=1024 29.8 / 26.2, T=2048 50.4 / 41.6, T=3072 77.2 / 60.0, T=4096
         // 105.5 / 91.8, T=5120 131.1 / 138.7, T=8192 276.2 / 291.7; B=2 T=2048 60.0 / 57.0; H=8 T=4096 89.7 / 70.8.
+        // Long dense sequences, whose heads differ in how far they look, somewhat beyond (mean logits 0 .. -6 over the heads): T=4400
+        // (r 3.6) 99 / 87, T=5000 (3.1) 119 / 105, H=12 T=6500 (3.3) 148 / 121, H=8 T=10000 (3.2) 206 / 179, but H=16 T=6000 (2.7) 148 / 141 and
+        // at head_dim 80 112 / 119, H=4 T=20000 (3.2) 397 / 388 and 335 / 348, H=32 T=2500 (3.1) 66 / 72.
         if (sba_two_step_env() >= 0) return grid <= (unsigned)sba_two_step_env() ? 2 : 0;
-        return grid <= 2u * (unsigned)sba_cu_count() && sba_tail_ratio(kp, grid) >= 3.7 ? 2 : 0;
+        const double r = sba_tail_ratio(kp, grid);
+        if (!kp.cu_seqlens && kp.n_heads >= 8 && kp.seq_len > 32 * sba::kRowBlock && r >= 3.1) return 2;
+        return grid <= 2u * (unsigned)sba_cu_count() && r >= 3.7 ? 2 : 0;
     }
     const char* e = getenv("SBA_FWD_GROUPS");
     const int forced = e ? atoi(e) : 0;
