@@ -546,8 +546,8 @@ __global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Project
 // 1.42 with 256 rows, every CU busy).  The copies run through the list of (tile, stage) pairs without a break, so a tile's results
 // are stored while the next tile's first stages arrive.  TM = 256 has two buffers of 64 KB, TM = 128, whose stages pass in half the
 // time, three of 48 KB; the fetch addresses move from buffer to buffer, one add per address and stage.
-// 8192 tokens, k = 1024, TM = 256: 5632 features in 79 us (1.2 PFLOP/s; the library's kernel 96), with swiglu in 108 (its pass of its
-// own would read and write 230 MB more); TM = 128: 1024 features in 18 us (library: 21), with the residual for k = 2816 46 us (40 + 15).
+// 8192 tokens, k = 1024: 5632 features with swiglu in 83 us with TM = 256 (1.14 PFLOP/s; 89 with 128, 92 in 128 x 128 tiles), 3072 features in
+// 46 with TM = 128 (50; 49); k = 5632, W's rows: 1024 features in 77 with TM = 128 (104; 80).
 template <int TM, bool kRowsW, int kEpi>
 __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) {
     constexpr int NB = TM == 256 ? 2 : 3;

@@ -2,7 +2,7 @@
 // as the bf16 kernels, with every product on v_mfma_f32_32x32x2_f32.  The reference runs fp32
 // inputs through its one tiled kernel as well (stickbreaking_attention/utils.py:8 ALLOW_TF32,
 // sb_attn/sb_fwd.py:139-253); here fp32 stays fp32 end to end (the 1e-4 tolerance class), the
-// backward has no atomics and is bit-reproducible.
+// backward is bit-reproducible (its only atomics add two numbers to a zero).
 //
 // What bounds them is the matrix pipe, which runs fp32 at 1/16 of its bf16 rate: a 32 x 64 tile of scores and its product
 // with V keep one SIMD busy for 8192 cycles.  So fp32 runs, which are small, need their work spread over all SIMDs, and
