@@ -79,10 +79,10 @@ constexpr size_t kErrorWordBytes = 256;     // tail of the bf16 matrix-core back
 // that every lane of the backward starts its chain from its own carry - and the dQ pass the two prefix tables
 // (`gtab`, `gmid`).  fp32, two in all: the forward writes `rtab`, the dQ pass `gtab`.
 int forward_tables(const SbaParams* p) { return is_16bit(p) ? 2 : 1; }
-// save_for_backward = 2: the forward keeps `rtab` alone, and the dQ pass, whose chains cross a step from right to left as the forward's,
+// SBA_SAVE_ONE_TABLE: the forward keeps `rtab` alone, and the dQ pass, whose chains cross a step from right to left as the forward's,
 // makes `rmid` itself.  (Sequences of one row block have a kernel that reads both.)
 bool one_table(const SbaParams* p) {
-    return p->save_for_backward == 2 && is_16bit(p) && (p->head_dim == 64 || p->head_dim == 128) && p->seq_len > sba::kRowBlock && use_mfma_bwd(p);
+    return p->save_for_backward == SBA_SAVE_ONE_TABLE && is_16bit(p) && (p->head_dim == 64 || p->head_dim == 128) && p->seq_len > sba::kRowBlock && use_mfma_bwd(p);
 }
 int kept_tables(const SbaParams* p) { return one_table(p) ? 1 : forward_tables(p); }
 // tables in the backward's scratch: the dQ pass's own, plus the forward's that no workspace brings

@@ -61,7 +61,7 @@ struct KParams {
     int n_cus;
     int spread;                    // heads change their place from round to round of the CUs, see head_of_block()
     int turn;                      // jobs after which the order of a dense launch turns round (0: never), see turned()
-    int makes_mid;                 // dQ pass: rmid is not there yet (SbaParams::save_for_backward = 2)
+    int makes_mid;                 // dQ pass: rmid is not there yet (SBA_SAVE_ONE_TABLE)
     int cut_keys;                  // fp32 dQ pass: clear the rows of dK and dV that two workgroups will add to
     int early_end;                 // forward sweeps end once nothing is left of any of their rows' sticks
     int* gave_up;                  // backward error word (set if a kernel abandoned a bounded internal wait)

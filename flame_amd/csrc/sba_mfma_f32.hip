@@ -588,7 +588,9 @@ void launch_f32_bwd(const KParams& kp, int phases, hipStream_t s) {
     // passes and the forward, with against without, by that measure: 8.0 0.90, 6.1-7.1 0.69-0.77, 3.2-3.6 0.70-0.78, 2.3 0.85-0.88,
     // 1.8-1.9 0.74-0.92 (H=16, T=1024: 168 -> 155 us, D=128 304 -> 267), 1.7 0.85-0.92;  1.6 0.90 (a pack) ... 1.09 (B=4, T=512, whose
     // sweeps have two steps), 1.4 1.01-1.05, 1.2 1.00-1.04, 0.9 1.05-1.10: the second workgroup's prologue and the additions in memory.
-    const bool cut = !one_block && sba_tail_ratio(kp, jobs) >= 13.0;
+    // (Not where dK or dV takes the place of an input, which the clearing would wipe out.)
+    const auto input = [&](const char* out) { return out == kp.q.ptr || out == kp.k.ptr || out == kp.v.ptr || out == kp.d_o.ptr; };
+    const bool cut = !one_block && sba_tail_ratio(kp, jobs) >= 13.0 && !input(kp.dk.ptr) && !input(kp.dv.ptr);
     KParams dq = sba_turning(kp, D == 64 ? 2 : 1, 4);
     dq.cut_keys = cut && phases == 0;
     if (phases != 2 && one_block) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 1>), dim3(jobs), dim3(kThreads), 0, s, kp);

@@ -235,7 +235,7 @@ Tensor attention_forward(const Problem& pr, const Tensor& o, const Tensor& rem, 
         if (recompute_carries(n)) {
             // half of it, where the backward makes the other half (its dQ pass takes 5 % longer; a sweep for the carries alone would
             // take half of a forward)
-            p.save_for_backward = 2;
+            p.save_for_backward = SBA_SAVE_ONE_TABLE;
             const size_t half = std::max<size_t>(sba_workspace_bytes(&p), 16);
             if (half >= n || recompute_carries(half)) p.save_for_backward = 0;
             n = half;
@@ -259,7 +259,7 @@ void attention_backward(const Problem& pr, const Tensor& tables, const Tensor& d
     p.dk = describe(dk);
     p.dv = describe(dv);
     if (tables.defined() && tables.numel() > 16) {
-        if ((size_t)tables.numel() < sba_workspace_bytes(&p)) p.save_for_backward = 2;
+        if ((size_t)tables.numel() < sba_workspace_bytes(&p)) p.save_for_backward = SBA_SAVE_ONE_TABLE;
         p.workspace = tables.data_ptr();
         p.workspace_bytes = tables.numel();
     }

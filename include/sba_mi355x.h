@@ -45,6 +45,7 @@ extern "C" {
 
 #define SBA_ABI_VERSION 6
 #define SBA_SCHEDULE_INTS 8   /* int32 per scheduled job, see sba_build_schedule() */
+#define SBA_SAVE_ONE_TABLE 0x4f4e4531 /* a value of SbaParams::save_for_backward, see there */
 #define SBA_DOC_MAJOR_GRID 8192 /* workgroups from which the schedule is document-major */
 
 enum { SBA_DTYPE_F32 = 0, SBA_DTYPE_BF16 = 1, SBA_DTYPE_F16 = 2 };   /* (the reference's kernels take whatever dtype the tensors have, sb_attn/sb_fwd.py:144-146) */
@@ -87,10 +88,10 @@ typedef struct SbaParams {
     int32_t  head_dim;         /* D <= 256 */
     int32_t  attend_current;   /* 0: keys j < i;  1: keys j <= i */
     float    scale;            /* logit scale ("inv_temp") in natural-log units */
-    int32_t  save_for_backward;/* 1 (forward): also fill the carry tables in workspace.  2 (forward and backward, 16-bit dtypes at
-                                  head_dim 64 and 128 with sequences of more than 128 tokens, 1 elsewhere): only the first of the
-                                  two, half the bytes between the calls; the backward makes the second on its way, into one table
-                                  more of its scratch */
+    int32_t  save_for_backward;/* forward only: also fill the carry tables in workspace.  SBA_SAVE_ONE_TABLE, to be given to the
+                                  backward too: only the first of the two of 16-bit dtypes (at head_dim 64 and 128 with sequences
+                                  of more than 128 tokens, the same as 1 elsewhere), half the bytes between the calls; the backward
+                                  makes the second on its way, into one table more of its scratch */
     int32_t  bwd_phases;       /* backward only: 0 = whole backward; 1 = first kernel only (dq and the
                                   prefix table), 2 = second kernel only (dk, dv; needs phase 1 done on
                                   the same workspace).  Lets a profiler time the kernels one by one */
