@@ -59,6 +59,7 @@ struct KParams {
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)
     Divisor heads, seqs, cus;      // n_heads, n_seq and n_cus, for the way from a workgroup's index to its job
     int n_cus;
+    int stride;                    // heads that the dense layout's turn moves on by from slot to slot, coprime with n_heads
     int spread;                    // heads change their place from round to round of the CUs, see head_of_block()
     int turn;                      // jobs after which the order of a dense launch turns round (0: never), see turned()
     int makes_mid;                 // dQ pass: rmid is not there yet (SBA_SAVE_ONE_TABLE)
@@ -96,11 +97,21 @@ struct Job { int tok0, len, rb, seq, tab0; };
 // 0.77, 0.87; B=1 H=8 T=16384 0.90, 0.95; B=1 H=16 T=8192 0.92, 0.95; B=8 H=4 T=4096 0.88, 0.92; B=1 H=32 T=4096 0.92, 0.98; packs of 30000 and
 // 65536 tokens 0.97 ... 0.99.  Up to 3000 tokens, whose sweeps end near their starts in no head, and on packs of fewer rounds 0.98 ... 1.02:
 // not there.  Kernels with one workgroup a CU lose by it (key owners at d=128 223 -> 237 us, 566 -> 617).
-template <bool kShared = false>
+//
+// Those turn by KParams::stride heads a slot in the dense layout, 5 where the heads are no multiple of it, so that the heads that follow
+// each other on an XCD are no neighbours either: forward + backward B=2 H=8 T=16384 d=128 0.96, B=1 H=32 T=4096 0.95, H=16 T=8192 0.986,
+// B=2 H=16 T=3000 0.986, H=16 T=4096 d=64 0.986, 0.99 ... 1.003 at 20 other shapes.  The stream's items, two slots to a job and dealt
+// out beforehand, turn by one head in 16 slots: H=16 T=5000 0.96, H=8 T=7000 0.98, H=32 T=1800 0.98, 0.99 ... 1.00 elsewhere; with fewer than
+// eight heads every slot (H=4 T=12000 would be 1.04).
+enum Sharing { kOnePerCu, kSharedCu, kStreamItems };
+template <Sharing kSharing = kOnePerCu>
 __device__ inline int head_of_block(const KParams& p, int block) {
     const int slot = divided(block, p.heads);
-    int turn = p.cu_seqlens ? slot >> 3 : slot;
-    if (kShared && p.spread) {
+    int turn = slot;
+    if (p.cu_seqlens) turn = slot >> 3;
+    else if (kSharing == kOnePerCu) turn = p.stride * slot;
+    else if (kSharing == kStreamItems && p.n_heads >= 8) turn = slot >> 4;
+    if (kSharing == kSharedCu && p.spread) {
         const int round = divided(slot * p.n_heads, p.cus), of_round = slot - divided(round * p.n_cus + p.n_heads - 1, p.heads);
         turn = (p.cu_seqlens ? of_round >> 3 : of_round) + (int)__umulhi(__builtin_bitreverse32((uint32_t)round), (uint32_t)p.n_heads);
     }

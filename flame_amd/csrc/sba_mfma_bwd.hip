@@ -61,7 +61,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     LaneOffsets<D> lo;
     lo.init(lane);
     lo.rebase(lds);                        // absolute addresses: the loop below runs in one copy per tile buffer
-    const int head = head_of_block<D <= 128>(p, blockIdx.x);
+    const int head = head_of_block<D <= 128 ? kSharedCu : kOnePerCu>(p, blockIdx.x);
     const Job job = decode_job<D == 64>(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
@@ -650,7 +650,7 @@ __device__ inline KeyItem decode_item(const KParams& p, int idx) {
     KeyItem r;
     r.valid = idx >= 0;
     if (idx < 0) idx = 0;
-    r.head = head_of_block(p, idx);
+    r.head = head_of_block<kStreamItems>(p, idx);
     const int slot = slot_of_block(p, idx);          // two 64-key blocks per scheduled 128-row job
     r.job = decode_key_job(p, slot >> 1);
     r.kb = 2 * r.job.rb + (slot & 1);
@@ -1194,7 +1194,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
     lo.init(lane);
     LaneOffsets<64> lz;
     lz.init(lane);
-    const int head = head_of_block<D == 64>(p, blockIdx.x);
+    const int head = head_of_block<D == 64 ? kSharedCu : kOnePerCu>(p, blockIdx.x);
     const Job job = decode_key_job<D == 64>(p, slot_of_block(p, blockIdx.x));
     const int strict = p.attend_current ? 0 : 1;
     const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it

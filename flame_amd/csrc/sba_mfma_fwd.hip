@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
-    const int head = head_of_block<true>(p, blockIdx.x);
+    const int head = head_of_block<kSharedCu>(p, blockIdx.x);
     const Job job = decode_job<D == 64>(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(G * kThreads) void mfma_fwd_seg_kernel(KParams p) {
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
-    const int head = head_of_block<G == 2 && D == 64>(p, blockIdx.x);
+    const int head = head_of_block<G == 2 && D == 64 ? kSharedCu : kOnePerCu>(p, blockIdx.x);
     const Job job = decode_job<D == 64 && G == 2>(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;

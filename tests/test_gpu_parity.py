@@ -715,7 +715,7 @@ def test_key_owner_kernel_of_long_and_short_tails(B, H, T):
     _check_dense(B, H, T, 64, torch.bfloat16, seed=B + H + T)
 
 
-@pytest.mark.parametrize("B,H,T,D", [(1, 8, 3200, 64), (1, 12, 3300, 64), (1, 5, 3080, 128), (1, 12, 6300, 128)])
+@pytest.mark.parametrize("B,H,T,D", [(1, 8, 3200, 64), (1, 12, 3300, 64), (1, 5, 3080, 128), (1, 12, 6300, 128), (1, 10, 1200, 128), (2, 35, 300, 96), (1, 9, 2500, 64)])
 def test_heads_spread_over_the_rounds(B, H, T, D):
     # heads whose cycle divides a round of the CUs and heads whose does not, a single round; keys without queries' help: forward and
     # gradients against those of one head alone, which has other neighbours
