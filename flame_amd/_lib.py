@@ -335,9 +335,11 @@ def workspace_upper_bound(n_heads: int, columns: int) -> int:
     return 2 * table_bytes(n_heads, columns)
 
 
-def bwd_scratch_upper_bound(n_heads: int, columns: int, tab_tokens: int, head_dim: int) -> int:
+def bwd_scratch_upper_bound(n_heads: int, columns: int, tab_tokens: int, head_dim: int, fp32: bool = False) -> int:
     """Four tables (the recompute mode's count) or the generic path's fp32 dk|dv accumulators."""
     dp = 32 if head_dim <= 32 else (64 if head_dim <= 64 else (128 if head_dim <= 128 else 256))
     acc = (2 * tab_tokens * n_heads * dp * 4 + 255) & ~255
     scaled_q = (tab_tokens * n_heads * 64 * 2 + 255) & ~255      # bf16 at head_dim 64: the dQ pass's scaled copy of q
-    return max(4 * table_bytes(n_heads, columns) + scaled_q + 256, acc)      # + the backward's error word
+    # fp32: the sums of two workgroups that share a key block, which only launches of few workgroups do (less room is no error)
+    halves = min(4 * tab_tokens * n_heads * dp * 4, 64 << 20) if fp32 else 0
+    return max(4 * table_bytes(n_heads, columns) + scaled_q + 256 + halves, acc)      # + the backward's error word

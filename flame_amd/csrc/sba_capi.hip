@@ -97,6 +97,15 @@ size_t scaled_q_bytes(const SbaParams* p) {
     return (b + 255) & ~(size_t)255;
 }
 
+// fp32: sums of the two workgroups that share a key block's steps, [workgroup][dV, dK][head][token][column].  They are not
+// needed: without room for them every key block has one workgroup.  (The limit: packs of one long document among very many short ones.)
+constexpr size_t kMaxHalfSumsBytes = 256u << 20;
+size_t half_sums_bytes(const SbaParams* p) {
+    if (!use_mfma_bwd(p) || p->dtype != SBA_DTYPE_F32 || !sba_f32_halves_keys(p->seq_len, table_columns(p), p->n_heads)) return 0;
+    const size_t b = (size_t)4 * tab_tokens(p) * p->n_heads * p->head_dim * sizeof(float);
+    return b <= kMaxHalfSumsBytes ? (b + 255) & ~(size_t)255 : 0;
+}
+
 sba::TensorArg cvt(const SbaTensor& t) { return sba::TensorArg{(char*)t.ptr, t.stride_b, t.stride_h, t.stride_t}; }
 sba::VectorArg cvt(const SbaVector& t) { return sba::VectorArg{(char*)t.ptr, t.stride_b, t.stride_h}; }
 
@@ -194,6 +203,7 @@ KParams make_kparams(const SbaParams* p) {
             tail += scaled_q_bytes(p);
         }
         if (has_error_word(p)) kp.gave_up = (int*)tail;
+        if (half_sums_bytes(p) && p->bwd_scratch_bytes >= sba_bwd_scratch_bytes(p) && ((uintptr_t)tail & 15) == 0) kp.halves = (float*)tail;
     } else if (bs) {
         kp.dkv32 = (float*)bs;
     }
@@ -250,7 +260,7 @@ size_t sba_bwd_scratch_bytes(const SbaParams* p) {
     if (p->cu_seqlens && p->table_cols <= 0 && use_mfma_bwd(p)) return 0;
     // without a workspace the backward recomputes the forward's tables first, into slots of its own
     if (!use_mfma_bwd(p)) return generic_acc_bytes(p);
-    return scratch_tables(p) * table_bytes(p) + scaled_q_bytes(p) + (has_error_word(p) ? kErrorWordBytes : 0);
+    return scratch_tables(p) * table_bytes(p) + scaled_q_bytes(p) + (has_error_word(p) ? kErrorWordBytes : 0) + half_sums_bytes(p);
 }
 
 int sba_row_block(void) { return sba::kRowBlock; }
@@ -338,7 +348,7 @@ int sba_bwd(const SbaParams* p) {
     if (!p->d_o.ptr || !p->dq.ptr || !p->dk.ptr || !p->dv.ptr) return SBA_ERR_NULL;
     if (p->bwd_phases < 0 || p->bwd_phases > 2) return SBA_ERR_SHAPE;
     if (use_mfma_bwd(p) && p->workspace && p->workspace_bytes < sba_workspace_bytes(p)) return SBA_ERR_WORKSPACE;
-    if (!p->bwd_scratch || p->bwd_scratch_bytes < sba_bwd_scratch_bytes(p)) return SBA_ERR_WORKSPACE;
+    if (!p->bwd_scratch || p->bwd_scratch_bytes < sba_bwd_scratch_bytes(p) - half_sums_bytes(p)) return SBA_ERR_WORKSPACE;
     KParams kp = make_kparams(p);
     hipStream_t s = (hipStream_t)p->stream;
     if (use_mfma_bwd(p) && !p->workspace && p->bwd_phases != 2) {
@@ -381,7 +391,7 @@ int sba_bwd_gave_up(const SbaParams* p, int static_scratch_used, int* gave_up) {
 int sba_bwd_static(const SbaParams* p) {
     int rc = check_common(p);
     if (rc) return rc;
-    if (sba_bwd_scratch_bytes(p) > (size_t)SBA_STATIC_SCRATCH_BYTES) return SBA_ERR_STATIC_LIMIT;
+    if (sba_bwd_scratch_bytes(p) - half_sums_bytes(p) > (size_t)SBA_STATIC_SCRATCH_BYTES) return SBA_ERR_STATIC_LIMIT;
     void* ptr = nullptr;
     rc = static_scratch(&ptr);
     if (rc) return rc;

@@ -56,6 +56,7 @@ struct KParams {
     TensorArg q_scaled;            // bf16 head_dim 64 backward: q times scale2, rounded to bf16, written by the dQ pass for
                                    //   the key-owner stream kernel (ptr NULL: not wanted)
     float* dkv32;                  // generic path: fp32 dk|dv accumulators
+    float* halves;                 // fp32 key-owner pass: sums of two workgroups that share a key block (null: none does)
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)
     Divisor heads, seqs, cus;      // n_heads, n_seq and n_cus, for the way from a workgroup's index to its job
     int n_cus;
@@ -63,11 +64,10 @@ struct KParams {
     int spread;                    // heads change their place from round to round of the CUs, see head_of_block()
     int turn;                      // jobs after which the order of a dense launch turns round (0: never), see turned()
     int makes_mid;                 // dQ pass: rmid is not there yet (SBA_SAVE_ONE_TABLE)
-    int cut_keys;                  // fp32 dQ pass: clear the rows of dK and dV that two workgroups will add to
     int early_end;                 // forward sweeps end once nothing is left of any of their rows' sticks
     int* gave_up;                  // backward error word (set if a kernel abandoned a bounded internal wait)
     int64_t tab_head_stride;       // floats per head in each carry table
-    int64_t tab_tokens;            // generic path: tokens per head in the fp32 accumulators (n_seq*T dense, sumT packed)
+    int64_t tab_tokens;            // tokens per head in dkv32 and halves (n_seq*T dense, sumT packed)
 };
 
 // tab0: first carry-table column of the job's sequence
@@ -186,7 +186,7 @@ __device__ inline Job decode_key_job(const KParams& p, int i) {
     return j;
 }
 
-// Token index inside the generic path's fp32 accumulators.
+// Token index inside dkv32 and halves.
 __device__ inline int64_t tab_token(const KParams& p, const Job& j, int local) {
     return (p.cu_seqlens == nullptr) ? (int64_t)j.seq * p.seq_len + local : (int64_t)j.tok0 + local;
 }
@@ -301,12 +301,16 @@ inline int sba_cu_count() {
 // one sweep and a CU holds four of them:  r = longest sweep x (4 x CUs) / all sweep steps of the launch  (steps of
 // 64 keys; a sequence of n row blocks has n (n + 1) of them per head, which is also its number of carry-table
 // columns).  A launch cannot end before its longest sweep has; for r well above 1 most of the chip idles behind
-// it, and the kernels that cut a sweep into pieces pay.  seq_len is the longest sequence of the launch.
-inline double sba_tail_ratio(const sba::KParams& kp, unsigned grid) {
-    const double longest = 2.0 * ((kp.seq_len + sba::kRowBlock - 1) / sba::kRowBlock);
-    double steps = (double)(kp.tab_head_stride / sba::kRowBlock) * kp.n_heads;
+// it, and the kernels that cut a sweep into pieces pay.  seq_len is the longest sequence of the launch, columns its carry-table
+// columns per head.
+inline double sba_tail_ratio(int seq_len, int64_t columns, int n_heads, unsigned grid) {
+    const double longest = 2.0 * ((seq_len + sba::kRowBlock - 1) / sba::kRowBlock);
+    double steps = (double)columns * n_heads;
     if (steps <= 0) steps = (double)grid * (longest / 2 + 1);          // (no table size given: every sweep half the longest)
     return longest * 4.0 * sba_cu_count() / steps;
+}
+inline double sba_tail_ratio(const sba::KParams& kp, unsigned grid) {
+    return sba_tail_ratio(kp.seq_len, kp.tab_head_stride / sba::kRowBlock, kp.n_heads, grid);
 }
 
 // The same launch with KParams::turn set, for a kernel of which a CU holds `resident` workgroups and that takes `per_job` of them for
@@ -333,4 +337,5 @@ int sba_launch_mfma_f16_fwd(const sba::KParams& kp, hipStream_t s);       // the
 int sba_launch_mfma_f16_bwd(const sba::KParams& kp, int phases, hipStream_t s);
 int sba_launch_mfma_f32_fwd(const sba::KParams& kp, hipStream_t s);
 int sba_launch_mfma_f32_bwd(const sba::KParams& kp, int phases, hipStream_t s);
+bool sba_f32_halves_keys(int seq_len, int64_t columns, int n_heads);        // whether the fp32 key-owner pass cuts sweeps in two
 bool sba_mfma_bwd_available();

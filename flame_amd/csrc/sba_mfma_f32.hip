@@ -2,7 +2,7 @@
 // as the bf16 kernels, with every product on v_mfma_f32_32x32x2_f32.  The reference runs fp32
 // inputs through its one tiled kernel as well (stickbreaking_attention/utils.py:8 ALLOW_TF32,
 // sb_attn/sb_fwd.py:139-253); here fp32 stays fp32 end to end (the 1e-4 tolerance class), the
-// backward is bit-reproducible (its only atomics add two numbers to a zero).
+// backward is bit-reproducible.
 //
 // What bounds them is the matrix pipe, which runs fp32 at 1/16 of its bf16 rate: a 32 x 64 tile of scores and its product
 // with V keep one SIMD busy for 8192 cycles.  So fp32 runs, which are small, need their work spread over all SIMDs, and
@@ -314,22 +314,14 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void fwd_kernel(KParams 
 __device__ inline int first_half(const Job& job) {
     return ((job.len - job.rb * kRowBlock + 511) >> 9) << 8;
 }
-// zeros in rows row0 .. row0 + kRows - 1 of dK and dV where two workgroups add to them
-template <int D, int kRows>
-__device__ inline void clear_cut_rows(const KParams& p, const Job& job, int head, int row0) {
-    if (job.len <= job.rb * kRowBlock + first_half(job)) return;
-    const Slice dk(p.dk, job, head), dv(p.dv, job, head);
-    for (int c = threadIdx.x; c < kRows * D / 4; c += kThreads) {
-        const int row = row0 + c / (D / 4), at = 16 * (c % (D / 4));
-        if (row >= job.len) return;
-        *(f32x4*)(const_cast<char*>(dk.row(row)) + at) = f32x4{0};
-        *(f32x4*)(const_cast<char*>(dv.row(row)) + at) = f32x4{0};
-    }
+// end of the queries that the job's keys have weights in
+__device__ inline int live_end(const KParams& p, int head, const Job& job) {
+    return min(job.len, (last_live_row_block(p, head, job) + 1) * kRowBlock);
 }
+// a key's row of the sums that workgroup `part` of two leaves of dK or dV
 template <int D>
-__global__ __launch_bounds__(kThreads) void clear_cut_kernel(KParams p) {
-    const Job job = decode_job(p, slot_of_block(p, blockIdx.x));
-    clear_cut_rows<D, kRowBlock>(p, job, head_of_block(p, blockIdx.x), job.rb * kRowBlock);
+__device__ inline float* half_row(const KParams& p, int part, bool is_dk, const Job& job, int head, int key) {
+    return p.halves + (((2 * part + is_dk) * (int64_t)p.n_heads + head) * p.tab_tokens + tab_token(p, job, key)) * D;
 }
 
 // ---------------------------------------------------------------- backward pass 1: dQ + prefix table
@@ -343,7 +335,6 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void bwd_dq_kernel(KPara
     const RowGroup<S> grp(p, wave);
     const Job& job = grp.job;
     if (grp.q0 >= job.len) return;                         // (S = 4: the whole workgroup)
-    if (S == 4 && p.cut_keys) clear_cut_rows<D, 32>(p, job, grp.head, grp.q0);
     const int strict = p.attend_current ? 0 : 1;
     const int qi = grp.q0 + n;
     const bool row_ok = qi < job.len;
@@ -420,8 +411,11 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void bwd_dq_kernel(KPara
 // weights and logit gradients (carries from the two tables) and leaves them in LDS as [query][key] rows; after a barrier
 // it reduces [32 keys x 32 d] tiles of dV (W = 8: waves 0-3) and dK (waves 4-7) over all queries of the step: key half
 // w & 1, column blocks (w >> 1 & 1) + 2*j.
-// kCut: two workgroups per (64-key block, head), one for each half of its steps, that add their sums to zeroed dK and dV.  Of two
-// addends the order makes no difference; the cut lies at a step that the sequence's length alone decides.
+// kCut: two workgroups per (64-key block, head), one for each half of its steps, which leave their sums in KParams::halves for
+// add_halves_kernel (where the second half has steps at all; otherwise the first stores the rows).  The cut lies at a step that the
+// sequence's length alone decides.  B=2, H=8, T=1024, d=64, both passes and the forward: 168 us with one workgroup a key block, 159 so; 164
+// if the second workgroup to finish adds the sums itself (their round trips through memory), 246 with fences around that, which empty
+// the L2; 155 with float atomics on cleared rows of dK and dV, which are not defined on every memory that a gradient may lie in.
 template <int D, int W, bool kCut = false>
 __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
     constexpr int kMine = D / 64;              // output tiles per wave and tensor
@@ -448,7 +442,7 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
     for (int t = 0; t < kBoth; ++t)
 #pragma unroll
         for (int j = 0; j < kMine; ++j) acc[t][j] = f32x16{0};
-    const int q_live = min(job.len, (last_live_row_block(p, head, job) + 1) * kRowBlock);
+    const int q_live = live_end(p, head, job);
     const int cut = kCut ? first_half(job) : 0;
     const int q_start = job.rb * kRowBlock + part * cut, q_end = kCut && part == 0 ? min(q_live, q_start + cut) : q_live;
     if (kCut && part == 1 && q_start >= q_end) return;         // uniform over the workgroup
@@ -542,24 +536,41 @@ __global__ __launch_bounds__(W * 64, 2) void bwd_dkv_kernel(KParams p) {
         }
         __syncthreads();                       // the weight tiles are free
     }
-    const bool adds = kCut && job.len > job.rb * kRowBlock + cut;
     // accumulator rows are keys 32*kh + 8*(r/4) + 4*h + r%4, columns d = 32*(dbw + 2j) + n: dk = scale * dZ^T Q
 #pragma unroll
     for (int t = 0; t < kBoth; ++t) {
         const bool is_dk = kBoth == 2 ? t == 1 : wave >= 4;
         const Slice out(is_dk ? p.dk : p.dv, job, head);
-        const float s = is_dk ? p.scale : 1.0f;
+        const bool halved = kCut && q_live > job.rb * kRowBlock + cut;
+        const float s = is_dk && !halved ? p.scale : 1.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int key = key0 + 32 * kh + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (key < job.len)
+            if (key >= job.len) continue;
+            float* const row = halved ? half_row<D>(p, part, is_dk, job, head, key) : (float*)const_cast<char*>(out.row(key));
 #pragma unroll
-                for (int j = 0; j < kMine; ++j) {
-                    float* at = (float*)(const_cast<char*>(out.row(key)) + 4 * (32 * (dbw + 2 * j) + n));
-                    if (adds) unsafeAtomicAdd(at, acc[t][j][r] * s);
-                    else *at = acc[t][j][r] * s;
-                }
+            for (int j = 0; j < kMine; ++j) row[32 * (dbw + 2 * j) + n] = acc[t][j][r] * s;
         }
+    }
+}
+
+// dK and dV of the key blocks that two workgroups shared, 32 rows a workgroup: what bounds it is its launch (4 us in all at
+// B=2, H=8, T=1024, d=64, of 159).
+template <int D>
+__global__ __launch_bounds__(kThreads) void add_halves_kernel(KParams p) {
+    const int slot = slot_of_block(p, blockIdx.x), head = head_of_block(p, blockIdx.x);
+    const Job job = decode_key_job(p, slot >> 2);
+    if (live_end(p, head, job) <= job.rb * kRowBlock + first_half(job)) return;
+    const int row0 = job.rb * kRowBlock + 32 * (slot & 3);
+    constexpr int kChunks = 32 * D / 4;                    // of 16 bytes, per tensor
+#pragma unroll
+    for (int c = threadIdx.x; c < 2 * kChunks; c += kThreads) {
+        const bool is_dk = c >= kChunks;
+        const int key = row0 + c % kChunks / (D / 4), at = 4 * (c % (D / 4));
+        if (key >= job.len) continue;
+        const f32x4 a = *(const f32x4*)(half_row<D>(p, 0, is_dk, job, head, key) + at), b = *(const f32x4*)(half_row<D>(p, 1, is_dk, job, head, key) + at);
+        const Slice out(is_dk ? p.dk : p.dv, job, head);
+        *(f32x4*)(const_cast<char*>(out.row(key)) + 4 * at) = (a + b) * (is_dk ? p.scale : 1.0f);
     }
 }
 
@@ -583,25 +594,25 @@ void launch_f32_bwd(const KParams& kp, int phases, hipStream_t s) {
     // 16 .. 128 take 193 us forward + backward this way, 276 with S = 4 and W = 8.  Longer ones are 4-15 % ahead with eight
     // waves per workgroup in the key-owner pass.
     const bool one_block = kp.seq_len <= kRowBlock;
-    // A key-owner workgroup has its CU to itself, so a launch of few lasts as long as the one with the most steps.  Where that is more
-    // than 1.6 times the average share of a CU (an eighth of the tail ratio), two workgroups take half of the steps each.  Both
-    // passes and the forward, with against without, by that measure: 8.0 0.90, 6.1-7.1 0.69-0.77, 3.2-3.6 0.70-0.78, 2.3 0.85-0.88,
-    // 1.8-1.9 0.74-0.92 (H=16, T=1024: 168 -> 155 us, D=128 304 -> 267), 1.7 0.85-0.92;  1.6 0.90 (a pack) ... 1.09 (B=4, T=512, whose
-    // sweeps have two steps), 1.4 1.01-1.05, 1.2 1.00-1.04, 0.9 1.05-1.10: the second workgroup's prologue and the additions in memory.
-    // (Not where dK or dV takes the place of an input, which the clearing would wipe out.)
-    const auto input = [&](const char* out) { return out == kp.q.ptr || out == kp.k.ptr || out == kp.v.ptr || out == kp.d_o.ptr; };
-    const bool cut = !one_block && sba_tail_ratio(kp, jobs) >= 13.0 && !input(kp.dk.ptr) && !input(kp.dv.ptr);
-    KParams dq = sba_turning(kp, D == 64 ? 2 : 1, 4);
-    dq.cut_keys = cut && phases == 0;
     if (phases != 2 && one_block) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 1>), dim3(jobs), dim3(kThreads), 0, s, kp);
-    else if (phases != 2) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 4>), dim3(4 * jobs), dim3(kThreads), 0, s, dq);
+    else if (phases != 2) hipLaunchKernelGGL((f32::bwd_dq_kernel<D, 4>), dim3(4 * jobs), dim3(kThreads), 0, s, sba_turning(kp, D == 64 ? 2 : 1, 4));
     if (phases != 1 && one_block) hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 4>), dim3(2 * jobs), dim3(4 * 64), 0, s, kp);
-    else if (phases != 1 && cut) {
-        if (phases == 2) hipLaunchKernelGGL((f32::clear_cut_kernel<D>), dim3(jobs), dim3(kThreads), 0, s, kp);
+    else if (phases != 1 && kp.halves) {
         hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 8, true>), dim3(4 * jobs), dim3(8 * 64), 0, s, kp);
+        hipLaunchKernelGGL((f32::add_halves_kernel<D>), dim3(4 * jobs), dim3(kThreads), 0, s, kp);
     } else if (phases != 1) hipLaunchKernelGGL((f32::bwd_dkv_kernel<D, 8>), dim3(2 * jobs), dim3(8 * 64), 0, s, kp);
 }
 }  // namespace
+
+// A key-owner workgroup has its CU to itself, so a launch of few lasts as long as the one with the most steps.  Where that is more
+// than 1.6 times the average share of a CU (an eighth of the tail ratio), two workgroups take half of the steps each (sequences of at most 256 tokens
+// have a single step).  Both passes and the forward, with against without, by that measure: 7.1-7.8 0.71-0.78 (1.05-1.07 where hardly
+// a sweep reaches its second half: one head of logits near 0, 72 us), 3.8 0.71-0.74, 3.2 0.78-0.84, 4.0 at T=300 0.93-0.97, 1.9 0.80-0.84, 1.8
+// 0.90-0.95 (H=16, T=1024: 168 -> 159 us, D=128 305 -> 273);  1.6 1.05-1.10, 1.3 1.10-1.13, 1.2 0.95-1.08, 0.9-1.0 1.08-1.27: the second
+// workgroup's prologue and the sums' way through memory.
+bool sba_f32_halves_keys(int seq_len, int64_t columns, int n_heads) {
+    return seq_len > 256 && columns > 0 && sba_tail_ratio(seq_len, columns, n_heads, 0) >= 13.0;
+}
 
 int sba_launch_mfma_f32_fwd(const sba::KParams& kp, hipStream_t s) {
     const bool one_block = kp.seq_len <= kRowBlock;

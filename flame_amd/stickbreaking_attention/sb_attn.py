@@ -58,7 +58,7 @@ def bwd_scratch_bytes(q, have_workspace=True) -> int:
     kept none)."""
     if torch.compiler.is_compiling():
         B, H, T, D = q.shape
-        return _lib.bwd_scratch_upper_bound(H, _lib.dense_columns(B, T), B * T, D)
+        return _lib.bwd_scratch_upper_bound(H, _lib.dense_columns(B, T), B * T, D, q.dtype == torch.float32)
     key = _size_key(q, 1 if have_workspace else 2)
     n = _SIZES.get(key)
     if n is None:

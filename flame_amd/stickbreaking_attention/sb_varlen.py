@@ -105,7 +105,7 @@ def bwd_scratch_bytes(q, cu_seqlens, max_seqlens: int, have_workspace=True) -> i
     cols = _columns(q, cu_seqlens, max_seqlens)
     if torch.compiler.is_compiling():
         H, N, D = q.shape
-        return _lib.bwd_scratch_upper_bound(H, cols, N, D)
+        return _lib.bwd_scratch_upper_bound(H, cols, N, D, q.dtype == torch.float32)
     p = _params(q, q, q, 1, max_seqlens, 1.0, False)
     p.cu_seqlens, p.table_cols = 1, cols
     p.workspace = 1 if have_workspace else None       # only NULL or not is looked at
