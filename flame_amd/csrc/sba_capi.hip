@@ -166,9 +166,6 @@ KParams make_kparams(const SbaParams* p) {
     }
     kp.n_cus = sba_cu_count();
     kp.cus = sba::divisor(kp.n_cus);
-    kp.stride = 1;
-    if (p->n_heads >= 8)                       // (stride * slot stays below 2^31 with the workgroups' index)
-        for (int s : {5, 7}) if (kp.stride == 1 && p->n_heads % s) kp.stride = s;
     kp.spread = p->cu_seqlens ? (int64_t)kp.n_jobs * kp.n_heads >= (int64_t)8 * kp.n_cus : p->seq_len > 24 * sba::kRowBlock;
     kp.q = cvt(p->q); kp.k = cvt(p->k); kp.v = cvt(p->v); kp.o = cvt(p->o);
     kp.d_o = cvt(p->d_o); kp.dq = cvt(p->dq); kp.dk = cvt(p->dk); kp.dv = cvt(p->dv);

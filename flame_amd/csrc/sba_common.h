@@ -60,7 +60,6 @@ struct KParams {
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)
     Divisor heads, seqs, cus;      // n_heads, n_seq and n_cus, for the way from a workgroup's index to its job
     int n_cus;
-    int stride;                    // heads that the dense layout's turn moves on by from slot to slot, coprime with n_heads
     int spread;                    // heads change their place from round to round of the CUs, see head_of_block()
     int turn;                      // jobs after which the order of a dense launch turns round (0: never), see turned()
     int makes_mid;                 // dQ pass: rmid is not there yet (SBA_SAVE_ONE_TABLE)
@@ -90,26 +89,29 @@ struct Job { int tok0, len, rb, seq, tab0; };
 // length (longest first); `longest_last` walks the list from its other end (the key-owner
 // pass, whose work grows as the row-block index falls).
 //
-// kShared: kernels of which a CU holds several workgroups.  The CU that gets a round's i-th workgroup gets the next round's i-th, too, so
+// kSharedCu: kernels of which a CU holds several workgroups.  The CU that gets a round's i-th workgroup gets the next round's i-th, too, so
 // by the turn above a head's longest sweeps meet on the same CUs where a round is a multiple of the heads' cycle (2 ... 16 heads on 256
 // CUs).  With KParams::spread the heads of round r start the binary fractions' bit-reversed r-th on instead (0, 1/2, 1/4, 3/4, ... of
-// them).  Forward + backward against the plain turn, mean logits 0 .. -6 over the heads: B=2 H=4 T=16384 d=64 0.73, d=128 0.86; B=4 H=4 T=8192
-// 0.77, 0.87; B=1 H=8 T=16384 0.90, 0.95; B=1 H=16 T=8192 0.92, 0.95; B=8 H=4 T=4096 0.88, 0.92; B=1 H=32 T=4096 0.92, 0.98; packs of 30000 and
-// 65536 tokens 0.97 ... 0.99.  Up to 3000 tokens, whose sweeps end near their starts in no head, and on packs of fewer rounds 0.98 ... 1.02:
-// not there.  Kernels with one workgroup a CU lose by it (key owners at d=128 223 -> 237 us, 566 -> 617).
+// them).  Forward + backward against the plain turn, mean logits 0 .. -6 over the heads, in this order / two random ones / all at -6:
+//     B=2 H=4 T=16384 d=64 0.87 / 0.88 0.87 / 1.01, d=128 0.88 / 0.88 0.87 / 1.01     B=4 H=4 T=8192 d=64 0.90 / 0.91 0.90 / 1.00
+//     B=1 H=8 T=16384 d=128 0.96 / 0.96 0.98 / 1.00     B=1 H=16 T=8192 d=64 0.91 / 0.99 0.99 / 1.00, d=128 0.94 / 1.00 1.01 / 1.01
+//     B=1 H=32 T=4096 d=64 0.89 / 0.99 1.00 / 0.99     B=1 H=16 T=16384 d=128 1.00 / 1.01 1.00 / 1.00
+// so it pays in any order of up to eight heads, where few heads make a cycle, and costs at most 1 % with more of them in no order; packs
+// of 30000 and 65536 tokens 0.97 ... 0.99.  Up to 3000 tokens, whose sweeps end near their starts in no head, and on packs of fewer rounds
+// 0.98 ... 1.02: not there.  Kernels with one workgroup a CU lose by it (key owners at d=128 223 -> 237 us, 566 -> 617).
+// (A turn of several heads a slot, so that those that follow each other on an XCD are no neighbours: ahead where the neighbours reach
+// equally far - over ten shapes 0.99 of the time in the order above, 1.004 in random ones.  Heads have no such order in general.)
 //
-// Those turn by KParams::stride heads a slot in the dense layout, 5 where the heads are no multiple of it, so that the heads that follow
-// each other on an XCD are no neighbours either: forward + backward B=2 H=8 T=16384 d=128 0.96, B=1 H=32 T=4096 0.95, H=16 T=8192 0.986,
-// B=2 H=16 T=3000 0.986, H=16 T=4096 d=64 0.986, 0.99 ... 1.003 at 20 other shapes.  The stream's items, two slots to a job and dealt
-// out beforehand, turn by one head in 16 slots: H=16 T=5000 0.96, H=8 T=7000 0.98, H=32 T=1800 0.98, 0.99 ... 1.00 elsewhere; with fewer than
-// eight heads every slot (H=4 T=12000 would be 1.04).
+// The stream's items, two slots to a job and dealt out beforehand, turn by one head in 16 slots, for the sake of the XCD's L2, against one
+// a slot in the same orders:  H=16 T=4096 0.99 / 0.98 0.99 / 0.97     H=16 T=5000 0.98 / 0.97 1.00 / 0.99     H=8 T=7000 0.98 / 1.01 1.00 / 0.97
+//     H=32 T=1800 1.00 / 1.00 0.99 / 0.97     H=12 T=3000, H=16 T=3500 1.00 / 1.00 / 1.00, 0.99
+// With fewer than eight heads they turn every slot (H=4 T=12000 would be 1.04).
 enum Sharing { kOnePerCu, kSharedCu, kStreamItems };
 template <Sharing kSharing = kOnePerCu>
 __device__ inline int head_of_block(const KParams& p, int block) {
     const int slot = divided(block, p.heads);
     int turn = slot;
     if (p.cu_seqlens) turn = slot >> 3;
-    else if (kSharing == kOnePerCu) turn = p.stride * slot;
     else if (kSharing == kStreamItems && p.n_heads >= 8) turn = slot >> 4;
     if (kSharing == kSharedCu && p.spread) {
         const int round = divided(slot * p.n_heads, p.cus), of_round = slot - divided(round * p.n_cus + p.n_heads - 1, p.heads);
