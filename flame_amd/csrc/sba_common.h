@@ -97,7 +97,7 @@ struct Job { int tok0, len, rb, seq, tab0; };
 //     B=1 H=8 T=16384 d=128 0.96 / 0.96 0.98 / 1.00     B=1 H=16 T=8192 d=64 0.91 / 0.99 0.99 / 1.00, d=128 0.94 / 1.00 1.01 / 1.01
 //     B=1 H=32 T=4096 d=64 0.89 / 0.99 1.00 / 0.99     B=1 H=16 T=16384 d=128 1.00 / 1.01 1.00 / 1.00
 // so it pays in any order of up to eight heads, where few heads make a cycle, and costs at most 1 % with more of them in no order; packs
-// of 30000 and 65536 tokens 0.97 ... 0.99.  Up to 3000 tokens, whose sweeps end near their starts in no head, and on packs of fewer rounds
+// of 30000 to 65536 tokens, seven of them, 0.93 ... 1.00 in this order and 0.96 ... 1.01 in random ones.  Up to 3000 tokens, whose sweeps end near their starts in no head, and on packs of fewer rounds
 // 0.98 ... 1.02: not there.  Kernels with one workgroup a CU lose by it (key owners at d=128 223 -> 237 us, 566 -> 617).
 // (A turn of several heads a slot, so that those that follow each other on an XCD are no neighbours: ahead where the neighbours reach
 // equally far - over ten shapes 0.99 of the time in the order above, 1.004 in random ones.  Heads have no such order in general.)

@@ -1932,17 +1932,23 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     if (!kp.makes_mid && (const char*)kp.gmid - (const char*)kp.rtab != (const char*)kp.gtab - (const char*)kp.rmid) return SBA_ERR_WORKSPACE;
     // Key-owner pass.  head_dim 64: the kernel whose waves own their keys outright, one sweep per workgroup, unless the launch hangs
     // on its longest sweeps; then the resident producer/consumer stream, which splits the work into twice as many items and deals
-    // them out itself.  Own-keys time over the stream's by tail ratio r, both passes, dense and packed alike:  longest sequence up
-    // to 4096 tokens  r 2.5 0.94, 2.7 0.90, 2.9 0.92-0.97, 3.1 0.92, 3.2 0.90-0.95, 3.4 0.99-1.02, 3.6 1.04, 3.9 1.13;  longer ones
-    // r 2.0 0.87, 2.2 0.93, 2.6 0.985, 2.7-2.8 1.00, 3.05 1.02, 3.2 1.04-1.06; with fewer heads, of which one that looks far is a larger
-    // part, B=2 H=4 T=16384 (2.0) 1.02, H=4 T=34000 (1.9) 1.03, T=26000 (2.5) 1.09, H=6 T=20000 (2.2) 1.01, H=2 T=50000 (2.6) 0.96.
+    // them out itself.  Forward + backward with the stream over the same with own keys, by tail ratio r, mean logits 0 .. -6 over the heads in
+    // this order and in random ones / all at -6:
+    //     longest sequence up to 4096 tokens, dense  r 2.7 1.04-1.05 / 1.04, 2.9 1.00 / 1.01, 3.1 0.99-1.015 / 0.99-1.00, 3.2 1.00-1.02 / 1.01, 3.3 0.98-1.00 /
+    //         0.99, 3.4 1.01-1.02 / 1.01, 3.9 0.93 / 0.94, 4.0 0.89-0.90 / 0.92;  packs  1.9 1.14-1.15, 2.5 1.08-1.13, 2.8 1.09-1.11, 3.3 1.04-1.06, 4.4 0.98
+    //     longer, dense, twelve and sixteen heads  r 2.1 0.99-1.07 / 0.98, 2.5 0.97-1.04 / 1.00, 2.6 1.01 / 0.99, 2.7 0.96-1.01 / 1.02, 2.9 0.96-1.00 /
+    //         1.01, 3.0 0.975 / 0.97, 3.1 0.96-0.98 / 0.97, 3.3 0.97 / 0.96
+    //     longer, dense, up to eight heads  r 1.6-1.7 0.975-1.12 / 1.00, 1.9 (H=4) 0.98 / 0.97, 2.0 H=8 0.96-1.03 / 0.96-0.99, H=4 0.99 / 0.97, H=1 and 2 1.09-1.18 /
+    //         0.95-0.97, 2.2 (H=6) 0.98-1.06 / 0.97, 2.3 (H=8) 0.95-1.00 / 0.96-0.98, 2.5 0.92-0.95 / 0.98, 2.7 0.93-0.985 / 0.97-0.98, 2.8-3.2 0.86-0.95 /
+    //         0.94-0.97, 3.6-4.0 0.79-0.91 / 0.88-0.90; behind only H=2 T=50000 (2.6) 1.02 / 0.98 and H=1 T=65536 (4.0), whose sweeps end early, 1.12 / 0.90
+    //     longer, packs  r 0.7-1.7 1.07-1.22, 2.4 1.09, 3.2 1.02-1.03 and (H=2) 0.90, 3.3 0.96, 3.9 0.97
     // Batches of short sequences (sweeps of at most 16 steps) also take the own-keys kernel at any size: on 512 workgroups B=8,
     // T=512 takes 27.3 us against the stream's 33.0, B=4, T=1024 44.0 against 45.3.
     // head_dim 128: the paired kernel at every size (on 64 ... 256 workgroups of B=1, H=16 it takes 27 / 44 / 62 / 81 us where the
     // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103); SBA_DKV_KERNEL=other still selects that one.
     const unsigned cus = (unsigned)sba_cu_count();
     const bool short_sweeps = kp.seq_len <= 8 * kRowBlock && grid.x >= 2u * cus;
-    const double own_up_to = kp.seq_len <= 32 * kRowBlock ? 3.35 : kp.n_heads < 8 ? 1.9 : 2.75;
+    const double own_up_to = kp.seq_len <= 32 * kRowBlock ? 3.35 : kp.n_heads <= 8 && !kp.cu_seqlens ? 2.2 : 2.75;
     const bool own = own_keys_kernel(kp.head_dim == 64 ? short_sweeps || sba_tail_ratio(kp, grid.x) <= own_up_to : true);
     const char* which = getenv("SBA_DKV_KERNEL");
     const bool plain = which && !strcmp(which, "plain");
@@ -1978,8 +1984,10 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         // The register-lean arrangement (three waves per SIMD) from five workgroups per CU on, unless the launch hangs on
         // one long sweep (tail ratio above 2.5: there the plain arrangement's shorter step is ahead, e.g. 111 against 118 us
         // on an 8192-token pack with a 4096-token document); from eight workgroups per CU on always.  On 1280-3232
-        // workgroups of 15 dense and packed shapes it is 0-5 % ahead of the plain one; at four workgroups per CU (six
-        // shapes of 1024 workgroups) the plain one is, by 1-3 %.
+        // workgroups of 15 dense shapes it takes 0.98-1.00 of the plain one's forward + backward where all heads look far and 0.98-1.02 where
+        // they differ, but for single sequences of 10000 tokens and more (1.00-1.07: B=1 H=12 T=16384 1690 against 1580 us, H=16 T=10240 898
+        // and 865; from T=14000 on 0.99-1.02); on packs 0.96-1.00.  At four workgroups per CU (six shapes of 1024 workgroups) the
+        // plain one is ahead by 1-3 %.
         else if (p1 && lean_dq_kernel(grid.x >= 8u * cus || (grid.x >= 5u * cus && sba_tail_ratio(kp, grid.x) <= 2.5)))
             hipLaunchKernelGGL((mfma_bwd_dq_kernel<64, true>), grid, dim3(kThreads), 0, s, sba_turning(kp, 3));
         else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<64>), grid, dim3(kThreads), 0, s, sba_turning(kp, 2));

@@ -440,9 +440,12 @@ static int forward_segments(const sba::KParams& kp, unsigned grid) {
         // LDS) one; it pays while the grid is at most two rounds of those and the longest sweep dominates.  B=1,
         // H=16, one sweep / two segments in us: T=1024 29.8 / 26.2, T=2048 50.4 / 41.6, T=3072 77.2 / 60.0, T=4096
         // 105.5 / 91.8, T=5120 131.1 / 138.7, T=8192 276.2 / 291.7; B=2 T=2048 60.0 / 57.0; H=8 T=4096 89.7 / 70.8.
-        // Long dense sequences, whose heads differ in how far they look, somewhat beyond (mean logits 0 .. -6 over the heads): T=4400
-        // (r 3.6) 99 / 87, T=5000 (3.1) 119 / 105, H=12 T=6500 (3.3) 148 / 121, H=8 T=10000 (3.2) 206 / 179, but H=16 T=6000 (2.7) 148 / 141 and
-        // at head_dim 80 112 / 119, H=4 T=20000 (3.2) 397 / 388 and 335 / 348, H=32 T=2500 (3.1) 66 / 72.
+        // Long dense sequences somewhat beyond.  Two segments over one sweep, mean logits 0 .. -6 over the heads in this order and in two random
+        // ones / all at -6:  T=4400 (r 3.6) 0.83-0.86 / 0.86, T=4800 (3.3) 0.87-0.92 / 0.90, T=5000 (3.1) 0.88-0.94 / 0.915, H=12 T=6500 (3.3)
+        // 0.79-0.82 / 0.90, H=10 T=8000 (3.2) 0.82-0.97 / 0.885, H=8 T=10000 (3.2) 0.92-1.00 / 0.89, B=2 H=8 T=4800 (3.3) 0.98 / 0.92; beyond that
+        // H=8 T=11000 (2.9) 0.90-1.09 / 0.93;  with fewer heads H=4 T=20000 (3.2) 0.97-0.98 / 0.88;  shorter ones H=32 T=2500 (3.1) 1.02-1.08 / 1.02.
+        // At head_dim 80, whose steps are shorter, the same rule is about even: T=4400 0.91-0.93 / 0.97, T=4800 0.94-0.99 / 1.05, T=5000 0.97-1.01 / 1.07,
+        // H=12 T=6500 0.85-0.87 / 1.01, H=10 T=8000 0.90-1.06 / 1.03, H=8 T=10000 0.96-1.06 / 1.00, B=2 H=8 T=4800 1.08 / 1.03.
         if (sba_two_step_env() >= 0) return grid <= (unsigned)sba_two_step_env() ? 2 : 0;
         const double r = sba_tail_ratio(kp, grid);
         if (!kp.cu_seqlens && kp.n_heads >= 8 && kp.seq_len > 32 * sba::kRowBlock && r >= 3.1) return 2;
