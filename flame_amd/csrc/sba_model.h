@@ -30,8 +30,6 @@ int norm_bwd(const NormBwd& a, bool f16, hipStream_t stream);
 // out[i][c] = sum over the parts of part[i], for one or two of them in a launch
 int sum_parts(const float* const (&part)[2], float* const (&out)[2], int n, int parts, int cols, hipStream_t stream);
 
-int add_residual(const float* x, const void* h, float* out, int64_t n, bool f16, hipStream_t stream);
-
 // y = [rows][2 * width] = gate | up;  out = silu(gate) * up
 int swiglu_fwd(const void* y, void* out, int64_t rows, int width, bool f16, hipStream_t stream);
 int swiglu_bwd(const void* y, const void* d_out, void* dy, int64_t rows, int width, bool f16, hipStream_t stream);
@@ -74,7 +72,7 @@ int weight_grads_f16(const WeightGrads& g, int splits, hipStream_t stream);
 
 // y[t][n] = sum over k of x[t][k] w[n][k] (rows_w: w[k][n]) for m token rows, k a multiple of 32, n of 8, and what follows:
 //   kStore        out = y                                    16-bit [m][n]
-//   kAddResidual  out = residual + y                         fp32   [m][n]
+//   kAddResidual  out = residual + y                         fp32   [m][n]; y is the fp32 sum, not rounded to 16 bits first
 //   kSwigluFwd    w = gate rows | up rows: out = silu(gate) * up, 16-bit [m][n/2]; pre = y if given
 //   kSwigluBwd    y = gradient of silu(gate) * up, pre = gate | up [m][2n]: out = their gradients, 16-bit [m][2n]
 // x and w are 16-byte aligned with leading dimensions that are multiples of 8; outputs are dense.

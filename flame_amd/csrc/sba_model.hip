@@ -149,18 +149,6 @@ __global__ __launch_bounds__(1024) void sum_parts_kernel(const float* part0, con
     }
 }
 
-template <typename E>
-__global__ __launch_bounds__(kThreads) void add_residual_kernel(const float* x, const E* h, float* out, int64_t n4) {
-    typedef typename Vec<E>::x4 e4;
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n4; i += (int64_t)gridDim.x * kThreads) {
-        f32x4 v = *(const f32x4*)(x + i * 4);
-        const e4 a = *(const e4*)(h + i * 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] += (float)a[j];
-        *(f32x4*)(out + i * 4) = v;
-    }
-}
-
 // ------------------------------------------------------------------------------------------------- SwiGLU
 // silu(gate) and d_out * up are rounded to 16 bits where the module path holds them as tensors: both paths give the same bits.
 template <typename E>
@@ -473,13 +461,6 @@ int norm_bwd_parts(int rows) {
 
 int sum_parts(const float* const (&part)[2], float* const (&out)[2], int n, int parts, int cols, hipStream_t s) {
     hipLaunchKernelGGL(sum_parts_kernel, dim3((cols + 15) / 16, n), dim3(1024), 0, s, part[0], part[1], out[0], out[1], parts, cols);
-    return launched();
-}
-
-int add_residual(const float* x, const void* h, float* out, int64_t n, bool f16, hipStream_t s) {
-    const dim3 grid(grid_for(n / 4)), block(kThreads);
-    if (f16) hipLaunchKernelGGL(add_residual_kernel<_Float16>, grid, block, 0, s, x, (const _Float16*)h, out, n / 4);
-    else hipLaunchKernelGGL(add_residual_kernel<__bf16>, grid, block, 0, s, x, (const __bf16*)h, out, n / 4);
     return launched();
 }
 

@@ -144,3 +144,17 @@ def test_the_input_gradient_of_a_head_is_shared_out():
     x = torch.randn(700, 16000, generator=g, device="cuda").bfloat16()
     w = (torch.randn(16000, 512, generator=g, device="cuda") / 126).bfloat16()
     assert rel_l2(_lib.native().project(x, w, True).float(), x.float() @ w.float()) <= 4e-3
+
+
+# the product is added to the residual as its fp32 sum, for contractions that the kernels take as they are and for others: rounded to 16
+# bits first it would be off by a thousandth (bf16) or a ten-thousandth
+@pytest.mark.parametrize("m,n,k,dtype", [(65, 80, 64, torch.bfloat16), (300, 512, 1000, torch.bfloat16), (257, 64, 8, torch.float16), (1, 128, 328, torch.float16)])
+def test_the_residual_meets_an_unrounded_product(m, n, k, dtype):
+    from flame_amd import _lib
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(n, k, generator=g, device="cuda") / k ** 0.5).to(dtype)
+    residual = torch.randn(m, n, generator=g, device="cuda")
+    got = _lib.native().project_add(x, w, residual)
+    # products of 16-bit values are exact in fp32, their sums carry at most k + 1 roundings of 2^-24
+    assert rel_l2(got.double(), residual.double() + x.double() @ w.double().t()) <= 1e-5
