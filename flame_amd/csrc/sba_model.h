@@ -83,7 +83,8 @@ struct Projection {
     const float* residual; void* pre; void* out;
     int splits; float* partial;          // kStore, rows_w: so many workgroups share a tile's contraction (0, 1: none); [splits][m][n]
 };
-bool projects(const Projection& p, int cus);             // whether the kernels take it
+bool addresses(const Projection& p);                     // whether the kernels can take it
+bool projects(const Projection& p, int cus);             // whether they do
 enum ProjectionTile { kTile256, kTile128x256, kTile128, kTile128Halves, kTile64, kTile64Halves };
 ProjectionTile projection_tile(const Projection& p, int cus);
 double tile_time(const Projection& p, ProjectionTile tile, int cus);    // an estimate, us; 1e30 where its kernel does not take it

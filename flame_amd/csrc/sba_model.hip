@@ -559,11 +559,14 @@ double tile_time(const Projection& p, ProjectionTile tile, int cus) {
     return us;
 }
 
+bool addresses(const Projection& p) {
+    return p.k % 32 == 0 && p.k > 0 && p.n % (p.epilogue == kSwigluFwd ? 16 : 8) == 0 && p.n > 0 && p.m > 0 && p.ldx % 8 == 0 &&
+           p.ldw % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.w & 15) == 0 && p.ldx < (1 << 22) && p.ldw < (1 << 22) &&
+           (int64_t)(p.rows_w ? p.k : p.n) * p.ldw < (INT64_C(1) << 31);
+}
+
 bool projects(const Projection& p, int cus) {
-    if (!(p.k % 32 == 0 && p.k > 0 && p.n % (p.epilogue == kSwigluFwd ? 16 : 8) == 0 && p.n > 0 && p.m > 0 && p.ldx % 8 == 0 &&
-          p.ldw % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.w & 15) == 0 && p.ldx < (1 << 22) && p.ldw < (1 << 22) &&
-          (int64_t)(p.rows_w ? p.k : p.n) * p.ldw < (INT64_C(1) << 31)))
-        return false;
+    if (!addresses(p)) return false;
     if (p.epilogue == kSwigluBwd) {
         // against the plain product and a pass of its own, which reads and writes 12 bytes per product at 7.7 TB/s (much of it still in
         // the last-level cache): 8192 x 2816, k = 1024 76 against 48 + 36 us

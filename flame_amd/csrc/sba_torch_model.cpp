@@ -69,6 +69,8 @@ int compute_units() {
     return cus;
 }
 
+void check_on_gpu(const Tensor& x) { TORCH_CHECK_VALUE(x.is_cuda(), "the model's kernels run on the GPU only"); }
+
 // d_weight = d_out^T . in, in fp32, of several products over the same rows at once
 std::vector<Tensor> weight_grads(at::ArrayRef<std::pair<Tensor, Tensor>> pairs) {
     WeightGrads g = {};
@@ -84,6 +86,7 @@ std::vector<Tensor> weight_grads(at::ArrayRef<std::pair<Tensor, Tensor>> pairs) 
     }
     const Tensor& like = pairs[0].first;
     ok(weight_grads_fit(g) ? 0 : SBA_ERR_SHAPE);
+    check_on_gpu(like);
     const int splits = weight_grad_splits(g, compute_units());
     const Tensor out = empty({g.total}, like, at::kFloat);
     Tensor partial;
@@ -190,12 +193,33 @@ bool try_project(const Tensor& x, const Tensor& w, bool rows_w, int epilogue, co
     return true;
 }
 
+// What the kernels take for granted and the nodes see to before they call: the entries by themselves check it.
+void check_operands(const Tensor& x, const Tensor& w, bool rows_w) {
+    const auto t = x.scalar_type();
+    TORCH_CHECK_TYPE((t == at::kBFloat16 || t == at::kHalf) && w.scalar_type() == t, "x and w must both be bfloat16 or both float16");
+    TORCH_CHECK_VALUE(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(rows_w ? 0 : 1), "x and w must be matrices that share k");
+    TORCH_CHECK_VALUE(x.stride(1) == 1 && w.stride(1) == 1 && (x.size(0) < 2 || x.stride(0) >= x.size(1)) && (w.size(0) < 2 || w.stride(0) >= w.size(1)), "rows of x and w must be dense");
+    TORCH_CHECK_VALUE(x.device() == w.device(), "x and w must be on the same device");
+}
+void check_dense(const Tensor& t, at::IntArrayRef sizes, at::ScalarType type, const Tensor& like, const char* name) {
+    TORCH_CHECK_VALUE(t.defined() && t.sizes() == sizes && t.is_contiguous() && t.device() == like.device() && ((uintptr_t)t.data_ptr() & 15) == 0,
+                      name, " must be a dense tensor of shape ", sizes, " on 16 bytes beside x");
+    TORCH_CHECK_TYPE(t.scalar_type() == type, name, " must be ", type);
+}
 // The same with the tile of a caller's choice, where that tile's kernel takes the problem (tests of kernels that the rule picks elsewhere).
 bool project_with(int64_t tile, const Tensor& x, const Tensor& w, bool rows_w, int64_t epilogue, const std::optional<Tensor>& residual,
                   const std::optional<Tensor>& pre, const Tensor& out, int64_t splits) {
+    TORCH_CHECK(tile >= kTile256 && tile <= kTile64Halves && epilogue >= kStore && epilogue <= kSwigluBwd && splits >= 1, "project_with: no such tile, epilogue or share");
+    check_operands(x, w, rows_w);
+    const int64_t m = x.size(0), n = w.size(rows_w ? 1 : 0);
+    const auto t = x.scalar_type();
+    check_dense(out, {m, epilogue == kSwigluFwd ? n / 2 : epilogue == kSwigluBwd ? 2 * n : n}, epilogue == kAddResidual ? at::kFloat : t, x, "out");
+    if (epilogue == kAddResidual) check_dense(residual.value_or(Tensor()), {m, n}, at::kFloat, x, "residual");
+    if (epilogue == kSwigluBwd || (epilogue == kSwigluFwd && pre)) check_dense(pre.value_or(Tensor()), {m, epilogue == kSwigluBwd ? 2 * n : n}, t, x, "pre");
+    check_on_gpu(x);
+    c10::DeviceGuard guard(x.device());
     Projection p = projection_of(x, w, rows_w, (int)epilogue, residual.value_or(Tensor()), pre.value_or(Tensor()), out);
-    TORCH_CHECK(tile >= kTile256 && tile <= kTile64Halves && p.k % 32 == 0 && p.n % 16 == 0 && p.ldx % 8 == 0 && p.ldw % 8 == 0 && p.m > 0,
-                "project_with: sizes that no tile takes");
+    TORCH_CHECK(addresses(p), "project_with: sizes or places that no tile takes");
     if (tile_time(p, (ProjectionTile)tile, compute_units()) >= 1e30) return false;
     Tensor partial;
     if (splits > 1) {
@@ -610,18 +634,48 @@ void bind_model(py::module& m) {
     m.def("head", &head);
     m.def("next_token_loss", &next_token_loss);
     m.def("clip_and_step", &clip_and_step);
-    m.def("project", &project);
+    m.def("project", [](const Tensor& x, const Tensor& w, bool rows_w) {
+        check_operands(x, w, rows_w);
+        check_on_gpu(x);
+        c10::DeviceGuard guard(x.device());
+        return project(x, w, rows_w);
+    });
     m.def("project_with", &project_with, py::arg("tile"), py::arg("x"), py::arg("w"), py::arg("rows_w"), py::arg("epilogue"), py::arg("residual"),
           py::arg("pre"), py::arg("out"), py::arg("splits") = 1);
     m.attr("projection_tiles") = (int)kTile64Halves + 1;
-    m.def("project_add", &project_add);
+    m.def("project_add", [](const Tensor& x, const Tensor& w, const Tensor& residual) {
+        check_operands(x, w, false);
+        check_dense(residual, {x.size(0), w.size(0)}, at::kFloat, x, "residual");
+        check_on_gpu(x);
+        c10::DeviceGuard guard(x.device());
+        return project_add(x, w, residual);
+    });
     m.def("project_swiglu", [](const Tensor& x, const Tensor& w) {
+        check_operands(x, w, false);
+        TORCH_CHECK_VALUE(w.size(0) % 16 == 0, "gate and up must have a multiple of 8 rows each");
+        check_on_gpu(x);
+        c10::DeviceGuard guard(x.device());
         Tensor pre;
         const Tensor out = project_swiglu(x, w, pre, true);
         return std::make_pair(out, pre);
     });
-    m.def("project_swiglu_grad", &project_swiglu_grad);
-    m.def("weight_grad", [](const Tensor& d_out, const Tensor& in) { return weight_grads({{d_out, in}})[0]; });
+    m.def("project_swiglu_grad", [](const Tensor& d, const Tensor& w, const Tensor& pre) {
+        check_operands(d, w, true);
+        check_dense(pre, {d.size(0), 2 * w.size(1)}, d.scalar_type(), d, "pre");
+        TORCH_CHECK_VALUE(w.size(1) % 8 == 0, "gate and up must have a multiple of 8 columns each");
+        check_on_gpu(d);
+        c10::DeviceGuard guard(d.device());
+        return project_swiglu_grad(d, w, pre);
+    });
+    m.def("weight_grad", [](const Tensor& d_out, const Tensor& in) {
+        const auto t = d_out.scalar_type();
+        TORCH_CHECK_TYPE((t == at::kBFloat16 || t == at::kHalf) && in.scalar_type() == t, "d_out and in must both be bfloat16 or both float16");
+        TORCH_CHECK_VALUE(d_out.dim() == 2 && in.dim() == 2 && d_out.size(0) == in.size(0) &&
+                          (d_out.numel() == 0 || (d_out.stride(1) == 1 && in.stride(1) == 1)) && d_out.device() == in.device(),
+                          "d_out and in must be matrices of the same rows, which are dense");
+        c10::OptionalDeviceGuard guard(d_out.device());
+        return weight_grads({{d_out, in}})[0];
+    });
     m.attr("max_norm_width") = kMaxNormWidth;
 }
 

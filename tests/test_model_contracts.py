@@ -126,3 +126,32 @@ def test_clip_and_step_leaves_other_tensor_classes_and_observed_steps_alone(nati
     p.grad = plain
     opt.state[p]["exp_avg"] = opt.state[p]["exp_avg"].as_subclass(Other)
     assert fused.clip_and_step([p], opt, 1.0) is None and not native.calls
+
+
+# The projection kernels' entries by themselves: what the kernels take for granted is refused before anything is launched.
+@pytest.mark.parametrize("change,error,says", [
+    ({"x": torch.zeros(4, 64)}, TypeError, "float16"),
+    ({"w": torch.zeros(32, 64, dtype=torch.float16)}, TypeError, "float16"),
+    ({"w": torch.zeros(32, 96, dtype=torch.bfloat16)}, ValueError, "share k"),
+    ({"x": torch.zeros(64, 4, dtype=torch.bfloat16).t()}, ValueError, "dense"),
+    ({"residual": None}, ValueError, "residual"),
+    ({"residual": torch.zeros(4, 16)}, ValueError, "residual"),
+    ({"residual": torch.zeros(4, 32, dtype=torch.bfloat16)}, TypeError, "residual"),
+    ({"out": torch.zeros(4, 16)}, ValueError, "out"),
+    ({"out": torch.zeros(32, 4).t()}, ValueError, "out"),
+    ({"out": torch.zeros(4, 32, dtype=torch.bfloat16)}, TypeError, "out"),
+    ({"epilogue": 3, "out": torch.zeros(4, 64, dtype=torch.bfloat16), "w": torch.zeros(64, 32, dtype=torch.bfloat16), "rows_w": True}, ValueError, "pre"),
+    ({"epilogue": 4}, RuntimeError, "epilogue"),
+    ({"tile": 6}, RuntimeError, "tile"),
+    ({}, ValueError, "GPU only"),
+])
+def test_what_the_projection_kernels_take_for_granted_is_checked(change, error, says):
+    from flame_amd import _lib
+    a = dict(tile=2, x=torch.zeros(4, 64, dtype=torch.bfloat16), w=torch.zeros(32, 64, dtype=torch.bfloat16), rows_w=False, epilogue=1,
+             residual=torch.zeros(4, 32), pre=None, out=torch.zeros(4, 32))
+    a.update(change)
+    with pytest.raises(error, match=says):
+        _lib.native().project_with(**a)
+    if not set(change) - {"x", "w", "residual"} and a["residual"] is not None:
+        with pytest.raises(error, match=says):
+            _lib.native().project_add(a["x"], a["w"], a["residual"])
