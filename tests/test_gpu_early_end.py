@@ -93,3 +93,39 @@ def test_a_gradient_of_rem_that_is_no_number_shows_where_the_stick_is_used_up(B,
     assert torch.equal(dq.isnan(), full.isnan()) and torch.equal(dq.nan_to_num(7), full.nan_to_num(7))
     assert bool(dq[0, 0, [700, 901, 1099]].isnan().all())
     assert bool(dk[0, 0, [690, 890, 1090]].isnan().all())        # the keys that these rows still reach
+
+
+# with room for one of the forward's two tables, the other made by the dQ pass on its way
+@pytest.mark.parametrize("B,H,T,D,dtype", [
+    (1, 4, 2047, 64, torch.bfloat16),
+    (3, 16, 1100, 64, torch.float16),
+    (1, 4, 2100, 128, torch.float16),
+    (1, 4, 1500, 80, torch.bfloat16),
+    (0, 4, [1, 700, 129, 2500, 64, 1000], 64, torch.bfloat16),
+    (0, 4, [1, 700, 129, 1500, 64], 128, torch.bfloat16),
+    (0, 4, [1, 700, 129, 1500, 64], 96, torch.float16),
+])
+def test_same_bits_as_full_sweeps_with_one_kept_table(B, H, T, D, dtype, monkeypatch):
+    from flame_amd import _lib
+    lens = T if isinstance(T, list) else None
+    x = _inputs(H, (B,) if B else (), sum(T) if lens else T, D, dtype, 60 + D)
+    one = 4 * 128 * H * sum(n * (n + 1) for n in ((t + 127) // 128 for t in (lens or [T] * B)))
+    kept = []
+
+    def note(t):
+        if t.dtype == torch.uint8:
+            kept.append(t.numel())
+        return t
+
+    try:
+        _lib.set_workspace_budget(1.5 * one)
+        with torch.autograd.graph.saved_tensors_hooks(note, lambda t: t):
+            _run(x, lens, False)
+        assert kept == [one]
+        short = _run(x, lens, False)
+        monkeypatch.setenv("SBA_FULL_SWEEPS", "1")
+        full = _run(x, lens, False)
+    finally:
+        _lib.set_workspace_budget(None)
+    for a, b in zip(short, full):
+        assert torch.equal(a, b)
