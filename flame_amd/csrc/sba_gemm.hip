@@ -542,12 +542,13 @@ __global__ __launch_bounds__(256 * G, G * kPerCu) void projection_kernel(Project
 // Stages of 64 k: rows of 64 k are whole 128-byte lines (with 32 k every line is fetched twice: -12 %).  A stage is four slices of
 // TM/16 MFMAs a wave; the operands of a slice are fetched under the MFMAs of the one before.  After the third slice the waves meet:
 // the stage's buffer has been read, the next stage has landed, and the copies of the stage NB ahead start into it, spread over the
-// slices that follow (all under one they ask for 1024 cycles of the CU's memory pipe in 544 of MFMAs: 1.55 us per stage against
-// 1.42 with 256 rows, every CU busy).  The copies run through the list of (tile, stage) pairs without a break, so a tile's results
-// are stored while the next tile's first stages arrive.  TM = 256 has two buffers of 64 KB, TM = 128, whose stages pass in half the
-// time, three of 48 KB; the fetch addresses move from buffer to buffer, one add per address and stage.
-// 8192 tokens, k = 1024: 5632 features with swiglu in 83 us with TM = 256 (1.14 PFLOP/s; 89 with 128, 92 in 128 x 128 tiles), 3072 features in
-// 46 with TM = 128 (50; 49); k = 5632, W's rows: 1024 features in 77 with TM = 128 (104; 80).
+// slices that follow (all under one they ask for 1024 cycles of the CU's memory pipe in 544 of MFMAs: 1.09 of the time per stage,
+// which with 256 rows and every CU busy is 1.33 us in products of 90 us and 1.56 in products of 400, where the chip's power limit has
+// taken the clock down).  The copies run through the list of (tile, stage) pairs without a break, so a tile's results are stored while
+// the next tile's first stages arrive.  TM = 256 has two buffers of 64 KB, TM = 128, whose stages pass in half the time, three of
+// 48 KB; the fetch addresses move from buffer to buffer, one add per address and stage.
+// 8192 tokens, k = 1024: 5632 features with swiglu in 92 us with TM = 256 (1.03 PFLOP/s; 99 with 128, 102 in 128 x 128 tiles), 3072 features in
+// 47 with TM = 128 (49; 50); k = 5632, W's rows: 1024 features in 79.6 with TM = 128 (103.5; 79.2).
 template <int TM, bool kRowsW, int kEpi>
 __global__ __launch_bounds__(256, 1) void large_projection_kernel(Projection p) {
     constexpr int NB = TM == 256 ? 2 : 3;

@@ -1459,9 +1459,9 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
 // where the two passes read them twice, no prefix table is written or read, and it is one launch.
 // What bounds it is memory (seven tensors' bytes): two workgroups of four waves (80 KB of LDS) or four of two waves (sequences
 // of at most 64 tokens) share a CU at head_dim 64, so that one's loads and stores run under the other's arithmetic; the next key
-// block's K and V are requested into the tile just used.  On 65536 tokens in documents of 16 .. 128 (H=16, d=64) it takes 256 us where
-// its copies and stores alone take 200 and its arithmetic, on rows that the caches hold, about 230: 1650 instructions per wave of
-// which the two chains are 600.  (Two documents in turn per workgroup, the next one's rows requested into registers meanwhile, are
+// block's K and V are requested into the tile just used.  On 65536 tokens in documents of 16 .. 128 (H=16, d=64) it takes 257 us and executes
+// 800 vector and 410 scalar instructions a wave, 144 us of issue at the measured rates.  (When it took 268 us, its copies and stores alone
+// took 200 and the whole of it, on rows that the caches held, 241.  Two documents in turn per workgroup, the next one's rows requested into registers meanwhile, are
 // behind at every size: 64 registers and the second document's scalars spill, and the loads were not what was waited for.)
 template <int D, int W>
 __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel(KParams p) {
@@ -1941,6 +1941,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     //     longer, dense, up to eight heads  r 1.6-1.7 0.975-1.12 / 1.00, 1.9 (H=4) 0.98 / 0.97, 2.0 H=8 0.96-1.03 / 0.96-0.99, H=4 0.99 / 0.97, H=1 and 2 1.09-1.18 /
     //         0.95-0.97, 2.2 (H=6) 0.98-1.06 / 0.97, 2.3 (H=8) 0.95-1.00 / 0.96-0.98, 2.5 0.92-0.95 / 0.98, 2.7 0.93-0.985 / 0.97-0.98, 2.8-3.2 0.86-0.95 /
     //         0.94-0.97, 3.6-4.0 0.79-0.91 / 0.88-0.90; behind only H=2 T=50000 (2.6) 1.02 / 0.98 and H=1 T=65536 (4.0), whose sweeps end early, 1.12 / 0.90
+    //         backward alone at the line and above, by the longest document: 3.4-3.8 0.92-1.04 (2000 to 4096 tokens), 3.5 1.09-1.11 (1387); 4.0 0.96 (3562), 1.08
+    //         (1539); 4.4-5.2 0.78-0.96
     //     longer, packs  r 0.7-1.7 1.07-1.22, 2.4 1.09, 3.2 1.02-1.03 and (H=2) 0.90, 3.3 0.96, 3.9 0.97
     // Batches of short sequences (sweeps of at most 16 steps) also take the own-keys kernel at any size: on 512 workgroups B=8,
     // T=512 takes 27.3 us against the stream's 33.0, B=4, T=1024 44.0 against 45.3.

@@ -13,7 +13,7 @@
 //     16 MFMAs (1024 cycles) of which the next is always on its way;
 //   * a workgroup of the key-owner pass owns 64 keys and has eight waves, 256 queries per step.
 // B=2, H=8, T=1024, d=64, forward / dQ / dK,dV in us: 85 / 120 / 103 with 128 rows per workgroup, one step at a time and
-// tiles through LDS; now 36 / 54 / 95 (the MFMAs alone, evenly spread over the chip: 14 / 20 / 27).
+// tiles through LDS; now 31 / 49 / 87 (the MFMAs alone, evenly spread over the chip: 14 / 20 / 27).
 //
 // Geometry as in sba_mfma.h: a step covers 64 keys, score tiles are computed transposed (S^T = K Q^T), and MFMA row M of
 // tile t holds key

@@ -532,9 +532,10 @@ int weight_grad_splits(WeightGrads& g, int cus) {
 // each k / 64 times `rate` of a full CU, then a last one at the rate of as many workgroups a CU as are left (one on half of the CUs or
 // less: `half` of that rate, what lies between in proportion); `round` and what the epilogue adds that nothing hides, per round
 // and in proportion to its fill; `launch`.
-// Where each is ahead (us): 256 x 256 8192 x 5632 of swiglu, k = 1024 (92, next 101); 128 x 256 8192 x 3072, k = 1024 (49; 52);
-// 128 x 128 two a CU 4096 x 1024, k = 1024 (12; 15); by halves 4096 x 1024, k = 5632 (49; 59); 64 x 64 three a CU 2048 x 2304,
-// k = 768 (13.0; 14.0), 1500 x 2816 with the swiglu gradient, k = 1024 (21; 24); by halves 1024 x 768, k = 4096 (15.8; 19.8).
+// Where each is ahead (us): 256 x 256 8192 x 5632 of swiglu, k = 1024 (92, next 99); 128 x 256 8192 x 3072, k = 1024 (47; 49);
+// 128 x 128 two a CU 8192 x 2816 with the swiglu gradient, k = 1024 (69; 86), 8192 x 1024 with the residual, k = 2816 (47; 49); by halves
+// 4096 x 1024, k = 5632 (49; 59); 64 x 64 three a CU 2048 x 2304, k = 768 (12.4; 13.3), 1500 x 2816 with the swiglu gradient, k = 1024 (20.8;
+// 23.4); by halves 1024 x 768, k = 4096 (14.6; 18.5).
 double tile_time(const Projection& p, ProjectionTile tile, int cus) {
     struct { int rows, features, per_cu; double rate[3], half, round, launch, add, swiglu_fwd, swiglu_bwd; } static const cost[] = {
         {256, 256, 1, {1.24}, 0.87, 3.8, 7.0, 0.0, 2.4, 0.0},                   // kTile256
@@ -569,7 +570,7 @@ bool projects(const Projection& p, int cus) {
     if (!addresses(p)) return false;
     if (p.epilogue == kSwigluBwd) {
         // against the plain product and a pass of its own, which reads and writes 12 bytes per product at 7.7 TB/s (much of it still in
-        // the last-level cache): 8192 x 2816, k = 1024 76 against 48 + 36 us
+        // the last-level cache): 8192 x 2816, k = 1024 69 against 48 + 36 us (91 in a training step)
         Projection plain = p;
         plain.epilogue = kStore;
         return tile_time(p, projection_tile(p, cus), cus) < tile_time(plain, projection_tile(plain, cus), cus) + 12e-6 * p.m * p.n / 7.7 + 1.5;
@@ -590,7 +591,8 @@ ProjectionTile projection_tile(const Projection& p, int cus) {
 }
 
 // Long contractions over few tiles (the input gradient of a language model's head): the large tiles' kernels with as many workgroups to a
-// tile as the CUs allow, their fp32 sums written, read and added at 5.5 TB/s.  k = 32000, one workgroup a tile against several (us): 300 x 768
+// tile as the CUs allow, their fp32 sums written, read and added at 5.5 TB/s.  (1.4 us a stage of 256 rows: a full chip slows from 1.38 to
+// 1.59 in contractions as long as these, and tile_time()'s 1.24 fits shorter ones.)  k = 32000, one workgroup a tile against several (us): 300 x 768
 // 94, 57;  1024 x 1024 121, 76;  2048 x 1024 208, 120;  3000 x 768 244, 150;  4096 x 1024 355, 237;  8192 x 1024 436, 423;  k = 8192:
 // 2048 x 1024 52, 43;  4096 x 1024 68 either way;  k = 5632: 3000 x 768 48, 39.
 int projection_splits(const Projection& p, int cus, ProjectionTile& tile) {

@@ -231,7 +231,8 @@ int sba_bwd_gave_up(const SbaParams* p, int static_scratch_used, int* gave_up);
  * p->bwd_scratch / p->bwd_scratch_bytes are ignored: the scratch is an array of
  * SBA_STATIC_SCRATCH_BYTES that the library itself holds on every GPU it runs on, until the
  * process ends.  Problems with sba_bwd_scratch_bytes(p) above that limit are refused with
- * SBA_ERR_STATIC_LIMIT and nothing is launched.  The call allocates nothing and frees nothing;
+ * SBA_ERR_STATIC_LIMIT and nothing is launched (the room for two fp32 workgroups' sums, which need
+ * not be there, does not count).  The call allocates nothing and frees nothing;
  * the very first call on a device looks up the array's address there (make one call before a
  * graph capture starts).  All calls on one GPU share the one array, which keeps the previous
  * call's contents: calls that overlap on the same GPU (different streams or threads) race and
