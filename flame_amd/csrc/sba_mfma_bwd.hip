@@ -1643,36 +1643,40 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
 // [32 keys x 128] accumulators of dK and dV - is 190 registers: one wave per SIMD.  Here TWO waves share
 // 32 keys.  Both hold the K and V fragments; wave r of the pair turns query tile r of the step (32 of
 // its 64 queries) into weights and logit gradients and writes them to the pair's tile in LDS; after a
-// barrier each wave reduces ALL 64 queries of the step for ITS half of the head dim (column blocks
-// 2r, 2r + 1 at head_dim 128), so it accumulates [32 keys x D/2] of dK and of dV only.  The vector work
-// of a step is split between the two, the reductions too: eight waves per workgroup (128 keys), two per
-// SIMD.  Two workgroup barriers per step (weights complete; tiles handed over).
-template <int D>
-__global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KParams p) {
+// barrier wave 0 reduces the weights of ALL 64 queries with dO into dV, wave 1 the logit gradients with Q into
+// dK, so each accumulates [32 keys x D] of one output.  (A split of both outputs' columns fetches both kinds of
+// weights in both waves - six operands a 16 queries instead of five - and leaves head_dim 96 with two column blocks in one wave and
+// one in the other: 12 heads, 20011 tokens, d = 80 222 -> 213 us.)  Two workgroup barriers per step (weights complete; tiles handed over).
+// What bounds it is instruction issue (MFMA and vector instructions keep a SIMD busy 84 to 94 % of the time in which its CU has
+// work) and the waits of waves that run in step.  kPairs = 2: a workgroup is 64 keys, four waves and exactly half of a CU's LDS, so
+// that two of them share a CU and one's barriers and round trips pass under the other's work, and the diagonal and the end of a
+// sequence are cut off by 64 keys.  Against one workgroup of kPairs = 4 a CU (128 keys, eight waves, half the tile copies):
+// B=4 H=16 T=2047 d=128 181 -> 163 us, B=1 H=16 T=16384 1690 -> 1530, d = 80 as above 249 -> 213.
+template <int D, int kPairs>
+__global__ __launch_bounds__(128 * kPairs, 2) void mfma_bwd_dkv_pair_kernel(KParams p) {
     constexpr int kQTile = 64 * kPitch<D> * 2;           // Q or dO tile of one step (64 queries)
     constexpr int kZTile = 64 * 64 * 2;          // per pair: [64 queries][32 a | 32 dz] bf16
     constexpr int kStep = 64;
-    constexpr bool kPairPin = true;              // LDS fetch bases pinned in registers: 3 % faster here
-    constexpr int kBlocks = (D + 63) / 64;       // 32-wide column blocks of dK / dV per wave (head_dim 96: two or one)
-    static_assert(32 * D * 2 <= kZTile, "the pair's tile doubles as the staging of its [32 keys x D] outputs");
-    __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + 4 * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
+    constexpr int kBlocks = D / 32;              // 32-wide column blocks of dK or dV
+    static_assert(2 * kPairs * 32 * D * 2 <= 4 * kQTile, "every wave stages its [32 keys x D] output in the tiles");
+    __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + kPairs * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = wave >> 1, r = wave & 1;
-    // this wave's column blocks: kBlocks * half ..; at head_dim 96 the second half is one block, and the pairs take turns at which
-    // of their waves (r: which SIMD) has it
-    const int half = D == 96 ? r ^ (grp >> 1) : r;
-    const bool both = D != 96 || half == 0;
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
     LaneOffsets<64> lz;
     lz.init(lane);
-    const int head = head_of_block(p, blockIdx.x);
-    const Job job = decode_key_job(p, slot_of_block(p, blockIdx.x));
+    constexpr int kParts = 4 / kPairs;                 // workgroups of a scheduled 128-row job
+    const int slot = slot_of_block(p, blockIdx.x);
+    const int head = head_of_block<kPairs == 4 ? kOnePerCu : kSharedCu>(p, blockIdx.x);
+    const Job job = decode_key_job(p, slot / kParts);
     const int strict = p.attend_current ? 0 : 1;
-    const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it
+    const int first_kb = 2 * job.rb + slot % kParts;   // first 64-key block of the workgroup's keys
+    const int q_begin = first_kb * kKeyBlock;          // first key = first query that may see it
+    if (q_begin >= job.len) return;
     const int kb0 = q_begin + 32 * grp;                // first key of this pair
     char* ztile = lds + 4 * kQTile + grp * kZTile;
 
@@ -1691,19 +1695,28 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
         load_row_frags<D>(vfr, p.v, vbase, kb0, key, job.len, lane, p.cols);
         prescale_frags(kfr, p.scale2);
     }
-    f32x16 dkacc[kBlocks], dvacc[kBlocks];
+    f32x16 acc[kBlocks];         // r = 0: dV, r = 1: dK
 #pragma unroll
-    for (int j = 0; j < kBlocks; ++j) { dkacc[j] = f32x16{0}; dvacc[j] = f32x16{0}; }
+    for (int j = 0; j < kBlocks; ++j) acc[j] = f32x16{0};
 
-    const int n_steps = min((job.len - q_begin + kStep - 1) / kStep, 2 * (last_live_row_block(p, head, job) + 1 - job.rb));
+    const int n_steps = min((job.len - q_begin + kStep - 1) / kStep, 2 * (last_live_row_block(p, head, job) + 1) - first_kb);
 
-    // waves 0-3 copy the Q tiles, waves 4-7 the dO tiles
-    TileDma<D, true> tc;
-    tc.init(lane, wave & 3, wave < 4 ? p.q : p.d_o, wave < 4 ? qbase : dobase, p.cols);
-    const int my_tile = wave < 4 ? 0 : kQTile;
-    tc.clear(lds + my_tile);
-    tc.clear(lds + 2 * kQTile + my_tile);
-    if (n_steps > 0) tc.issue(q_begin, job.len, lds + my_tile);
+    // copies of a step's Q and dO tiles: with eight waves the first four take Q and the others dO, four waves take both
+    const bool q_first = kPairs == 2 || wave < 4;
+    TileDma<D, true> tc, tc2;
+    tc.init(lane, wave & 3, q_first ? p.q : p.d_o, q_first ? qbase : dobase, p.cols);
+    if (kPairs == 2) tc2.init(lane, wave, p.d_o, dobase, p.cols);
+    const int my_tile = q_first ? 0 : kQTile;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        tc.clear(lds + b * 2 * kQTile + my_tile);
+        if (kPairs == 2) tc2.clear(lds + b * 2 * kQTile + kQTile);
+    }
+    auto issue_tiles = [&](int row0, char* tiles) __attribute__((always_inline)) {
+        tc.issue(row0, job.len, tiles + my_tile);
+        if (kPairs == 2) tc2.issue(row0, job.len, tiles + kQTile);
+    };
+    if (n_steps > 0) issue_tiles(q_begin, lds);
 
     // carries of a (query, this pair's 32 keys) pair, see the own-keys kernel
     const int kb64 = kb0 / kKeyBlock;
@@ -1729,31 +1742,22 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
     // made once, and the loop runs in two copies, one per tile buffer, so that buffer and row offsets are compile-time
     // numbers that go into the offset fields of the fetches.  (With the tile address in a scalar register each
     // fetch costs one or two vector adds with a scalar operand, 1.8 ns each: 40 of them per step.)
-    const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
-    uint32_t row_at[D / 16], nat_at[2][kBlocks], z_at[2][2];
+    uint32_t row_at[D / 16], nat_at[2][kBlocks], z_at[2];
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) row_at[ks] = lds_lane_base(lds + r * 32 * kPitch<D> * 2, lo.rows[ks]);
-    {
-        const int hh = lane >> 5, G1 = (lane >> 4) & 1, sl = lane & 15;
 #pragma unroll
-        for (int a2 = 0; a2 < 2; ++a2) {
+    for (int a2 = 0; a2 < 2; ++a2) {
 #pragma unroll
-            for (int j = 0; j < kBlocks; ++j) {
-                const int chunk = 4 * (kBlocks * half + j) + 2 * G1 + ((sl & 3) >> 1);
-                nat_at[a2][j] = lds_lane_base(lds, tile_offset<D>(8 * hh + 4 * a2 + (sl >> 2), chunk) + ((sl & 1) << 3));
-            }
-#pragma unroll
-            for (int cb = 0; cb < 2; ++cb) z_at[a2][cb] = lds_lane_base(ztile, lz.nat[a2][cb]);
-        }
+        for (int j = 0; j < kBlocks; ++j) nat_at[a2][j] = lds_lane_base(lds + (r ? 0 : kQTile), lo.nat[a2][j]);
+        z_at[a2] = lds_lane_base(ztile, r ? lz.nat[a2][1] : lz.nat[a2][0]);
     }
-    (void)lds0;
     auto rows_at = [&](uint32_t base, int imm) __attribute__((always_inline)) {
         return *(const __attribute__((address_space(3))) h16x8*)((__attribute__((address_space(3))) char*)(uintptr_t)base + imm);
     };
-    auto nat_pair = [&](const uint32_t (&at)[2][2], int col, int imm) __attribute__((always_inline)) {
+    auto transposed = [&](uint32_t at0, uint32_t at1, int imm) __attribute__((always_inline)) {
         union { s16x4 v[2]; h16x8 b; } u;
-        u.v[0] = lds_read_tr_at(at[0][col], imm);
-        u.v[1] = lds_read_tr_at(at[1][col], imm);
+        u.v[0] = lds_read_tr_at(at0, imm);
+        u.v[1] = lds_read_tr_at(at1, imm);
         return u.b;
     };
 
@@ -1769,7 +1773,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
         for (int ks = 0; ks < D / 16; ++ks) bq[ks] = rows_at(row_at[ks], kQ);
         __builtin_amdgcn_sched_barrier(0);
         if (step + 1 < n_steps) {     // next tiles, straight into the other buffer (nobody reads it since the last barrier)
-            tc.issue(q0 + kStep, job.len, lds + (buf ^ 1) * 2 * kQTile + my_tile);
+            issue_tiles(q0 + kStep, lds + (buf ^ 1) * 2 * kQTile);
             request_carries(q0 + kStep);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1791,11 +1795,11 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
                 float beta[16];
                 __builtin_amdgcn_s_setprio(3);     // paced like the two-step dQ kernel's chain: the wave behind goes first
                 {
-                    f32x16 acc = {0};
+                    f32x16 sacc = {0};
 #pragma unroll
-                    for (int ks = 0; ks < D / 16; ++ks) acc = mfma(kfr[ks], bq[ks], acc);
+                    for (int ks = 0; ks < D / 16; ++ks) sacc = mfma(kfr[ks], bq[ks], sacc);
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) x[i] = acc[i];
+                    for (int i = 0; i < 16; ++i) x[i] = sacc[i];
                 }
                 if (kb0 + 31 + strict > qt0 || qt0 + 31 >= job.len) {     // diagonal or ragged tile
 #pragma unroll
@@ -1838,19 +1842,14 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
         }
         __syncthreads();                       // the pair's weights are complete
         if (!skip) {
-            // dV += A^T dO, dK += dZ^T Q over the step's 64 queries, this wave's column blocks.  The operands of
-            // 16 queries are requested while the MFMAs of the 16 before them run (left to itself the compiler
-            // requests them right before their MFMA, which then waits for the LDS round trip: 16 per step).
-            h16x8 w[2][2], o[2][2 * kBlocks];
-            auto fetch_kk = [&](int kk, h16x8 (&ww)[2], h16x8 (&oo)[2 * kBlocks]) __attribute__((always_inline)) {
-                ww[0] = nat_pair(z_at, 0, 16 * kk * 64 * 2);
-                ww[1] = nat_pair(z_at, 1, 16 * kk * 64 * 2);
+            // dV += A^T dO (r = 0) or dK += dZ^T Q (r = 1) over the step's 64 queries.  The operands of 16 queries are
+            // requested while the MFMAs of the 16 before them run (left to itself the compiler requests them right before
+            // their MFMA, which then waits for the LDS round trip).
+            h16x8 w[2], o[2][kBlocks];
+            auto fetch_kk = [&](int kk, h16x8& ww, h16x8 (&oo)[kBlocks]) __attribute__((always_inline)) {
+                ww = transposed(z_at[0], z_at[1], 16 * kk * 64 * 2);
 #pragma unroll
-                for (int j = 0; j < kBlocks; ++j) {
-                    if (j > 0 && !both) break;
-                    oo[2 * j] = nat_pair(nat_at, j, kDO + 16 * kk * kPitch<D> * 2);
-                    oo[2 * j + 1] = nat_pair(nat_at, j, kQ + 16 * kk * kPitch<D> * 2);
-                }
+                for (int j = 0; j < kBlocks; ++j) oo[j] = transposed(nat_at[0][j], nat_at[1][j], kQ + 16 * kk * kPitch<D> * 2);
             };
             fetch_kk(0, w[0], o[0]);
 #pragma unroll
@@ -1858,11 +1857,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
                 if (kk < 3) fetch_kk(kk + 1, w[(kk + 1) & 1], o[(kk + 1) & 1]);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = 0; j < kBlocks; ++j) {
-                    if (j > 0 && !both) break;
-                    dvacc[j] = mfma(w[kk & 1][0], o[kk & 1][2 * j], dvacc[j]);
-                    dkacc[j] = mfma(w[kk & 1][1], o[kk & 1][2 * j + 1], dkacc[j]);
-                }
+                for (int j = 0; j < kBlocks; ++j) acc[j] = mfma(w[kk & 1], o[kk & 1][j], acc[j]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -1874,22 +1869,17 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dkv_pair_kernel(KPar
         if (step + 1 < n_steps) do_step(step + 1, std::integral_constant<int, 1>{});
     }
 
-    // ---- rows kb0.. of dK (scaled) and dV: each wave stages its column blocks in the pair's tile, the pair
-    // stores whole rows as coalesced 16-byte chunks
+    // ---- this wave's output, rows kb0.. of dV or of dK (scaled), staged in its share of the tiles and stored as coalesced
+    // 16-byte chunks
+    const TensorArg& out = r ? p.dk : p.dv;
+    const int64_t ob = slice_offset(out, job.seq, head, job.tok0);
+    char* const stage = lds + wave * (32 * D * 2);
 #pragma unroll
-    for (int which = 0; which < 2; ++which) {
-        const TensorArg& out = which == 0 ? p.dk : p.dv;
-        const int64_t ob = slice_offset(out, job.seq, head, job.tok0);
-#pragma unroll
-        for (int j = 0; j < kBlocks; ++j)
-            if (j == 0 || both) stage_acc_tile<D>(ztile, 0, 32 * (kBlocks * half + j), which == 0 ? dkacc[j] : dvacc[j], which == 0 ? p.scale : 1.0f, lane);
-        __syncthreads();
-        for (int c = lane + 64 * r; c < 32 * D / 8; c += 128) {
-            const int row = c / (D / 8), cc = c % (D / 8);
-            if (kb0 + row < job.len && (D != 96 || cc * 8 < p.cols))
-                *(u32x4*)(out.ptr + 2 * (ob + (int64_t)(kb0 + row) * out.st + cc * 8)) = *(const u32x4*)(ztile + row * (D * 2) + cc * 16);
-        }
-        __syncthreads();
+    for (int j = 0; j < kBlocks; ++j) stage_acc_tile<D>(stage, 0, 32 * j, acc[j], r ? p.scale : 1.0f, lane);
+    for (int c = lane; c < 32 * D / 8; c += 64) {
+        const int row = c / (D / 8), cc = c % (D / 8);
+        if (kb0 + row < job.len && (D != 96 || cc * 8 < p.cols))
+            *(u32x4*)(out.ptr + 2 * (ob + (int64_t)(kb0 + row) * out.st + cc * 8)) = *(const u32x4*)(stage + row * (D * 2) + cc * 16);
     }
 }
 
@@ -1904,7 +1894,7 @@ bool sba_mfma_bwd_available() { return true; }
 // both on the same inputs).
 static bool own_keys_kernel(bool by_size) {
     const char* e = getenv("SBA_DKV_KERNEL");
-    if (e && (!strcmp(e, "own") || !strcmp(e, "pair"))) return true;
+    if (e && (!strcmp(e, "own") || !strcmp(e, "pair") || !strcmp(e, "pair4"))) return true;
     if (e && !strcmp(e, "other")) return false;
     return by_size;
 }
@@ -1946,7 +1936,7 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     //     longer, packs  r 0.7-1.7 1.07-1.22, 2.4 1.09, 3.2 1.02-1.03 and (H=2) 0.90, 3.3 0.96, 3.9 0.97
     // Batches of short sequences (sweeps of at most 16 steps) also take the own-keys kernel at any size: on 512 workgroups B=8,
     // T=512 takes 27.3 us against the stream's 33.0, B=4, T=1024 44.0 against 45.3.
-    // head_dim 128: the paired kernel at every size (on 64 ... 256 workgroups of B=1, H=16 it takes 27 / 44 / 62 / 81 us where the
+    // head_dim 128: the paired kernel at every size (B=1, H=16, T=512 ... 2048: with four pairs 27 / 44 / 62 / 81 us where the
     // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103); SBA_DKV_KERNEL=other still selects that one.
     const unsigned cus = (unsigned)sba_cu_count();
     const bool short_sweeps = kp.seq_len <= 8 * kRowBlock && grid.x >= 2u * cus;
@@ -1959,6 +1949,12 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     const bool stream8 = which && !strcmp(which, "stream8");
     // the scaled copy of q is for the stream kernel: no other key-owner kernel reads it, so the dQ pass skips it
     const bool stream = kp.head_dim == 64 && !plain && !own;
+    // Paired kernel: workgroups of two pairs, two a CU, but for launches of short sweeps that do not fill the chip with them, where the
+    // prologue counts.  Forward + backward with two pairs over the same with four, d=128 / 96:  T=300 B=16 1.04 / 1.03,
+    // T=512 B=2 1.06 / 1.00, B=4 1.04 / 0.99, B=8 (512 row blocks) 1.05 / 1.05, B=16 (1024) 1.00 / 1.00;  T=640 B=4 1.00 / 0.98;
+    // T=768 B=2 0.93 / 0.945;  T=1024 B=1 0.88, B=2 0.95 / 0.95, B=8 0.98 / 1.00;  T=4096 0.97;  packs of documents of at most 512 tokens 0.95
+    // (65536 tokens), 256 0.98 (16384).
+    const bool four_pairs = which && !strncmp(which, "pair", 4) ? !strcmp(which, "pair4") : kp.seq_len <= 4 * kRowBlock && grid.x < 4u * cus;
     if (stream && !kp.q_scaled.ptr) return SBA_ERR_WORKSPACE;
     if (!stream) kp.q_scaled.ptr = nullptr;
     // Sequences of at most 128 tokens: one kernel for both passes (it all runs in phase 1).  A kernel asked for by name is one of
@@ -2009,7 +2005,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     } else if (kp.head_dim == 96) {
         if (p1 && kp.makes_mid) hipLaunchKernelGGL((mfma_bwd_dq_kernel<96, false, true>), grid, dim3(kThreads), 0, s, kp);
         else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<96>), grid, dim3(kThreads), 0, s, kp);
-        if (p2) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<96>), grid, dim3(2 * kThreads), 0, s, kp);
+        if (p2 && four_pairs) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<96, 4>), grid, dim3(2 * kThreads), 0, s, kp);
+        else if (p2) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<96, 2>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
     } else if (kp.head_dim == 256) {
         // one wave per SIMD in both passes; every wave of the key-owner pass on its own 32 keys, two workgroups per
         // key block that each accumulate one half of the columns of dK and dV - the other key-owner kernels do not
@@ -2024,7 +2021,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         // key owners at head_dim 128: two waves per 32 keys (6-9 % faster than one wave per 32 keys,
         // which SBA_DKV_KERNEL=own still selects)
         const bool pair = !(which && !strcmp(which, "own"));
-        if (p2 && own && pair) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<128>), grid, dim3(2 * kThreads), 0, s, kp);
+        if (p2 && own && pair && four_pairs) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<128, 4>), grid, dim3(2 * kThreads), 0, s, kp);
+        else if (p2 && own && pair) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<128, 2>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
         else if (p2 && own) hipLaunchKernelGGL((mfma_bwd_dkv_own_kernel<128>), grid, dim3(kThreads), 0, s, kp);
         else if (p2) hipLaunchKernelGGL((mfma_bwd_dkv_kernel<128>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
     }
