@@ -9,7 +9,7 @@ namespace sba_model {
 
 constexpr int kMaxNormWidth = 2048;      // columns of a row that a wave keeps in registers
 constexpr int kCastTensors = 8;
-constexpr int kOptChunk = 16384;         // weights that one workgroup of the optimizer kernels takes
+constexpr int kOptChunk = 16384;         // weights to a partial sum of squares
 
 // y = rms_norm(x) * w as 16-bit
 struct NormFwd {
