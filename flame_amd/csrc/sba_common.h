@@ -65,6 +65,9 @@ struct KParams {
     int makes_mid;                 // dQ pass: rmid is not there yet (SBA_SAVE_ONE_TABLE)
     int early_end;                 // forward sweeps end once nothing is left of any of their rows' sticks
     int* gave_up;                  // backward error word (set if a kernel abandoned a bounded internal wait)
+    int* queue;                    // where the launch's workgroups draw their jobs, see draw_jobs(): queue i's counter lies i strides further
+    int64_t queue_stride;
+    int queue_blocks;              // jobs of such a launch
     int64_t tab_head_stride;       // floats per head in each carry table
     int64_t tab_tokens;            // tokens per head in dkv32 and halves (n_seq*T dense, sumT packed)
 };
@@ -106,12 +109,16 @@ struct Job { int tok0, len, rb, seq, tab0; };
 // a slot in the same orders:  H=16 T=4096 0.99 / 0.98 0.99 / 0.97     H=16 T=5000 0.98 / 0.97 1.00 / 0.99     H=8 T=7000 0.98 / 1.01 1.00 / 0.97
 //     H=32 T=1800 1.00 / 1.00 0.99 / 0.97     H=12 T=3000, H=16 T=3500 1.00 / 1.00 / 1.00, 0.99
 // With fewer than eight heads they turn every slot (H=4 T=12000 would be 1.04).
-enum Sharing { kOnePerCu, kSharedCu, kStreamItems };
+// Launches that draw their jobs (draw_jobs()) turn by one head in eight slots: an XCD that is through early takes jobs of the others, and
+// the turn by slots costs the L2 more than the unequal heads do.  Forward + backward, turn by slots / by eighths / fixed heads over the launch that
+// does not draw, heads in order / in a random one / all at -6:  H=16 T=16384 d=128 0.959 0.933 0.952 / 0.957 0.930 0.981 / 0.992 0.964 0.964
+//     T=8192 0.987 1.010 1.044 / 0.994 1.003 1.011 / 0.987 0.946 0.935     packs of 65536 tokens d=80 0.964 0.959 0.984 / 0.963 0.986 0.979 / 0.983 0.979 0.971
+enum Sharing { kOnePerCu, kSharedCu, kStreamItems, kDrawn };
 template <Sharing kSharing = kOnePerCu>
 __device__ inline int head_of_block(const KParams& p, int block) {
     const int slot = divided(block, p.heads);
     int turn = slot;
-    if (p.cu_seqlens) turn = slot >> 3;
+    if (p.cu_seqlens || kSharing == kDrawn) turn = slot >> 3;
     else if (kSharing == kStreamItems && p.n_heads >= 8) turn = slot >> 4;
     if (kSharing == kSharedCu && p.spread) {
         const int round = divided(slot * p.n_heads, p.cus), of_round = slot - divided(round * p.n_cus + p.n_heads - 1, p.heads);
@@ -246,6 +253,71 @@ __device__ inline void close_live_ranges(const KParams& p, int head, const Job& 
     }
 }
 
+// Workgroups that draw their jobs.  The dispatcher deals workgroups to the XCDs in turn and in order: where one XCD has no room for its
+// next one, all others wait.  With sweeps of unequal lengths a fifth of the chip's slots is empty from the first round to the last.  So a
+// launch of many rounds has as many workgroups as the chip holds, which draw their jobs: job i belongs to queue i % 8 and workgroups draw from
+// the queue of their own XCD, whose L2 holds the heads of its jobs, and, once that is empty, from the next one that is not.
+// A queue is a counter of the jobs taken beyond the first round, which are dealt out by index.  The counters lie in the tables, behind the words
+// of live_index() of eight row blocks: the forward's in rtab, the two backward passes' in gtab.
+constexpr int kQueues = 8, kForwardQueue = 32, kDqQueue = 32, kKeyQueue = 48;       // entries of live_index()'s column
+__device__ inline int queued_block(int queue, int ticket) { return queue + kQueues * (ticket + (int)gridDim.x / kQueues); }
+__device__ inline int* queue_counter(const KParams& p, int queue) { return p.queue + queue * p.queue_stride; }
+__device__ inline int take_ticket(const KParams& p, int queue) {
+    return __hip_atomic_fetch_add(queue_counter(p, queue), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline int lane_index() { return __builtin_amdgcn_mbcnt_hi(-1, __builtin_amdgcn_mbcnt_lo(-1, 0)); }
+// (first wave) the job of the ticket that lane 0 took from its home queue, or one from another queue that has some left, or -1.  Counters
+// only grow, so the search ends.
+__device__ inline int drawn_block(const KParams& p, int home, int ticket, int lane) {
+    int block = queued_block(home, __builtin_amdgcn_readfirstlane(ticket));
+    while (block >= p.queue_blocks) {
+        const int queue = (home + lane) & (kQueues - 1);
+        const int next = queued_block(queue, __hip_atomic_load(queue_counter(p, queue), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        const uint64_t left = __builtin_amdgcn_ballot_w64(lane < kQueues && next < p.queue_blocks);
+        if (!left) return -1;
+        const int other = (home + __builtin_ctzll(left)) & (kQueues - 1);
+        block = queued_block(other, __builtin_amdgcn_readfirstlane(lane == 0 ? take_ticket(p, other) : 0));
+    }
+    return block;
+}
+// Runs run(parameters, block, wave, lane, draw) for the workgroup's jobs.  Parameters and lane are given as if they were others each time, so
+// that nothing computed from them stays in registers from job to job (without this the forward at head_dim 64 takes 165 registers in place of
+// 124).  A job calls draw() behind its last step: the ticket is on its way while the results are stored.  (Asked for before the job, it
+// would be bound to the end of a long sweep while others find no work: 8192-token packs 1.15 of the time.)
+// words: two ints of LDS that a job does not use behind its last barrier.
+template <class Run>
+__device__ __forceinline__ void draw_jobs(int* words, Run&& run) {
+    typedef const __attribute__((address_space(4))) KParams* Arguments;
+    int block = blockIdx.x;
+    const int home = block & (kQueues - 1);
+    int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int parity = 0;; parity ^= 1) {
+        Arguments args = (Arguments)__builtin_amdgcn_kernarg_segment_ptr();
+        int lane = lane_index();
+        asm volatile("" : "+s"(args), "+v"(lane), "+s"(wave));
+        __builtin_assume(lane >= 0 && lane < 64);
+        const KParams& p = *(const KParams*)args;
+        int ticket = 0;
+        run(p, block, wave, lane, [&]() __attribute__((always_inline)) {
+            if (wave == 0 && lane_index() == 0) ticket = take_ticket(p, home);
+        });
+        if (wave == 0) {
+            const int l = lane_index();
+            const int next = drawn_block(p, home, ticket, l);
+            if (l == 0) words[parity] = next;
+        }
+        __syncthreads();                       // (everybody is through with this job's LDS, too)
+        block = __builtin_amdgcn_readfirstlane(words[parity]);
+        if (block < 0) return;
+    }
+}
+// In front of a dQ pass that draws its jobs, or of a key-owner pass by itself: the dQ pass clears the key owners' queues.
+__global__ static void clear_queues_kernel(int* queue, int64_t stride) { queue[threadIdx.x * stride] = 0; }
+__device__ inline void clear_words(const KParams& p, int lane) {
+    if (lane == 0 && p.gave_up) *p.gave_up = 0;
+    if (lane < kQueues && p.queue_stride) ((int*)p.gtab)[kRowBlock + kKeyQueue + lane * p.queue_stride] = 0;
+}
+
 __device__ inline float bf16_to_f32(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
 __device__ inline uint16_t f32_to_bf16(float f) {   // round to nearest even
     uint32_t u = __float_as_uint(f);
@@ -326,6 +398,47 @@ inline sba::KParams sba_turning(const sba::KParams& kp, int resident, int per_jo
     const int64_t cus = sba_cu_count(), per = (int64_t)kp.n_heads * per_job, grid = kp.n_jobs * per, round = cus / per;
     if (!kp.cu_seqlens && grid > cus && grid <= resident * cus && round > kp.n_seq && kp.n_jobs % round == 0) r.turn = (int)round;
     return r;
+}
+
+// Distance of the eight queues' counters: they are in eight heads' or eight sequences' first row blocks (0: there are not so many).
+inline int64_t sba_queue_stride(const sba::KParams& kp) {
+    if (kp.n_heads >= sba::kQueues) return kp.tab_head_stride;
+    return !kp.cu_seqlens && kp.n_seq >= sba::kQueues ? kp.tab_head_stride / kp.n_seq : 0;
+}
+// Whether a pass of a 16-bit launch draws its jobs.  Forward + backward over the same with a workgroup per job, mean logits 0 .. -6 over the heads in
+// order / in a random one / all at -6; work = carry-table columns (64-key steps of all sweeps) x heads:
+//     head dims 72 to 128, all three passes   H=16 d=128 T=16384 (work 264000) 0.91 / 0.93 / 0.94, T=12000 0.92 / 0.92 / 0.93, T=8192 (67000) 0.98 / 0.97 / 0.92,
+//         H=32 T=8192 0.90 / 0.93 / 0.93, B=2 H=8 T=16384 0.925 / 0.81 / 0.97, B=4 T=4096 (68000) 0.97 / 0.99 / 1.01, B=16 T=4096 0.96 / 0.97 / 0.97;
+//         d=80 T=16384 0.93 / 0.94 / 0.94, B=8 H=12 T=4096 0.965 / 0.98 / 1.00;  packs  65536 tokens d=128 0.96 / 0.97 / 0.99, d=80 0.96 / 0.97 / 0.99, documents up
+//         to 16384 0.915 / 0.94 / 0.98, up to 1024 d=96 0.99 / 0.98 / 0.97, 32768 tokens 1.00 / 0.98 / 1.01;  below the line B=8 T=2048 (35000) 1.01 / 1.03 / 1.015
+//     head_dim 64, the backward's two passes (the forward's, of which a CU holds four, gains nothing)   packs  65536 tokens 0.97 / 1.00 / 1.00, H=32 0.94 / 0.95 / 0.98,
+//         131072 tokens 0.96 / 0.96 / 0.98, documents up to 16384 0.94 / 0.94 / 0.97, up to 1024 0.99 / 1.00 / 0.98;  B=16 H=16 T=4096 0.98 / 0.98 / 0.98, B=4
+//         T=16384 0.97 / 0.98 / 0.99;  below the line B=4 T=4096 (2048 workgroups) 1.03 / 1.03 / 1.03
+// Short sweeps lose by it: documents up to 256 tokens 1.02 to 1.03 for the forward and the dQ pass at head_dim 64.
+// SBA_DRAW=1 / =0 (experiments and tests): wherever there are more jobs than the chip holds workgroups, or nowhere.
+inline bool sba_draws(const sba::KParams& kp, unsigned blocks, unsigned slots) {
+    if (!kp.queue_stride || slots == 0 || blocks <= slots) return false;
+    const char* e = getenv("SBA_DRAW");
+    if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
+    const int64_t grid = (int64_t)kp.n_jobs * kp.n_heads, columns = kp.tab_head_stride / sba::kRowBlock, mean_sweep = columns / kp.n_jobs;
+    return kp.head_dim == 64 ? grid >= SBA_DOC_MAJOR_GRID && mean_sweep >= 8 : columns * kp.n_heads >= 60000 && mean_sweep >= 4;
+}
+// Launches `drawing` with `resident` workgroups a CU where that pays, else `plain` with a workgroup per job.  table, entry: where its queues lie
+// (null: nowhere).
+template <class Kernel>
+inline void sba_launch_drawing(Kernel plain, Kernel drawing, unsigned blocks, int threads, int resident, const sba::KParams& kp, float* table, int entry,
+                               bool cleared, hipStream_t s) {
+    const unsigned slots = (unsigned)(resident * kp.n_cus) & ~(unsigned)(sba::kQueues - 1);
+    if (!table || !sba_draws(kp, blocks, slots)) {
+        hipLaunchKernelGGL(plain, dim3(blocks), dim3(threads), 0, s, kp);
+        return;
+    }
+    sba::KParams r = kp;
+    r.queue = (int*)table + sba::kRowBlock + entry;
+    r.queue_blocks = (int)blocks;
+    r.turn = 0;
+    if (!cleared) hipLaunchKernelGGL(sba::clear_queues_kernel, dim3(1), dim3(sba::kQueues), 0, s, r.queue, r.queue_stride);
+    hipLaunchKernelGGL(drawing, dim3(slots), dim3(threads), 0, s, r);
 }
 
 // Launchers implemented in the kernel translation units.

@@ -49,20 +49,18 @@ __device__ inline void store_scaled_q(const KParams& p, const Job& job, int head
 // -6 %); on launches that last as long as their longest sweep the plain arrangement's shorter step is ahead.
 // kMid: the forward kept `rtab` alone (KParams::makes_mid).  The left half-wave starts its chain from 1, the right half-wave's product
 // completes it, and is the entry of `rmid`: 32 multiplications a step.
-template <int D, bool kLean = false, bool kMid = false>
-__global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 1)) void mfma_bwd_dq_kernel(KParams p) {
+template <int D, bool kLean, bool kMid, Sharing kSharing, class Draw>
+__device__ __forceinline__ void dq_job(const KParams& p, const int block, const int wave, const int lane, Draw draw) {
     static_assert(!kMid || kWide<D> || kLean, "the arrangement that takes the carry into g alone");
     constexpr int kTile = 64 * kPitch<D> * 2;
     __shared__ __attribute__((aligned(16))) char lds[4 * kTile];   // K0 V0 K1 V1
 
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform, keep it scalar
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
     lo.rebase(lds);                        // absolute addresses: the loop below runs in one copy per tile buffer
-    const int head = head_of_block<D <= 128 ? kSharedCu : kOnePerCu>(p, blockIdx.x);
-    const Job job = decode_job<D == 64>(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
+    const int head = head_of_block<kSharing>(p, block);
+    const Job job = decode_job<D == 64>(p, order_job(slot_of_block(p, block), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * wave;
@@ -73,7 +71,7 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
     const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
     const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
 
-    if (blockIdx.x == 0 && threadIdx.x == 0 && p.gave_up) *p.gave_up = 0;     // error word of the launch pair, see wait_for_count()
+    if (block == 0 && wave == 0) clear_words(p, lane);     // error word of the launch pair, see wait_for_count(), and the second one's queues
     h16x8 qf[D / 16], dof[D / 16];
     load_row_frags<D>(qf, p.q, qbase, q0w, n, job.len, lane, p.cols);
     prescale_frags(qf, p.scale2);          // the score MFMAs then deliver base-2 logits
@@ -232,9 +230,21 @@ __global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 
         if (step + 1 < n_steps) do_step(step + 1, std::integral_constant<int, 1>{});
     }
     store_prefixes();
+    draw();
 
     store_query_rows<D>(lds + wave * kRowStage<D>, dqacc, p.scale, p.dq,                 // (the tiles are free)
                         slice_offset(p.dq, job.seq, head, job.tok0), q0w, job.len, lane, p.cols);
+}
+
+template <int D, bool kLean = false, bool kMid = false>
+__global__ __launch_bounds__(kThreads, (D == 64 && kLean) ? 3 : (D <= 128 ? 2 : 1)) void mfma_bwd_dq_kernel(KParams p) {
+    dq_job<D, kLean, kMid, D <= 128 ? kSharedCu : kOnePerCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {});
+}
+
+template <int D, bool kLean, bool kMid>
+__global__ __launch_bounds__(kThreads, kLean ? 3 : 2) void mfma_bwd_dq_drawing_kernel(KParams) {
+    __shared__ int words[2];
+    draw_jobs(words, [&](const KParams& p, int block, int wave, int lane, auto draw) { dq_job<D, kLean, kMid, kDrawn>(p, block, wave, lane, draw); });
 }
 
 // ---------------------------------------------------------------- pass 1, two steps per iteration
@@ -272,7 +282,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void mfma_bwd_dq2_kernel(KParams p
     const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
     const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
 
-    if (blockIdx.x == 0 && threadIdx.x == 0 && p.gave_up) *p.gave_up = 0;     // error word of the launch pair, see wait_for_count()
+    if (blockIdx.x == 0 && wave == 0) clear_words(p, lane);     // as in mfma_bwd_dq_kernel
     h16x8 qf[D / 16], dof[D / 16];
     load_row_frags<D>(qf, p.q, qbase, q0w, n, job.len, lane);
     prescale_frags(qf, p.scale2);          // the score MFMAs then deliver base-2 logits
@@ -1169,8 +1179,8 @@ __global__ __launch_bounds__((NP + 4) * 64, NP == 4 ? 2 : 3) void mfma_bwd_dkv_s
 // for the K and V fragments.  There the grid has kSplit = 2 workgroups per (key block, head), blockIdx.y = 0, 1, and
 // workgroup `part` accumulates and stores columns 128 * part .. 128 * part + 127 of dK and dV only; scores, weights and
 // logit gradients are formed in both.
-template <int D, int kSplit = 1>
-__global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_kernel(KParams p) {
+template <int D, int kSplit, Sharing kSharing, class Draw>
+__device__ __forceinline__ void own_keys_job(const KParams& p, const int block, const int wave, const int lane, Draw draw) {
     constexpr int kNB = D / 32 / kSplit;         // 32-wide column blocks of dK / dV accumulated here
     const int part = kSplit > 1 ? (int)blockIdx.y : 0;
     static_assert(32 * (D / kSplit) * 2 <= 64 * 64 * 2, "a wave stages its [32 keys x columns] outputs in its weight tile");
@@ -1187,15 +1197,13 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
     constexpr int kNBuf = kDefer ? 3 : 2;
     __shared__ __attribute__((aligned(16))) char lds[2 * kNBuf * kQTile + 4 * kZTile];   // Q, dO per buffer | one Z tile per wave
 
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
     LaneOffsets<64> lz;
     lz.init(lane);
-    const int head = head_of_block<D == 64 ? kSharedCu : kOnePerCu>(p, blockIdx.x);
-    const Job job = decode_key_job<D == 64>(p, slot_of_block(p, blockIdx.x));
+    const int head = head_of_block<kSharing>(p, block);
+    const Job job = decode_key_job<D == 64>(p, slot_of_block(p, block));
     const int strict = p.attend_current ? 0 : 1;
     const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it
     const int kb0 = q_begin + 32 * wave;               // first key of this wave
@@ -1432,6 +1440,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
         else second_tile_reduction(TileAt{(kNBuf - 1) * 2 * kQTile}, TileAt{(kNBuf - 1) * 2 * kQTile + kQTile});
     }
 
+    draw();
     // ---- rows kb0.. of dK (scaled) and dV, through the wave's own tile as coalesced 16-byte stores
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
@@ -1447,6 +1456,17 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_ke
                 *(u32x4*)(out.ptr + 2 * (ob + (int64_t)(kb0 + row) * out.st + part * kCols + cc * 8)) = *(const u32x4*)(ztile + row * (kCols * 2) + cc * 16);
         }
     }
+}
+
+template <int D, int kSplit = 1>
+__global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_kernel(KParams p) {
+    own_keys_job<D, kSplit, D == 64 ? kSharedCu : kOnePerCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {});
+}
+
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void mfma_bwd_dkv_own_drawing_kernel(KParams) {
+    __shared__ int words[2];
+    draw_jobs(words, [&](const KParams& p, int block, int wave, int lane, auto draw) { own_keys_job<D, 1, kDrawn>(p, block, wave, lane, draw); });
 }
 
 
@@ -1652,17 +1672,14 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
 // that two of them share a CU and one's barriers and round trips pass under the other's work, and the diagonal and the end of a
 // sequence are cut off by 64 keys.  Against one workgroup of kPairs = 4 a CU (128 keys, eight waves, half the tile copies):
 // B=4 H=16 T=2047 d=128 181 -> 163 us, B=1 H=16 T=16384 1690 -> 1530, d = 80 as above 249 -> 213.
-template <int D, int kPairs>
-__global__ __launch_bounds__(128 * kPairs, 2) void mfma_bwd_dkv_pair_kernel(KParams p) {
+template <int D, int kPairs, Sharing kSharing, class Draw>
+__device__ __forceinline__ void paired_keys_job(const KParams& p, const int block, const int wave, const int lane, Draw draw, char* const lds) {
     constexpr int kQTile = 64 * kPitch<D> * 2;           // Q or dO tile of one step (64 queries)
     constexpr int kZTile = 64 * 64 * 2;          // per pair: [64 queries][32 a | 32 dz] bf16
     constexpr int kStep = 64;
     constexpr int kBlocks = D / 32;              // 32-wide column blocks of dK or dV
     static_assert(2 * kPairs * 32 * D * 2 <= 4 * kQTile, "every wave stages its [32 keys x D] output in the tiles");
-    __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + kPairs * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
 
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = wave >> 1, r = wave & 1;
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
@@ -1670,13 +1687,16 @@ __global__ __launch_bounds__(128 * kPairs, 2) void mfma_bwd_dkv_pair_kernel(KPar
     LaneOffsets<64> lz;
     lz.init(lane);
     constexpr int kParts = 4 / kPairs;                 // workgroups of a scheduled 128-row job
-    const int slot = slot_of_block(p, blockIdx.x);
-    const int head = head_of_block<kPairs == 4 ? kOnePerCu : kSharedCu>(p, blockIdx.x);
+    const int slot = slot_of_block(p, block);
+    const int head = head_of_block<kSharing>(p, block);
     const Job job = decode_key_job(p, slot / kParts);
     const int strict = p.attend_current ? 0 : 1;
     const int first_kb = 2 * job.rb + slot % kParts;   // first 64-key block of the workgroup's keys
     const int q_begin = first_kb * kKeyBlock;          // first key = first query that may see it
-    if (q_begin >= job.len) return;
+    if (q_begin >= job.len) {
+        draw();
+        return;
+    }
     const int kb0 = q_begin + 32 * grp;                // first key of this pair
     char* ztile = lds + 4 * kQTile + grp * kZTile;
 
@@ -1869,6 +1889,7 @@ __global__ __launch_bounds__(128 * kPairs, 2) void mfma_bwd_dkv_pair_kernel(KPar
         if (step + 1 < n_steps) do_step(step + 1, std::integral_constant<int, 1>{});
     }
 
+    draw();
     // ---- this wave's output, rows kb0.. of dV or of dK (scaled), staged in its share of the tiles and stored as coalesced
     // 16-byte chunks
     const TensorArg& out = r ? p.dk : p.dv;
@@ -1881,6 +1902,20 @@ __global__ __launch_bounds__(128 * kPairs, 2) void mfma_bwd_dkv_pair_kernel(KPar
         if (kb0 + row < job.len && (D != 96 || cc * 8 < p.cols))
             *(u32x4*)(out.ptr + 2 * (ob + (int64_t)(kb0 + row) * out.st + cc * 8)) = *(const u32x4*)(stage + row * (D * 2) + cc * 16);
     }
+}
+
+template <int D, int kPairs>
+__global__ __launch_bounds__(128 * kPairs, 2) void mfma_bwd_dkv_pair_kernel(KParams p) {
+    constexpr int kQTile = 64 * kPitch<D> * 2, kZTile = 64 * 64 * 2;
+    __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + kPairs * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
+    paired_keys_job<D, kPairs, kPairs == 4 ? kOnePerCu : kSharedCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {}, lds);
+}
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void mfma_bwd_dkv_pair_drawing_kernel(KParams) {
+    constexpr int kQTile = 64 * kPitch<D> * 2, kZTile = 64 * 64 * 2;
+    __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + 2 * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
+    draw_jobs((int*)(lds + 4 * kQTile), [&](const KParams& p, int block, int wave, int lane, auto draw) { paired_keys_job<D, 2, kDrawn>(p, block, wave, lane, draw, lds); });
 }
 
 }  // inline namespace SBA_ELEM_NS
@@ -1917,6 +1952,7 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     KParams kp = kp_in;
     dim3 grid((unsigned)kp.n_jobs * kp.n_heads);
     const bool p1 = phases != 2, p2 = phases != 1;
+    kp.queue_stride = sba_queue_stride(kp);
     // the dQ kernels reach a lane's prefix entry from its carry entry by one uniform distance (see there)
     if (!kp.rtab || !kp.rmid || !kp.gtab || !kp.gmid) return SBA_ERR_WORKSPACE;
     if (!kp.makes_mid && (const char*)kp.gmid - (const char*)kp.rtab != (const char*)kp.gtab - (const char*)kp.rmid) return SBA_ERR_WORKSPACE;
@@ -1977,7 +2013,7 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         // 23.8 us with one step per iteration against 27.4, B=4, T=1024 36.0 against 37.7).
         const bool two_steps = sba_two_step_env() >= 0 ? grid.x <= (unsigned)sba_two_step_env()
                                                        : grid.x <= kTwoStepDqMaxGrid && sba_tail_ratio(kp, grid.x) >= 3.7;
-        if (p1 && kp.makes_mid) hipLaunchKernelGGL((mfma_bwd_dq_kernel<64, true, true>), grid, dim3(kThreads), 0, s, sba_turning(kp, 3));
+        if (p1 && kp.makes_mid) sba_launch_drawing((mfma_bwd_dq_kernel<64, true, true>), (mfma_bwd_dq_drawing_kernel<64, true, true>), grid.x, kThreads, 3, sba_turning(kp, 3), kp.gtab, kDqQueue, false, s);
         else if (p1 && two_steps) hipLaunchKernelGGL((mfma_bwd_dq2_kernel<64>), grid, dim3(2 * kThreads), 0, s, kp);
         // The register-lean arrangement (three waves per SIMD) from five workgroups per CU on, unless the launch hangs on
         // one long sweep (tail ratio above 2.5: there the plain arrangement's shorter step is ahead, e.g. 111 against 118 us
@@ -1987,12 +2023,12 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         // and 865; from T=14000 on 0.99-1.02); on packs 0.96-1.00.  At four workgroups per CU (six shapes of 1024 workgroups) the
         // plain one is ahead by 1-3 %.
         else if (p1 && lean_dq_kernel(grid.x >= 8u * cus || (grid.x >= 5u * cus && sba_tail_ratio(kp, grid.x) <= 2.5)))
-            hipLaunchKernelGGL((mfma_bwd_dq_kernel<64, true>), grid, dim3(kThreads), 0, s, sba_turning(kp, 3));
+            sba_launch_drawing((mfma_bwd_dq_kernel<64, true>), (mfma_bwd_dq_drawing_kernel<64, true, false>), grid.x, kThreads, 3, sba_turning(kp, 3), kp.gtab, kDqQueue, false, s);
         else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<64>), grid, dim3(kThreads), 0, s, sba_turning(kp, 2));
         if (p2 && plain) {
             hipLaunchKernelGGL((mfma_bwd_dkv_kernel<64>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
         } else if (p2 && own) {
-            hipLaunchKernelGGL((mfma_bwd_dkv_own_kernel<64>), grid, dim3(kThreads), 0, s, sba_turning(kp, 2));
+            sba_launch_drawing((mfma_bwd_dkv_own_kernel<64>), (mfma_bwd_dkv_own_drawing_kernel<64>), grid.x, kThreads, 2, sba_turning(kp, 2), kp.gtab, kKeyQueue, p1, s);
         } else if (p2) {
             // one resident workgroup per CU, in whole rounds of the 8 XCDs (surplus workgroups
             // find no item)
@@ -2003,10 +2039,10 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
             else hipLaunchKernelGGL((mfma_bwd_dkv_stream_kernel<64, 4>), dim3(n_wg), dim3(8 * 64), 0, s, kp);
         }
     } else if (kp.head_dim == 96) {
-        if (p1 && kp.makes_mid) hipLaunchKernelGGL((mfma_bwd_dq_kernel<96, false, true>), grid, dim3(kThreads), 0, s, kp);
-        else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<96>), grid, dim3(kThreads), 0, s, kp);
+        if (p1 && kp.makes_mid) sba_launch_drawing((mfma_bwd_dq_kernel<96, false, true>), (mfma_bwd_dq_drawing_kernel<96, false, true>), grid.x, kThreads, 2, kp, kp.gtab, kDqQueue, false, s);
+        else if (p1) sba_launch_drawing((mfma_bwd_dq_kernel<96>), (mfma_bwd_dq_drawing_kernel<96, false, false>), grid.x, kThreads, 2, kp, kp.gtab, kDqQueue, false, s);
         if (p2 && four_pairs) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<96, 4>), grid, dim3(2 * kThreads), 0, s, kp);
-        else if (p2) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<96, 2>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
+        else if (p2) sba_launch_drawing((mfma_bwd_dkv_pair_kernel<96, 2>), (mfma_bwd_dkv_pair_drawing_kernel<96>), 2 * grid.x, kThreads, 2, kp, kp.gtab, kKeyQueue, p1, s);
     } else if (kp.head_dim == 256) {
         // one wave per SIMD in both passes; every wave of the key-owner pass on its own 32 keys, two workgroups per
         // key block that each accumulate one half of the columns of dK and dV - the other key-owner kernels do not
@@ -2016,13 +2052,13 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
             hipLaunchKernelGGL((mfma_bwd_dkv_own_kernel<256, 2>), dim3(grid.x, 2), dim3(kThreads), 0, s, kp);
         }
     } else {
-        if (p1 && kp.makes_mid) hipLaunchKernelGGL((mfma_bwd_dq_kernel<128, false, true>), grid, dim3(kThreads), 0, s, kp);
-        else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<128>), grid, dim3(kThreads), 0, s, kp);
+        if (p1 && kp.makes_mid) sba_launch_drawing((mfma_bwd_dq_kernel<128, false, true>), (mfma_bwd_dq_drawing_kernel<128, false, true>), grid.x, kThreads, 2, kp, kp.gtab, kDqQueue, false, s);
+        else if (p1) sba_launch_drawing((mfma_bwd_dq_kernel<128>), (mfma_bwd_dq_drawing_kernel<128, false, false>), grid.x, kThreads, 2, kp, kp.gtab, kDqQueue, false, s);
         // key owners at head_dim 128: two waves per 32 keys (6-9 % faster than one wave per 32 keys,
         // which SBA_DKV_KERNEL=own still selects)
         const bool pair = !(which && !strcmp(which, "own"));
         if (p2 && own && pair && four_pairs) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<128, 4>), grid, dim3(2 * kThreads), 0, s, kp);
-        else if (p2 && own && pair) hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<128, 2>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
+        else if (p2 && own && pair) sba_launch_drawing((mfma_bwd_dkv_pair_kernel<128, 2>), (mfma_bwd_dkv_pair_drawing_kernel<128>), 2 * grid.x, kThreads, 2, kp, kp.gtab, kKeyQueue, p1, s);
         else if (p2 && own) hipLaunchKernelGGL((mfma_bwd_dkv_own_kernel<128>), grid, dim3(kThreads), 0, s, kp);
         else if (p2) hipLaunchKernelGGL((mfma_bwd_dkv_kernel<128>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
     }

@@ -58,19 +58,17 @@ __device__ inline void store_o_rows(char* stage, const KParams& p, const Job& jo
 
 // kCarryOnly: write the carry table and nothing else (no P*V, no o / rem): the backward's way of
 // getting the table when the forward kept none.
-template <int D, bool kCarryOnly>
-__global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
+template <int D, bool kCarryOnly, Sharing kSharing, class Draw>
+__device__ __forceinline__ void fwd_job(const KParams& p, const int block, const int wave, const int lane, Draw draw) {
     constexpr int kTile = 64 * kPitch<D> * 2;            // bytes per K or V tile
     __shared__ __attribute__((aligned(16))) char lds[4 * kTile + (kCarryOnly ? 0 : 32)];   // K0 V0 K1 V1 | words
     int (*const done_waves)[4] = (int (*)[4])(lds + (kCarryOnly ? kTile : 4 * kTile));     // [parity of the step][wave]
 
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform, keep it scalar
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
-    const int head = head_of_block<kSharedCu>(p, blockIdx.x);
-    const Job job = decode_job<D == 64>(p, order_job(slot_of_block(p, blockIdx.x), p.n_jobs, false));
+    const int head = head_of_block<kSharing>(p, block);
+    const Job job = decode_job<D == 64>(p, order_job(slot_of_block(p, block), p.n_jobs, false));
     const int strict = p.attend_current ? 0 : 1;
     const int m0 = job.rb * kRowBlock;
     const int q0w = m0 + 32 * wave;              // first query of this wave
@@ -90,7 +88,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
     float R = qi < job.len ? 1.0f : 0.0f;
     // This wave has no more weights to give: its rows' carries are exactly 0, or it has no rows at all.
     bool done = q0w >= job.len;
-    if (threadIdx.x < 8) done_waves[threadIdx.x >> 2][threadIdx.x & 3] = 0;
+    if (wave == 0 && lane < 8) done_waves[lane >> 2][lane & 3] = 0;
 
     const int imax = min(m0 + kRowBlock - 1, job.len - 1);
     const int kmax = imax - strict;                       // last key any row of the block sees
@@ -191,14 +189,26 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
         }
         close_step(step, buf);
     }
+    draw();
     store_carries();
-    if (p.save && threadIdx.x == 0) set_first_live(p, head, job, n_steps - iterations);
+    if (p.save && wave == 0 && lane == 0) set_first_live(p, head, job, n_steps - iterations);
 
     if (!kCarryOnly) {
         store_o_rows<D>(lds + wave * kRowStage<D>, p, job, head, q0w, lane, oacc);       // (the tiles are free)
         if (h == 0 && qi < job.len)
             Elem16::store(p.rem.ptr, (int64_t)job.seq * p.rem.sb + (int64_t)head * p.rem.sh + job.tok0 + qi, R);
     }
+}
+
+template <int D, bool kCarryOnly>
+__global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
+    fwd_job<D, kCarryOnly, kSharedCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {});
+}
+
+template <int D, bool kCarryOnly>
+__global__ __launch_bounds__(kThreads, 2) void mfma_fwd_drawing_kernel(KParams) {
+    __shared__ int words[2];
+    draw_jobs(words, [&](const KParams& p, int block, int wave, int lane, auto draw) { fwd_job<D, kCarryOnly, kDrawn>(p, block, wave, lane, draw); });
 }
 
 // ---------------------------------------------------------------- small grids: G segments per sweep
@@ -471,13 +481,16 @@ static void launch_seg(int groups, dim3 grid, hipStream_t s, const sba::KParams&
 }
 
 #ifdef SBA_ELEM_F16
-int sba_launch_mfma_f16_fwd(const sba::KParams& kp, hipStream_t s) {
+int sba_launch_mfma_f16_fwd(const sba::KParams& kp_in, hipStream_t s) {
 #else
-int sba_launch_mfma_fwd(const sba::KParams& kp, hipStream_t s) {
+int sba_launch_mfma_fwd(const sba::KParams& kp_in, hipStream_t s) {
 #endif
     using namespace sba;
-    dim3 grid((unsigned)kp.n_jobs * kp.n_heads);
-    const int segments = forward_segments(kp, grid.x);
+    dim3 grid((unsigned)kp_in.n_jobs * kp_in.n_heads);
+    const int segments = forward_segments(kp_in, grid.x);
+    KParams kp = kp_in;
+    kp.queue_stride = sba_queue_stride(kp);
+    float* const table = kp.save ? kp.rtab : nullptr;
     if (segments) {
         if (kp.carry_only) launch_seg<true>(segments, grid, s, kp);
         else launch_seg<false>(segments, grid, s, kp);
@@ -485,11 +498,11 @@ int sba_launch_mfma_fwd(const sba::KParams& kp, hipStream_t s) {
         if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<64, true>), grid, dim3(kThreads), 0, s, sba_turning(kp, 4));
         else hipLaunchKernelGGL((mfma_fwd_kernel<64, false>), grid, dim3(kThreads), 0, s, sba_turning(kp, 4));
     } else if (kp.head_dim == 96) {
-        if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<96, true>), grid, dim3(kThreads), 0, s, kp);
-        else hipLaunchKernelGGL((mfma_fwd_kernel<96, false>), grid, dim3(kThreads), 0, s, kp);
+        if (kp.carry_only) sba_launch_drawing((mfma_fwd_kernel<96, true>), (mfma_fwd_drawing_kernel<96, true>), grid.x, kThreads, 2, kp, table, kForwardQueue, false, s);
+        else sba_launch_drawing((mfma_fwd_kernel<96, false>), (mfma_fwd_drawing_kernel<96, false>), grid.x, kThreads, 2, kp, table, kForwardQueue, false, s);
     } else if (kp.head_dim == 128) {
-        if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<128, true>), grid, dim3(kThreads), 0, s, kp);
-        else hipLaunchKernelGGL((mfma_fwd_kernel<128, false>), grid, dim3(kThreads), 0, s, kp);
+        if (kp.carry_only) sba_launch_drawing((mfma_fwd_kernel<128, true>), (mfma_fwd_drawing_kernel<128, true>), grid.x, kThreads, 2, kp, table, kForwardQueue, false, s);
+        else sba_launch_drawing((mfma_fwd_kernel<128, false>), (mfma_fwd_drawing_kernel<128, false>), grid.x, kThreads, 2, kp, table, kForwardQueue, false, s);
     } else {
         if (kp.carry_only) hipLaunchKernelGGL((mfma_fwd_kernel<256, true>), grid, dim3(kThreads), 0, s, kp);
         else hipLaunchKernelGGL((mfma_fwd_kernel<256, false>), grid, dim3(kThreads), 0, s, kp);
