@@ -626,7 +626,7 @@ __device__ inline void wait_for_count(int* counter, int target, int* gave_up) {
 }
 
 // Weights and logit gradients of ONE [32 keys x 32 queries] tile whose lanes hold 16 consecutive keys
-// (the own-keys kernel and the eight-producer stream): the carries enter per 32 keys.
+// (the own-keys and paired kernels and the eight-producer stream): the carries enter per 32 keys.
 template <class Between>
 __device__ inline void own_tile_weights(float (&x)[16], float (&beta)[16], float Rin, int lane, Between&& between) {
     const float L = product_chain_with<true, 16>(x, beta, between);
@@ -1175,12 +1175,14 @@ __global__ __launch_bounds__((NP + 4) * 64, NP == 4 ? 2 : 3) void mfma_bwd_dkv_s
 // a 64-key block that touches the edge, the mid-block ones for the other half.  Weights and
 // logit gradients go as bf16 [query][32 a | 32 dz] rows into a tile private to the wave and
 // come back transposed as the A operands of  dV += A^T dO  and  dK += dZ^T Q.
+// At head_dim 256; at 128 behind the paired kernel and there to test it against, as at 64, where it took 97 us on a pack of 8192 tokens and 745 on one
+// of 65536 (H=16) that the paired kernel takes 89 and 732 on.
 // kSplit: at head_dim 256 the [32 keys x 256] accumulators of dK and dV alone are 256 registers a lane, on top of 128
 // for the K and V fragments.  There the grid has kSplit = 2 workgroups per (key block, head), blockIdx.y = 0, 1, and
 // workgroup `part` accumulates and stores columns 128 * part .. 128 * part + 127 of dK and dV only; scores, weights and
 // logit gradients are formed in both.
-template <int D, int kSplit, Sharing kSharing, class Draw>
-__device__ __forceinline__ void own_keys_job(const KParams& p, const int block, const int wave, const int lane, Draw draw) {
+template <int D, int kSplit = 1>
+__global__ __launch_bounds__(kThreads, 1) void mfma_bwd_dkv_own_kernel(KParams p) {
     constexpr int kNB = D / 32 / kSplit;         // 32-wide column blocks of dK / dV accumulated here
     const int part = kSplit > 1 ? (int)blockIdx.y : 0;
     static_assert(32 * (D / kSplit) * 2 <= 64 * 64 * 2, "a wave stages its [32 keys x columns] outputs in its weight tile");
@@ -1192,18 +1194,18 @@ __device__ __forceinline__ void own_keys_job(const KParams& p, const int block, 
     // and goes between the segments of that step's first chain.  The Q / dO tiles of a step then
     // have to outlive it by one step: three tile buffers instead of two.
     constexpr bool kDefer = D == 128;
-    // LDS fetches with the pinned base (see fetch_cols_o): -1.6 % at head_dim 64, +2.5 % at 128 (registers)
-    constexpr bool kOwnPin = D == 64;
     constexpr int kNBuf = kDefer ? 3 : 2;
     __shared__ __attribute__((aligned(16))) char lds[2 * kNBuf * kQTile + 4 * kZTile];   // Q, dO per buffer | one Z tile per wave
 
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 31, h = lane >> 5;
     LaneOffsets<D> lo;
     lo.init(lane);
     LaneOffsets<64> lz;
     lz.init(lane);
-    const int head = head_of_block<kSharing>(p, block);
-    const Job job = decode_key_job<D == 64>(p, slot_of_block(p, block));
+    const int head = head_of_block(p, blockIdx.x);
+    const Job job = decode_key_job(p, slot_of_block(p, blockIdx.x));
     const int strict = p.attend_current ? 0 : 1;
     const int q_begin = job.rb * kRowBlock;            // first key of the block = first query that may see it
     const int kb0 = q_begin + 32 * wave;               // first key of this wave
@@ -1440,7 +1442,6 @@ __device__ __forceinline__ void own_keys_job(const KParams& p, const int block, 
         else second_tile_reduction(TileAt{(kNBuf - 1) * 2 * kQTile}, TileAt{(kNBuf - 1) * 2 * kQTile + kQTile});
     }
 
-    draw();
     // ---- rows kb0.. of dK (scaled) and dV, through the wave's own tile as coalesced 16-byte stores
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
@@ -1456,17 +1457,6 @@ __device__ __forceinline__ void own_keys_job(const KParams& p, const int block, 
                 *(u32x4*)(out.ptr + 2 * (ob + (int64_t)(kb0 + row) * out.st + part * kCols + cc * 8)) = *(const u32x4*)(ztile + row * (kCols * 2) + cc * 16);
         }
     }
-}
-
-template <int D, int kSplit = 1>
-__global__ __launch_bounds__(kThreads, D == 64 ? 2 : 1) void mfma_bwd_dkv_own_kernel(KParams p) {
-    own_keys_job<D, kSplit, D == 64 ? kSharedCu : kOnePerCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {});
-}
-
-template <int D>
-__global__ __launch_bounds__(kThreads, 2) void mfma_bwd_dkv_own_drawing_kernel(KParams) {
-    __shared__ int words[2];
-    draw_jobs(words, [&](const KParams& p, int block, int wave, int lane, auto draw) { own_keys_job<D, 1, kDrawn>(p, block, wave, lane, draw); });
 }
 
 
@@ -1672,12 +1662,19 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
 // that two of them share a CU and one's barriers and round trips pass under the other's work, and the diagonal and the end of a
 // sequence are cut off by 64 keys.  Against one workgroup of kPairs = 4 a CU (128 keys, eight waves, half the tile copies):
 // B=4 H=16 T=2047 d=128 181 -> 163 us, B=1 H=16 T=16384 1690 -> 1530, d = 80 as above 249 -> 213.
+// At head_dim 64 a wave holds one output's [32 keys x 64] and needs 165 registers, three waves to a SIMD, and a workgroup 48 KB of LDS, three to a
+// CU.  A sweep's step is two tiles in a row there in the own-keys kernel, one in each wave here, which the longest sweeps of a launch gain most from
+// (H=16 T=4096: 97 us, the resident stream 114).  With three workgroups to fill each other's gaps the pacing of a workgroup's own waves costs more than
+// it gives: without it T=4096 109 -> 97 us, 65536 packed tokens 746 -> 732; at head dims 96 and 128 it makes no difference.
+// Rounded are the scaled K where the stream takes the forward's scaled Q; errors of dK / dV against 64 bits at B=1 H=8 T=2048 (2-norms, 1e-3, this kernel and the
+// stream's): mean logits 0 .. -6 over the heads 2.44 / 2.42 and 2.90 / 2.41, all at -6 2.90 / 2.91 and 3.07 / 2.64, of standard deviation 2 3.40 / 2.74 and 3.66 / 2.73.
 template <int D, int kPairs, Sharing kSharing, class Draw>
 __device__ __forceinline__ void paired_keys_job(const KParams& p, const int block, const int wave, const int lane, Draw draw, char* const lds) {
     constexpr int kQTile = 64 * kPitch<D> * 2;           // Q or dO tile of one step (64 queries)
     constexpr int kZTile = 64 * 64 * 2;          // per pair: [64 queries][32 a | 32 dz] bf16
     constexpr int kStep = 64;
     constexpr int kBlocks = D / 32;              // 32-wide column blocks of dK or dV
+    constexpr bool kPaced = D != 64;
     static_assert(2 * kPairs * 32 * D * 2 <= 4 * kQTile, "every wave stages its [32 keys x D] output in the tiles");
 
     const int grp = wave >> 1, r = wave & 1;
@@ -1813,7 +1810,7 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
                 const float Rt = sees ? Rin : 1.0f;      // table entries of invisible pairs are not written
                 const float Gt = sees ? Gin : 0.0f;
                 float beta[16];
-                __builtin_amdgcn_s_setprio(3);     // paced like the two-step dQ kernel's chain: the wave behind goes first
+                if (kPaced) __builtin_amdgcn_s_setprio(3);     // paced like the two-step dQ kernel's chain: the wave behind goes first
                 {
                     f32x16 sacc = {0};
 #pragma unroll
@@ -1846,9 +1843,9 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
                         const int ks = kPer * seg + i;
                         if (ks < D / 16) dacc = mfma(vfr[ks], cur[i], ks == 0 ? f32x16{0} : dacc);
                     }
-                    if (seg == 1) __builtin_amdgcn_s_setprio(2);
+                    if (kPaced && seg == 1) __builtin_amdgcn_s_setprio(2);
                 });
-                __builtin_amdgcn_s_setprio(1);
+                if (kPaced) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int i = 0; i < 16; ++i) dp[i] = dacc[i];
                 // a -> columns 16h.. of row (32r + n) now, dz -> columns 32 + 16h.. below
@@ -1857,7 +1854,7 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
                 own_tile_grads(x, beta, dp, Gt, lane);
                 *(h16x8*)(ztile + tile_offset<64>(32 * r + n, 4 + 2 * h)) = pack8(&dp[0]);
                 *(h16x8*)(ztile + tile_offset<64>(32 * r + n, 4 + 2 * h + 1)) = pack8(&dp[8]);
-                __builtin_amdgcn_s_setprio(0);
+                if (kPaced) __builtin_amdgcn_s_setprio(0);
             }
         }
         __syncthreads();                       // the pair's weights are complete
@@ -1905,14 +1902,14 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
 }
 
 template <int D, int kPairs>
-__global__ __launch_bounds__(128 * kPairs, 2) void mfma_bwd_dkv_pair_kernel(KParams p) {
+__global__ __launch_bounds__(128 * kPairs, D == 64 ? 3 : 2) void mfma_bwd_dkv_pair_kernel(KParams p) {
     constexpr int kQTile = 64 * kPitch<D> * 2, kZTile = 64 * 64 * 2;
     __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + kPairs * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
     paired_keys_job<D, kPairs, kPairs == 4 ? kOnePerCu : kSharedCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {}, lds);
 }
 
 template <int D>
-__global__ __launch_bounds__(256, 2) void mfma_bwd_dkv_pair_drawing_kernel(KParams) {
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void mfma_bwd_dkv_pair_drawing_kernel(KParams) {
     constexpr int kQTile = 64 * kPitch<D> * 2, kZTile = 64 * 64 * 2;
     __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + 2 * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
     draw_jobs((int*)(lds + 4 * kQTile), [&](const KParams& p, int block, int wave, int lane, auto draw) { paired_keys_job<D, 2, kDrawn>(p, block, wave, lane, draw, lds); });
@@ -1956,28 +1953,21 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     // the dQ kernels reach a lane's prefix entry from its carry entry by one uniform distance (see there)
     if (!kp.rtab || !kp.rmid || !kp.gtab || !kp.gmid) return SBA_ERR_WORKSPACE;
     if (!kp.makes_mid && (const char*)kp.gmid - (const char*)kp.rtab != (const char*)kp.gtab - (const char*)kp.rmid) return SBA_ERR_WORKSPACE;
-    // Key-owner pass.  head_dim 64: the kernel whose waves own their keys outright, one sweep per workgroup, unless the launch hangs
-    // on its longest sweeps; then the resident producer/consumer stream, which splits the work into twice as many items and deals
-    // them out itself.  Forward + backward with the stream over the same with own keys, by tail ratio r, mean logits 0 .. -6 over the heads in
-    // this order and in random ones / all at -6:
-    //     longest sequence up to 4096 tokens, dense  r 2.7 1.04-1.05 / 1.04, 2.9 1.00 / 1.01, 3.1 0.99-1.015 / 0.99-1.00, 3.2 1.00-1.02 / 1.01, 3.3 0.98-1.00 /
-    //         0.99, 3.4 1.01-1.02 / 1.01, 3.9 0.93 / 0.94, 4.0 0.89-0.90 / 0.92;  packs  1.9 1.14-1.15, 2.5 1.08-1.13, 2.8 1.09-1.11, 3.3 1.04-1.06, 4.4 0.98
-    //     longer, dense, twelve and sixteen heads  r 2.1 0.99-1.07 / 0.98, 2.5 0.97-1.04 / 1.00, 2.6 1.01 / 0.99, 2.7 0.96-1.01 / 1.02, 2.9 0.96-1.00 /
-    //         1.01, 3.0 0.975 / 0.97, 3.1 0.96-0.98 / 0.97, 3.3 0.97 / 0.96
-    //     longer, dense, up to eight heads  r 1.6-1.7 0.975-1.12 / 1.00, 1.9 (H=4) 0.98 / 0.97, 2.0 H=8 0.96-1.03 / 0.96-0.99, H=4 0.99 / 0.97, H=1 and 2 1.09-1.18 /
-    //         0.95-0.97, 2.2 (H=6) 0.98-1.06 / 0.97, 2.3 (H=8) 0.95-1.00 / 0.96-0.98, 2.5 0.92-0.95 / 0.98, 2.7 0.93-0.985 / 0.97-0.98, 2.8-3.2 0.86-0.95 /
-    //         0.94-0.97, 3.6-4.0 0.79-0.91 / 0.88-0.90; behind only H=2 T=50000 (2.6) 1.02 / 0.98 and H=1 T=65536 (4.0), whose sweeps end early, 1.12 / 0.90
-    //         backward alone at the line and above, by the longest document: 3.4-3.8 0.92-1.04 (2000 to 4096 tokens), 3.5 1.09-1.11 (1387); 4.0 0.96 (3562), 1.08
-    //         (1539); 4.4-5.2 0.78-0.96
-    //     longer, packs  r 0.7-1.7 1.07-1.22, 2.4 1.09, 3.2 1.02-1.03 and (H=2) 0.90, 3.3 0.96, 3.9 0.97
-    // Batches of short sequences (sweeps of at most 16 steps) also take the own-keys kernel at any size: on 512 workgroups B=8,
-    // T=512 takes 27.3 us against the stream's 33.0, B=4, T=1024 44.0 against 45.3.
-    // head_dim 128: the paired kernel at every size (B=1, H=16, T=512 ... 2048: with four pairs 27 / 44 / 62 / 81 us where the
-    // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103); SBA_DKV_KERNEL=other still selects that one.
+    // Key-owner pass.  head_dim 64: the paired kernel, but for fewer than one and a half row blocks a CU (all heads), where three workgroups a CU do not
+    // come together and the resident producer/consumer stream is ahead.  Forward + backward with the paired kernel over the same with the stream,
+    // by workgroups of the row-owner passes, mean logits 0 .. -6 over the heads in order / in a random one / all at -6:
+    //     192 (H=16 T=1500) 1.11 / 1.08 / 1.085    256 (H=16 T=2048) 1.07 / 1.07 / 1.08, (H=8 T=4096) 1.13 / 1.13 / 1.13, (H=4 T=8192) 1.15 / 1.16 / 1.15
+    //     320 (H=16 T=2500) 1.02 / 1.015 / 1.01, (H=8 T=5000) 1.05 / 1.05 / 1.05, packs of 2000 tokens 1.02 / 1.02 / 1.02, of 4096 tokens, H=8 1.04 / 1.02 / 1.03
+    //     376 (H=8 T=6000) 1.04 / 1.02 / 1.03    384 (H=12 T=4096) 1.00 / 1.00 / 1.00, (H=16 T=3000) 0.98 / 0.97 / 0.975, (B=3 H=16 T=1024) 0.96 / 0.97 / 0.95
+    //     440 (H=8 T=7000) 1.00 / 0.98 / 1.01, (H=4 T=14000) 1.04 / 1.05 / 1.01    512 (H=16 T=4096) 0.94 / 0.95 / 0.98, (B=2 H=16 T=2048) 0.92 / 0.91 / 0.96, (H=8 T=8192)
+    //     0.95 / 0.95 / 0.96, (H=4 T=16384) 1.03 / 1.03 / 1.00, (H=2 T=32768) 0.94 / 0.94 / 1.00    640 (H=16 T=5000) 0.94 / 0.92 / 1.00, packs of 4096 tokens 0.90 / 0.90 / 0.89
+    // and over the kernel whose waves own 32 keys each (two waves per SIMD at 215 registers), which was there before for launches that do not hang on their longest
+    // sweeps: 1024 (H=32 T=4096) 0.95 / 0.94 / 0.935, (H=16 T=8192) 0.96 / 0.94 / 0.93, (B=8 T=2048) 0.935 / 0.94 / 0.98, (B=4 T=1024) 0.97 / 0.95 / 0.97,
+    // packs of 8192 tokens 0.95 / 0.93 / 0.93, 16384 0.93 / 0.95 / 0.93, 65536 0.98 / 0.97 / 0.98, documents up to 1024 0.96 / 0.96 / 0.95, up to 256 0.98 / 0.975 / 0.97.
+    // head_dim 72 to 128: the paired kernel at every size (B=1, H=16, T=512 ... 2048: with four pairs 27 / 44 / 62 / 81 us where the
+    // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103).  SBA_DKV_KERNEL=pair / =other (the stream at head_dim 64) picks one.
     const unsigned cus = (unsigned)sba_cu_count();
-    const bool short_sweeps = kp.seq_len <= 8 * kRowBlock && grid.x >= 2u * cus;
-    const double own_up_to = kp.seq_len <= 32 * kRowBlock ? 3.35 : kp.n_heads <= 8 && !kp.cu_seqlens ? 2.2 : 2.75;
-    const bool own = own_keys_kernel(kp.head_dim == 64 ? short_sweeps || sba_tail_ratio(kp, grid.x) <= own_up_to : true);
+    const bool own = own_keys_kernel(kp.head_dim == 64 ? 2 * grid.x >= 3 * cus : true);
     const char* which = getenv("SBA_DKV_KERNEL");
     const bool plain = which && !strcmp(which, "plain");
     // the stream with eight half-block producers (12 waves): behind the one with four full-block producers
@@ -2028,7 +2018,7 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         if (p2 && plain) {
             hipLaunchKernelGGL((mfma_bwd_dkv_kernel<64>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
         } else if (p2 && own) {
-            sba_launch_drawing((mfma_bwd_dkv_own_kernel<64>), (mfma_bwd_dkv_own_drawing_kernel<64>), grid.x, kThreads, 2, sba_turning(kp, 2), kp.gtab, kKeyQueue, p1, s);
+            sba_launch_drawing((mfma_bwd_dkv_pair_kernel<64, 2>), (mfma_bwd_dkv_pair_drawing_kernel<64>), 2 * grid.x, kThreads, 3, kp, kp.gtab, kKeyQueue, p1, s);
         } else if (p2) {
             // one resident workgroup per CU, in whole rounds of the 8 XCDs (surplus workgroups
             // find no item)
