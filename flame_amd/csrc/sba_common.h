@@ -411,17 +411,17 @@ inline int64_t sba_queue_stride(const sba::KParams& kp) {
 //         H=32 T=8192 0.90 / 0.93 / 0.93, B=2 H=8 T=16384 0.925 / 0.81 / 0.97, B=4 T=4096 (68000) 0.97 / 0.99 / 1.01, B=16 T=4096 0.96 / 0.97 / 0.97;
 //         d=80 T=16384 0.93 / 0.94 / 0.94, B=8 H=12 T=4096 0.965 / 0.98 / 1.00;  packs  65536 tokens d=128 0.96 / 0.97 / 0.99, d=80 0.96 / 0.97 / 0.99, documents up
 //         to 16384 0.915 / 0.94 / 0.98, up to 1024 d=96 0.99 / 0.98 / 0.97, 32768 tokens 1.00 / 0.98 / 1.01;  below the line B=8 T=2048 (35000) 1.01 / 1.03 / 1.015
-//     head_dim 64, the backward's two passes (the forward's, of which a CU holds four, gains nothing)   packs  65536 tokens 0.97 / 1.00 / 1.00, H=32 0.94 / 0.95 / 0.98,
-//         131072 tokens 0.96 / 0.96 / 0.98, documents up to 16384 0.94 / 0.94 / 0.97, up to 1024 0.99 / 1.00 / 0.98;  B=16 H=16 T=4096 0.98 / 0.98 / 0.98, B=4
-//         T=16384 0.97 / 0.98 / 0.99;  below the line B=4 T=4096 (2048 workgroups) 1.03 / 1.03 / 1.03
-// Short sweeps lose by it: documents up to 256 tokens 1.02 to 1.03 for the forward and the dQ pass at head_dim 64.
+//     head_dim 64, the backward's two passes (the forward, of which a CU holds four, gains nothing)   packs  65536 tokens 0.99 / 0.98 / 1.00, H=32 0.96 / 0.95 / 0.99,
+//         131072 tokens 0.97 / 0.96 / 0.98, documents up to 16384 0.97 / 0.95 / 0.98;  B=16 H=16 T=4096 0.97 / 0.98 / 0.97, B=4 T=16384 0.98 / 0.98 / 0.99;  below the
+//         lines packs of documents up to 1024 1.005 / 1.01 / 1.01, 32768 tokens 1.01 / - / 1.02, B=4 T=4096 (2048 workgroups) 1.01 / - / 1.02
+// Short sweeps lose by it: documents up to 300 tokens 1.14.
 // SBA_DRAW=1 / =0 (experiments and tests): wherever there are more jobs than the chip holds workgroups, or nowhere.
 inline bool sba_draws(const sba::KParams& kp, unsigned blocks, unsigned slots) {
     if (!kp.queue_stride || slots == 0 || blocks <= slots) return false;
     const char* e = getenv("SBA_DRAW");
     if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
     const int64_t grid = (int64_t)kp.n_jobs * kp.n_heads, columns = kp.tab_head_stride / sba::kRowBlock, mean_sweep = columns / kp.n_jobs;
-    return kp.head_dim == 64 ? grid >= SBA_DOC_MAJOR_GRID && mean_sweep >= 8 : columns * kp.n_heads >= 60000 && mean_sweep >= 4;
+    return kp.head_dim == 64 ? grid >= SBA_DOC_MAJOR_GRID && mean_sweep >= 12 : columns * kp.n_heads >= 60000 && mean_sweep >= 4;
 }
 // Launches `drawing` with `resident` workgroups a CU where that pays, else `plain` with a workgroup per job.  table, entry: where its queues lie
 // (null: nowhere).
