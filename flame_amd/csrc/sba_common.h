@@ -186,9 +186,8 @@ __device__ inline Job decode_job(const KParams& p, int job) {
 // their longest sweeps are the FIRST row-blocks of the longest sequences.  i-th job in that
 // order: arithmetic for the dense layout, the second half of row i of the host-built schedule
 // for the packed.
-template <bool kTurns = false>
 __device__ inline Job decode_key_job(const KParams& p, int i) {
-    if (p.cu_seqlens == nullptr) return dense_job(p, p.n_jobs - 1 - (kTurns ? turned(p, i) : i));
+    if (p.cu_seqlens == nullptr) return dense_job(p, p.n_jobs - 1 - i);
     const ScheduleRow s = schedule_row(p, i, 4);
     Job j;
     j.tok0 = s[0]; j.len = s[1]; j.rb = s[2]; j.seq = 0; j.tab0 = s[3];
@@ -350,9 +349,6 @@ inline int sba_two_step_env() {
         return e ? atoi(e) : -1;
     }();
     return v;
-}
-inline unsigned sba_two_step_max_grid(unsigned by_default) {
-    return sba_two_step_env() >= 0 ? (unsigned)sba_two_step_env() : by_default;
 }
 // The two-steps-per-iteration dQ kernel up to 544 workgroups (measured at H = 16: 103.9 us against the one-step
 // kernel's 106.4 at 528 workgroups, 122.0 against 120.6 at 576).  The forward's rule is in sba_launch_mfma_fwd().

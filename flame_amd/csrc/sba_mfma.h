@@ -559,22 +559,6 @@ __device__ inline void score_raw_o(f32x16 (&raw)[2], Tile ktile, const LaneOffse
     }
 }
 
-// base-2 logits from the raw accumulators: x[16*t + r] = scale2 * raw[t][r].
-__device__ inline void scale_scores(float (&x)[32], const f32x16 (&raw)[2], float scale2) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[16 * t + r] = raw[t][r] * scale2;
-}
-
-template <int D, bool kBatch = kWide<D>, class Tile>
-__device__ inline void score_tiles_o(float (&x)[32], Tile ktile, const LaneOffsets<D>& o,
-                                     const h16x8 (&qf)[D / 16], float scale2) {
-    f32x16 raw[2];
-    score_raw_o<D, kBatch>(raw, ktile, o, qf);
-    scale_scores(x, raw, scale2);
-}
-
 // Score tiles from pre-scaled fragments: x[16*t + r] = raw accumulator, no vector work.
 template <int D, bool kBatch = kWide<D>, class Tile>
 __device__ inline void score_tiles_ps(float (&x)[32], Tile ktile, const LaneOffsets<D>& o,
@@ -750,55 +734,8 @@ __device__ inline void stick_weights(float (&x)[32], float (&beta)[kNeedBeta ? 3
     R = R * Llo * Lup;
 }
 
-// stick_weights<true> with a hook between the eight segments of the chain (see product_chain_with).
-template <class Between>
-__device__ inline void stick_weights_hooked(float (&x)[32], float (&beta)[32], float& R, int lane, float* lane_carry,
-                                            Between&& between) {
-    const float L = product_chain_with<true, 32>(x, beta, between);
-    float Llo, Lup;
-    half_values(L, Llo, Lup);
-    const float F = (lane >= 32) ? R : R * Lup;
-    if (lane_carry) *lane_carry = F;
-    scale_clamped<32>(x, F);
-    R = R * Llo * Lup;
-}
-
-// stick_weights<true> with the dP MFMAs of the step (dp[16t + r] = (V dO^T)[key][query], see
-// dp_tiles_o) issued between the segments of the chain, their operands fetched one segment ahead.
-template <int D, class Tile>
-__device__ inline void stick_weights_and_dp(float (&x)[32], float (&beta)[32], float (&dp)[32], float& R, int lane,
-                                            float* lane_carry, Tile vtile, const LaneOffsets<D>& o,
-                                            const h16x8 (&dof)[D / 16]) {
-    constexpr int kPer = (D / 8 + 7) / 8;      // MFMAs per segment: 2 tiles x D/16 slices over 8 segments
-    f32x16 dacc[2];
-    h16x8 nx[kPer];
-    // MFMA m (0 .. D/8 - 1): tile t = m & 1, slice ks = m >> 1 (neighbours use different accumulators)
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) nx[i] = fetch_rows_o<D>(vtile, o, i & 1, i >> 1);
-    stick_weights_hooked(x, beta, R, lane, lane_carry, [&](int seg) {
-        h16x8 cur[kPer];
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) cur[i] = nx[i];
-        if (seg < 7) {
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const int m = kPer * (seg + 1) + i;
-                if (m < D / 8) nx[i] = fetch_rows_o<D>(vtile, o, m & 1, m >> 1);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int m = kPer * seg + i, t = m & 1, ks = m >> 1;
-            if (m < D / 8) dacc[t] = mfma(cur[i], dof[ks], ks == 0 ? f32x16{0} : dacc[t]);
-        }
-    });
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) dp[16 * t + r] = dacc[t][r];
-}
-
-// The same from this lane's own carry F (carried_chain_with): finished weights, beta and dP; returns the carry
+// The chain from this lane's own carry F (carried_chain_with) with the dP MFMAs of the step (dp[16t + r] = (V dO^T)[key][query], see
+// dp_tiles_o) issued between its segments, their operands fetched one segment ahead: finished weights, beta and dP; returns the carry
 // leaving the lane's keys.
 // kPaced: the wave lowers its issue priority as it moves through the chain (3 for the first two 4-key segments, then 2,
 // 1, 0).  Two waves of a SIMD that run this chain side by side otherwise issue oldest first: the older one runs as if
@@ -865,11 +802,6 @@ __device__ inline void mask_step(float (&x)[32], int key_first, int qi, int stri
 #pragma unroll
     for (int idx = 0; idx < 32; ++idx)
         if (idx >= nvis) x[idx] = -INFINITY;
-}
-
-// Row fetch from a natural-order tile: 8 bf16 of row `row`, columns 16*ks + 8*h .. +7.
-template <int ROWD> __device__ inline h16x8 fetch_row_nat(const char* tile, int row, int ks, int lane) {
-    return *(const h16x8*)(tile + tile_offset<ROWD>(row, 2 * ks + (lane >> 5)));
 }
 
 // dP^T tile pair: dp[16*t + r] = (V dO^T)[key_local][query].  The gradient of `rem` is not
@@ -950,14 +882,9 @@ __device__ inline void logit_grads_from(const float (&a)[N], const float (&beta)
 
 // Register-lean form of the backward's per-step arithmetic for the row-owner kernel at head_dim
 // 128, where registers decide between one and two waves per SIMD: two arrays of 32 instead of
-// four.  Part 1 runs the reciprocal-per-key chain right-to-left and leaves, in place of the
-// logits, beta, and in place of dP, g' = a' * dP with a' the weight relative to the right edge of
-// the lane's 32 keys (the finished weight is F * a', F the carry entering the lane's keys, which
-// only the exchange after the chain supplies).  Returns the lane's product of (1 - beta) (clamped,
-// see product_chain) and in `gsum` the lane's sum of g'.  Part 2 walks left-to-right from the
-// prefix `G` entering the lane's keys:  t = F g',  G += t,  dz = t - beta G,  packed as it goes.
-// chain_beta_gprime from this lane's own carry F (see carried_chain_with): dp[idx] <- g = a * dP with the finished
-// weight, gsum their sum; returns the carry leaving the lane's keys.
+// four.  Part 1 runs the reciprocal-per-key chain right-to-left from this lane's own carry F (see carried_chain_with) and leaves, in
+// place of the logits, beta, and in place of dP, g = a * dP with the finished weight a, gsum their sum; returns the carry leaving the
+// lane's keys.  Part 2 walks left-to-right from the prefix `G` entering the lane's keys:  G += g,  dz = g - beta G,  packed as it goes.
 __device__ inline float carried_beta_g(float (&x)[32], float (&dp)[32], float F, float& gsum) {
     float W = __builtin_amdgcn_rcpf(F), L = F, c = 0.f;
 #pragma unroll
@@ -980,7 +907,7 @@ __device__ inline void scale_all(float (&g)[32], float by) {
 #pragma unroll
     for (int i = 0; i < 32; ++i) g[i] *= by;
 }
-// dz from beta, g and the prefix G entering the lane's keys
+// dz from beta, g and the prefix G entering the lane's keys; zf[c] = dz of keys 8c .. 8c+7 packed (the B operand of dQ^T += K^T dZ^T)
 // (The running sum must stay a plain add: fused with the product that made g - which the compiler does across
 // function boundaries when allowed to - it would need the two factors of every g alive instead of g itself,
 // 32 registers more than this kernel has.)
@@ -997,37 +924,6 @@ __device__ inline void walk_logit_grads_g(const float (&beta)[32], const float (
         zf[c] = pack8(dz);
     }
 }
-__device__ inline float chain_beta_gprime(float (&x)[32], float (&dp)[32], float& gsum) {
-    float W = 1.0f, L = 1.0f, c = 0.f;
-#pragma unroll
-    for (int idx = 31; idx >= 0; --idx) {
-        const float e = __builtin_amdgcn_exp2f(x[idx]);
-        const float Wn = __builtin_fmaf(W, e, W);
-        const float Ln = __builtin_amdgcn_rcpf(Wn);
-        x[idx] = clamp01(__builtin_fmaf(-W, Ln, 1.0f));       // beta
-        dp[idx] = clamp01(L - Ln) * dp[idx];                  // g' (the clamps map the NaN of an overflowed chain to 0)
-        c += dp[idx];
-        W = Wn;
-        L = Ln;
-    }
-    gsum = c;
-    return clamp01(L);
-}
-// Out: zf[c] = dz of keys 8c .. 8c+7 packed to bf16 (the B operand of dQ^T += K^T dZ^T).
-__device__ inline void walk_logit_grads(const float (&beta)[32], const float (&g)[32], float F, float G, h16x8 (&zf)[4]) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        float dz[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float t = F * g[8 * c + i];
-            G += t;
-            dz[i] = __builtin_fmaf(-beta[8 * c + i], G, t);
-        }
-        zf[c] = pack8(dz);
-    }
-}
-
 // logit_grads in two parts (see stick_weights_local): part 1 forms g in place of dp and
 // returns this lane's offset inside the step (0 for the lower half-wave, the lower half's
 // sum for the upper) and, in `total`, the step's sum of g; part 2 applies the prefix.
