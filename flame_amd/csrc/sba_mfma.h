@@ -396,6 +396,39 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
         if (kCut) dma16_lanes(tile_base, o, lds_address(tile + (w4 + 4 * i) * 1024), live[i]);
         else dma16(tile_base, o, lds_address(tile + (w4 + 4 * i) * 1024));
     }
+    // For loops that are short of scalar registers (the dQ pass), whose sums known in front of the loop are spilled into vector lanes and come back
+    // one by one: the origin moves along with the tiles, and the wave's part of the tile is an unknown at each tile, so that
+    // the copies' LDS addresses - 8 at head_dim 64, 16 above - are formed where they are used.  dQ at d=128, float16, B=4 H=16 T=2047: 15 lane reads a
+    // step, 118.7 us, and 6, 116; d=80, 20011 tokens packed: 16, 147, and none, 144; d=64, 65536 tokens packed 551 and 538.  (The forward and the
+    // key owners have the registers: T=16384, d=128 1.005 and 1.008 of the time with it.)
+    __device__ inline void seek(int row0) { origin += ((uint64_t)(uint32_t)row0 * (uint32_t)st) << 1; }
+    __device__ inline void forth() { origin += (uint32_t)st << 7; }
+    __device__ inline void issue_here(int row0, int len, char* tile) const {
+        uint32_t part = (uint32_t)w4 << 10;
+        asm volatile("" : "+s"(part));
+        auto copy_here = [&](int i, uint32_t o) __attribute__((always_inline)) {
+            if (kCut) dma16_lanes(origin, o, lds_address(tile) + part + 4096 * i, live[i]);
+            else dma16(origin, o, lds_address(tile) + part + 4096 * i);
+        };
+        if (row0 + 64 <= len) {
+#pragma unroll
+            for (int i = 0; i < kPerWave; ++i) copy_here(i, off[i]);
+        } else {
+            each_ragged(row0, len, copy_here);
+        }
+    }
+    // offsets of a tile that ends beyond the sequence, whose last row stands in for the rows that are not there
+    template <class Copy> __device__ inline void each_ragged(int row0, int len, Copy&& copy_of) const {
+        int lane_here = lane;
+        if (kLateRagged) asm volatile("" : "+v"(lane_here));
+        int kl, c;
+        where(w4, lane_here, kl, c);
+#pragma unroll
+        for (int i = 0; i < kPerWave; ++i) {
+            if (!kSameChunk) where(w4 + 4 * i, lane_here, kl, c);
+            copy_of(i, offset(min(kl + (kSameChunk ? rows_on(i) : 0), len - 1 - row0), c, st));
+        }
+    }
     // Zeros where this wave's copies into `tile` write (and, in rows shorter than 96 columns, never will): once per tile buffer,
     // before its first copy.
     __device__ inline void clear(char* tile) const {
@@ -421,15 +454,7 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
 #pragma unroll
             for (int i = 0; i < kPerWave; ++i) copy(i, tile_base, off[i], tile);
         } else {
-            int lane_here = lane;
-            if (kLateRagged) asm volatile("" : "+v"(lane_here));
-            int kl, c;
-            where(w4, lane_here, kl, c);
-#pragma unroll
-            for (int i = 0; i < kPerWave; ++i) {
-                if (!kSameChunk) where(w4 + 4 * i, lane_here, kl, c);
-                copy(i, tile_base, offset(min(kl + (kSameChunk ? rows_on(i) : 0), len - 1 - row0), c, st), tile);
-            }
+            each_ragged(row0, len, [&](int i, uint32_t o) __attribute__((always_inline)) { copy(i, tile_base, o, tile); });
         }
     }
 };

@@ -96,8 +96,10 @@ __device__ __forceinline__ void dq_job(const KParams& p, const int block, const 
         vc.clear(lds + b * 2 * kTile + kTile);
     }
     if (n_steps > 0) {
-        kc.issue(first * kKeyBlock, job.len, lds);
-        vc.issue(first * kKeyBlock, job.len, lds + kTile);
+        kc.seek(first * kKeyBlock);
+        kc.issue_here(first * kKeyBlock, job.len, lds);
+        vc.seek(first * kKeyBlock);
+        vc.issue_here(first * kKeyBlock, job.len, lds + kTile);
     }
     if (wave == 3) close_live_ranges(p, head, job, lane, first);
 
@@ -168,8 +170,10 @@ __device__ __forceinline__ void dq_job(const KParams& p, const int block, const 
             if (row_ok && kByBase && h) Rnext = entry_of(p.rtab, column + tstride);
             if (row_ok && !kByBase && (!kMid || h)) Rnext = rcur[tstride];
             // next tiles, straight into the other buffer (free since the last barrier)
-            kc.issue((step + 1) * kKeyBlock, job.len, lds + (buf ^ 1) * 2 * kTile);
-            vc.issue((step + 1) * kKeyBlock, job.len, lds + (buf ^ 1) * 2 * kTile + kTile);
+            kc.forth();
+            kc.issue_here((step + 1) * kKeyBlock, job.len, lds + (buf ^ 1) * 2 * kTile);
+            vc.forth();
+            vc.issue_here((step + 1) * kKeyBlock, job.len, lds + (buf ^ 1) * 2 * kTile + kTile);
         }
         if (!skip) {
             h16x8 zf[4];
