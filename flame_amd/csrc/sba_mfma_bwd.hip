@@ -1203,8 +1203,8 @@ __global__ __launch_bounds__((NP + 4) * 64, NP == 4 ? 2 : 3) void mfma_bwd_dkv_s
 // a 64-key block that touches the edge, the mid-block ones for the other half.  Weights and
 // logit gradients go as bf16 [query][32 a | 32 dz] rows into a tile private to the wave and
 // come back transposed as the A operands of  dV += A^T dO  and  dK += dZ^T Q.
-// At head_dim 256; at 128 behind the paired kernel and there to test it against, as at 64, where it took 97 us on a pack of 8192 tokens and 745 on one
-// of 65536 (H=16) that the paired kernel takes 89 and 732 on.
+// At head_dim 256; at 128 behind the paired kernel and there to test it against.  (At 64, where the paired kernel has replaced it, it took 97 us on a
+// pack of 8192 tokens and 745 on one of 65536 (H=16) that the paired kernel takes 89 and 732 on.)
 // kSplit: at head_dim 256 the [32 keys x 256] accumulators of dK and dV alone are 256 registers a lane, on top of 128
 // for the K and V fragments.  There the grid has kSplit = 2 workgroups per (key block, head), blockIdx.y = 0, 1, and
 // workgroup `part` accumulates and stores columns 128 * part .. 128 * part + 127 of dK and dV only; scores, weights and
