@@ -54,7 +54,7 @@ struct KParams {
     float* gmid;                   // the prefix entering the block's RIGHT 32 keys (written by the dQ pass, like gtab);
                                    //   the bf16 dQ kernels rely on gmid - rtab == gtab - rmid
     TensorArg q_scaled;            // bf16 head_dim 64 backward: q times scale2, rounded to bf16, written by the dQ pass for
-                                   //   the key-owner stream kernel (ptr NULL: not wanted)
+                                   //   the key-owner stream and paired kernels (ptr NULL: not wanted)
     float* dkv32;                  // generic path: fp32 dk|dv accumulators
     float* halves;                 // fp32 key-owner pass: sums of two workgroups that share a key block (null: none does)
     float* weights;                // sba_attention_weights(): the attention weights, fp32 (debug output)

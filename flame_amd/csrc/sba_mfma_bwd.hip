@@ -30,8 +30,8 @@ namespace sba {
 inline namespace SBA_ELEM_NS {
 
 // The dQ pass leaves its pre-scaled Q fragments (q times scale * log2 e, rounded to bf16: the operand every
-// row-owner kernel multiplies with) behind for the key-owner stream kernel, which then needs no scaling of its
-// own and sees bit for bit the logits that the forward's carries were made from.  Row qi of q_scaled gets this
+// row-owner kernel multiplies with) behind for the key-owner stream and the paired kernel in its place, which then need no scaling of their
+// own and see bit for bit the logits that the forward's carries were made from.  Row qi of q_scaled gets this
 // lane's four 16-byte chunks (columns 16 ks + 8 h ..).  head_dim 64 only, and only where the launcher asks for it.
 template <int D>
 __device__ inline void store_scaled_q(const KParams& p, const Job& job, int head, int qi, int lane,
@@ -1694,9 +1694,11 @@ __global__ __launch_bounds__(W * 64, D == 64 ? 2 : 1) void mfma_bwd_short_kernel
 // CU.  A sweep's step is two tiles in a row there in the own-keys kernel, one in each wave here, which the longest sweeps of a launch gain most from
 // (H=16 T=4096: 97 us, the resident stream 114).  With three workgroups to fill each other's gaps the pacing of a workgroup's own waves costs more than
 // it gives: without it T=4096 109 -> 97 us, 65536 packed tokens 746 -> 732; at head dims 96 and 128 it makes no difference.
-// Rounded are the scaled K where the stream takes the forward's scaled Q; errors of dK / dV against 64 bits at B=1 H=8 T=2048 (2-norms, 1e-3, this kernel and the
-// stream's): mean logits 0 .. -6 over the heads 2.44 / 2.42 and 2.90 / 2.41, all at -6 2.90 / 2.91 and 3.07 / 2.64, of standard deviation 2 3.40 / 2.74 and 3.66 / 2.73.
-template <int D, int kPairs, Sharing kSharing, class Draw>
+// kScaledQ (head_dim 64): which operand of the scores is scaled and rounded.  Without it K, in registers; with it the tiles are the scaled copy of q that the
+// dQ pass leaves behind, for the scores and for dK, as in the stream: the weights are those behind the forward's carries, but q is rounded twice where dK is formed.
+// Errors of dK / dV against 64 bits (2-norms, 1e-3, bf16, H=4 T=2048), K and scaled q, the latter the stream's to four digits:  all heads' mean logits at -6
+// 2.93 / 2.92 and 3.08 / 2.65, logits of standard deviation 3 3.41 / 2.62 and 3.79 / 2.63, mean logits 0 .. -6 over the heads 2.44 / 2.42 and 2.90 / 2.41.
+template <int D, int kPairs, bool kScaledQ, Sharing kSharing, class Draw>
 __device__ __forceinline__ void paired_keys_job(const KParams& p, const int block, const int wave, const int lane, Draw draw, char* const lds) {
     constexpr int kQTile = 64 * kPitch<D> * 2;           // Q or dO tile of one step (64 queries)
     constexpr int kZTile = 64 * 64 * 2;          // per pair: [64 queries][32 a | 32 dz] bf16
@@ -1725,7 +1727,8 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
     const int kb0 = q_begin + 32 * grp;                // first key of this pair
     char* ztile = lds + 4 * kQTile + grp * kZTile;
 
-    const int64_t qbase = slice_offset(p.q, job.seq, head, job.tok0);
+    const TensorArg& q = kScaledQ ? p.q_scaled : p.q;
+    const int64_t qbase = slice_offset(q, job.seq, head, job.tok0);
     const int64_t kbase = slice_offset(p.k, job.seq, head, job.tok0);
     const int64_t vbase = slice_offset(p.v, job.seq, head, job.tok0);
     const int64_t dobase = slice_offset(p.d_o, job.seq, head, job.tok0);
@@ -1738,7 +1741,7 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
         const int key = 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
         load_row_frags<D>(kfr, p.k, kbase, kb0, key, job.len, lane, p.cols);
         load_row_frags<D>(vfr, p.v, vbase, kb0, key, job.len, lane, p.cols);
-        prescale_frags(kfr, p.scale2);
+        if (!kScaledQ) prescale_frags(kfr, p.scale2);
     }
     f32x16 acc[kBlocks];         // r = 0: dV, r = 1: dK
 #pragma unroll
@@ -1749,7 +1752,7 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
     // copies of a step's Q and dO tiles: with eight waves the first four take Q and the others dO, four waves take both
     const bool q_first = kPairs == 2 || wave < 4;
     TileDma<D, true> tc, tc2;
-    tc.init(lane, wave & 3, q_first ? p.q : p.d_o, q_first ? qbase : dobase, p.cols);
+    tc.init(lane, wave & 3, q_first ? q : p.d_o, q_first ? qbase : dobase, p.cols);
     if (kPairs == 2) tc2.init(lane, wave, p.d_o, dobase, p.cols);
     const int my_tile = q_first ? 0 : kQTile;
 #pragma unroll
@@ -1920,8 +1923,9 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
     const TensorArg& out = r ? p.dk : p.dv;
     const int64_t ob = slice_offset(out, job.seq, head, job.tok0);
     char* const stage = lds + wave * (32 * D * 2);
+    const float dk_scale = kScaledQ ? p.scale / p.scale2 : p.scale;
 #pragma unroll
-    for (int j = 0; j < kBlocks; ++j) stage_acc_tile<D>(stage, 0, 32 * j, acc[j], r ? p.scale : 1.0f, lane);
+    for (int j = 0; j < kBlocks; ++j) stage_acc_tile<D>(stage, 0, 32 * j, acc[j], r ? dk_scale : 1.0f, lane);
     for (int c = lane; c < 32 * D / 8; c += 64) {
         const int row = c / (D / 8), cc = c % (D / 8);
         if (kb0 + row < job.len && (D != 96 || cc * 8 < p.cols))
@@ -1929,18 +1933,18 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
     }
 }
 
-template <int D, int kPairs>
+template <int D, int kPairs, bool kScaledQ = false>
 __global__ __launch_bounds__(128 * kPairs, D == 64 ? 3 : 2) void mfma_bwd_dkv_pair_kernel(KParams p) {
     constexpr int kQTile = 64 * kPitch<D> * 2, kZTile = 64 * 64 * 2;
     __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + kPairs * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
-    paired_keys_job<D, kPairs, kPairs == 4 ? kOnePerCu : kSharedCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {}, lds);
+    paired_keys_job<D, kPairs, kScaledQ, kPairs == 4 ? kOnePerCu : kSharedCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {}, lds);
 }
 
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void mfma_bwd_dkv_pair_drawing_kernel(KParams) {
     constexpr int kQTile = 64 * kPitch<D> * 2, kZTile = 64 * 64 * 2;
     __shared__ __attribute__((aligned(16))) char lds[4 * kQTile + 2 * kZTile];   // (Q, dO) x 2 buffers | one Z tile per pair
-    draw_jobs((int*)(lds + 4 * kQTile), [&](const KParams& p, int block, int wave, int lane, auto draw) { paired_keys_job<D, 2, kDrawn>(p, block, wave, lane, draw, lds); });
+    draw_jobs((int*)(lds + 4 * kQTile), [&](const KParams& p, int block, int wave, int lane, auto draw) { paired_keys_job<D, 2, false, kDrawn>(p, block, wave, lane, draw, lds); });
 }
 
 }  // inline namespace SBA_ELEM_NS
@@ -1950,13 +1954,25 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void mfma_bwd_dkv_pair_drawin
 bool sba_mfma_bwd_available() { return true; }
 #endif
 
-// SBA_DKV_KERNEL=own / =other overrides the choice between the key-owner kernels (tests run
-// both on the same inputs).
+// SBA_DKV_KERNEL overrides the choice between the key-owner kernels (tests run them on the same inputs).  =pair, =other, =plain and =stream8 are explained where
+// the choice is made; =own is the own-keys kernel at head_dim 128 and the paired one at 64 to 96, =pair4 has four pairs from 72 on and two at 64.
 static bool own_keys_kernel(bool by_size) {
     const char* e = getenv("SBA_DKV_KERNEL");
-    if (e && (!strcmp(e, "own") || !strcmp(e, "pair") || !strcmp(e, "pair4"))) return true;
+    if (e && (!strcmp(e, "own") || !strncmp(e, "pair", 4))) return true;
     if (e && !strcmp(e, "other")) return false;
     return by_size;
+}
+
+// Whether the paired kernel at head_dim 64 takes the dQ pass's scaled copy of q (kScaledQ): for launches that hang on their longest sweeps, which the stream had
+// before it and still has where they are small, so that neither gradient is further off for the change of kernel.  The others round K, as the kernel did that
+// they had before.  (For them the copy would be a write of q in the dQ pass and a larger error of dK: forward + backward of packs of 65536 tokens 1.007 / 1.024 / 1.009,
+// B=4 T=8192 1.006 / 1.013 / 1.004 of the time, T=4096 0.997 / 0.998 / 1.003: the heads' mean logits 0 .. -6 in order / in a random one / all at -6.)
+// SBA_DKV_KERNEL=pairq / =pair picks one.
+static bool paired_scaled_q(const sba::KParams& kp, unsigned grid) {
+    const char* e = getenv("SBA_DKV_KERNEL");
+    if (e && (!strcmp(e, "own") || !strncmp(e, "pair", 4))) return !strcmp(e, "pairq");
+    if (kp.seq_len <= 8 * sba::kRowBlock && grid >= 2u * (unsigned)sba_cu_count()) return false;
+    return sba_tail_ratio(kp, grid) > (kp.seq_len <= 32 * sba::kRowBlock ? 3.35 : kp.n_heads <= 8 && !kp.cu_seqlens ? 2.2 : 2.75);
 }
 
 // SBA_DQ_KERNEL=lean / =plain overrides the choice between the two arrangements of the one-step dQ kernel at
@@ -1996,12 +2012,13 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103).  SBA_DKV_KERNEL=pair / =other (the stream at head_dim 64) picks one.
     const unsigned cus = (unsigned)sba_cu_count();
     const bool own = own_keys_kernel(kp.head_dim == 64 ? 2 * grid.x >= 3 * cus : true);
+    const bool scaled_q = kp.head_dim == 64 && own && paired_scaled_q(kp, grid.x);
     const char* which = getenv("SBA_DKV_KERNEL");
     const bool plain = which && !strcmp(which, "plain");
     // the stream with eight half-block producers (12 waves): behind the one with four full-block producers
     // (107 against 99.5 us at B=1 H=16 T=4096), which stays the default
     const bool stream8 = which && !strcmp(which, "stream8");
-    // the scaled copy of q is for the stream kernel: no other key-owner kernel reads it, so the dQ pass skips it
+    // the scaled copy of q is for the stream and for the paired kernel in its place: nobody else reads it, so the dQ pass skips it
     const bool stream = kp.head_dim == 64 && !plain && !own;
     // Paired kernel: workgroups of two pairs, two a CU, but for launches of short sweeps that do not fill the chip with them, where the
     // prologue counts.  Forward + backward with two pairs over the same with four, d=128 / 96:  T=300 B=16 1.04 / 1.03,
@@ -2009,8 +2026,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     // T=768 B=2 0.93 / 0.945;  T=1024 B=1 0.88, B=2 0.95 / 0.95, B=8 0.98 / 1.00;  T=4096 0.97;  packs of documents of at most 512 tokens 0.95
     // (65536 tokens), 256 0.98 (16384).
     const bool four_pairs = which && !strncmp(which, "pair", 4) ? !strcmp(which, "pair4") : kp.seq_len <= 4 * kRowBlock && grid.x < 4u * cus;
-    if (stream && !kp.q_scaled.ptr) return SBA_ERR_WORKSPACE;
-    if (!stream) kp.q_scaled.ptr = nullptr;
+    if ((stream || scaled_q) && !kp.q_scaled.ptr) return SBA_ERR_WORKSPACE;
+    if (!stream && !scaled_q) kp.q_scaled.ptr = nullptr;
     // Sequences of at most 128 tokens: one kernel for both passes (it all runs in phase 1).  A kernel asked for by name is one of
     // the two-pass ones.
     if (kp.seq_len <= kRowBlock && kp.head_dim <= 128 && !which && !getenv("SBA_DQ_KERNEL") && sba_two_step_env() < 0) {
@@ -2045,6 +2062,8 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<64>), grid, dim3(kThreads), 0, s, sba_turning(kp, 2));
         if (p2 && plain) {
             hipLaunchKernelGGL((mfma_bwd_dkv_kernel<64>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
+        } else if (p2 && scaled_q) {
+            hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<64, 2, true>), dim3(2 * grid.x), dim3(256), 0, s, kp);
         } else if (p2 && own) {
             sba_launch_drawing((mfma_bwd_dkv_pair_kernel<64, 2>), (mfma_bwd_dkv_pair_drawing_kernel<64>), 2 * grid.x, kThreads, 3, kp, kp.gtab, kKeyQueue, p1, s);
         } else if (p2) {

@@ -25,8 +25,9 @@ def test_paired_kernel_at_head_dim_64(lens, current, D, dtype, monkeypatch):
         o, rem = sb_attn_varlen(qg, kg, vg, cu.cuda(), max(lens), attend_current=current)
         return torch.autograd.grad((o, rem), (qg, kg, vg), (do.cuda(), dr.cuda()))
 
-    paired = run("pair")
     ref = O.sb_attn_grads_oracle(q, k, v, do, dr, cu_seqlens=cu.tolist(), attend_current=current)[2:]
-    for g, other, r in zip(paired, run("plain"), ref):          # (the bounds of the other packed tests of these kernels)
-        assert max_abs(g.float().cpu(), r) <= 5e-2 and rel_l2(g.float().cpu(), r) <= 2e-2
-        assert rel_l2(g.float(), other.float()) <= 2e-2
+    plain = run("plain")
+    for kernel in ("pair", "pairq"):                            # (scores of scaled K and of the dQ pass's scaled q)
+        for g, other, r in zip(run(kernel), plain, ref):        # (the bounds of the other packed tests of these kernels)
+            assert max_abs(g.float().cpu(), r) <= 5e-2 and rel_l2(g.float().cpu(), r) <= 2e-2
+            assert rel_l2(g.float(), other.float()) <= 2e-2
