@@ -1998,21 +1998,32 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     if (!kp.rtab || !kp.rmid || !kp.gtab || !kp.gmid) return SBA_ERR_WORKSPACE;
     if (!kp.makes_mid && (const char*)kp.gmid - (const char*)kp.rtab != (const char*)kp.gtab - (const char*)kp.rmid) return SBA_ERR_WORKSPACE;
     // Key-owner pass.  head_dim 64: the paired kernel, but for fewer than one and a half row blocks a CU (all heads), where three workgroups a CU do not
-    // come together and the resident producer/consumer stream is ahead.  Forward + backward with the paired kernel over the same with the stream,
-    // by workgroups of the row-owner passes, mean logits 0 .. -6 over the heads in order / in a random one / all at -6:
-    //     192 (H=16 T=1500) 1.11 / 1.08 / 1.085    256 (H=16 T=2048) 1.07 / 1.07 / 1.08, (H=8 T=4096) 1.13 / 1.13 / 1.13, (H=4 T=8192) 1.15 / 1.16 / 1.15
-    //     320 (H=16 T=2500) 1.02 / 1.015 / 1.01, (H=8 T=5000) 1.05 / 1.05 / 1.05, packs of 2000 tokens 1.02 / 1.02 / 1.02, of 4096 tokens, H=8 1.04 / 1.02 / 1.03
-    //     376 (H=8 T=6000) 1.04 / 1.02 / 1.03    384 (H=12 T=4096) 1.00 / 1.00 / 1.00, (H=16 T=3000) 0.98 / 0.97 / 0.975, (B=3 H=16 T=1024) 0.96 / 0.97 / 0.95
-    //     440 (H=8 T=7000) 1.00 / 0.98 / 1.01, (H=4 T=14000) 1.04 / 1.05 / 1.01    512 (H=16 T=4096) 0.94 / 0.95 / 0.98, (B=2 H=16 T=2048) 0.92 / 0.91 / 0.96, (H=8 T=8192)
-    //     0.95 / 0.95 / 0.96, (H=4 T=16384) 1.03 / 1.03 / 1.00, (H=2 T=32768) 0.94 / 0.94 / 1.00    640 (H=16 T=5000) 0.94 / 0.92 / 1.00, packs of 4096 tokens 0.90 / 0.90 / 0.89
+    // come together, and for launches that hang on few long sweeps, whose steps are longer in it; there the resident producer/consumer stream is ahead.  Forward +
+    // backward with the paired kernel (scaled q) over the same with the stream, by workgroups of the row-owner passes and tail ratio, mean logits 0 .. -6
+    // over the heads in order / in a random one / all at -6:
+    //     fewer than 384 (K rounded)  192 (H=16 T=1500) 1.11 / 1.08 / 1.085    256 (H=16 T=2048) 1.07 / 1.07 / 1.08, (H=4 T=8192) 1.15 / 1.16 / 1.15    320 (H=16 T=2500) 1.02 /
+    //         1.015 / 1.01, (H=8 T=5000) 1.05 / 1.05 / 1.05, packs of 2000 tokens 1.02 / 1.02 / 1.02    376 (H=8 T=6000) 1.04 / 1.02 / 1.03
+    //     longest sequence up to 4096 tokens  384 (H=12 T=4096, 5.2) 0.99 / 0.99 / 0.99, (H=16 T=3072, 5.1) 0.98 / 0.975 / 1.00, (B=6 H=4 T=2048, 5.0) 0.95 / 0.96 / 0.96    408 (H=24 T=2176,
+    //         4.7) 0.97 / 0.97 / 0.97    512 (H=16 T=4096, 3.9) 0.955 / 0.95 / 0.96, (B=4 H=4 T=4096) 0.93 / 0.94 / 0.97, (B=16 H=2 T=2048, 3.8) 0.96 / 0.96 / 0.97, (H=32 T=2048) 0.94 / 0.95 /
+    //         0.95;  packs  4096 + 2048 H=8 (384, 6.2) 1.02 / 1.02 / 1.03, 4096 to 400 H=4 (500, 5.7) 1.02 / 1.01 / 1.02, 4096 to 1000 H=8 (544, 5.3) 0.98 / 0.97 / 0.98, 2048 to 400
+    //         H=16 (512, 5.3) 0.94 / 0.96 / 0.965;  one document among short ones  4096 and 100s H=4 (528, 13) 1.04 / 1.05 / 1.05, 4096 and 300s H=2 (664, 14.5) 1.03, H=4 (848, 9.2) 0.98,
+    //         4096 and 200s H=8 (896, 6.3) 1.01, 3500 and 300s H=8 (944, 6.1) 0.98, 3000 and 128s H=8 (512, 9.0) 1.05, 2500 and 128s H=8 (480, 10.2) 1.07, 2048 and 100s (424, 18) 1.04, (448,
+    //         11.6) 1.045, 2048 and 300s H=4 (784, 8.3) 0.88, 2048 and 256s H=8 (928, 7.2) 0.91, 2048 and 128s H=16 (896, 5.8) 0.93, 4096 and 128s H=16 (1472, 3.5) 0.89 / 0.89 / 0.90
+    //     longer  384 (H=4 T=12288, 5.3) 1.06 / 1.06 / 1.04, (H=8 T=6144) 1.03 / 1.01 / 1.03, (H=6 T=8192) 1.015 / 1.00 / 1.03, (B=2 H=2 T=12288) 1.00 / 1.00 / 1.02    440 (H=4 T=14000, 4.6) 1.045 / 1.045 /
+    //         1.03    480 (H=12 T=5120, 4.2) 0.97 / 0.975 / 0.98    512 (3.9 to 4.0) (H=4 T=16384) 1.03 / 1.03 / 1.00, (H=2 T=32768) 0.94 / 0.94 / 1.01, heads at 0 and -6 1.07 / 1.08 / 0.99,
+    //         (H=8 T=8192) 0.96 / 0.96 / 0.98, (B=2 H=2 T=16384) 0.94 / 0.94 / 1.01, (B=2 H=4 T=8192) 0.94 / 0.945 / 0.99    628 (H=4 T=20000, 3.2) 0.97 / 0.97 / 1.02    640 (H=16 T=5000, 3.1)
+    //         0.935 / 0.91 / 1.00    784 (H=4 T=25000, 2.6) 0.95 / 0.95 / 1.00, (B=2 H=2 T=25000) 0.83 / 0.83 / 0.98;  packs  8192 + 4096 + 2048 H=4 (448, 6.0) 1.04 / 1.05 / 1.05, 16384 + 8192
+    //         H=2 (384, 6.3) 1.11 / 1.11 / 1.07, 11000 and short ones H=4 (436, 5.8) 1.04 / 1.05 / 1.05, 6000 and 300s H=4 (908, 8.1) 1.04, 8192 and 512s H=8 (1152, 3.6) 0.89 / 0.925 / 0.95
     // and over the kernel whose waves own 32 keys each (two waves per SIMD at 215 registers), which was there before for launches that do not hang on their longest
     // sweeps: 1024 (H=32 T=4096) 0.95 / 0.94 / 0.935, (H=16 T=8192) 0.96 / 0.94 / 0.93, (B=8 T=2048) 0.935 / 0.94 / 0.98, (B=4 T=1024) 0.97 / 0.95 / 0.97,
     // packs of 8192 tokens 0.95 / 0.93 / 0.93, 16384 0.93 / 0.95 / 0.93, 65536 0.98 / 0.97 / 0.98, documents up to 1024 0.96 / 0.96 / 0.95, up to 256 0.98 / 0.975 / 0.97.
     // head_dim 72 to 128: the paired kernel at every size (B=1, H=16, T=512 ... 2048: with four pairs 27 / 44 / 62 / 81 us where the
-    // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103).  SBA_DKV_KERNEL=pair / =other (the stream at head_dim 64) picks one.
+    // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103).  SBA_DKV_KERNEL=pair / =pairq (see paired_scaled_q()) / =other (the stream at
+    // head_dim 64) picks one.
     const unsigned cus = (unsigned)sba_cu_count();
-    const bool own = own_keys_kernel(kp.head_dim == 64 ? 2 * grid.x >= 3 * cus : true);
-    const bool scaled_q = kp.head_dim == 64 && own && paired_scaled_q(kp, grid.x);
+    const bool scaled_q = kp.head_dim == 64 && paired_scaled_q(kp, grid.x);
+    const double paired_up_to = kp.seq_len > 32 * kRowBlock ? (kp.n_heads <= 4 && kp.n_seq == 1 ? 3.5 : 4.5) : grid.x >= 3 * cus ? 9.5 : 5.5;
+    const bool own = own_keys_kernel(kp.head_dim == 64 ? 2 * grid.x >= 3 * cus && (!scaled_q || sba_tail_ratio(kp, grid.x) <= paired_up_to) : true);
     const char* which = getenv("SBA_DKV_KERNEL");
     const bool plain = which && !strcmp(which, "plain");
     // the stream with eight half-block producers (12 waves): behind the one with four full-block producers
@@ -2026,8 +2037,9 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     // T=768 B=2 0.93 / 0.945;  T=1024 B=1 0.88, B=2 0.95 / 0.95, B=8 0.98 / 1.00;  T=4096 0.97;  packs of documents of at most 512 tokens 0.95
     // (65536 tokens), 256 0.98 (16384).
     const bool four_pairs = which && !strncmp(which, "pair", 4) ? !strcmp(which, "pair4") : kp.seq_len <= 4 * kRowBlock && grid.x < 4u * cus;
-    if ((stream || scaled_q) && !kp.q_scaled.ptr) return SBA_ERR_WORKSPACE;
-    if (!stream && !scaled_q) kp.q_scaled.ptr = nullptr;
+    const bool needs_scaled_q = stream || (own && scaled_q);
+    if (needs_scaled_q && !kp.q_scaled.ptr) return SBA_ERR_WORKSPACE;
+    if (!needs_scaled_q) kp.q_scaled.ptr = nullptr;
     // Sequences of at most 128 tokens: one kernel for both passes (it all runs in phase 1).  A kernel asked for by name is one of
     // the two-pass ones.
     if (kp.seq_len <= kRowBlock && kp.head_dim <= 128 && !which && !getenv("SBA_DQ_KERNEL") && sba_two_step_env() < 0) {
@@ -2062,7 +2074,7 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<64>), grid, dim3(kThreads), 0, s, sba_turning(kp, 2));
         if (p2 && plain) {
             hipLaunchKernelGGL((mfma_bwd_dkv_kernel<64>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
-        } else if (p2 && scaled_q) {
+        } else if (p2 && own && scaled_q) {
             hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<64, 2, true>), dim3(2 * grid.x), dim3(256), 0, s, kp);
         } else if (p2 && own) {
             sba_launch_drawing((mfma_bwd_dkv_pair_kernel<64, 2>), (mfma_bwd_dkv_pair_drawing_kernel<64>), 2 * grid.x, kThreads, 3, kp, kp.gtab, kKeyQueue, p1, s);
