@@ -58,8 +58,12 @@ __device__ inline void store_o_rows(char* stage, const KParams& p, const Job& jo
 
 // kCarryOnly: write the carry table and nothing else (no P*V, no o / rem): the backward's way of
 // getting the table when the forward kept none.
-template <int D, bool kCarryOnly, Sharing kSharing, class Draw>
-__device__ __forceinline__ void fwd_job(const KParams& p, const int block, const int wave, const int lane, Draw draw) {
+// Params, wave_, lane_: launches that draw their jobs hand them in anew for each job (see draw_jobs()).  The others take the parameters by value and their own thread
+// index: then the compiler makes of it what it makes of a kernel's body (head_dim 256 by reference and from outside: 721 -> 725 us at H=16 T=10008, 46.8 -> 47.4 at B=4 H=8 T=1024).
+template <int D, bool kCarryOnly, Sharing kSharing, class Params, class Draw>
+__device__ __forceinline__ void fwd_job(Params p, const int block, const int wave_, const int lane_, Draw draw) {
+    const int lane = kSharing == kDrawn ? lane_ : (int)(threadIdx.x & 63);
+    const int wave = kSharing == kDrawn ? wave_ : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int kTile = 64 * kPitch<D> * 2;            // bytes per K or V tile
     __shared__ __attribute__((aligned(16))) char lds[4 * kTile + (kCarryOnly ? 0 : 32)];   // K0 V0 K1 V1 | words
     int (*const done_waves)[4] = (int (*)[4])(lds + (kCarryOnly ? kTile : 4 * kTile));     // [parity of the step][wave]
@@ -88,7 +92,8 @@ __device__ __forceinline__ void fwd_job(const KParams& p, const int block, const
     float R = qi < job.len ? 1.0f : 0.0f;
     // This wave has no more weights to give: its rows' carries are exactly 0, or it has no rows at all.
     bool done = q0w >= job.len;
-    if (wave == 0 && lane < 8) done_waves[lane >> 2][lane & 3] = 0;
+    const int thread = kSharing == kDrawn ? 64 * wave + lane : (int)threadIdx.x;
+    if (thread < 8) done_waves[thread >> 2][thread & 3] = 0;
 
     const int imax = min(m0 + kRowBlock - 1, job.len - 1);
     const int kmax = imax - strict;                       // last key any row of the block sees
@@ -191,7 +196,7 @@ __device__ __forceinline__ void fwd_job(const KParams& p, const int block, const
     }
     draw();
     store_carries();
-    if (p.save && wave == 0 && lane == 0) set_first_live(p, head, job, n_steps - iterations);
+    if (p.save && thread == 0) set_first_live(p, head, job, n_steps - iterations);
 
     if (!kCarryOnly) {
         store_o_rows<D>(lds + wave * kRowStage<D>, p, job, head, q0w, lane, oacc);       // (the tiles are free)
@@ -202,13 +207,13 @@ __device__ __forceinline__ void fwd_job(const KParams& p, const int block, const
 
 template <int D, bool kCarryOnly>
 __global__ __launch_bounds__(kThreads) void mfma_fwd_kernel(KParams p) {
-    fwd_job<D, kCarryOnly, kSharedCu>(p, blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63, [] {});
+    fwd_job<D, kCarryOnly, kSharedCu, KParams>(p, blockIdx.x, 0, 0, [] {});
 }
 
 template <int D, bool kCarryOnly>
 __global__ __launch_bounds__(kThreads, 2) void mfma_fwd_drawing_kernel(KParams) {
     __shared__ int words[2];
-    draw_jobs(words, [&](const KParams& p, int block, int wave, int lane, auto draw) { fwd_job<D, kCarryOnly, kDrawn>(p, block, wave, lane, draw); });
+    draw_jobs(words, [&](const KParams& p, int block, int wave, int lane, auto draw) { fwd_job<D, kCarryOnly, kDrawn, const KParams&>(p, block, wave, lane, draw); });
 }
 
 // ---------------------------------------------------------------- small grids: G segments per sweep
