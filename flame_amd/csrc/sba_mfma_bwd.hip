@@ -1956,8 +1956,7 @@ bool sba_mfma_bwd_available() { return true; }
 
 // SBA_DKV_KERNEL overrides the choice between the key-owner kernels (tests run them on the same inputs).  =pair, =other, =plain and =stream8 are explained where
 // the choice is made; =own is the own-keys kernel at head_dim 128 and the paired one at 64 to 96, =pair4 has four pairs from 72 on and two at 64.
-static bool own_keys_kernel(bool by_size) {
-    const char* e = getenv("SBA_DKV_KERNEL");
+static bool own_keys_kernel(const char* e, bool by_size) {
     if (e && (!strcmp(e, "own") || !strncmp(e, "pair", 4))) return true;
     if (e && !strcmp(e, "other")) return false;
     return by_size;
@@ -1968,8 +1967,7 @@ static bool own_keys_kernel(bool by_size) {
 // they had before.  (For them the copy would be a write of q in the dQ pass and a larger error of dK: forward + backward of packs of 65536 tokens 1.007 / 1.024 / 1.009,
 // B=4 T=8192 1.006 / 1.013 / 1.004 of the time, T=4096 0.997 / 0.998 / 1.003: the heads' mean logits 0 .. -6 in order / in a random one / all at -6.)
 // SBA_DKV_KERNEL=pairq / =pair picks one.
-static bool paired_scaled_q(const sba::KParams& kp, unsigned grid) {
-    const char* e = getenv("SBA_DKV_KERNEL");
+static bool paired_scaled_q(const char* e, const sba::KParams& kp, unsigned grid) {
     if (e && (!strcmp(e, "own") || !strncmp(e, "pair", 4))) return !strcmp(e, "pairq");
     if (kp.seq_len <= 8 * sba::kRowBlock && grid >= 2u * (unsigned)sba_cu_count()) return false;
     return sba_tail_ratio(kp, grid) > (kp.seq_len <= 32 * sba::kRowBlock ? 3.35 : kp.n_heads <= 8 && !kp.cu_seqlens ? 2.2 : 2.75);
@@ -2020,11 +2018,11 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
     // head_dim 72 to 128: the paired kernel at every size (B=1, H=16, T=512 ... 2048: with four pairs 27 / 44 / 62 / 81 us where the
     // kernel with one workgroup per 64-key block takes 33 / 55 / 73 / 103).  SBA_DKV_KERNEL=pair / =pairq (see paired_scaled_q()) / =other (the stream at
     // head_dim 64) picks one.
-    const unsigned cus = (unsigned)sba_cu_count();
-    const bool scaled_q = kp.head_dim == 64 && paired_scaled_q(kp, grid.x);
-    const double paired_up_to = kp.seq_len > 32 * kRowBlock ? (kp.n_heads <= 4 && kp.n_seq == 1 ? 3.5 : 4.5) : grid.x >= 3 * cus ? 9.5 : 5.5;
-    const bool own = own_keys_kernel(kp.head_dim == 64 ? 2 * grid.x >= 3 * cus && (!scaled_q || sba_tail_ratio(kp, grid.x) <= paired_up_to) : true);
     const char* which = getenv("SBA_DKV_KERNEL");
+    const unsigned cus = (unsigned)sba_cu_count();
+    const bool scaled_q = kp.head_dim == 64 && paired_scaled_q(which, kp, grid.x);
+    const double paired_up_to = kp.seq_len > 32 * kRowBlock ? (kp.n_heads <= 4 && kp.n_seq == 1 ? 3.5 : 4.5) : grid.x >= 3 * cus ? 9.5 : 5.5;
+    const bool own = own_keys_kernel(which, kp.head_dim == 64 ? 2 * grid.x >= 3 * cus && (!scaled_q || sba_tail_ratio(kp, grid.x) <= paired_up_to) : true);
     const bool plain = which && !strcmp(which, "plain");
     // the stream with eight half-block producers (12 waves): behind the one with four full-block producers
     // (107 against 99.5 us at B=1 H=16 T=4096), which stays the default
