@@ -36,7 +36,8 @@ CASES = [  # B, H, T or lengths, D, dtype, options
     (1, 4, 2048, 64, torch.bfloat16, {}),
     (1, 4, 2048, 64, torch.bfloat16, {"SBA_RECOMPUTE_CARRIES": "1"}),
     (1, 4, 2048, 64, torch.bfloat16, {"SBA_FWD_GROUPS": "2"}),
-    (1, 4, 2047, 64, torch.bfloat16, {"SBA_DKV_KERNEL": "own"}),
+    (1, 4, 2047, 64, torch.bfloat16, {"SBA_DKV_KERNEL": "pair"}),
+    (1, 4, 2047, 64, torch.bfloat16, {"SBA_DKV_KERNEL": "pairq"}),
     (1, 4, 2047, 64, torch.float16, {"SBA_DKV_KERNEL": "plain"}),
     (1, 4, 2047, 64, torch.bfloat16, {"SBA_DKV_KERNEL": "stream8"}),
     (3, 16, 1537, 64, torch.bfloat16, {}),

@@ -508,7 +508,7 @@ def test_config4_size_invariants():
     _full_size_properties(fwd_bwd, ups)
 
 
-@pytest.mark.parametrize("dkv_kernel,D", [("", 64), ("own", 64), ("other", 64), ("stream8", 64), ("plain", 64),
+@pytest.mark.parametrize("dkv_kernel,D", [("", 64), ("pair", 64), ("pairq", 64), ("other", 64), ("stream8", 64), ("plain", 64),
                                           ("own", 128), ("other", 128), ("pair", 128)])
 def test_randomized_packed_batches_mfma_vs_generic_backward(dkv_kernel, D, monkeypatch):
     # Seeded random packed batches (document counts, lengths around the 64/128 block edges,

@@ -44,5 +44,5 @@ def test_short_dense_batches_agree_with_the_two_passes(T, D, dtype, monkeypatch)
 
     one = run()
     assert torch.equal(one, run())
-    monkeypatch.setenv("SBA_DKV_KERNEL", "own")
+    monkeypatch.setenv("SBA_DKV_KERNEL", "own" if D == 128 else "pair")
     assert rel_l2(one.float(), run().float()) <= (4e-3 if dtype == torch.bfloat16 else 5e-4)
