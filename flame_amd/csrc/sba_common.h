@@ -280,8 +280,8 @@ __device__ inline int drawn_block(const KParams& p, int home, int ticket, int la
     return block;
 }
 // Runs run(parameters, block, wave, lane, draw) for the workgroup's jobs.  Parameters and lane are given as if they were others each time, so
-// that nothing computed from them stays in registers from job to job (without this the forward at head_dim 64 takes 165 registers in place of
-// 124).  A job calls draw() behind its last step: the ticket is on its way while the results are stored.  (Asked for before the job, it
+// that nothing computed from them stays in registers from job to job (without this the forward at head_dim 128 takes 253 registers in place of 214, the dQ pass
+// there spills 48 and the key owners 17).  A job calls draw() behind its last step: the ticket is on its way while the results are stored.  (Asked for before the job, it
 // would be bound to the end of a long sweep while others find no work: 8192-token packs 1.15 of the time.)
 // words: two ints of LDS that a job does not use behind its last barrier.
 template <class Run>
@@ -386,8 +386,8 @@ inline double sba_tail_ratio(const sba::KParams& kp, unsigned grid) {
 // The same launch with KParams::turn set, for a kernel of which a CU holds `resident` workgroups and that takes `per_job` of them for
 // each (job, head).  Only for dense batches in whole rounds of the CUs, several row blocks to a round.  Time against the plain order:
 // 16-bit forward at head_dim 64 0.99 ... 0.91 on 512 and 768 workgroups of 9 shapes (1.08 where a round is one row block of every
-// sequence: the turn only parts the row blocks of a sequence that meet on a CU), both passes of its backward 0.95 ... 1.00 together on
-// 512 workgroups of 10 shapes, float32 0.91 ... 1.00 on 512 workgroups of 9.  On 384 ... 640 workgroups that are no whole rounds
+// sequence: the turn only parts the row blocks of a sequence that meet on a CU), the dQ pass of its backward 0.995 ... 1.005 (forward + backward, nine
+// shapes of 512; the key owners, whose launch gained from it, have a kernel that is not turned), float32 0.91 ... 1.00 on 512 workgroups of 9.  On 384 ... 640 workgroups that are no whole rounds
 // 1.00 ... 1.03, and at head_dim 96 and 128 in 16 bits 0.98 ... 1.02: left as they come.
 inline sba::KParams sba_turning(const sba::KParams& kp, int resident, int per_job = 1) {
     sba::KParams r = kp;

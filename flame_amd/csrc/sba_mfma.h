@@ -398,7 +398,7 @@ template <int D, bool kNatural = false, bool kLateRagged = false> struct TileDma
     }
     // For loops that are short of scalar registers (the dQ pass), whose sums known in front of the loop are spilled into vector lanes and come back
     // one by one: the origin moves along with the tiles, and the wave's part of the tile is an unknown at each tile, so that
-    // the copies' LDS addresses - 8 at head_dim 64, 16 above - are formed where they are used.  dQ at d=128, float16, B=4 H=16 T=2047: 15 lane reads a
+    // the copies' LDS addresses - 8 at head_dim 64, 16 at 96 and 128, 32 at 256 - are formed where they are used.  dQ at d=128, float16, B=4 H=16 T=2047: 15 lane reads a
     // step, 118.7 us, and 6, 116; d=80, 20011 tokens packed: 16, 147, and none, 144; d=64, 65536 tokens packed 551 and 538.  (The forward and the
     // key owners have the registers: T=16384, d=128 1.005 and 1.008 of the time with it.)
     __device__ inline void seek(int row0) { origin += ((uint64_t)(uint32_t)row0 * (uint32_t)st) << 1; }

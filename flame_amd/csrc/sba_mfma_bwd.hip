@@ -1786,7 +1786,7 @@ __device__ __forceinline__ void paired_keys_job(const KParams& p, const int bloc
     __syncthreads();
 
     // Every LDS address of the loop is "a register that is fixed for the whole sweep + a constant": the sums of
-    // LDS base, lane offset and this wave's share (query tile r, column blocks 2r.., the pair's weight tile) are
+    // LDS base, lane offset and this wave's share (query tile r, the Q or the dO tiles, the pair's weight tile) are
     // made once, and the loop runs in two copies, one per tile buffer, so that buffer and row offsets are compile-time
     // numbers that go into the offset fields of the fetches.  (With the tile address in a scalar register each
     // fetch costs one or two vector adds with a scalar operand, 1.8 ns each: 40 of them per step.)
@@ -2072,7 +2072,7 @@ int sba_launch_mfma_bwd(const sba::KParams& kp_in, int phases, hipStream_t s) {
         else if (p1) hipLaunchKernelGGL((mfma_bwd_dq_kernel<64>), grid, dim3(kThreads), 0, s, sba_turning(kp, 2));
         if (p2 && plain) {
             hipLaunchKernelGGL((mfma_bwd_dkv_kernel<64>), dim3(2 * grid.x), dim3(kThreads), 0, s, kp);
-        } else if (p2 && own && scaled_q) {
+        } else if (p2 && own && scaled_q) {        // (has no drawing form: a launch that hangs on its longest sweeps has not the work that pays)
             hipLaunchKernelGGL((mfma_bwd_dkv_pair_kernel<64, 2, true>), dim3(2 * grid.x), dim3(256), 0, s, kp);
         } else if (p2 && own) {
             sba_launch_drawing((mfma_bwd_dkv_pair_kernel<64, 2>), (mfma_bwd_dkv_pair_drawing_kernel<64>), 2 * grid.x, kThreads, 3, kp, kp.gtab, kKeyQueue, p1, s);
